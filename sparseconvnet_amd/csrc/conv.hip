@@ -5,12 +5,15 @@
 // (CPU/Convolution.cpp:45-79,117-150, CPU/Deconvolution.cpp:7-41); they differ only in
 // the table they pass.
 //
-// Three MFMA kernels (groups == 1, fp32 v_mfma_f32_16x16x4_f32, accumulators in registers
-// for the whole filter, taps skipped per 16-row granule), chosen by the output width:
+// MFMA kernels (groups == 1, accumulators in registers for the whole filter, taps skipped per
+// 16-row granule).  From 20 input planes on fp32 layers run in
+//   k_conv_split     fp32 operands as three bf16 pieces each, rows through LDS
+// and the others (fewer planes, plane counts that are no multiple of four, arrays not 16-byte aligned or
+// of 2 GiB and more, the allocation-free entry point, bf16 operands) are chosen by the output width:
 //   k_conv_resident  nOut <= 32   all taps' weights resident in LDS, wavefronts run alone
 //   k_conv_rows      nOut <= 128  wavefronts own rows, the weight slab goes through LDS
 //   k_conv_mfma      wider        wavefronts own columns, rows and weights go through LDS
-// and k_conv_generic for everything else (groups > 1).  Positions arrive in Z-order and
+// (v_mfma_f32_16x16x4_f32, or 16x16x32_bf16), and k_conv_generic for everything else (groups > 1).  Positions arrive in Z-order and
 // pattern-sorted, so a granule's rows mostly share one neighbour pattern and the skipped
 // (granule, tap) pairs carry almost all of the sparsity.  Template flag BUF: the gathers are
 // buffer loads, for which an absent row is an offset past the end that reads as zeros;
@@ -269,6 +272,7 @@ template <bool PRE>
 static bool conv_mfma_paths(Metadata &m, const Table &t, const float *in, float *out, const float *w,
                             Epi epi, int n_in, int n_out, PreArgs pre, hipStream_t s) {
   if (!PRE && try_few(m, t, in, out, w, epi, n_in, n_out, s)) return true;
+  if (conv_split_dispatch(PRE, m, t, in, out, w, epi, n_in, n_out, pre, s)) return true;
   if (!PRE && try_resident(m, t, in, out, w, epi, n_in, n_out, s)) return true;
   const bool vec4 = n_in % 4 == 0 && ((uintptr_t)in % 16 == 0);
   if (n_out <= 128 && t.K <= 1024 && conv_rows_dispatch(vec4, PRE, m, t, in, out, w, epi, n_in, n_out, pre, s)) return true;

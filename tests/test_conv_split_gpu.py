@@ -1,0 +1,95 @@
+"""The convolution kernel that takes fp32 operands as three bf16 pieces each: every tile shape, at sizes
+around the ends of tiles and of the ranges a tile shape serves, against sums in 64 bits over the exported
+rules; and rows and weights that are no finite numbers.
+
+Tolerance: the pieces hold every operand exactly, the products left out are below 2^-24 of a product and of
+either sign, and the sums of 32 channels are added in fp32, so that a result of m additions is off by at most
+about (m + 4) 2^-24 of the sum of the products' magnitudes; 2-norm over the output: a tenth of that and less."""
+import numpy as np
+import pytest
+
+from sparseconvnet_amd import synthetic
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(n, seed):
+    from hip_path import HipPath
+    spatial = 126 if n < 30000 else 1022
+    coords = synthetic.room_scene(seed=seed, target=max(n, 2000), spatial=spatial)[:n]
+    p = HipPath(3)
+    assert p.input_layer(spatial, coords, 0, 0) == len(coords) == n
+    return p, spatial
+
+
+def _reference(rules, x, w):
+    """sum over rules (tap, in, out), and the same of the magnitudes; on the GPU, in 64 bits."""
+    import torch
+    x, w = torch.as_tensor(x).cuda().double(), torch.as_tensor(w).cuda().double()
+    y = torch.zeros((len(x), w.shape[-1]), dtype=torch.float64, device="cuda")
+    a = torch.zeros_like(y)
+    for k in range(w.shape[0]):
+        r = torch.as_tensor(rules[k]).cuda().long()
+        if len(r):
+            y.index_add_(0, r[:, 1], x[r[:, 0]] @ w[k, 0])
+            a.index_add_(0, r[:, 1], x[r[:, 0]].abs() @ w[k, 0].abs())
+    return y.cpu().numpy(), a.cpu().numpy()
+
+
+# widths at and beside every number of 16-column blocks; sites around 16, 32, 64 and 128 rows, 1024, and 300 k
+@pytest.mark.parametrize("n,cin,cout", [
+    (1, 20, 5), (15, 32, 32), (17, 36, 33), (33, 64, 64), (65, 100, 96), (127, 32, 128), (129, 48, 130), (1023, 64, 192),
+    (1023, 40, 209), (1023, 224, 224), (1023, 32, 256), (1024, 64, 48), (1024, 52, 80), (1025, 96, 112), (1500, 160, 160),
+    (1500, 20, 177), (2000, 44, 200), (2100, 256, 256), (5000, 64, 24), (20011, 32, 64), (33333, 64, 32), (33333, 24, 96),
+    (299999, 32, 40), (300001, 32, 17), (300001, 36, 64), (300001, 32, 90), (300001, 64, 128)])
+def test_split_operands_against_64_bits(n, cin, cout):
+    p, spatial = _scene(n, 9000 + n % 97)
+    rng = np.random.default_rng(cin * 1000 + cout)
+    x = rng.normal(size=(n, cin)).astype(np.float32)
+    x *= np.exp(rng.normal(size=(n, 1))).astype(np.float32)  # rows of different size
+    w = (rng.normal(size=(27, 1, cin, cout)) * (2.0 / (cin * 27)) ** 0.5).astype(np.float32)
+    got, _ = p.subm_conv(spatial, 3, x, w)
+    want, mag = _reference(p.submanifold_rules(spatial, 3), x, w)
+    err = np.abs(got - want)
+    additions = 27 * -(-cin // 32)
+    assert (err <= (additions + 4) * 2.0 ** -24 * mag).all(), err.max()
+    assert np.linalg.norm(err) <= 0.1 * (additions + 4) * 2.0 ** -24 * np.linalg.norm(mag)
+
+
+@pytest.mark.parametrize("n,cin,cout", [(700, 32, 64), (3000, 24, 32), (3000, 64, 160)])
+def test_values_that_are_not_finite_spread_as_the_sum_says(n, cin, cout):
+    """An infinity reaches exactly the outputs whose rules read it, with the sign the sum gives; so does a NaN; sums
+    past the largest float are infinite; everything else stays as it was.  Weights likewise."""
+    p, spatial = _scene(n, 9500 + n)
+    rng = np.random.default_rng(n + cout)
+    rules = p.submanifold_rules(spatial, 3)
+
+    def check(x, w):
+        got, _ = p.subm_conv(spatial, 3, x, w)
+        with np.errstate(all="ignore"):
+            want = np.zeros((n, cout), np.float64)
+            for k in range(27):
+                i, o = rules[k][:, 0], rules[k][:, 1]  # (an output occurs once per tap)
+                for c in range(cin):
+                    want[o] += x[i, c:c + 1].astype(np.float64) * w[k, 0, c][None, :].astype(np.float64)
+        assert (np.isnan(got) == np.isnan(want)).all()
+        big = np.abs(want) > 3.5e38
+        assert big.any() or np.isnan(want).any()
+        assert (got[big] == np.sign(want[big]) * np.inf).all()
+        rest = np.abs(want) < 3e38
+        np.testing.assert_allclose(got[rest], want[rest], rtol=1e-4, atol=1e-5 * min(np.abs(x[np.isfinite(x)]).max(), 1e36))
+
+    x = rng.normal(size=(n, cin)).astype(np.float32)
+    w = (rng.normal(size=(27, 1, cin, cout)) * 0.05).astype(np.float32)
+    w[:, 0, 3, :7] = 1.0  # a weight whose lower pieces are zero
+    a = x.copy()
+    a[5, 3], a[n // 2, 7], a[n - 1, 3] = np.inf, np.nan, -np.inf
+    check(a, w)
+    b = x.copy()
+    b[:, 0] = np.where(np.arange(n) % 5 == 0, 3.4e38, 0.0)  # near the largest float: rounding it to bf16 would overflow
+    v = w * np.float32(1e-3)
+    v[13, 0, 0, :] = 2.0
+    check(b, v)
+    v = w.copy()
+    v[13, 0, 2, 4], v[13, 0, 1, 6] = np.inf, np.nan
+    check(x, v)
