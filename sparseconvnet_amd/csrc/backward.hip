@@ -214,6 +214,10 @@ static void column_sums(Metadata &m, const float *x, int64_t rows, int planes, f
   LAUNCH_CHECK();
 }
 
+// conv_dw_split.hip
+int64_t conv_dw_split(Metadata &m, const Table &t, const float *a, int64_t a_rows, int n_a, const float *b, int64_t b_rows,
+                      int n_b, hipStream_t s);
+
 // ---- weight gradient ---------------------------------------------------------------------------
 // dW[k][c][o] = sum over positions t with nbr[k][t] >= 0 of a[nbr[k][t]][c] * b[row(t)][o].
 // One workgroup (4 wavefronts): tap k, positions [chunk * chunk_len, ...), channel tile 64 x 64.
@@ -854,6 +858,11 @@ static void weight_gradient(Metadata &m, const Table &t, const float *a, int64_t
       LAUNCH_CHECK();
       return;
     }
+  }
+  if (const int64_t shares = conv_dw_split(m, t, a, a_rows, n_a, b, b_rows, n_b, s)) {
+    k_sum_blocks<float, float><<<dim3((unsigned)ceil_div(per_chunk, 64)), sum_threads(shares), 0, s>>>(m.partial.p, (int)shares, per_chunk, per_chunk, dw);
+    LAUNCH_CHECK();
+    return;
   }
   // up to 32 channels on both sides; from there on the per-wavefront kernel below is faster
   // (64 -> 64 at 1 M sites: 1.97 against 1.3 ms)

@@ -4,45 +4,6 @@
 
 namespace scn {
 
-// ---- fp32 operands as three bf16 pieces -------------------------------------------------
-// x = h + m + l exactly, eight significant bits each: h is x cut off after eight bits (never rounded
-// up, so it cannot overflow), m the remainder rounded to bf16, l what is left of it (signed).  Of the nine
-// products of two such numbers the three below 2^-24 of the product are left out; the other six are one
-// v_mfma_f32_16x16x32_bf16 each, 96 cycles of the matrix unit for 32 channels where eight
-// v_mfma_f32_16x16x4_f32 take 256.  (The matrix unit sustains 1700 TFLOP/s on the former and 140
-// on the latter, operands in registers: twice the rate after the six-fold work.)
-// The six products of 32 channels are summed from zero and then added to the accumulator in fp32: a
-// chain of them straight into the accumulator rounds with the accumulator's exponent every time, and
-// not to nearest.  Against sums in 64 bits, 16 x 16 tiles, 1728 channels (relative 2-norm): fp32
-// matrix instructions 7.5e-7 (signed values) / 5.3e-7 (ReLU outputs) / 4.2e-7 (all positive), six
-// products into the accumulator 6.4e-7 / 6.2e-7 / 7.7e-7, summed apart 1.5e-7 / 1.5e-7 / 1.1e-7.
-__device__ inline void split_pair(float x0, float x1, unsigned &h, unsigned &m, unsigned &l) {
-  typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-  typedef float v2f __attribute__((ext_vector_type(2)));
-  const unsigned u0 = __builtin_bit_cast(unsigned, x0), u1 = __builtin_bit_cast(unsigned, x1);
-  h = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
-  const float r0 = x0 - __builtin_bit_cast(float, u0 & 0xFFFF0000u), r1 = x1 - __builtin_bit_cast(float, u1 & 0xFFFF0000u);
-  m = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f){r0, r1}, v2bf));
-  const float l0 = r0 - __builtin_bit_cast(float, m << 16), l1 = r1 - __builtin_bit_cast(float, m & 0xFFFF0000u);
-  l = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f){l0, l1}, v2bf));
-}
-struct Split8 {  // eight channels of a lane: the operands of the three pieces
-  v8s h, m, l;
-};
-__device__ inline Split8 split8(v4f a, v4f b) {
-  typedef unsigned v4u __attribute__((ext_vector_type(4)));
-  unsigned h[4], m[4], l[4];
-  split_pair(a.x, a.y, h[0], m[0], l[0]);
-  split_pair(a.z, a.w, h[1], m[1], l[1]);
-  split_pair(b.x, b.y, h[2], m[2], l[2]);
-  split_pair(b.z, b.w, h[3], m[3], l[3]);
-  Split8 s;
-  s.h = __builtin_bit_cast(v8s, (v4u){h[0], h[1], h[2], h[3]});
-  s.m = __builtin_bit_cast(v8s, (v4u){m[0], m[1], m[2], m[3]});
-  s.l = __builtin_bit_cast(v8s, (v4u){l[0], l[1], l[2], l[3]});
-  return s;
-}
-
 // wp[k][slab of 32 channels][piece][column block][lane]: 16 bytes, the lane's eight channels
 // (slab*32 + 16*(e/4) + 4*(lane/16) + e%4, e < 8) of column 16*cb + lane%16; zeros outside
 // [nIn) x [nOut).  A weight that is no finite number is all in its first piece.

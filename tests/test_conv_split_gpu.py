@@ -93,3 +93,56 @@ def test_values_that_are_not_finite_spread_as_the_sum_says(n, cin, cout):
     v = w.copy()
     v[13, 0, 2, 4], v[13, 0, 1, 6] = np.inf, np.nan
     check(x, v)
+
+
+def _weight_gradient(rules, x, d, cin, cout):
+    import torch
+    x, d = torch.as_tensor(x).cuda().double(), torch.as_tensor(d).cuda().double()
+    w, a = np.zeros((27, 1, cin, cout)), np.zeros((27, 1, cin, cout))
+    for k in range(27):
+        r = torch.as_tensor(rules[k]).cuda().long()
+        if len(r):
+            i, o = x[r[:, 0]], d[r[:, 1]]
+            w[k, 0], a[k, 0] = (i.t() @ o).cpu().numpy(), (i.abs().t() @ o.abs()).cpu().numpy()
+    return w, a
+
+
+# a tile of 64, 96 or 128 channels per side, one to three of them; sites around a granule, a block of eight and
+# the ranges of the shares
+@pytest.mark.parametrize("n,cin,cout", [
+    (1, 68, 36), (17, 36, 100), (129, 96, 128), (1000, 128, 96), (1025, 160, 64), (2100, 196, 132), (5000, 64, 260),
+    (29999, 72, 72), (30001, 64, 64), (30001, 36, 60), (30001, 132, 40), (60011, 64, 96), (300001, 64, 64), (300001, 100, 36)])
+def test_weight_gradient_from_split_operands_against_64_bits(n, cin, cout):
+    """Sums of m rules, 32 positions at a time from zero, then shares: within (m / 32 + 200) additions in fp32 of
+    the sum of magnitudes, and in the 2-norm a tenth of that."""
+    p, spatial = _scene(n, 9700 + n % 89)
+    rng = np.random.default_rng(cin * 1000 + cout)
+    x = rng.normal(size=(n, cin)).astype(np.float32)
+    d = (rng.normal(size=(n, cout)) * np.exp(rng.normal(size=(n, 1)))).astype(np.float32)
+    w = np.zeros((27, 1, cin, cout), np.float32)
+    p.subm_conv(spatial, 3, x, w)
+    got = p.subm_conv_bwd(spatial, 3, x, d, w)[1]
+    want, mag = _weight_gradient(p.submanifold_rules(spatial, 3), x, d, cin, cout)
+    err = np.abs(got.reshape(want.shape) - want)
+    bound = (n / 32 + 200) * 2.0 ** -24 * mag
+    assert (err <= bound).all(), err.max()
+    assert np.linalg.norm(err) <= 0.1 * np.linalg.norm(bound)
+
+
+def test_weight_gradient_with_values_that_are_not_finite():
+    n, cin, cout = 3000, 100, 64
+    p, spatial = _scene(n, 9800)
+    rng = np.random.default_rng(9)
+    x, d = rng.normal(size=(n, cin)).astype(np.float32), rng.normal(size=(n, cout)).astype(np.float32)
+    x[11, 5], x[n - 1, 70] = np.inf, np.nan
+    w = np.zeros((27, 1, cin, cout), np.float32)
+    p.subm_conv(spatial, 3, x, w)
+    got = p.subm_conv_bwd(spatial, 3, x, d, w)[1].reshape(w.shape)
+    for k, r in enumerate(p.submanifold_rules(spatial, 3)):
+        i, o = x[r[:, 0]].astype(np.float64), d[r[:, 1]].astype(np.float64)
+        for c in (4, 5, 6, 70, 99):
+            with np.errstate(all="ignore"):
+                want = (i[:, c:c + 1] * o).sum(0) if len(r) else np.zeros(cout)
+            assert (np.isnan(got[k, 0, c]) == np.isnan(want)).all()
+            ok = ~np.isnan(want)
+            np.testing.assert_allclose(got[k, 0, c][ok], want[ok], rtol=1e-4, atol=1e-3)
