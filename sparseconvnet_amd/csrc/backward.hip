@@ -14,11 +14,10 @@
 //     over the positions that have the tap: MFMA tiles over chunks of positions, partial sums per
 //     chunk, then a reduction in fixed order (no float atomics, deterministic);
 //   * column sums (bias gradients, batch-norm statistics) are two-stage reductions in fixed order.
-#include "metadata.h"
+#include "conv_common.h"
 
 namespace scn {
 
-typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v3f __attribute__((ext_vector_type(3)));
 static const int TB = 256;
@@ -1040,11 +1039,21 @@ static bool taps_mirror(Metadata &m, Table &t, const int64_t *filter, hipStream_
 // d_in = (table read from the output side) convolution of d_out with transposed weights.
 static void input_gradient(Metadata &m, const Table &t, const float *d_out, int64_t d_out_rows, float *d_in,
                            const float *w, int n_in, int n_out, int groups, bool mirror, hipStream_t s) {
+  m.frozen = nullptr;  // the transposed weights are this call's
+  // Where the split-operand kernel takes the call, its packing reads the weights transposed.  (Tables of one
+  // rule per position go to another kernel first, more than 256 planes run as ranges of copied columns, and
+  // many taps may not fit its tile set-up.)
+  if (groups == 1 && n_in <= 256 && t.K <= 64 && !t.few_tap.p && !t.identity_few &&
+      conv_split_serves(m, t, d_out, d_out_rows, n_out)) {
+    m.pack_transposed = w;
+    m.pack_mirror = mirror;
+    conv_forward(m, t, d_out, d_out_rows, d_in, w, nullptr, n_out, n_in, groups, nullptr, nullptr, s);
+    return;
+  }
   const int64_t wn = (int64_t)t.K * (n_in / groups) * (n_out / groups) * groups;
   m.wt.reserve(wn);
   k_transpose_weights<<<grid_for(wn), TB, 0, s>>>(w, m.wt.p, t.K, groups, n_in / groups, n_out / groups, mirror ? 1 : 0);
   LAUNCH_CHECK();
-  m.frozen = nullptr;  // the transposed weights are scratch of this call
   conv_forward(m, t, d_out, d_out_rows, d_in, m.wt.p, nullptr, n_out, n_in, groups, nullptr, nullptr, s);
 }
 

@@ -7,7 +7,11 @@ namespace scn {
 // wp[k][slab of 32 channels][piece][column block][lane]: 16 bytes, the lane's eight channels
 // (slab*32 + 16*(e/4) + 4*(lane/16) + e%4, e < 8) of column 16*cb + lane%16; zeros outside
 // [nIn) x [nOut).  A weight that is no finite number is all in its first piece.
-__global__ void k_pack_weights_split(const float *w, v8s *wp, int K, int n_in, int n_out, int n_slab, int NCB, CoefJobs jobs) {
+// transposed: `w` is [K][nOut][nIn] (an input gradient's weights as the forward pass has them); mirror: the
+// taps in reverse order.  (A transposed copy was a launch per layer of its own, 232 us of the million-site
+// U-Net's training step.)
+__global__ void k_pack_weights_split(const float *w, v8s *wp, int K, int n_in, int n_out, int n_slab, int NCB, CoefJobs jobs,
+                                     bool transposed, bool mirror) {
   coef_jobs(jobs);
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t per_slab = (int64_t)NCB * 64;
@@ -20,7 +24,9 @@ __global__ void k_pack_weights_split(const float *w, v8s *wp, int K, int n_in, i
 #pragma unroll
   for (int e = 0; e < 8; e++) {
     const int ch = sl * 32 + 16 * (e >> 2) + 4 * (lane >> 4) + (e & 3);
-    const float v = (ch < n_in && col < n_out) ? w[((int64_t)k * n_in + ch) * n_out + col] : 0.0f;
+    float v = 0.0f;
+    if (ch < n_in && col < n_out)
+      v = transposed ? w[((int64_t)(mirror ? K - 1 - k : k) * n_out + col) * n_in + ch] : w[((int64_t)k * n_in + ch) * n_out + col];
     unsigned ph, pm, pl;
     split_pair(v, 0.0f, ph, pm, pl);
     if (!(fabsf(v) < INFINITY)) {
@@ -273,7 +279,8 @@ static bool launch_split(Metadata &m, const Table &t, const float *in, float *ou
   float *wpack = packed_weights(m, {3, (int64_t)(uintptr_t)w, t.K, n_in, n_out, NCB}, packed, [&](float *dst) {
     const int64_t threads = (int64_t)t.K * n_slab * NCB * 64;
     k_pack_weights_split<<<dim3((unsigned)ceil_div(threads, 256)), 256, 0, s>>>(
-        w, reinterpret_cast<v8s *>(dst), t.K, n_in, n_out, n_slab, NCB, take_jobs(m));
+        m.pack_transposed ? m.pack_transposed : w, reinterpret_cast<v8s *>(dst), t.K, n_in, n_out, n_slab, NCB, take_jobs(m),
+        m.pack_transposed != nullptr, m.pack_mirror);
     LAUNCH_CHECK();
   });
   constexpr int CUT = !PRE || OCC == 4 ? OCC : OCC == 5 ? 3 : 2;  // the batch norm's coefficients take 16 registers more
@@ -356,11 +363,14 @@ static bool dispatch_split(Metadata &m, const Table &t, const float *in, float *
 // Inputs of up to 16 planes stay with the fp32 kernels: half of a 32-channel slab would be empty (a
 // million sites 16 -> 16 146 us there, 193 here; 24 -> 24 265 there, 243 here, and 67 / 21 at 20 k sites).
 // The allocation-free entry point too: its fixed array holds fp32 weights, not half as many again.
-bool conv_split_dispatch(bool pre_fused, Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi,
-                         int n_in, int n_out, PreArgs pre, hipStream_t s) {
+bool conv_split_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in) {
   if (m.bf16 || m.fixed_scratch) return false;
   if (n_in <= 16 || n_in % 4 || (uintptr_t)in % 16 || t.K > 1024 || n_in * 4 >= (1 << 24)) return false;
-  if (m.cur_in_rows <= 0 || m.cur_in_rows >= (1 << 24) || m.cur_in_rows * n_in * 4 >= ((int64_t)1 << 31)) return false;
+  return in_rows > 0 && in_rows < (1 << 24) && in_rows * n_in * 4 < ((int64_t)1 << 31);
+}
+bool conv_split_dispatch(bool pre_fused, Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi,
+                         int n_in, int n_out, PreArgs pre, hipStream_t s) {
+  if (!conv_split_serves(m, t, in, m.cur_in_rows, n_in)) return false;
   return pre_fused ? dispatch_split<true>(m, t, in, out, w, epi, n_in, n_out, pre, s)
                    : dispatch_split<false>(m, t, in, out, w, epi, n_in, n_out, pre, s);
 }

@@ -89,8 +89,9 @@ struct Table {
   // each XCD a contiguous range.
   bool spread = false;
   const int *rowmap_ptr() const { return identity_rows ? nullptr : rowmap.p; }
-  // Submanifold tables, decided on first use by a backward pass: does rule (k, i -> j) imply
-  // rule (K-1-k, j -> i)?  (Odd filter sizes on a level without repeated points.)
+  // Submanifold tables: does rule (k, i -> j) imply rule (K-1-k, j -> i)?  (Odd filter sizes on a level
+  // without repeated points: known when the table is made, or, where points may repeat, decided on the
+  // device on first use by a backward pass.)
   bool mirror_known = false, mirror = false;
   std::shared_ptr<Counts> cnt;  // never null once the table has been built
   const std::vector<int64_t> &counts(hipStream_t s) {
@@ -232,6 +233,10 @@ struct Metadata {
   DevBuf<int> scan_tiles;  // exclusive_scan: the tiles' sums
   DevBuf<int> ob_words, ob_list, ob_part;  // strided rulebooks by lookup: counters, the coarse level's blocks, partial ranks
   uint64_t level_gen = 0;
+  // The running convolution's weights are those at `pack_transposed`, each tap's slice transposed (and the taps
+  // in reverse order): the packing reads them so (k_pack_weights_split), no transposed copy is made.
+  const float *pack_transposed = nullptr;
+  bool pack_mirror = false;
   std::function<void()> before_pack;  // work the packing of the running convolution's weights needs first (the column-range path's copy), run at most once
   // while a column range of a wide layer runs: addresses in the scratch copy (from wkey_from) stand for
   // addresses from wkey_ptr in the caller's weights in a frozen set's keys

@@ -1660,6 +1660,10 @@ Table &submanifold_rules(Metadata &m, const int64_t *spatial, const int64_t *fil
   Level &L = lit->second;
   t.n = L.n;
   t.npad = L.npad;
+  if (!L.dups) {  // every key once: a backward pass need not look (Table::mirror)
+    t.mirror_known = t.mirror = true;
+    for (int d = 0; d < m.dim; d++) t.mirror = t.mirror && f.size[d] % 2 == 1;
+  }
   bool all3 = true;
   for (int d = 0; d < m.dim; d++) all3 = all3 && f.size[d] == 3;
   if (all3 && (m.dim == 2 || m.dim == 3) && t.n <= TINY_MAX && !L.dups) {
