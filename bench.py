@@ -26,6 +26,7 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0      # MI355X HBM3E
 MFMA_FP32_TFLOPS = 157.3   # MI355X dense fp32 matrix peak
 MFMA_BF16_TFLOPS = 2500.0  # MI355X dense bf16 matrix peak
+MFMA_SPLIT_TFLOPS = MFMA_BF16_TFLOPS / 6  # fp32 operands as three bf16 pieces each: six bf16 products per fp32 one
 PAIRS = [(3, 32), (32, 32), (64, 64), (128, 128), (256, 256)]
 TRAFFIC_FILE = os.path.join("profiles", "conv_sweep1M_pmc.txt")
 
@@ -76,15 +77,16 @@ def roofline_for(cin, cout, R, n, K, ms, traffic=None):
     """traffic: (bytes, kernel name) from the committed counter summary, or None."""
     flops = 2.0 * R * cin * cout
     byts = conv_bytes(R, n, K, cin, cout)
-    t_mfma = flops / (MFMA_FP32_TFLOPS * 1e12)
+    mfma = round(MFMA_SPLIT_TFLOPS, 1) if cin > 16 and cin % 4 == 0 else MFMA_FP32_TFLOPS  # the kernels that serve them
+    t_mfma = flops / (mfma * 1e12)
     t_hbm = byts / (HBM_PEAK_GBS * 1e9)
     tr = {"traffic": traffic[0] if traffic else None}
     if traffic:
         tr["traffic_source"] = {"file": TRAFFIC_FILE, "kernel": traffic[1]}
     if t_mfma >= t_hbm:
         ach = flops / (ms * 1e-3) / 1e12
-        return dict({"bound": "mfma", "achieved": round(ach, 3), "peak": MFMA_FP32_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(ach / MFMA_FP32_TFLOPS, 4)}, **tr)
+        return dict({"bound": "mfma", "achieved": round(ach, 3), "peak": mfma, "unit": "TFLOP/s",
+                     "frac": round(ach / mfma, 4)}, **tr)
     ach = byts / (ms * 1e-3) / 1e9
     return dict({"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                  "frac": round(ach / HBM_PEAK_GBS, 4)}, **tr)
@@ -292,8 +294,8 @@ def unet_scene(sites, seed, reps=7, residual=False, batch=1):
 def unet_layer_table(torch, scn, model, x, reps=5):
     """Every convolution of one warm U-Net pass, in call order: HIP events on the launch stream
     around each call (median of `reps` passes), the kernel the library chose, the layer's
-    multiply-adds as the reference counts them and its roofline (fp32 MFMA peak or HBM,
-    whichever bounds the layer)."""
+    multiply-adds as the reference counts them and its roofline (MFMA peak of the arithmetic that serves
+    it or HBM, whichever bounds the layer)."""
     from sparseconvnet_amd import metadata as M
     recs = []
     orig = M.Metadata._conv
