@@ -91,6 +91,10 @@ __device__ inline void split_pair(float x0, float x1, unsigned &h, unsigned &m, 
   const float l0 = r0 - __builtin_bit_cast(float, m << 16), l1 = r1 - __builtin_bit_cast(float, m & 0xFFFF0000u);
   l = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f){l0, l1}, v2bf));
 }
+__device__ inline float join_pieces(short h, short m, short l) {
+  auto as_float = [](short b) { return __builtin_bit_cast(float, (unsigned)(unsigned short)b << 16); };
+  return (as_float(h) + as_float(m)) + as_float(l);
+}
 struct Split8 {  // eight channels of a lane: the operands of the three pieces
   v8s h, m, l;
 };

@@ -57,7 +57,7 @@ __global__ void k_pack_weights_split(const float *w, v8s *wp, int K, int n_in, i
 // the staging writes (lane = row * 4 + chunk) nor the operand reads (lane = chunk * 16 + row) meet in
 // a bank.
 // Rows or weights that are no finite numbers make the pieces' sums NaN: a wavefront that finds any
-// sum not finite computes its whole tile again as the definition says, in fp32 (see the end).
+// sum not finite computes its part of the tile again in fp32 (see the end).
 template <int NCBW, int WC, int GW, int CG, int NB, int OCC, bool PRE>
 __global__ __launch_bounds__(256, OCC) void k_conv_split(
     const int *__restrict__ nbr, const int *__restrict__ rowmap, int K, int64_t n, int64_t npad,
@@ -200,20 +200,78 @@ __global__ __launch_bounds__(256, OCC) void k_conv_split(
     }
   }
 
-  // acc[q][c][r] = result for position tbase + 16*(wr*GW+q) + 4*g + r, column 16*(wc*NCBW+c) + r16
-  float *pt = partial ? partial + ((int64_t)blockIdx.y * n_tiles * TM + tbase) * (NCB * 16) : nullptr;
-  const bool post = epi.sc != nullptr;
-  auto store = [&](int p, int64_t row, int col, float v, float bias, float sc, float sh) {
-    if (pt) {  // [n_split][n_tiles * TM][NCB * 16]
-      pt[(int64_t)p * (NCB * 16) + col] = v;
-      return;
+  float probe = 0.f;  // stays zero while every sum is finite
+#pragma unroll
+  for (int q = 0; q < GW; q++)
+#pragma unroll
+    for (int c = 0; c < NCBW; c++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) probe = __builtin_fmaf(acc[q][c][r], 0.f, probe);
+  if (__ballot(probe != 0.f) != 0ull) {
+    // Infinities, NaNs or sums past the largest number: the wavefront's part of the tile again on the fp32
+    // matrix instructions, rows as they are and weights put back together from their pieces (the packed
+    // layout is the operand order of these instructions too: element e of step s is the lane's channel of one
+    // of them).  A row that does not have the tap is left out of the sum, not multiplied as zeros: its
+    // weights may be infinite.  Where every tile has to, a pass takes 1.4 (20 k sites 32 -> 32), 1.9 (64 -> 64),
+    // 2.9 (128 -> 128) or 3.9 times (256 -> 256) an ordinary one; a loop over single values took 27 to 216 times.
+#pragma unroll
+    for (int q = 0; q < GW; q++)
+#pragma unroll
+      for (int c = 0; c < NCBW; c++) acc[q][c] = (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int it = 0; it < total; it++) {
+      const int ti = it / n_slab, sl = it - ti * n_slab;
+      const int k = __builtin_amdgcn_readfirstlane(taplist[ti]);
+      const unsigned gm = __builtin_amdgcn_readfirstlane(gmask[k]);
+#pragma unroll
+      for (int c = 0; c < NCBW; c++) {
+        const v8s *src = wp + ((int64_t)k * n_slab + sl) * (3 * NCB * 64) + (wc * NCBW + c) * 64 + lane;
+        const v8s wh = src[0], wm = src[NCB * 64], wl = src[2 * NCB * 64];
+        float w[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) w[e] = join_pieces(wh[e], wm[e], wl[e]);
+#pragma unroll
+        for (int q = 0; q < GW; q++) {
+          const int gr = wr * GW + q;
+          if (!((gm >> gr) & 1u)) continue;  // uniform over the wavefront
+          const int *rows = jtab + (gr * K + k) * 16;
+          const int j = rows[r16];
+          v4f t = (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int s = 0; s < 2; s++) {
+            const int ch = (sl * 2 + s) * 16 + 4 * g;
+            const bool there = j >= 0 && ch < n_in;  // n_in is a multiple of four
+            v4f x = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
+                                                rsrc, there ? (unsigned)j * row_bytes + 4u * (unsigned)ch : 0x80000000u, 0, 0));
+            if (PRE) {
+              x = pre_act<PRE>(x, *reinterpret_cast<const v4f *>(pre_sc + ch), *reinterpret_cast<const v4f *>(pre_sh + ch), pre_leak);
+              if (!there) x = (v4f){0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) t = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], w[4 * s + e], t, 0, 0, 0);
+          }
+#pragma unroll
+          for (int r = 0; r < 4; r++) acc[q][c][r] += rows[4 * g + r] >= 0 ? t[r] : 0.f;
+        }
+      }
     }
-    if (col >= n_out) return;
-    v += bias;
-    if (epi.out2) epi_second(epi, row, col, v);
-    if (post) v = epi_act(v, sc, sh, epi.leak);
-    out[row * (epi.out_stride ? epi.out_stride : n_out) + col] = v;
-  };
+  }
+
+  // acc[q][c][r] = result for position tbase + 16*(wr*GW+q) + 4*g + r, column 16*(wc*NCBW+c) + r16
+  if (partial) {  // [n_split][n_tiles * TM][NCB * 16]
+    float *pt = partial + ((int64_t)blockIdx.y * n_tiles * TM + tbase) * (NCB * 16);
+#pragma unroll
+    for (int q = 0; q < GW; q++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int p = (wr * GW + q) * 16 + 4 * g + r;
+        if (tbase + p >= n) continue;
+#pragma unroll
+        for (int c = 0; c < NCBW; c++) pt[(int64_t)p * (NCB * 16) + 16 * (wc * NCBW + c) + r16] = acc[q][c][r];
+      }
+    return;
+  }
+  const bool post = epi.sc != nullptr;
   float bv[NCBW], es[NCBW], eh[NCBW];
 #pragma unroll
   for (int c = 0; c < NCBW; c++) {
@@ -222,49 +280,23 @@ __global__ __launch_bounds__(256, OCC) void k_conv_split(
     es[c] = (post && col < n_out) ? epi.sc[col] : 1.0f;
     eh[c] = (post && col < n_out) ? epi.sh[col] : 0.0f;
   }
-  float probe = 0.f;  // stays zero while every sum is finite
 #pragma unroll
   for (int q = 0; q < GW; q++) {
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int p = (wr * GW + q) * 16 + 4 * g + r;
-      const int64_t pos = tbase + p;
-#pragma unroll
-      for (int c = 0; c < NCBW; c++) probe = __builtin_fmaf(acc[q][c][r], 0.f, probe);
+      const int64_t pos = tbase + (wr * GW + q) * 16 + 4 * g + r;
       if (pos >= n) continue;
-      const int64_t row = rowmap && !pt ? rowmap[pos] : pos;
+      const int64_t row = rowmap ? rowmap[pos] : pos;
 #pragma unroll
-      for (int c = 0; c < NCBW; c++) store(p, row, 16 * (wc * NCBW + c) + r16, acc[q][c][r], bv[c], es[c], eh[c]);
-    }
-  }
-  if (__ballot(probe != 0.f) == 0ull) return;
-  // Infinities, NaNs or sums past the largest number: every value of the wavefront's part of the tile
-  // again, rows as they are and weights put back together from their pieces, in fp32 (one lane per value).
-  const short *ws = reinterpret_cast<const short *>(wp);
-  auto as_float = [](short b) { return __builtin_bit_cast(float, (unsigned)(unsigned short)b << 16); };
-  for (int e = 0; e < GW * 4 * NCBW; e++) {
-    const int c = e % NCBW, r = (e / NCBW) & 3, q = e / (4 * NCBW);
-    const int gr = wr * GW + q, cb = wc * NCBW + c, p = gr * 16 + 4 * g + r, col = 16 * cb + r16;
-    const int64_t pos = tbase + p;
-    if (pos >= n) continue;
-    float v = 0.f;
-    for (int ti = 0; ti < ntaps; ti++) {
-      const int k = taplist[ti], j = jtab[(gr * K + k) * 16 + 4 * g + r];
-      if (j < 0) continue;
-      for (int ch = 0; ch < n_in; ch++) {
-        float x = in[(int64_t)j * n_in + ch];
-        if (PRE) {
-          x = x * pre_sc[ch] + pre_sh[ch];
-          x *= x > 0.f ? 1.f : pre_leak;
-        }
-        const short *wc_ = ws + ((((int64_t)k * n_slab + ch / 32) * 3 * NCB + cb) * 64 + ((ch >> 2) & 3) * 16 + r16) * 8 +
-                           ((ch >> 4) & 1) * 4 + (ch & 3);
-        const float w = (as_float(wc_[0]) + as_float(wc_[NCB * 512])) + as_float(wc_[2 * NCB * 512]);
-        v = __builtin_fmaf(x, w, v);
+      for (int c = 0; c < NCBW; c++) {
+        const int col = 16 * (wc * NCBW + c) + r16;
+        if (col >= n_out) continue;
+        float v = acc[q][c][r] + bv[c];
+        if (epi.out2) epi_second(epi, row, col, v);
+        if (post) v = epi_act(v, es[c], eh[c], epi.leak);
+        out[row * (epi.out_stride ? epi.out_stride : n_out) + col] = v;
       }
     }
-    store(p, rowmap && !pt ? rowmap[pos] : pos, col, v, epi.bias != nullptr && col < n_out ? epi.bias[col] : 0.0f,
-          post && col < n_out ? epi.sc[col] : 1.0f, post && col < n_out ? epi.sh[col] : 0.0f);
   }
 }
 

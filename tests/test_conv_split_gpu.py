@@ -146,3 +146,132 @@ def test_weight_gradient_with_values_that_are_not_finite():
             assert (np.isnan(got[k, 0, c]) == np.isnan(want)).all()
             ok = ~np.isnan(want)
             np.testing.assert_allclose(got[k, 0, c][ok], want[ok], rtol=1e-4, atol=1e-3)
+
+
+def _rules_of(md):
+    from hip_path import HipPath
+
+    class Rules(HipPath):
+        def __init__(self):
+            self.L, self.dim, self.h = md._L, 3, md._h
+
+        def __del__(self):
+            pass
+    return Rules()
+
+
+def _close_where_finite(got, want, mag, terms):
+    """NaNs where the sum in 64 bits has them, infinities of its sign where it is past the largest float, and elsewhere within
+    `terms` additions in fp32 of the sum of magnitudes."""
+    import torch
+    got = got.double()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    big = want.abs() > 3.5e38
+    assert torch.equal(got[big], torch.sign(want[big]) * float("inf"))
+    rest = want.abs() < 3e38
+    assert rest.any() and not rest.all()
+    assert ((got - want).abs()[rest] <= terms * 2.0 ** -24 * mag[rest] + 1e-37).all()
+
+
+# 512 tiles and more (stored by the tile itself) and fewer (its taps dealt out), 32-, 64- and 128-row tiles, each
+# form of the call, tables with and without a row map
+@pytest.mark.parametrize("kind,n,cin,cout,pre", [
+    ("subm", 900, 64, 96, False), ("subm", 1500, 64, 64, True), ("subm", 33333, 24, 48, False), ("subm", 33333, 36, 160, True),
+    ("subm", 70001, 20, 32, False), ("subm", 300001, 32, 40, False), ("subm", 300001, 32, 40, True),
+    ("down", 20011, 32, 64, False), ("down", 160001, 32, 64, False), ("up", 33333, 64, 48, False), ("up", 3001, 64, 48, True)])
+def test_values_that_are_not_finite_in_every_form_of_the_call(kind, n, cin, cout, pre):
+    import torch
+    import sparseconvnet_amd as scn
+    spatial = 126 if n < 30000 else 1022
+    coords = synthetic.room_scene(seed=9600 + n % 91, target=max(n, 2000), spatial=spatial)[:n]
+    t = scn.InputLayer(3, spatial, mode=4)([torch.as_tensor(coords), torch.zeros((n, 1)).cuda()])
+    md, size, half = t.metadata, t.spatial_size, (t.spatial_size - 2) // 2 + 1
+    two, three = torch.LongTensor([2] * 3), torch.LongTensor([3] * 3)
+    g = torch.Generator().manual_seed(n + cout)
+
+    def normal(*shape):
+        return torch.randn(*shape, generator=g).cuda()
+
+    def bn(c):
+        return normal(c) * 0.3, torch.rand(c, generator=g).cuda() + 0.5, torch.rand(c, generator=g).cuda() + 0.5, normal(c) * 0.3, 1e-4, 0.2
+
+    def normalise(y, mag, p):
+        mean, var, gamma, beta, eps, leak = p
+        sc = (gamma.double() / torch.sqrt(var.double() + eps))
+        y, mag = (y - mean.double()) * sc + beta.double(), mag * sc + (mean.abs().double() * sc + beta.abs().double())
+        return torch.where(y > 0, y, leak * y), mag
+    taps = 27 if kind == "subm" else 8
+    p = _rules_of(md)
+    if kind == "subm":
+        rules = p.submanifold_rules(size, 3)
+
+        def conv(*a, **k):
+            return md.submanifoldConvolution(size, three, *a, want_macs=False, **k)[0]
+    else:
+        md.convolution(size, half, two, two, torch.zeros((n, 1)).cuda(), torch.zeros(8, 1, 1, 1).cuda(), None, want_macs=False)
+        rules = p.strided_rules(size, half, 2, 2)
+        if kind == "up":
+            rules = [r[:, ::-1].copy() for r in rules]
+
+        def conv(*a, **k):
+            f, sizes = (md.convolution, (size, half)) if kind == "down" else (md.deconvolution, (half, size))
+            return f(*sizes, two, two, *a, want_macs=False, **k)[0]
+    rows_in, rows_out = (md.getNActive(half) if kind == "up" else n), (md.getNActive(half) if kind == "down" else n)
+    w, bias, front, post, second = normal(taps, 1, cin, cout) * 0.05, normal(cout), bn(cin) if pre else None, bn(cout), bn(cout)
+    for case in ("rows", "weights", "overflow"):
+        x, v = normal(rows_in, cin), w.clone()
+        if case == "rows":
+            x[5, 3], x[rows_in // 2, 7], x[rows_in - 1, 3] = float("inf"), float("nan"), float("-inf")
+        elif case == "weights":
+            v[taps // 2, 0, 2, 4], v[taps - 1, 0, 1, 6] = float("inf"), float("nan")
+        else:
+            v *= 1e-3
+            x[::5, 0], v[taps // 2, 0, 0] = 1e38, 16.0
+        f, fm = x.double(), x.double().abs()
+        if pre:
+            f, fm = normalise(f, fm, front)
+        want = bias.double().expand(rows_out, -1).clone()
+        mag = want.abs()
+        for k, r in enumerate(rules):
+            r = torch.as_tensor(r).cuda().long()
+            want.index_add_(0, r[:, 1], f[r[:, 0]] @ v[k, 0].double())
+            mag.index_add_(0, r[:, 1], fm[r[:, 0]] @ v[k, 0].double().abs())
+        terms = taps * cin + 16
+        _close_where_finite(conv(x, v, bias, bn=front), want, mag, terms)
+        wide, other = torch.full((rows_out, cout + 24), 7.0).cuda(), torch.full((rows_out, cout + 12), 5.0).cuda()
+        conv(x, v, bias, bn=front, post=post, out=wide[:, 8:8 + cout], second=(second, other[:, 4:4 + cout]))
+        assert (wide[:, :8] == 7.0).all() and (wide[:, 8 + cout:] == 7.0).all()
+        assert (other[:, :4] == 5.0).all() and (other[:, 4 + cout:] == 5.0).all()
+        raw = torch.where(want.abs() > 3.5e38, torch.sign(want) * float("inf"), want)  # as the fp32 sum in front has it
+        for got, p in ((wide[:, 8:8 + cout], post), (other[:, 4:4 + cout], second)):
+            y, m = normalise(raw, mag, p)
+            _close_where_finite(got, y, m, terms)
+
+
+def test_rows_of_nans_cost_a_few_times_an_ordinary_pass():
+    """Every tile computed twice, the second time on fp32 matrix instructions with nothing prefetched: 1.9 times an ordinary
+    pass at 64 -> 64, 2.9 at 128 -> 128.  The bound tells that from a loop over single values (60 and 136 times)."""
+    import torch
+    import sparseconvnet_amd as scn
+    coords = synthetic.room_scene(seed=9650, target=20011, spatial=126)
+    t = scn.InputLayer(3, 126, mode=4)([torch.as_tensor(coords), torch.zeros((len(coords), 1)).cuda()])
+    for planes in (64, 128):
+        conv = scn.SubmanifoldConvolution(3, planes, planes, 3, False).cuda()
+
+        def time(x):
+            best = float("inf")
+            for _ in range(4):
+                a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                a.record()
+                with torch.no_grad():
+                    y = conv(scn.SparseConvNetTensor(x, t.metadata, t.spatial_size)).features
+                b.record()
+                b.synchronize()
+                best = min(best, a.elapsed_time(b))
+            return best, y
+        x = torch.randn(len(coords), planes).cuda()
+        ordinary, _ = time(x)
+        x[:, 3] = float("nan")
+        nans, y = time(x)
+        assert torch.isnan(y).all()
+        assert nans < 15 * ordinary, (nans, ordinary)
