@@ -70,9 +70,12 @@ __device__ inline v4f mfma_bf16(v8s a, v8s b, v4f acc) {
 }
 
 // ---- fp32 operands as three bf16 pieces -------------------------------------------------
-// x = h + m + l exactly, eight significant bits each: h is x cut off after eight bits (never rounded
-// up, so it cannot overflow), m the remainder rounded to bf16, l what is left of it (signed).  Of the nine
-// products of two such numbers the three below 2^-24 of the product are left out; the other six are one
+// x = h + m + l, each rounded to the eight bits of bf16 (G. Henry, P. T. P. Tang, A. Heinecke, "Leveraging the
+// bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", ARITH 2019).  For x in [2^e, 2^(e+1))
+// |m| <= 2^(e-8) and |l| <= 2^(e-17), so that of the nine products of two such numbers h l' + l h' + m m' and above
+// count and m l' + l m' + l l' <= 1.001 2^-24 2^(e+e') are left out (cut off instead of rounded, h would leave
+// an m of up to 2^(e-7) and four times as much: single products up to 4.8 2^-24 off, against 2.4 now and 1.0 on the
+// fp32 matrix instructions, which round to nearest).  The other six are one
 // v_mfma_f32_16x16x32_bf16 each, 96 cycles of the matrix unit for 32 channels where eight
 // v_mfma_f32_16x16x4_f32 take 256.  (The matrix unit sustains 1700 TFLOP/s on the former and 140
 // on the latter, operands in registers: twice the rate after the six-fold work.)
@@ -81,19 +84,32 @@ __device__ inline v4f mfma_bf16(v8s a, v8s b, v4f acc) {
 // not to nearest.  Against sums in 64 bits, 16 x 16 tiles, 1728 channels (relative 2-norm): fp32
 // matrix instructions 7.5e-7 (signed values) / 5.3e-7 (ReLU outputs) / 4.2e-7 (all positive), six
 // products into the accumulator 6.4e-7 / 6.2e-7 / 7.7e-7, summed apart 1.5e-7 / 1.5e-7 / 1.1e-7.
+// A number that no bf16 rounds (3.396e38 and more) has infinite pieces: whoever multiplies them finds a sum that is not
+// finite.
 __device__ inline void split_pair(float x0, float x1, unsigned &h, unsigned &m, unsigned &l) {
   typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
   typedef float v2f __attribute__((ext_vector_type(2)));
-  const unsigned u0 = __builtin_bit_cast(unsigned, x0), u1 = __builtin_bit_cast(unsigned, x1);
-  h = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
-  const float r0 = x0 - __builtin_bit_cast(float, u0 & 0xFFFF0000u), r1 = x1 - __builtin_bit_cast(float, u1 & 0xFFFF0000u);
+  h = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f){x0, x1}, v2bf));
+  const float r0 = x0 - __builtin_bit_cast(float, h << 16), r1 = x1 - __builtin_bit_cast(float, h & 0xFFFF0000u);
   m = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f){r0, r1}, v2bf));
   const float l0 = r0 - __builtin_bit_cast(float, m << 16), l1 = r1 - __builtin_bit_cast(float, m & 0xFFFF0000u);
   l = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f){l0, l1}, v2bf));
 }
-__device__ inline float join_pieces(short h, short m, short l) {
-  auto as_float = [](short b) { return __builtin_bit_cast(float, (unsigned)(unsigned short)b << 16); };
-  return (as_float(h) + as_float(m)) + as_float(l);
+// Packed weights: the pieces of v, or, of a number that has none, an infinity and its own two halves.
+constexpr short PIECE_WHOLE = 0x7F80;
+__device__ inline void split_weight(float v, short &h, short &m, short &l) {
+  unsigned ph, pm, pl;
+  split_pair(v, 0.0f, ph, pm, pl);
+  const bool whole = (ph & 0x7F80u) == 0x7F80u;
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  h = whole ? PIECE_WHOLE : (short)ph;
+  m = (short)(whole ? u >> 16 : pm);
+  l = (short)(whole ? u : pl);
+}
+__device__ inline float join_weight(short h, short m, short l) {
+  auto upper = [](short b) { return (unsigned)(unsigned short)b << 16; };
+  if (h == PIECE_WHOLE) return __builtin_bit_cast(float, upper(m) | (unsigned short)l);
+  return (__builtin_bit_cast(float, upper(h)) + __builtin_bit_cast(float, upper(m))) + __builtin_bit_cast(float, upper(l));
 }
 struct Split8 {  // eight channels of a lane: the operands of the three pieces
   v8s h, m, l;

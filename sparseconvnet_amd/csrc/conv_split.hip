@@ -6,7 +6,7 @@ namespace scn {
 
 // wp[k][slab of 32 channels][piece][column block][lane]: 16 bytes, the lane's eight channels
 // (slab*32 + 16*(e/4) + 4*(lane/16) + e%4, e < 8) of column 16*cb + lane%16; zeros outside
-// [nIn) x [nOut).  A weight that is no finite number is all in its first piece.
+// [nIn) x [nOut).
 // transposed: `w` is [K][nOut][nIn] (an input gradient's weights as the forward pass has them); mirror: the
 // taps in reverse order.  (A transposed copy was a launch per layer of its own, 232 us of the million-site
 // U-Net's training step.)
@@ -27,13 +27,9 @@ __global__ void k_pack_weights_split(const float *w, v8s *wp, int K, int n_in, i
     float v = 0.0f;
     if (ch < n_in && col < n_out)
       v = transposed ? w[((int64_t)(mirror ? K - 1 - k : k) * n_out + col) * n_in + ch] : w[((int64_t)k * n_in + ch) * n_out + col];
-    unsigned ph, pm, pl;
-    split_pair(v, 0.0f, ph, pm, pl);
-    if (!(fabsf(v) < INFINITY)) {
-      if (v != v) ph |= 0x40u;  // a NaN whose upper half would read as infinity stays one
-      pm = pl = 0u;
-    }
-    h[e] = (short)ph, m[e] = (short)pm, l[e] = (short)pl;
+    short ph, pm, pl;
+    split_weight(v, ph, pm, pl);
+    h[e] = ph, m[e] = pm, l[e] = pl;
   }
   v8s *dst = wp + ks * 3 * per_slab + (int64_t)cb * 64 + lane;
   dst[0] = h;
@@ -229,7 +225,7 @@ __global__ __launch_bounds__(256, OCC) void k_conv_split(
         const v8s wh = src[0], wm = src[NCB * 64], wl = src[2 * NCB * 64];
         float w[8];
 #pragma unroll
-        for (int e = 0; e < 8; e++) w[e] = join_pieces(wh[e], wm[e], wl[e]);
+        for (int e = 0; e < 8; e++) w[e] = join_weight(wh[e], wm[e], wl[e]);
 #pragma unroll
         for (int q = 0; q < GW; q++) {
           const int gr = wr * GW + q;

@@ -275,3 +275,39 @@ def test_rows_of_nans_cost_a_few_times_an_ordinary_pass():
         nans, y = time(x)
         assert torch.isnan(y).all()
         assert nans < 15 * ordinary, (nans, ordinary)
+
+
+def _hard_factors(n, seed):
+    """fp32 numbers in [1, 2): those whose bits below the first eight are all set or just over half, and any."""
+    bits = np.random.default_rng(seed).integers(0x3F800000, 0x40000000, n, dtype=np.uint32)
+    bits[:8] = [0x3F80FF7F, 0x3F80FF80, 0x3F807FFF, 0x3F808001, 0x3F807F7F, 0x3FFFFFFF, 0x3FFF7FFF, 0x3F817F80]
+    return bits.view(np.float32)
+
+
+def test_single_products():
+    """What the six products leave out is at most 1.001 2^-24 of a product with factors in [1, 2), and the sum of the six is
+    rounded to 24 bits, not to nearest: 2^-23 of the result."""
+    p, spatial = _scene(3000, 9900)
+    u, v = _hard_factors(3000, 1), _hard_factors(128, 2)
+    x, w = np.zeros((3000, 32), np.float32), np.zeros((27, 1, 32, 128), np.float32)
+    x[:, 5], w[13, 0, 5] = u, v
+    got, _ = p.subm_conv(spatial, 3, x, w)
+    want = u[:, None].astype(np.float64) * v[None].astype(np.float64)
+    assert (np.abs(got - want) <= 3.1 * 2.0 ** -24 * want).all(), (np.abs(got - want) / want).max() * 2.0 ** 24
+    x, d, w = np.zeros((3000, 128), np.float32), np.zeros((3000, 128), np.float32), np.zeros((27, 1, 128, 128), np.float32)
+    x[7], d[7] = u[:128], v
+    got = p.subm_conv_bwd(spatial, 3, x, d, w)[1].reshape(27, 128, 128)
+    want = want[:128]
+    assert (np.abs(got[13] - want) <= 3.1 * 2.0 ** -24 * want).all(), (np.abs(got[13] - want) / want).max() * 2.0 ** 24
+    assert (got[:13] == 0).all() and (got[14:] == 0).all()
+
+
+def test_weights_near_the_largest_float():
+    """Weights that no bf16 rounds, an infinity and a NaN beside them: packed whole."""
+    p, spatial = _scene(3000, 9901)
+    big = np.array([3.3962e38, -3.4028234e38, 3.39e38, np.inf, -np.inf, np.nan, 1e38, 1.0], np.float32)
+    x, w = np.zeros((3000, 32), np.float32), np.zeros((27, 1, 32, 8), np.float32)
+    x[:, 9], w[13, 0, 9] = np.linspace(0.25, 0.99, 3000), big
+    got, _ = p.subm_conv(spatial, 3, x, w)
+    want = (x[:, 9:10] * big[None]).astype(np.float32)
+    np.testing.assert_allclose(got, want, rtol=2.0 ** -22)
