@@ -84,11 +84,16 @@ __device__ inline v4f mfma_bf16(v8s a, v8s b, v4f acc) {
 // not to nearest.  Against sums in 64 bits, 16 x 16 tiles, 1728 channels (relative 2-norm): fp32
 // matrix instructions 7.5e-7 (signed values) / 5.3e-7 (ReLU outputs) / 4.2e-7 (all positive), six
 // products into the accumulator 6.4e-7 / 6.2e-7 / 7.7e-7, summed apart 1.5e-7 / 1.5e-7 / 1.1e-7.
-// A number that no bf16 rounds (3.396e38 and more) has infinite pieces: whoever multiplies them finds a sum that is not
-// finite.
+// The pieces are those of 2^24 x: bf16 ends at 2^-133 where fp32 ends at 2^-149, and pieces of x itself would lose bits of
+// every x below 2^-110 (4.7e-2 of the result at 2^-126, all of it at 2^-140).  Sums of products come out 2^48 times too
+// large (SPLIT_UNSCALE).  (Costs a multiplication per value staged: a stack of layers at a million sites 10.13 -> 10.19 ms,
+// training step 24.8 -> 24.9.)  A number that no bf16 then rounds (2e31 and more) has infinite pieces: whoever multiplies them,
+// or has a sum past 1.2e24, finds a sum that is not finite and computes it in fp32.
+constexpr float SPLIT_SCALE = 0x1p24f, SPLIT_UNSCALE = 0x1p-48f;
 __device__ inline void split_pair(float x0, float x1, unsigned &h, unsigned &m, unsigned &l) {
   typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
   typedef float v2f __attribute__((ext_vector_type(2)));
+  x0 *= SPLIT_SCALE, x1 *= SPLIT_SCALE;
   h = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f){x0, x1}, v2bf));
   const float r0 = x0 - __builtin_bit_cast(float, h << 16), r1 = x1 - __builtin_bit_cast(float, h & 0xFFFF0000u);
   m = __builtin_bit_cast(unsigned, __builtin_convertvector((v2f){r0, r1}, v2bf));
@@ -109,7 +114,8 @@ __device__ inline void split_weight(float v, short &h, short &m, short &l) {
 __device__ inline float join_weight(short h, short m, short l) {
   auto upper = [](short b) { return (unsigned)(unsigned short)b << 16; };
   if (h == PIECE_WHOLE) return __builtin_bit_cast(float, upper(m) | (unsigned short)l);
-  return (__builtin_bit_cast(float, upper(h)) + __builtin_bit_cast(float, upper(m))) + __builtin_bit_cast(float, upper(l));
+  return ((__builtin_bit_cast(float, upper(h)) + __builtin_bit_cast(float, upper(m))) + __builtin_bit_cast(float, upper(l))) *
+         (1.0f / SPLIT_SCALE);
 }
 struct Split8 {  // eight channels of a lane: the operands of the three pieces
   v8s h, m, l;

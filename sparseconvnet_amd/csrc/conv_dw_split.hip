@@ -212,8 +212,8 @@ __global__ __launch_bounds__(256, 2) void k_conv_dw_split(
 #pragma unroll
       for (int r = 0; r < 4; r++) probe = __builtin_fmaf(acc[i][j][r], 0.f, probe);
   if (__ballot(probe != 0.f) != 0ull) {
-    // Values that are no finite numbers make the pieces' sums NaN: the wavefront goes through the share
-    // again on the fp32 matrix instructions, 16 positions and one channel per lane and load.
+    // Values that are no finite numbers, or too large for pieces, make the pieces' sums infinite or NaN: the
+    // wavefront goes through the share again on the fp32 matrix instructions, 16 positions and one channel per lane and load.
 #pragma unroll
     for (int i = 0; i < NA; i++)
 #pragma unroll
@@ -246,6 +246,11 @@ __global__ __launch_bounds__(256, 2) void k_conv_dw_split(
           for (int j = 0; j < NB; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[i], vb[j], acc[i][j], 0, 0, 0);
       }
     }
+  } else {
+#pragma unroll
+    for (int i = 0; i < NA; i++)
+#pragma unroll
+      for (int j = 0; j < NB; j++) acc[i][j] *= SPLIT_UNSCALE;
   }
   float *pk = partial + ((size_t)share * K + k) * (size_t)n_a * n_b;
 #pragma unroll

@@ -52,8 +52,8 @@ __global__ void k_pack_weights_split(const float *w, v8s *wp, int K, int n_in, i
 // the registers are cut for.  An operand slot is moved by twice its lane group so that neither
 // the staging writes (lane = row * 4 + chunk) nor the operand reads (lane = chunk * 16 + row) meet in
 // a bank.
-// Rows or weights that are no finite numbers make the pieces' sums NaN: a wavefront that finds any
-// sum not finite computes its part of the tile again in fp32 (see the end).
+// Rows or weights that are no finite numbers, or too large for pieces, make the pieces' sums infinite or NaN: a
+// wavefront that finds any sum not finite computes its part of the tile again in fp32 (see the end).
 template <int NCBW, int WC, int GW, int CG, int NB, int OCC, bool PRE>
 __global__ __launch_bounds__(256, OCC) void k_conv_split(
     const int *__restrict__ nbr, const int *__restrict__ rowmap, int K, int64_t n, int64_t npad,
@@ -204,12 +204,12 @@ __global__ __launch_bounds__(256, OCC) void k_conv_split(
 #pragma unroll
       for (int r = 0; r < 4; r++) probe = __builtin_fmaf(acc[q][c][r], 0.f, probe);
   if (__ballot(probe != 0.f) != 0ull) {
-    // Infinities, NaNs or sums past the largest number: the wavefront's part of the tile again on the fp32
+    // Infinities, NaNs or values too large for pieces: the wavefront's part of the tile again on the fp32
     // matrix instructions, rows as they are and weights put back together from their pieces (the packed
     // layout is the operand order of these instructions too: element e of step s is the lane's channel of one
     // of them).  A row that does not have the tap is left out of the sum, not multiplied as zeros: its
-    // weights may be infinite.  Where every tile has to, a pass takes 1.4 (20 k sites 32 -> 32), 1.9 (64 -> 64),
-    // 2.9 (128 -> 128) or 3.9 times (256 -> 256) an ordinary one; a loop over single values took 27 to 216 times.
+    // weights may be infinite.  Where every tile has to, a pass takes 1.5 (20 k sites 32 -> 32), 2 (64 -> 64), 3
+    // (128 -> 128) or 4 to 5 times (256 -> 256) an ordinary one; a loop over single values took 27 to 216 times.
 #pragma unroll
     for (int q = 0; q < GW; q++)
 #pragma unroll
@@ -251,6 +251,11 @@ __global__ __launch_bounds__(256, OCC) void k_conv_split(
         }
       }
     }
+  } else {
+#pragma unroll
+    for (int q = 0; q < GW; q++)
+#pragma unroll
+      for (int c = 0; c < NCBW; c++) acc[q][c] *= SPLIT_UNSCALE;
   }
 
   // acc[q][c][r] = result for position tbase + 16*(wr*GW+q) + 4*g + r, column 16*(wc*NCBW+c) + r16

@@ -249,8 +249,8 @@ def test_values_that_are_not_finite_in_every_form_of_the_call(kind, n, cin, cout
 
 
 def test_rows_of_nans_cost_a_few_times_an_ordinary_pass():
-    """Every tile computed twice, the second time on fp32 matrix instructions with nothing prefetched: 1.9 times an ordinary
-    pass at 64 -> 64, 2.9 at 128 -> 128.  The bound tells that from a loop over single values (60 and 136 times)."""
+    """Every tile computed twice, the second time on fp32 matrix instructions with nothing prefetched: 2 times an ordinary
+    pass at 64 -> 64, 3 at 128 -> 128.  The bound tells that from a loop over single values (60 and 136 times)."""
     import torch
     import sparseconvnet_amd as scn
     coords = synthetic.room_scene(seed=9650, target=20011, spatial=126)
@@ -311,3 +311,29 @@ def test_weights_near_the_largest_float():
     got, _ = p.subm_conv(spatial, 3, x, w)
     want = (x[:, 9:10] * big[None]).astype(np.float32)
     np.testing.assert_allclose(got, want, rtol=2.0 ** -22)
+
+
+@pytest.mark.parametrize("ex,ew", [(-112, 60), (-126, 60), (-140, 80), (60, -112), (60, -126), (80, -140), (-100, -38), (-126, 0),
+                                   (100, -100), (110, -30), (50, 20)])
+def test_operands_of_any_size(ex, ew):
+    """Rows of 2^ex and weights (output gradients) of 2^ew: as exact as any others, down to numbers that fp32 holds with fewer bits
+    and past 2^104, where the pieces end.  Beside the bound of ordinary operands, each part of a sum that is stored by itself (a
+    tile's taps are dealt out over up to 27 workgroups, positions over up to 200 shares) may be off by half of the smallest
+    number, 2^-150."""
+    p, spatial = _scene(2000, 9910)
+    rng = np.random.default_rng(abs(ex * 1000 + ew))
+
+    def normal(e, *shape):
+        return np.ldexp(np.clip(rng.normal(size=shape), -4, 4), e).astype(np.float32)
+    for cin, cout in ((32, 64), (96, 64)):
+        x, w, d = normal(ex, 2000, cin), normal(ew, 27, 1, cin, cout), normal(ew, 2000, cout)
+        got, _ = p.subm_conv(spatial, 3, x, w)
+        rules = p.submanifold_rules(spatial, 3)
+        want, mag = _reference(rules, x, w)
+        assert np.linalg.norm(want) > 0
+        err = np.abs(got - want)
+        assert (err <= (27 * -(-cin // 32) + 4) * 2.0 ** -24 * mag + 27 * 2.0 ** -150).all(), (err / mag.max()).max()
+        got = p.subm_conv_bwd(spatial, 3, x, d, w)[1].reshape(w.shape)
+        want, mag = _weight_gradient(rules, x, d, cin, cout)
+        err = np.abs(got - want)
+        assert (err <= (2000 / 32 + 200) * 2.0 ** -24 * mag + 200 * 2.0 ** -150).all(), (err / mag.max()).max()
