@@ -257,7 +257,7 @@ bool conv_tiled_dispatch(bool vec4, bool pre_fused, Metadata &m, const Table &t,
 bool conv_rows_dispatch(bool vec4, bool pre_fused, Metadata &m, const Table &t, const float *in, float *out,
                         const float *w, Epi epi, int n_in, int n_out, PreArgs pre, hipStream_t s);
 // conv_split.hip: fp32 operands as three bf16 pieces each.
-bool conv_split_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in);
+bool conv_split_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in, int n_out);
 bool conv_split_dispatch(bool pre_fused, Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi,
                          int n_in, int n_out, PreArgs pre, hipStream_t s);
 // conv_few.hip: transposed convolutions of filter = stride = 2 rulebooks whose weights fit LDS.

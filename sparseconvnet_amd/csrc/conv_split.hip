@@ -393,17 +393,25 @@ static bool dispatch_split(Metadata &m, const Table &t, const float *in, float *
   return false;
 }
 
-// Inputs of up to 16 planes stay with the fp32 kernels: half of a 32-channel slab would be empty (a
-// million sites 16 -> 16 146 us there, 193 here; 24 -> 24 265 there, 243 here, and 67 / 21 at 20 k sites).
-// The allocation-free entry point too: its fixed array holds fp32 weights, not half as many again.
-bool conv_split_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in) {
+// What the fp32 kernels keep (us):
+//   inputs of up to 16 planes: half of a 32-channel slab would be empty (a million sites 16 -> 16 146 there, 193
+//     here; 24 -> 24 265 there, 243 here, and 67 / 21 at 20 k sites)
+//   up to 32 -> 16 planes at large levels, where half of the columns here would be empty too and staging all weights per
+//     workgroup does not show any more: 32 -> 16 a million sites 164 there, 222 here, 400 k 83 / 98, 200 k 62 / 64, 150 k
+//     63 / 55; 20 -> 16 a million 187 / 225, 300 k 83 / 83; eight taps the other way round (a million fine sites 70 / 36)
+//   more than 64 taps onto up to 32 planes: 128 rows of so many neighbour indices leave one workgroup per CU (5^3,
+//     100 k sites 32 -> 32 353 / 443, 64 -> 32 675 / 831, 1 k 25 / 34; 49 taps 50 k 32 -> 32 73 / 76, 24 -> 32 91 / 76)
+//   the allocation-free entry point: its fixed array holds fp32 weights, not half as many again
+bool conv_split_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in, int n_out) {
   if (m.bf16 || m.fixed_scratch) return false;
   if (n_in <= 16 || n_in % 4 || (uintptr_t)in % 16 || t.K > 1024 || n_in * 4 >= (1 << 24)) return false;
+  if (n_out <= 16 && n_in <= 32 && t.n >= (n_in > 24 ? 200000 : 300000) && t.K > 8 && resident_fits(m, t, n_in, n_out, false)) return false;
+  if (n_out <= 32 && t.K > 64) return false;
   return in_rows > 0 && in_rows < (1 << 24) && in_rows * n_in * 4 < ((int64_t)1 << 31);
 }
 bool conv_split_dispatch(bool pre_fused, Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi,
                          int n_in, int n_out, PreArgs pre, hipStream_t s) {
-  if (!conv_split_serves(m, t, in, m.cur_in_rows, n_in)) return false;
+  if (!conv_split_serves(m, t, in, m.cur_in_rows, n_in, n_out)) return false;
   return pre_fused ? dispatch_split<true>(m, t, in, out, w, epi, n_in, n_out, pre, s)
                    : dispatch_split<false>(m, t, in, out, w, epi, n_in, n_out, pre, s);
 }

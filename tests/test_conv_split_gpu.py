@@ -184,6 +184,37 @@ def _rules_of(md):
     return Rules()
 
 
+def _table(kind, n, seed):
+    """A layer of `kind` on a room of n sites: (call of its convolution, rules per tap (in, out), input rows, output rows,
+    Metadata)."""
+    import torch
+    import sparseconvnet_amd as scn
+    spatial = {"up3": 127, "down3": 127}.get(kind, 126) if n < 30000 else {"up3": 1023, "down3": 1023}.get(kind, 1022)
+    coords = synthetic.room_scene(seed=seed, target=max(n + n // 10, 2000), spatial=spatial)[:n]
+    t = scn.InputLayer(3, spatial, mode=4)([torch.as_tensor(coords), torch.zeros((n, 1)).cuda()])
+    md, size = t.metadata, t.spatial_size
+    assert md.getNActive(size) == n
+    p = _rules_of(md)
+    if kind == "nin":
+        rules = [np.stack([np.arange(n)] * 2, 1)]
+        return lambda x, w, b: md.networkInNetwork(x, w[0, 0], b, want_macs=False)[0], rules, n, n, md
+    if kind.startswith("subm"):
+        f = torch.LongTensor([int(kind[4:] or 3)] * 3)
+
+        def conv(*a, **k):
+            return md.submanifoldConvolution(size, f, *a, want_macs=False, **k)[0]
+        conv(torch.zeros((n, 1)).cuda(), torch.zeros(int(f.prod()), 1, 1, 1).cuda(), None)
+        return conv, p.submanifold_rules(size, int(f[0])), n, n, md
+    f = 3 if kind.endswith("3") else 2
+    fs, two, half = torch.LongTensor([f] * 3), torch.LongTensor([2] * 3), (size - f) // 2 + 1
+    md.convolution(size, half, fs, two, torch.zeros((n, 1)).cuda(), torch.zeros(f ** 3, 1, 1, 1).cuda(), None, want_macs=False)
+    rules, coarse = p.strided_rules(size, half, f, 2), md.getNActive(half)
+    if kind.startswith("down"):
+        return lambda *a, **k: md.convolution(size, half, fs, two, *a, want_macs=False, **k)[0], rules, n, coarse, md
+    rules = [r[:, ::-1].copy() for r in rules]
+    return lambda *a, **k: md.deconvolution(half, size, fs, two, *a, want_macs=False, **k)[0], rules, coarse, n, md
+
+
 def _close_where_finite(got, want, mag, terms):
     """NaNs where the sum in 64 bits has them, infinities of its sign where it is past the largest float, and elsewhere within
     `terms` additions in fp32 of the sum of magnitudes."""
@@ -205,12 +236,8 @@ def _close_where_finite(got, want, mag, terms):
     ("down", 20011, 32, 64, False), ("down", 160001, 32, 64, False), ("up", 33333, 64, 48, False), ("up", 3001, 64, 48, True)])
 def test_values_that_are_not_finite_in_every_form_of_the_call(kind, n, cin, cout, pre):
     import torch
-    import sparseconvnet_amd as scn
-    spatial = 126 if n < 30000 else 1022
-    coords = synthetic.room_scene(seed=9600 + n % 91, target=max(n, 2000), spatial=spatial)[:n]
-    t = scn.InputLayer(3, spatial, mode=4)([torch.as_tensor(coords), torch.zeros((n, 1)).cuda()])
-    md, size, half = t.metadata, t.spatial_size, (t.spatial_size - 2) // 2 + 1
-    two, three = torch.LongTensor([2] * 3), torch.LongTensor([3] * 3)
+    conv, rules, rows_in, rows_out, _ = _table(kind, n, 9600 + n % 91)
+    taps = len(rules)
     g = torch.Generator().manual_seed(n + cout)
 
     def normal(*shape):
@@ -224,23 +251,6 @@ def test_values_that_are_not_finite_in_every_form_of_the_call(kind, n, cin, cout
         sc = (gamma.double() / torch.sqrt(var.double() + eps))
         y, mag = (y - mean.double()) * sc + beta.double(), mag * sc + (mean.abs().double() * sc + beta.abs().double())
         return torch.where(y > 0, y, leak * y), mag
-    taps = 27 if kind == "subm" else 8
-    p = _rules_of(md)
-    if kind == "subm":
-        rules = p.submanifold_rules(size, 3)
-
-        def conv(*a, **k):
-            return md.submanifoldConvolution(size, three, *a, want_macs=False, **k)[0]
-    else:
-        md.convolution(size, half, two, two, torch.zeros((n, 1)).cuda(), torch.zeros(8, 1, 1, 1).cuda(), None, want_macs=False)
-        rules = p.strided_rules(size, half, 2, 2)
-        if kind == "up":
-            rules = [r[:, ::-1].copy() for r in rules]
-
-        def conv(*a, **k):
-            f, sizes = (md.convolution, (size, half)) if kind == "down" else (md.deconvolution, (half, size))
-            return f(*sizes, two, two, *a, want_macs=False, **k)[0]
-    rows_in, rows_out = (md.getNActive(half) if kind == "up" else n), (md.getNActive(half) if kind == "down" else n)
     w, bias, front, post, second = normal(taps, 1, cin, cout) * 0.05, normal(cout), bn(cin) if pre else None, bn(cout), bn(cout)
     for case in ("rows", "weights", "overflow"):
         x, v = normal(rows_in, cin), w.clone()
@@ -299,6 +309,45 @@ def test_rows_of_nans_cost_a_few_times_an_ordinary_pass():
         nans, y = time(x)
         assert torch.isnan(y).all()
         assert nans < 15 * ordinary, (nans, ordinary)
+
+
+# (kind of layer, sites of its fine level, planes, what the kernel that runs says of itself)
+@pytest.mark.parametrize("kind,n,cin,cout,says", [
+    # up to 32 -> 16 planes at large levels and many taps onto up to 32: the fp32 kernels
+    ("subm", 199999, 32, 16, ("split ",)), ("subm", 200000, 32, 16, ("resident",)), ("subm", 299999, 20, 12, ("split ",)),
+    ("subm", 300000, 20, 12, ("resident",)), ("subm5", 3000, 64, 32, ("rows",)), ("subm5", 3000, 64, 40, ("split ",))])
+def test_kernel_and_shares_by_size(kind, n, cin, cout, says):
+    import torch
+    conv, rules, rows_in, rows_out, md = _table(kind, n, 9700 + n % 83)
+    g = torch.Generator().manual_seed(n + cin)
+    x, w = torch.randn(rows_in, cin, generator=g).cuda(), torch.randn(len(rules), 1, cin, cout, generator=g).cuda()
+    bias = torch.randn(cout, generator=g).cuda()
+    got = conv(x, w, bias)
+    kernel = md._L.scn_md_last_conv_kernel(md._h).decode()
+    assert all(part in kernel + " " for part in says), kernel
+    want = bias.double().expand(rows_out, -1).clone()
+    mag = want.abs()
+    for k, r in enumerate(rules):
+        r = torch.as_tensor(r).cuda().long()
+        want.index_add_(0, r[:, 1], x[r[:, 0]].double() @ w[k, 0].double())
+        mag.index_add_(0, r[:, 1], x[r[:, 0]].double().abs() @ w[k, 0].double().abs())
+    # the fp32 kernels add products one by one
+    additions = len(rules) * (-(-cin // 32) if kernel.startswith("split") else cin) + 28
+    assert ((got.double() - want).abs() <= additions * 2.0 ** -24 * mag).all()
+
+
+@pytest.mark.parametrize("n,cin,cout", [(200000, 16, 32), (199999, 16, 32), (20011, 24, 64), (3000, 96, 36)])
+def test_input_gradients_whichever_kernel_takes_them(n, cin, cout):
+    """The packing of k_conv_split reads the forward weights transposed; the others get a transposed copy."""
+    import torch
+    p, spatial = _scene(n, 9800 + n % 61)
+    rng = np.random.default_rng(n + cin)
+    d = rng.normal(size=(n, cout)).astype(np.float32)
+    w = (rng.normal(size=(27, 1, cin, cout)) * 0.1).astype(np.float32)
+    got = p.subm_conv_bwd(spatial, 3, np.zeros((n, cin), np.float32), d, w)[0]
+    rules = [r[:, ::-1].copy() for r in p.submanifold_rules(spatial, 3)]
+    want, mag = _reference(rules, d, np.ascontiguousarray(w.transpose(0, 1, 3, 2)))
+    assert (np.abs(got - want) <= (27 * cout + 4) * 2.0 ** -24 * mag).all()
 
 
 def _hard_factors(n, seed):
