@@ -356,6 +356,9 @@ static bool launch_split(Metadata &m, const Table &t, const float *in, float *ou
 //   below 1024 sites, 32-row tiles beyond 32 planes: a launch is as long as one workgroup's chain; 300
 //     sites 64 -> 64 10.6 (64-row tiles 11.0, was 10.8), 768 192 -> 192 22.8 (25.7, was 29.6), 384 -> 192 32.4
 //     (36.3, was 46.1); 152 sites 224 -> 224 21.4 (23.3, was 19.1); at 3.3 k 320 -> 160 68 against 57
+//   and up to 24 k where a tile has only a few iterations (1x1 convolutions, the fine side of filter = stride tables, eight
+//     or nine taps of 32 planes), for the same reason: 64 -> 256 1x1 5 k rows 19.8 -> 12.1, 20 k 23.9 -> 16.8; transposed 96 -> 96
+//     10 k sites 16.8 -> 14.5; 40 k one way or the other
 //   wider: 64-row tiles, three wavefronts per SIMD: a million sites 256 -> 256 11561 -> 6851 (128-row
 //     tiles, two wavefronts 6856), 100 k 1553 -> 830 (880); 300 k 192 -> 192 2336 -> 1276 (1359), 60 k
 //     160 -> 160 507 -> 290 (304), 3.3 k 160 -> 160 42 -> 37
@@ -367,7 +370,8 @@ static bool dispatch_split(Metadata &m, const Table &t, const float *in, float *
                            int n_out, PreArgs pre, hipStream_t s) {
   const int ncb = (int)ceil_div(n_out, 16);
   const bool large = t.n >= 300000;
-  if (t.n < 1024) {
+  const bool short_chain = t.few_tap.p || t.K * ceil_div(n_in, 32) <= 9;
+  if (t.n < 1024 || (t.n < 24000 && short_chain)) {
     if (ncb > 2 && ncb <= 4) return launch_split<2, 2, 1, 2, 2, 2, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);
     if (ncb > 4 && ncb <= 6) return launch_split<3, 2, 1, 3, 2, 2, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);
     if (ncb > 6 && ncb <= 8) return launch_split<2, 4, 2, 2, 2, 2, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);

@@ -313,6 +313,9 @@ def test_rows_of_nans_cost_a_few_times_an_ordinary_pass():
 
 # (kind of layer, sites of its fine level, planes, what the kernel that runs says of itself)
 @pytest.mark.parametrize("kind,n,cin,cout,says", [
+    # 1x1: a tile is one to eight iterations
+    ("nin", 1023, 64, 256, ("wc=4 gw=2",)), ("nin", 1024, 64, 256, ("wc=4 gw=2",)), ("nin", 5000, 96, 160, ("gw=1",)),
+    ("nin", 23999, 160, 128, ("gw=2",)), ("nin", 24000, 160, 128, ("gw=4",)), ("nin", 5000, 320, 160, ("gw=2",)),
     # up to 32 -> 16 planes at large levels and many taps onto up to 32: the fp32 kernels
     ("subm", 199999, 32, 16, ("split ",)), ("subm", 200000, 32, 16, ("resident",)), ("subm", 299999, 20, 12, ("split ",)),
     ("subm", 300000, 20, 12, ("resident",)), ("subm5", 3000, 64, 32, ("rows",)), ("subm5", 3000, 64, 40, ("split ",))])
