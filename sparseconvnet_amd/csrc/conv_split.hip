@@ -82,7 +82,7 @@ __global__ __launch_bounds__(256, OCC) void k_conv_split(
   const int tile = tiles_per_xcd ? (blockIdx.x & 7) * tiles_per_xcd + (blockIdx.x >> 3) : blockIdx.x;  // see k_conv_mfma
   if (tile >= n_tiles) return;  // whole workgroup leaves: no barrier is skipped
   const int64_t tbase = (int64_t)tile * TM;
-  const int ntaps = tile_setup<256, G>(nbr, K, n, npad, tbase, n_split, (int)blockIdx.y, jtab, gmask, taplist, ntaps_p);
+  const int ntaps = tile_setup<256, G, true>(nbr, K, n, npad, tbase, n_split, (int)blockIdx.y, jtab, gmask, taplist, ntaps_p);
   const int total = ntaps * n_slab;
   v4f acc[GW][NCBW];
 #pragma unroll
@@ -327,12 +327,25 @@ static bool launch_split(Metadata &m, const Table &t, const float *in, float *ou
   const int n_tiles = (int)ceil_div(t.n, G * 16);
   const int tiles_per_xcd = t.spread ? 0 : (int)ceil_div(n_tiles, 8);  // 0: tile = workgroup index
   // Few tiles: the taps of a tile dealt over several workgroups, four of 64 rows (or two of 128) per CU in
-  // all.  (Two and only below 256 tiles, as the fp32 kernels have it, is slower: 20 k sites 64 -> 64 48 ->
-  // 29 us, 30 k 128 -> 128 126 -> 91, 14 k 256 -> 128 116 -> 91; six per CU the same within 5 % either
-  // way.)  Up to nine iterations in all stay together: the launch that adds the parts up costs what
-  // they would save.
+  // all, and a launch adds the parts up.  (Two and only below 256 tiles, as the fp32 kernels have it, is slower: 20 k
+  // sites 64 -> 64 48 -> 29 us, 30 k 128 -> 128 126 -> 91, 14 k 256 -> 128 116 -> 91; six per CU the same within
+  // 5 % either way.)  `chain`: iterations of a tile.  The fine side of a transposed table has K * (coarse sites / fine
+  // sites) rules per position at most, and its positions are ordered by tap or pattern, so that from some 50 tiles on a
+  // tile has about as few taps.  Not dealt out, in us (graph replays):
+  //   one rule per position and tiles that mostly have one tap: 5 k fine sites 64 -> 256 30.2 dealt out, 24.4 not;
+  //     20 k 64 -> 64 23.1 / 13.8, 96 -> 96 28.0 / 18.9; but 300 sites 96 -> 96 11.8 / 17
+  //   chains of up to 12 where the level itself has the workgroups: 20 k fine sites, filter 3 stride 2, 32 -> 64 23.0 / 18.9;
+  //     eight iterations, 1 k coarse sites 32 -> 64 10.0 / 13.3, 5 k 11 / 16, but 10 k 21.4 / 15.8
+  // Parts of three iterations and more keep the partial sums and the time to add them small: 2 k sites 32 -> 64 20.4 us
+  // with parts of one, 15.1; 64 -> 64 21.9 / 19.2; 128-row tiles and the shortest chains are better off without (1 k sites
+  // 64 -> 32 15.5 / 16.0, 1.2 k coarse sites 32 -> 64 10.0 / 11.4).
+  const int64_t taps = t.n < 768 * G ? t.K : std::min<int64_t>(t.K, ceil_div(t.K * m.cur_in_rows, t.n));
+  const int64_t chain = taps * n_slab;
+  const bool one_rule = t.few_tap.p && t.n >= 1024 * G;
+  const int part = NCB <= 2 || (chain <= 24 && t.n < 2500) ? 1 : 3;
   int n_split = 1;
-  if (n_tiles < 512 && t.K * n_slab > 9) n_split = (int)std::min<int64_t>(t.K, ceil_div(4096, (int64_t)n_tiles * G));
+  if (n_tiles < 512 && !one_rule && (chain > 12 || (chain > 7 && t.n < 6000)))
+    n_split = (int)std::min<int64_t>({t.K, ceil_div(t.n < 3000 ? 3072 : 4096, (int64_t)n_tiles * G), ceil_div(chain, part)});
   const int64_t split_stride = (int64_t)n_tiles * G * 16 * NCB * 16;
   float *partial = scratch_partial(m, n_split, split_stride);
   note_kernel(m, "split", {{"ncbw", NCBW}, {"wc", WC}, {"gw", GW}, {"pre", PRE}, {"split", n_split}});

@@ -313,6 +313,17 @@ def test_rows_of_nans_cost_a_few_times_an_ordinary_pass():
 
 # (kind of layer, sites of its fine level, planes, what the kernel that runs says of itself)
 @pytest.mark.parametrize("kind,n,cin,cout,says", [
+    # one rule per position: dealt out only while a tile has several taps; 32-row tiles up to 24 k
+    ("up", 301, 96, 96, ("split ", "gw=1", "split=8")), ("up", 1535, 64, 256, ("gw=2", "split=8")),
+    ("up", 1537, 64, 256, ("gw=2", "split=1")), ("up", 20011, 64, 256, ("gw=2", "split=1")), ("up", 24001, 64, 96, ("gw=2 ", "split=1")),
+    ("up", 6143, 96, 32, ("ncbw=2 wc=1", "split=8")), ("up", 6145, 96, 32, ("ncbw=2 wc=1", "split=1")),
+    # eight taps of 32 planes: dealt out on small levels only
+    ("down", 4001, 32, 64, ("gw=1", "split=8")), ("down", 12001, 32, 64, ("gw=1", "split=3")), ("down", 40011, 32, 64, ("gw=1", "split=1")),
+    # parts of three iterations and more
+    ("subm", 2000, 32, 64, ("gw=2", "split=9")), ("subm", 2000, 64, 64, ("gw=2", "split=18")), ("subm", 700, 64, 24, ("split=27",)),
+    # filter 3 stride 2, fine side: taps of one parity per tile
+    ("up3", 8001, 64, 64, ("gw=2", "split ")), ("up3", 20011, 32, 64, ("split=1",)), ("up3", 700, 64, 64, ("gw=1", "split=18")),
+    ("down3", 5001, 64, 96, ("split ",)),
     # 1x1: a tile is one to eight iterations
     ("nin", 1023, 64, 256, ("wc=4 gw=2",)), ("nin", 1024, 64, 256, ("wc=4 gw=2",)), ("nin", 5000, 96, 160, ("gw=1",)),
     ("nin", 23999, 160, 128, ("gw=2",)), ("nin", 24000, 160, 128, ("gw=4",)), ("nin", 5000, 320, 160, ("gw=2",)),
