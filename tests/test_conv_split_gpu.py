@@ -424,3 +424,43 @@ def test_operands_of_any_size(ex, ew):
         want, mag = _weight_gradient(rules, x, d, cin, cout)
         err = np.abs(got - want)
         assert (err <= (2000 / 32 + 200) * 2.0 ** -24 * mag + 200 * 2.0 ** -150).all(), (err / mag.max()).max()
+
+
+# where the staged kernel begins and ends: one tap, transposed tables, more than 32 taps, sides of 36 and 48 planes
+@pytest.mark.parametrize("kind,n,cin,cout", [
+    ("nin", 400003, 64, 96), ("nin", 31, 36, 36), ("nin", 40001, 192, 100), ("up", 60001, 96, 64), ("up", 299999, 64, 64),
+    ("up", 300000, 64, 64), ("up", 300000, 128, 128), ("up3", 20011, 96, 64), ("down", 160001, 64, 96), ("down3", 30001, 64, 96),
+    ("subm", 60011, 36, 48), ("subm", 299999, 48, 96), ("subm", 300000, 48, 96), ("subm5", 3001, 64, 96), ("subm5", 1000, 128, 128)])
+def test_weight_gradient_of_every_kind_of_table(kind, n, cin, cout):
+    """Within as many additions in fp32 as a tap has rules, of the sum of magnitudes, in whatever order (the fp32 kernels add them one
+    by one within a share), and in the 2-norm as the sums of either sign are (see above)."""
+    import torch
+    _, rules, rows_in, rows_out, md = _table(kind, n, 9900 + n % 79)
+    g = torch.Generator().manual_seed(n + cin)
+    x, d = torch.randn(rows_in, cin, generator=g).cuda(), torch.randn(rows_out, cout, generator=g).cuda()
+    w = torch.zeros(len(rules), 1, cin, cout).cuda()
+    two, size = torch.LongTensor([2] * 3), torch.LongTensor([{"up3": 127, "down3": 127}.get(kind, 126) if n < 30000 else
+                                                             {"up3": 1023, "down3": 1023}.get(kind, 1022)] * 3)
+    f = torch.LongTensor([round(len(rules) ** (1 / 3))] * 3)
+    half = (size - f) // 2 + 1
+    if kind == "nin":
+        got = md.networkInNetworkBackward(x, d, w[0, 0], False)[1][None]
+    elif kind.startswith("subm"):
+        got = md.submanifoldConvolutionBackward(size, f, x, d, w, False)[1]
+    elif kind.startswith("down"):
+        got = md.convolutionBackward(size, half, f, two, x, d, w, False)[1]
+    else:
+        got = md.deconvolutionBackward(half, size, f, two, x, d, w, False)[1]
+    got = got.reshape(len(rules), cin, cout).double()
+    error = total = 0.0
+    for k, r in enumerate(rules):
+        r = torch.as_tensor(r).cuda().long()
+        if not len(r):
+            assert (got[k] == 0).all()
+            continue
+        a, b = x[r[:, 0]].double(), d[r[:, 1]].double()
+        want, mag = a.t().contiguous() @ b, a.abs().t().contiguous() @ b.abs()
+        err = (got[k] - want).abs()
+        assert (err <= (len(r) + 4) * 2.0 ** -24 * mag).all(), k
+        error, total = error + float(err.norm()) ** 2, total + float(want.norm()) ** 2
+    assert error ** 0.5 <= ((min(n, 4096) / 2) ** 0.5 + 2) * 2.0 ** -24 * total ** 0.5
