@@ -335,7 +335,8 @@ static bool launch_split(Metadata &m, const Table &t, const float *in, float *ou
   //   one rule per position and tiles that mostly have one tap: 5 k fine sites 64 -> 256 30.2 dealt out, 24.4 not;
   //     20 k 64 -> 64 23.1 / 13.8, 96 -> 96 28.0 / 18.9; but 300 sites 96 -> 96 11.8 / 17
   //   chains of up to 12 where the level itself has the workgroups: 20 k fine sites, filter 3 stride 2, 32 -> 64 23.0 / 18.9;
-  //     eight iterations, 1 k coarse sites 32 -> 64 10.0 / 13.3, 5 k 11 / 16, but 10 k 21.4 / 15.8
+  //     eight iterations, 1 k coarse sites 32 -> 64 10.0 / 13.3, 5 k 11 / 16, but 10 k 21.4 / 15.8; up to 32 output planes gain
+  //     less on the device (nine taps 24 -> 32 16 / 11) than a second launch costs a host that issues them one by one
   // Parts of three iterations and more keep the partial sums and the time to add them small: 2 k sites 32 -> 64 20.4 us
   // with parts of one, 15.1; 64 -> 64 21.9 / 19.2; 128-row tiles and the shortest chains are better off without (1 k sites
   // 64 -> 32 15.5 / 16.0, 1.2 k coarse sites 32 -> 64 10.0 / 11.4).
@@ -344,7 +345,7 @@ static bool launch_split(Metadata &m, const Table &t, const float *in, float *ou
   const bool one_rule = t.few_tap.p && t.n >= 1024 * G;
   const int part = NCB <= 2 || (chain <= 24 && t.n < 2500) ? 1 : 3;
   int n_split = 1;
-  if (n_tiles < 512 && !one_rule && (chain > 12 || (chain > 7 && t.n < 6000)))
+  if (n_tiles < 512 && !one_rule && (chain > 12 || (chain > 7 && t.n < 6000 && NCB > 2)))
     n_split = (int)std::min<int64_t>({t.K, ceil_div(t.n < 3000 ? 3072 : 4096, (int64_t)n_tiles * G), ceil_div(chain, part)});
   const int64_t split_stride = (int64_t)n_tiles * G * 16 * NCB * 16;
   float *partial = scratch_partial(m, n_split, split_stride);
@@ -416,13 +417,17 @@ static bool dispatch_split(Metadata &m, const Table &t, const float *in, float *
 //   up to 32 -> 16 planes at large levels, where half of the columns here would be empty too and staging all weights per
 //     workgroup does not show any more: 32 -> 16 a million sites 164 there, 222 here, 400 k 83 / 98, 200 k 62 / 64, 150 k
 //     63 / 55; 20 -> 16 a million 187 / 225, 300 k 83 / 83; eight taps the other way round (a million fine sites 70 / 36)
+//   up to nine taps of up to 32 planes onto up to 16 on small levels (24 -> 16, 8 taps: 250 coarse sites 13.4 / 14.9, 10 k 15.5 /
+//     16.1, 20 k 17.4 / 16.3)
 //   more than 64 taps onto up to 32 planes: 128 rows of so many neighbour indices leave one workgroup per CU (5^3,
 //     100 k sites 32 -> 32 353 / 443, 64 -> 32 675 / 831, 1 k 25 / 34; 49 taps 50 k 32 -> 32 73 / 76, 24 -> 32 91 / 76)
 //   the allocation-free entry point: its fixed array holds fp32 weights, not half as many again
 bool conv_split_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in, int n_out) {
   if (m.bf16 || m.fixed_scratch) return false;
   if (n_in <= 16 || n_in % 4 || (uintptr_t)in % 16 || t.K > 1024 || n_in * 4 >= (1 << 24)) return false;
-  if (n_out <= 16 && n_in <= 32 && t.n >= (n_in > 24 ? 200000 : 300000) && t.K > 8 && resident_fits(m, t, n_in, n_out, false)) return false;
+  if (n_out <= 16 && n_in <= 32 && (t.K <= 9 ? t.n < 16000 : t.n >= (n_in > 24 ? 200000 : 300000)) &&
+      resident_fits(m, t, n_in, n_out, false))
+    return false;
   if (n_out <= 32 && t.K > 64) return false;
   return in_rows > 0 && in_rows < (1 << 24) && in_rows * n_in * 4 < ((int64_t)1 << 31);
 }

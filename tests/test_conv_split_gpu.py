@@ -329,7 +329,8 @@ def test_rows_of_nans_cost_a_few_times_an_ordinary_pass():
     ("nin", 23999, 160, 128, ("gw=2",)), ("nin", 24000, 160, 128, ("gw=4",)), ("nin", 5000, 320, 160, ("gw=2",)),
     # up to 32 -> 16 planes at large levels and many taps onto up to 32: the fp32 kernels
     ("subm", 199999, 32, 16, ("split ",)), ("subm", 200000, 32, 16, ("resident",)), ("subm", 299999, 20, 12, ("split ",)),
-    ("subm", 300000, 20, 12, ("resident",)), ("subm5", 3000, 64, 32, ("rows",)), ("subm5", 3000, 64, 40, ("split ",))])
+    ("subm", 300000, 20, 12, ("resident",)), ("subm5", 3000, 64, 32, ("rows",)), ("subm5", 3000, 64, 40, ("split ",)),
+    ("down", 12001, 24, 16, ("resident",)), ("down", 90001, 24, 16, ("split ", "split=1")), ("down", 4001, 24, 20, ("split ", "split=1"))])
 def test_kernel_and_shares_by_size(kind, n, cin, cout, says):
     import torch
     conv, rules, rows_in, rows_out, md = _table(kind, n, 9700 + n % 83)
