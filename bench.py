@@ -73,11 +73,13 @@ def conv_bytes(R, n_out_rows, K, cin, cout, s=4):
     return R * cin * s + 8 * R + n_out_rows * cout * s + K * cin * cout * s
 
 
-def roofline_for(cin, cout, R, n, K, ms, traffic=None):
-    """traffic: (bytes, kernel name) from the committed counter summary, or None."""
+def roofline_for(cin, cout, R, n, K, ms, traffic=None, kernel=None):
+    """traffic: (bytes, kernel name) from the committed counter summary, or None.  kernel: what the library says it ran; without
+    it, what serves large submanifold layers of this shape."""
     flops = 2.0 * R * cin * cout
     byts = conv_bytes(R, n, K, cin, cout)
-    mfma = round(MFMA_SPLIT_TFLOPS, 1) if cin > 16 and cin % 4 == 0 else MFMA_FP32_TFLOPS  # the kernels that serve them
+    split = kernel.startswith("split") if kernel else cin > 16 and cin % 4 == 0 and (cin > 32 or cout > 16)
+    mfma = round(MFMA_SPLIT_TFLOPS, 1) if split else MFMA_FP32_TFLOPS
     t_mfma = flops / (mfma * 1e12)
     t_hbm = byts / (HBM_PEAK_GBS * 1e9)
     tr = {"traffic": traffic[0] if traffic else None}
@@ -330,7 +332,7 @@ def unet_layer_table(torch, scn, model, x, reps=5):
                      "nIn": int(cin), "nOut": int(cout), "bn_in_front": bool(pre), "bn_behind": bool(post),
                      "kernel": kernel, "ms": round(float(t), 4),
                      "tflops": round(2.0 * macs / (float(t) * 1e-3) / 1e12, 2),
-                     "roofline": roofline_for(cin, cout, R, n_out_rows, K, float(t))})
+                     "roofline": roofline_for(cin, cout, R, n_out_rows, K, float(t), kernel=kernel)})
     return rows
 
 

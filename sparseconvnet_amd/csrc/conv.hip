@@ -9,7 +9,8 @@
 // 16-row granule).  From 20 input planes on fp32 layers run in
 //   k_conv_split     fp32 operands as three bf16 pieces each, rows through LDS
 // and the others (fewer planes, plane counts that are no multiple of four, arrays not 16-byte aligned or
-// of 2 GiB and more, the allocation-free entry point, bf16 operands) are chosen by the output width:
+// of 2 GiB and more, the allocation-free entry point, bf16 operands, and the narrow ranges conv_split_serves
+// lists) are chosen by the output width:
 //   k_conv_resident  nOut <= 32   all taps' weights resident in LDS, wavefronts run alone
 //   k_conv_rows      nOut <= 128  wavefronts own rows, the weight slab goes through LDS
 //   k_conv_mfma      wider        wavefronts own columns, rows and weights go through LDS
@@ -354,6 +355,7 @@ void conv_forward(Metadata &m, const Table &t, const float *in, int64_t n_in_row
     epi.sh = buf.p + n_out;
     epi.leak = post->leak;
   }
+  // (the resident kernel's shapes also where k_conv_split takes them, which could: not measured)
   const bool pre_fused = bn && groups == 1 && !resident_fits(m, t, n_in, n_out, true);
   PreArgs pre;
   if (pre_fused) {

@@ -448,7 +448,8 @@ static void launch_resident_c4(Metadata &m, const Table &t, const float *in, flo
 
 // Narrow layers: nOut <= 32, any nIn, K <= 32.  nIn is processed in parts of up to 32
 // channels so that every part's weights fit in LDS; parts after the first accumulate.
-// The resident kernel serves nOut <= 32 with up to 32 taps.  It takes the input channels in
+// The resident kernel serves nOut <= 32 with up to 32 taps (fp32 layers of 20 planes and more run in k_conv_split first,
+// but for what conv_split_serves leaves).  It takes the input channels in
 // parts of 32 (every part after the first re-reads and re-writes the output) and has no fused
 // batch norm, so from 64 input channels on the row-owner kernel is faster (measured).
 bool resident_fits(const Metadata &m, const Table &t, int n_in, int n_out, bool with_bn) {
