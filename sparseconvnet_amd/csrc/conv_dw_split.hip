@@ -278,17 +278,17 @@ int64_t conv_dw_split(Metadata &m, const Table &t, const float *a, int64_t a_row
   // Where the other kernels are faster (us, kernel and sums, room surfaces):
   //   a side of up to 32 channels (a million sites 64 x 32 671 there, 722 here; 32 x 32 471 / 651, both in the
   //     narrowest tile that is built, 64 x 64), small levels of up to 64 (20 k 48 x 48 35 / 39)
-  //   a side of 36 or 48 channels, for which they have a tile of 48: 60 k 36 x 36 76 / 92, 36 x 128 166 / 193, 48 x 96
-  //     132 / 163, 150 k 284 / 309; equal at 400 k
   //   more than 32 taps: no granule masks, so that a workgroup here stages every granule for every tap (5^3, 5 k sites
   //     64 x 96 159 / 178, 192 x 192 770 / 987, but 128 x 128 378 / 333; 7^3, 20 k 128 x 128 2770 / 5107)
-  //   large transposed tables: few of a position's rows are read twice (400 k fine sites, filter 3 stride 2, 64 x 96 351 /
-  //     463, 128 x 128 745 / 796; filter = stride = 2, 64 x 64 152 / 165 but 128 x 128 386 / 347)
-  auto tile48 = [](int planes) { return planes <= 48 && planes % 3 == 0; };
+  //   large transposed tables of many taps: few of a position's rows are read twice (400 k fine sites, filter 3 stride 2, 64 x 96
+  //     351 / 463, 128 x 128 745 / 796)
+  // Up to 32 taps the others wait for a new table's rule counts, which drains the queue: sides of 36 and 48 channels stay here although
+  // the tile of 48 is faster by itself (60 k 36 x 36 76 / 92, 48 x 96 132 / 163; but the training step of a U-Net with 24 planes on
+  // 150 k sites, new scene each, 7.26 ms with it and 7.09 without, 400 k 11.20 / 11.14), and so do large filter = stride tables
+  // (400 k 64 x 64 152 / 165, 96 x 64 144 / 149, 128 x 128 386 / 347).
   const bool transposed = a_rows < t.n;
   if (n_a <= 32 || n_b <= 32 || (t.n < 30000 && n_a <= 64 && n_b <= 64)) return 0;
-  if (t.K > 9 && t.n < 300000 && (tile48(n_a) || tile48(n_b))) return 0;
-  if (t.K > 32 || (transposed && t.n >= 300000 && (t.K > 9 || n_a < 128 || n_b < 128))) return 0;
+  if (t.K > 32 || (transposed && t.n >= 300000 && t.K > 9)) return 0;
   // 32 N channels per side: the fewest channels staged, a tile counted as 32 wider than it is
   auto width = [](int planes) {
     int best = 2;
@@ -304,9 +304,10 @@ int64_t conv_dw_split(Metadata &m, const Table &t, const float *a, int64_t a_row
   // of partial sums, 108 at 128.
   // Where a position has few rules, the sums weigh more than evenness does: one tap (1x1 convolutions), 512 / 1024 / 2048 /
   // 8192 workgroups, 400 k rows 64 x 96 108 / 118 / 136 / 162 us, 128 x 128 153 / 173 / 204 / 249; transposed tables
-  // and up to nine taps 1024 / 2048 / 4096 / 8192, 60 k sites 96 x 64 61 / 60 / 75 / 76, 2^3 / stride 2 400 k 99 / 99 / 120 / 146.
+  // and up to nine taps 1024 / 2048 / 4096 / 8192, 60 k sites 96 x 64 61 / 60 / 75 / 76, 2^3 / stride 2 400 k 99 / 99 / 120 / 146,
+  // large 2-D levels 400 k 64 x 96 463 / 404 / 386 / 433.
   const bool large = t.n >= 300000, small = t.n < 30000, few_rules = t.K <= 9 || transposed;
-  const int workgroups = t.K == 1 ? 512 : few_rules ? (large ? 4096 : 2048) : large ? 8192 : small ? 2048 : 4096;
+  const int workgroups = t.K == 1 ? 512 : few_rules ? (large && !transposed ? 4096 : 2048) : large ? 8192 : small ? 2048 : 4096;
   int64_t shares = ceil_div(workgroups, t.K * mt);
   shares = std::min(shares, std::max<int64_t>(1, ((int64_t)(large ? 256 : small ? 64 : 128) << 18) / per_share));
   shares = std::max<int64_t>(1, std::min(shares, ceil_div(t.n, 16 * DS_BLOCK)));
