@@ -1040,11 +1040,12 @@ static bool taps_mirror(Metadata &m, Table &t, const int64_t *filter, hipStream_
 static void input_gradient(Metadata &m, const Table &t, const float *d_out, int64_t d_out_rows, float *d_in,
                            const float *w, int n_in, int n_out, int groups, bool mirror, hipStream_t s) {
   m.frozen = nullptr;  // the transposed weights are this call's
-  // Where the split-operand kernel takes the call, its packing reads the weights transposed.  (Tables of one
+  // Where a split-operand kernel takes the call, its packing reads the weights transposed.  (Tables of one
   // rule per position go to another kernel first, more than 256 planes run as ranges of copied columns, and
   // many taps may not fit its tile set-up.)
-  if (groups == 1 && n_in <= 256 && t.K <= 64 && !t.few_tap.p && !t.identity_few &&
-      conv_split_serves(m, t, d_out, d_out_rows, n_out, n_in)) {
+  if (groups == 1 && n_in <= 256 &&
+      (conv_wave_serves(m, t, d_out, d_out_rows, n_out, n_in) ||
+       (t.K <= 64 && !t.few_tap.p && !t.identity_few && conv_split_serves(m, t, d_out, d_out_rows, n_out, n_in)))) {
     m.pack_transposed = w;
     m.pack_mirror = mirror;
     conv_forward(m, t, d_out, d_out_rows, d_in, w, nullptr, n_out, n_in, groups, nullptr, nullptr, s);

@@ -6,11 +6,12 @@
 // the table they pass.
 //
 // MFMA kernels (groups == 1, accumulators in registers for the whole filter, taps skipped per
-// 16-row granule).  From 20 input planes on fp32 layers run in
-//   k_conv_split     fp32 operands as three bf16 pieces each, rows through LDS
+// 16-row granule).  fp32 layers run on split operands (three bf16 pieces each) in
+//   k_conv_wave      nOut <= 32, from 8 input planes on: wavefronts own rows from the rule to the store
+//   k_conv_split     from 20 input planes on: rows through LDS
 // and the others (fewer planes, plane counts that are no multiple of four, arrays not 16-byte aligned or
-// of 2 GiB and more, the allocation-free entry point, bf16 operands, and the narrow ranges conv_split_serves
-// lists) are chosen by the output width:
+// of 2 GiB and more, the allocation-free entry point, bf16 operands, and the ranges conv_wave_serves and
+// conv_split_serves list) are chosen by the output width:
 //   k_conv_resident  nOut <= 32   all taps' weights resident in LDS, wavefronts run alone
 //   k_conv_rows      nOut <= 128  wavefronts own rows, the weight slab goes through LDS
 //   k_conv_mfma      wider        wavefronts own columns, rows and weights go through LDS
@@ -272,6 +273,7 @@ void launch_conv_reduce(const float *partial, int n_split, int64_t split_stride,
 template <bool PRE>
 static bool conv_mfma_paths(Metadata &m, const Table &t, const float *in, float *out, const float *w,
                             Epi epi, int n_in, int n_out, PreArgs pre, hipStream_t s) {
+  if (conv_wave_dispatch(PRE, m, t, in, out, w, epi, n_in, n_out, pre, s)) return true;
   if (!PRE && try_few(m, t, in, out, w, epi, n_in, n_out, s)) return true;
   if (conv_split_dispatch(PRE, m, t, in, out, w, epi, n_in, n_out, pre, s)) return true;
   if (!PRE && try_resident(m, t, in, out, w, epi, n_in, n_out, s)) return true;
@@ -355,8 +357,8 @@ void conv_forward(Metadata &m, const Table &t, const float *in, int64_t n_in_row
     epi.sh = buf.p + n_out;
     epi.leak = post->leak;
   }
-  // (the resident kernel's shapes also where k_conv_split takes them, which could: not measured)
-  const bool pre_fused = bn && groups == 1 && !resident_fits(m, t, n_in, n_out, true);
+  // in the gather where the kernel can: 32 -> 32 at 250 k sites 90 us with a pass of its own, 79 in k_conv_wave's gather, 5 k sites 18 / 8.4
+  const bool pre_fused = bn && groups == 1 && (conv_wave_serves(m, t, in, n_in_rows, n_in, n_out) || !resident_fits(m, t, n_in, n_out, true));
   PreArgs pre;
   if (pre_fused) {
     const int n_pad = (int)round_up(n_in, 64) + 64;

@@ -10,7 +10,10 @@ namespace scn {
 // transposed: `w` is [K][nOut][nIn] (an input gradient's weights as the forward pass has them); mirror: the
 // taps in reverse order.  (A transposed copy was a launch per layer of its own, 232 us of the million-site
 // U-Net's training step.)
-__global__ void k_pack_weights_split(const float *w, v8s *wp, int K, int n_in, int n_out, int n_slab, int NCB, CoefJobs jobs,
+// HALF (up to 16 input channels): wp[k][piece][column block][lane], 8 bytes: the lane's four channels 4*(lane/16) + e, of
+// which k_conv_wave puts those of two taps together.
+template <bool HALF>
+__global__ void k_pack_weights_split(const float *w, void *wp, int K, int n_in, int n_out, int n_slab, int NCB, CoefJobs jobs,
                                      bool transposed, bool mirror) {
   coef_jobs(jobs);
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -20,9 +23,10 @@ __global__ void k_pack_weights_split(const float *w, v8s *wp, int K, int n_in, i
   const int64_t ks = i / per_slab;
   const int sl = (int)(ks % n_slab), k = (int)(ks / n_slab);
   const int col = 16 * cb + (lane & 15);
-  v8s h, m, l;
+  typedef typename std::conditional<HALF, v4s, v8s>::type Operand;
+  Operand h, m, l;
 #pragma unroll
-  for (int e = 0; e < 8; e++) {
+  for (int e = 0; e < (HALF ? 4 : 8); e++) {
     const int ch = sl * 32 + 16 * (e >> 2) + 4 * (lane >> 4) + (e & 3);
     float v = 0.0f;
     if (ch < n_in && col < n_out)
@@ -31,10 +35,22 @@ __global__ void k_pack_weights_split(const float *w, v8s *wp, int K, int n_in, i
     split_weight(v, ph, pm, pl);
     h[e] = ph, m[e] = pm, l[e] = pl;
   }
-  v8s *dst = wp + ks * 3 * per_slab + (int64_t)cb * 64 + lane;
+  Operand *dst = static_cast<Operand *>(wp) + ks * 3 * per_slab + (int64_t)cb * 64 + lane;
   dst[0] = h;
   dst[per_slab] = m;
   dst[2 * per_slab] = l;
+}
+
+// The running convolution's weights in the layout of k_pack_weights_split.
+const float *split_weights(Metadata &m, int K, const float *w, int n_in, int n_out, int NCB, bool half, hipStream_t s) {
+  const int n_slab = (int)ceil_div(n_in, 32);
+  const int64_t threads = (int64_t)K * n_slab * NCB * 64;
+  return packed_weights(m, {half ? 5 : 3, (int64_t)(uintptr_t)w, K, n_in, n_out, NCB}, threads * 3 * (half ? 2 : 4), [&](float *dst) {
+    auto kern = half ? k_pack_weights_split<true> : k_pack_weights_split<false>;
+    kern<<<dim3((unsigned)ceil_div(threads, 256)), 256, 0, s>>>(m.pack_transposed ? m.pack_transposed : w, dst, K, n_in, n_out,
+                                                               n_slab, NCB, take_jobs(m), m.pack_transposed != nullptr, m.pack_mirror);
+    LAUNCH_CHECK();
+  });
 }
 
 // A workgroup of 4 wavefronts owns a tile of G = GW*WR granules (16 rows each).  The wavefronts form
@@ -308,14 +324,7 @@ static bool launch_split(Metadata &m, const Table &t, const float *in, float *ou
   const size_t lds_bytes = (size_t)NB * G * 3 * 64 * 16 + ((size_t)G * t.K * 16 + 2 * t.K + 4) * sizeof(int);
   if (lds_bytes > 160 * 1024) return false;
   const int n_slab = (int)ceil_div(n_in, 32);
-  const int64_t packed = (int64_t)t.K * n_slab * 3 * NCB * 64 * 4;
-  float *wpack = packed_weights(m, {3, (int64_t)(uintptr_t)w, t.K, n_in, n_out, NCB}, packed, [&](float *dst) {
-    const int64_t threads = (int64_t)t.K * n_slab * NCB * 64;
-    k_pack_weights_split<<<dim3((unsigned)ceil_div(threads, 256)), 256, 0, s>>>(
-        m.pack_transposed ? m.pack_transposed : w, reinterpret_cast<v8s *>(dst), t.K, n_in, n_out, n_slab, NCB, take_jobs(m),
-        m.pack_transposed != nullptr, m.pack_mirror);
-    LAUNCH_CHECK();
-  });
+  const float *wpack = split_weights(m, t.K, w, n_in, n_out, NCB, false, s);
   constexpr int CUT = !PRE || OCC == 4 ? OCC : OCC == 5 ? 3 : 2;  // the batch norm's coefficients take 16 registers more
   auto kern = k_conv_split<NCBW, WC, GW, CG, NB, CUT, PRE>;
   static bool attr_set = false;

@@ -1,0 +1,389 @@
+// The split-operand convolution onto up to 32 output planes: a wavefront owns its rows from the rule to the store.  The
+// arithmetic is that of conv_split.hip, to the bit where the additions come in the same order; see conv.hip for the family.
+#include "conv_common.h"
+
+namespace scn {
+
+// A wavefront owns GW granules (16 positions each) and NCB column blocks, and shares nothing with the others of its workgroup,
+// so that nothing waits at a barrier in the loop.  Per (slab of 32 input channels, tap) iteration:
+//   indices          two iterations ahead, straight from the table (16 consecutive entries per granule)
+//   gathered rows    an iteration ahead, four lanes reading 64 consecutive bytes of a row, turned into operand order through
+//                    2 KB of LDS per granule that only this wavefront touches, then split in registers: once per row and
+//                    tap, since no other wavefront needs it
+//   weights          requested behind the MFMAs of the iteration before, from L2 in operand order, once for all GW granules
+//   MFMAs            six per granule and column block, granules without the tap skipped by the table's masks
+// PAIR (up to 16 input channels): an iteration is two taps of 16 channels instead of one of 32; half an operand comes from
+// either, rows and weights alike.
+// DEAL = 4: the wavefronts of a workgroup share GW granules and take the iterations in turn; their sums meet in LDS and are
+// added in the wavefronts' order.  A small level is as long as one wavefront's chain of iterations, and this cuts it to a
+// quarter without partial sums in memory and a launch to add them up.
+// What bounds it: at large levels the vector instructions of the splitting (some 60 per granule and iteration) next to the
+// MFMAs: in a loop of nothing else the two overlap by a tenth only, 155 ns per granule and iteration of 2 x 16 columns against
+// 69 and 113 apart, and the clock falls to 1.9-2.1 GHz; 32 -> 32 at a million sites is 106 us of that.  Counters there:
+// vector unit 53 %, matrix unit 28 % of the time, 2.1 TB/s from beyond L2.
+// Against k_conv_split and k_conv_resident, which served these shapes (us, graph replays, room surfaces, 27 taps):
+//   sites       1 M        400 k      100 k      24 k       8 k        2 k
+//   32 -> 32    262 / 213  105 / 86   44 / 31    24 / 12    18 / 7.6   13 / 7.2
+//   16 -> 16    157 / 116  91 / 51    35 / 20    21 / 8.6   21 / 5.6   20 / 5.5
+//   48 -> 16    393 / 320  168 / 123  75 / 39    33 / 16    21 / 11    15 / 10
+// 8 taps, stride 2, 16 -> 32 from 60 k sites 14 / 5.8; transposed 24 -> 16 onto 20 k sites 8.0 / 4.4; 1x1 16 -> 32 60 k rows 17 / 8.
+// Sums of up to 16 channels were computed on fp32 matrix instructions before; against 64 bits (relative 2-norm) 16 -> 16 at
+// 20 k sites 2.6e-7 / 6.3e-8, 8 -> 8 1.8e-7 / 6.3e-8, 1x1 8 -> 8 5.7e-8 / 3.3e-8.
+template <int NCB, int GW, int DEAL, int OCC, bool PAIR, bool PRE>
+__global__ __launch_bounds__(64 * (DEAL > 4 ? DEAL : 4), OCC) void k_conv_wave(
+    const int *__restrict__ nbr, const int *__restrict__ rowmap, const unsigned *__restrict__ gmask, int64_t n, int64_t npad,
+    const float *__restrict__ in, float *__restrict__ out, const v8s *__restrict__ wp, Epi epi, int n_in, int n_out, int n_slab,
+    int ncb, int tiles_per_xcd, int n_tiles, const float *__restrict__ pre_sc, const float *__restrict__ pre_sh, float pre_leak,
+    unsigned in_bytes) {
+  constexpr int WAVES = DEAL > 4 ? DEAL : 4;
+  static_assert(DEAL == 1 || DEAL == WAVES, "a workgroup is one group of wavefronts that share granules");
+  constexpr int PART = DEAL > 1 && NCB > 2 ? NCB : 2;  // KB of LDS per wavefront and granule
+  __shared__ v4f turn[WAVES][GW][PART][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  const int ld_row = lane >> 2, ld_g = lane & 3;
+  const int wr_slot = ld_g * 16 + (ld_row ^ (2 * ld_g)), rd_slot = g * 16 + (r16 ^ (2 * g));
+  const int tile = tiles_per_xcd ? (blockIdx.x & 7) * tiles_per_xcd + (blockIdx.x >> 3) : blockIdx.x;  // see k_conv_mfma
+  if (tile >= n_tiles) return;
+  const int64_t pos0 = (DEAL > 1 ? (int64_t)tile : (int64_t)tile * 4 + wave) * (GW * 16);
+  if (pos0 >= n) return;  // a wavefront leaves by itself: there are no barriers (DEAL > 1: the whole workgroup)
+  const int cb0 = blockIdx.y * NCB;  // first of this wavefront's column blocks, of ncb
+  unsigned gm[GW], all = 0u;
+#pragma unroll
+  for (int q = 0; q < GW; q++) {
+    gm[q] = pos0 + 16 * q < n ? __builtin_amdgcn_readfirstlane(gmask[pos0 / 16 + q]) : 0u;
+    all |= gm[q];
+  }
+  const int its = PAIR ? (__popc(all) + 1) / 2 : __popc(all) * n_slab, total = DEAL > 1 ? max(0, (its - wave + DEAL - 1) / DEAL) : its;
+  v4f acc[GW][NCB];
+#pragma unroll
+  for (int q = 0; q < GW; q++)
+#pragma unroll
+    for (int c = 0; c < NCB; c++) acc[q][c] = (v4f){0.f, 0.f, 0.f, 0.f};
+
+  const __amdgpu_buffer_rsrc_t rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(in), 0, (int)in_bytes, 0x00020000);
+  const unsigned row_bytes = (unsigned)n_in * 4u;
+  const bool tail = n_in % 32 != 0;
+  const int last = (int)(n - 1 - pos0);  // positions behind the last one repeat its indices and are left out
+  // three cursors over the iterations (slab outer, tap inner), each staying on the last one
+  struct Cursor {
+    unsigned rest;
+    int sl, k, k2, left;  // k2 (PAIR): the second tap, -1: none
+  };
+  auto step = [&](Cursor &c) {
+    if (c.rest == 0u) c.rest = all, c.sl++;  // (PAIR: one slab, only the first step comes here)
+    c.k = __builtin_ctz(c.rest);
+    c.rest &= c.rest - 1u;
+    if (PAIR) {
+      c.k2 = c.rest ? __builtin_ctz(c.rest) : -1;
+      c.rest &= c.rest - 1u;  // stays 0 when it is
+    }
+  };
+  auto start = [&](Cursor &c) {
+    c = Cursor{0u, -1, 0, -1, total};
+    if (total > 0)
+      for (int i = 0; i <= (DEAL > 1 ? wave : 0); i++) step(c);
+  };
+  auto advance = [&](Cursor &c) {
+    if (c.left <= 1) return;
+    c.left--;
+#pragma unroll
+    for (int i = 0; i < DEAL; i++) step(c);
+  };
+  Cursor at, rows, idx;
+  int j[GW][PAIR ? 2 : 1];
+  v4f areg[GW][2];
+  v8s breg[NCB][3];
+  auto issue_indices = [&](const Cursor &c) {
+#pragma unroll
+    for (int q = 0; q < GW; q++)
+#pragma unroll
+      for (int h = 0; h < (PAIR ? 2 : 1); h++) {
+        const int p = min(16 * q + ld_row, last), k = h && c.k2 >= 0 ? c.k2 : c.k;
+        j[q][h] = (nbr + (int64_t)k * npad + pos0)[p];
+        if (h && c.k2 < 0) j[q][h] = -1;
+      }
+  };
+  unsigned aok = 0;  // PRE: bit 2q+s: this lane's chunk exists (zero must stay zero)
+  v4f psc[2], psh[2];
+  auto issue_rows = [&](const Cursor &c) {
+    aok = 0;
+#pragma unroll
+    for (int q = 0; q < GW; q++) {
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        const int row = j[q][PAIR ? s : 0], step = PAIR ? 0 : c.sl * 2 + s;  // step: of 16 channels
+        const bool past = (PAIR || tail) && step * 16 + 4 * ld_g >= n_in;    // channels past the last
+        const bool there = row >= 0 && !past;
+        const unsigned off = __umul24((unsigned)row, row_bytes) + 16u * (unsigned)ld_g;
+        areg[q][s] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, there ? off : 0x80000000u, step * 64, 0));
+        if (PRE && there) aok |= 1u << (2 * q + s);
+      }
+    }
+    if (PRE) {
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        const int ch = (PAIR ? 0 : (c.sl * 2 + s) * 16) + 4 * ld_g;
+        psc[s] = *reinterpret_cast<const v4f *>(pre_sc + ch);
+        psh[s] = *reinterpret_cast<const v4f *>(pre_sh + ch);
+      }
+    }
+  };
+  auto issue_weights = [&](const Cursor &c) {
+    if constexpr (PAIR) {  // half an operand from either tap
+      const v4s *src = reinterpret_cast<const v4s *>(wp) + lane;
+      const v4s *s0 = src + ((int64_t)c.k * (3 * ncb) + cb0) * 64, *s1 = src + ((int64_t)(c.k2 >= 0 ? c.k2 : c.k) * (3 * ncb) + cb0) * 64;
+#pragma unroll
+      for (int b = 0; b < NCB; b++)
+#pragma unroll
+        for (int p = 0; p < 3; p++)
+          breg[b][p] = __builtin_shufflevector(s0[(p * ncb + b) * 64], s1[(p * ncb + b) * 64], 0, 1, 2, 3, 4, 5, 6, 7);
+    } else {
+      const v8s *src = wp + (((int64_t)c.k * n_slab + c.sl) * (3 * ncb) + cb0) * 64 + lane;
+#pragma unroll
+      for (int b = 0; b < NCB; b++)
+#pragma unroll
+        for (int p = 0; p < 3; p++) breg[b][p] = src[(p * ncb + b) * 64];
+    }
+  };
+  start(at);
+  rows = at;
+  idx = at;
+  if (total > 0) {
+    issue_indices(idx);
+    issue_rows(rows);
+    issue_weights(rows);
+    advance(idx);
+    issue_indices(idx);
+  }
+  for (int it = 0; it < total; it++) {
+#pragma unroll
+    for (int q = 0; q < GW; q++)
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        v4f v = pre_act<PRE>(areg[q][s], psc[s], psh[s], pre_leak);
+        if (PRE && !((aok >> (2 * q + s)) & 1u)) v = (v4f){0.f, 0.f, 0.f, 0.f};
+        turn[wave][q][s][wr_slot] = v;
+      }
+    advance(rows);
+    issue_rows(rows);
+    advance(idx);
+    issue_indices(idx);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < GW; q++) {
+      if (!((gm[q] >> at.k) & 1u) && (!PAIR || at.k2 < 0 || !((gm[q] >> at.k2) & 1u))) continue;  // uniform over the wavefront
+      const Split8 a = split8(turn[wave][q][0][rd_slot], turn[wave][q][1][rd_slot]);
+      v4f t[NCB];
+#pragma unroll
+      for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.h, breg[c][2], (v4f){0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.l, breg[c][0], t[c]);
+#pragma unroll
+      for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.m, breg[c][1], t[c]);
+#pragma unroll
+      for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.h, breg[c][1], t[c]);
+#pragma unroll
+      for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.m, breg[c][0], t[c]);
+#pragma unroll
+      for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.h, breg[c][0], t[c]);
+#pragma unroll
+      for (int c = 0; c < NCB; c++) acc[q][c] += t[c];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    advance(at);
+    issue_weights(rows);
+  }
+
+  float probe = 0.f;  // stays zero while every sum is finite
+#pragma unroll
+  for (int q = 0; q < GW; q++)
+#pragma unroll
+    for (int c = 0; c < NCB; c++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) probe = __builtin_fmaf(acc[q][c][r], 0.f, probe);
+  if (__ballot(probe != 0.f) != 0ull) {
+    // infinities, NaNs or values too large for pieces: again on the fp32 matrix instructions (see k_conv_split)
+#pragma unroll
+    for (int q = 0; q < GW; q++)
+#pragma unroll
+      for (int c = 0; c < NCB; c++) acc[q][c] = (v4f){0.f, 0.f, 0.f, 0.f};
+    start(at);
+#pragma unroll 1
+    for (int it = 0; it < (PAIR ? 2 * total : total); it++) {
+      const int k = PAIR && (it & 1) ? at.k2 : at.k, sl = at.sl;
+#pragma unroll
+      for (int c = 0; c < NCB; c++) {
+        if (PAIR && k < 0) break;  // uniform
+        float w[8];
+        if constexpr (PAIR) {
+          const v4s *src = reinterpret_cast<const v4s *>(wp) + ((int64_t)k * (3 * ncb) + cb0 + c) * 64 + lane;
+          const v4s wh = src[0], wm = src[ncb * 64], wl = src[2 * ncb * 64];
+#pragma unroll
+          for (int e = 0; e < 4; e++) w[e] = join_weight(wh[e], wm[e], wl[e]);
+        } else {
+          const v8s *src = wp + (((int64_t)k * n_slab + sl) * (3 * ncb) + cb0 + c) * 64 + lane;
+          const v8s wh = src[0], wm = src[ncb * 64], wl = src[2 * ncb * 64];
+#pragma unroll
+          for (int e = 0; e < 8; e++) w[e] = join_weight(wh[e], wm[e], wl[e]);
+        }
+#pragma unroll
+        for (int q = 0; q < GW; q++) {
+          if (!((gm[q] >> k) & 1u)) continue;  // uniform over the wavefront
+          const int *src_j = nbr + (int64_t)k * npad + pos0;
+          const int row = 16 * q + r16 <= last ? src_j[16 * q + r16] : -1;
+          v4f t = (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int s = 0; s < (PAIR ? 1 : 2); s++) {
+            const int ch = (sl * 2 + s) * 16 + 4 * g;
+            const bool there = row >= 0 && ch < n_in;  // n_in is a multiple of four
+            v4f x = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
+                                                rsrc, there ? (unsigned)row * row_bytes + 4u * (unsigned)ch : 0x80000000u, 0, 0));
+            if (PRE) {
+              x = pre_act<PRE>(x, *reinterpret_cast<const v4f *>(pre_sc + ch), *reinterpret_cast<const v4f *>(pre_sh + ch), pre_leak);
+              if (!there) x = (v4f){0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) t = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], w[4 * s + e], t, 0, 0, 0);
+          }
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const int p = 16 * q + 4 * g + r;
+            acc[q][c][r] += p <= last && src_j[min(p, last)] >= 0 ? t[r] : 0.f;
+          }
+        }
+      }
+      if (!PAIR || (it & 1)) advance(at);
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < GW; q++)
+#pragma unroll
+      for (int c = 0; c < NCB; c++) acc[q][c] *= SPLIT_UNSCALE;
+  }
+
+  // acc[q][c][r] = result for position pos0 + 16*q + 4*g + r, column 16*c + r16
+  constexpr int R = DEAL == 1 ? 4 : 1;  // rows per lane and granule that this wavefront stores
+  int r0 = 0;
+  if constexpr (DEAL > 1) {
+    float *sums = reinterpret_cast<float *>(turn);  // [wave][q][c][r][lane]
+#pragma unroll
+    for (int q = 0; q < GW; q++)
+#pragma unroll
+      for (int c = 0; c < NCB; c++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) sums[(((wave * GW + q) * PART + c) * 4 + r) * 64 + lane] = acc[q][c][r];
+    __syncthreads();
+    if (wave >= 4) return;
+    r0 = wave;
+#pragma unroll
+    for (int q = 0; q < GW; q++)
+#pragma unroll
+      for (int c = 0; c < NCB; c++) {
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < DEAL; w++) v += sums[(((w * GW + q) * PART + c) * 4 + wave) * 64 + lane];
+        acc[q][c][0] = v;
+      }
+  }
+  const bool post = epi.sc != nullptr;
+  float bv[NCB], es[NCB], eh[NCB];
+#pragma unroll
+  for (int c = 0; c < NCB; c++) {
+    const int col = 16 * (cb0 + c) + r16;
+    bv[c] = (epi.bias != nullptr && col < n_out) ? epi.bias[col] : 0.0f;
+    es[c] = (post && col < n_out) ? epi.sc[col] : 1.0f;
+    eh[c] = (post && col < n_out) ? epi.sh[col] : 0.0f;
+  }
+  const int64_t stride = epi.out_stride ? epi.out_stride : n_out;
+  int orow[GW][R];
+#pragma unroll
+  for (int q = 0; q < GW; q++)
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int p = min(16 * q + 4 * g + r + r0, last);
+      orow[q][r] = rowmap ? rowmap[pos0 + p] : (int)pos0 + p;
+    }
+#pragma unroll
+  for (int q = 0; q < GW; q++) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      if (16 * q + 4 * g + r + r0 > last) continue;
+      float *o = out + orow[q][r] * stride + 16 * cb0 + r16;
+#pragma unroll
+      for (int c = 0; c < NCB; c++) {
+        if (16 * (cb0 + c) + r16 >= n_out) continue;
+        float v = acc[q][c][r] + bv[c];
+        if (epi.out2) epi_second(epi, orow[q][r], 16 * (cb0 + c) + r16, v);
+        if (post) v = epi_act(v, es[c], eh[c], epi.leak);
+        o[16 * c] = v;
+      }
+    }
+  }
+}
+
+template <int NCB, int GW, int DEAL, int OCC, bool PAIR, bool PRE>
+static void launch_wave(Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi, int n_in,
+                        int n_out, PreArgs pre, hipStream_t s) {
+  const int n_slab = (int)ceil_div(n_in, 32);
+  const int groups = (int)ceil_div(n_out, 16 * NCB), ncb = groups * NCB;
+  const float *wpack = split_weights(m, t.K, w, n_in, n_out, ncb, PAIR, s);
+  const int n_tiles = (int)ceil_div(t.n, (DEAL > 1 ? 1 : 4) * GW * 16);
+  const int tiles_per_xcd = t.spread ? 0 : (int)ceil_div(n_tiles, 8);
+  note_kernel(m, "split wave", {{"ncb", NCB}, {"gw", GW}, {"deal", DEAL}, {"pair", PAIR}, {"pre", PRE}, {"split", 1}});
+  k_conv_wave<NCB, GW, DEAL, OCC, PAIR, PRE><<<dim3((unsigned)(tiles_per_xcd ? tiles_per_xcd * 8 : n_tiles), groups), 64 * std::max(4, DEAL), 0, s>>>(
+      t.nbr.p, t.rowmap_ptr(), t.gmask.p, t.n, t.npad, in, out, reinterpret_cast<const v8s *>(wpack), epi, n_in, n_out, n_slab,
+      ncb, tiles_per_xcd, n_tiles, pre.sc, pre.sh, pre.leak, (unsigned)(m.cur_in_rows * n_in * 4));
+  LAUNCH_CHECK();
+}
+
+template <int NCB, bool PAIR, bool PRE>
+static void dispatch_wave(Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi, int n_in,
+                          int n_out, PreArgs pre, hipStream_t s) {
+  // the batch norm's coefficients take the registers of one wavefront per SIMD
+  constexpr int O1 = PRE && NCB == 2 ? 5 : 6, O2 = PRE && NCB == 2 ? 4 : 5;
+  const bool one_rule = t.few_tap.p || t.K == 1;
+  // The longer a wavefront's chain, the longer dealing it out pays; many granules per wavefront save weights' traffic where there
+  // are enough of them (us: one granule dealt out / two dealt out / two / four):
+  //   27 taps 32 -> 32: 8 k sites 7.6 / 9.8 / 25 / 41, 24 k 12.2 / 12.7 / 26 / 42, 100 k 36 / 31 / 36 / 47, 200 k 64 / 52 / 53 / 57,
+  //     400 k 120 / 99 / 86 / 90, 1 M 360 / 274 / 230 / 213
+  //   9 taps (2-D) 16 -> 16: 12 k 4.7 / 5.4 / 8.4 / 13, 50 k 9.4 / 8.5 / 9.4 / 14, 200 k 31 / 24 / 22 / 26
+  //   one rule per position 24 -> 16: 20 k 4.4 / 4.5 / 5.4 / 7.7, 60 k 7.3 / 6.6 / 6.2 / 8.5, 1 M 81 / 55 / 33 / 38
+#define WAVE(G, D, O) launch_wave<NCB, G, D, O, PAIR, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s)
+  if (t.n < 24000) WAVE(1, 4, O1);
+  else if (t.n < (one_rule ? 24000 : t.K <= 9 ? 100000 : 300000)) WAVE(2, 4, O2);
+  else if (t.K <= 9 || t.n < 600000) WAVE(2, 1, O2);
+  else WAVE(4, 1, 3);
+#undef WAVE
+}
+bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in, int n_out) {
+  if (m.bf16 || m.fixed_scratch || n_out > 32 || t.K > 32 || !t.gmask.p) return false;
+  if (n_in <= 4 || n_in % 4 || (uintptr_t)in % 16 || n_in * 4 >= (1 << 24)) return false;
+  // k_conv_resident keeps 20-32 -> up to 16 planes on small levels of few taps and on large ones
+  if (n_in > 16 && n_in <= 32 && n_out <= 16 && (t.K <= 9 ? t.n < 16000 : t.n >= (n_in > 24 ? 200000 : 300000))) return false;
+  // k_conv_split: wide inputs of one rule per position, and on the smallest levels chains that it cuts into more parts (500 sites
+  // 64 -> 32 11.9 there, 11.1 here, 128 -> 32 13.7 / 18.5)
+  if ((t.few_tap.p && n_in > 64) || (t.K > 9 && t.n < 1000 && n_in > 32)) return false;
+  // k_deconv_few, all weights in LDS (there / here): transposed 32 -> 32 onto 250 k sites 18.0 / 17.4, 500 k 28.0 / 28.5, 1 M 47 / 49, but
+  // 64 -> 32 1 M 71 / 64, 60 k 14.4 / 9.6; 1x1 32 -> 32 60 k rows 8.9 / 7.1, 120 k 10.1 / 10.2, 1 M 45 / 58; 64 -> 32 120 k 14.5 / 13.2,
+  // 250 k 22.3 / 22.1, 1 M 82 / 93
+  if (t.few_tap.p && n_in == 32 && t.n >= 400000) return false;
+  if (t.identity_few && (n_in == 32 || n_in == 64) && t.n >= (n_in == 32 ? 100000 : 200000)) return false;
+  return in_rows > 0 && in_rows < (1 << 24) && in_rows * n_in * 4 < ((int64_t)1 << 31);
+}
+bool conv_wave_dispatch(bool pre_fused, Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi,
+                        int n_in, int n_out, PreArgs pre, hipStream_t s) {
+  if (!conv_wave_serves(m, t, in, m.cur_in_rows, n_in, n_out)) return false;
+  auto run = [&](auto ncb, auto pair) {
+    if (pre_fused) dispatch_wave<decltype(ncb)::value, decltype(pair)::value, true>(m, t, in, out, w, epi, n_in, n_out, pre, s);
+    else dispatch_wave<decltype(ncb)::value, decltype(pair)::value, false>(m, t, in, out, w, epi, n_in, n_out, pre, s);
+  };
+  auto by_pair = [&](auto ncb) { n_in <= 16 ? run(ncb, std::true_type()) : run(ncb, std::false_type()); };
+  n_out <= 16 ? by_pair(std::integral_constant<int, 1>()) : by_pair(std::integral_constant<int, 2>());
+  return true;
+}
+
+}  // namespace scn

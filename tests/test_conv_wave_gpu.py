@@ -1,0 +1,93 @@
+"""The split-operand kernel of up to 32 output planes in which a wavefront owns its rows (k_conv_wave): every form of its
+dispatch, at sizes around granules, workgroups and the ends of its ranges, against sums in 64 bits over the exported rules.
+
+Tolerance, as for the other split-operand kernels: sums of a chain of six products of up to 32 channels are added in fp32, one per
+(tap, 32 channels), two taps of up to 16 channels together, so that one result is off by at most (m + 4) 2^-24 of the sum of the
+products' magnitudes, m the number of those additions; four wavefronts that share a row's taps add three."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind,n,cin,cout", [
+    # one wavefront, a ragged granule, a granule, one more, a workgroup and one more
+    ("subm", 1, 16, 16), ("subm", 15, 8, 8), ("subm", 16, 32, 24), ("subm", 17, 12, 20), ("subm", 63, 16, 32), ("subm", 65, 20, 17),
+    # taps dealt over four wavefronts of one granule, of two, and not dealt
+    ("subm", 1003, 96, 32), ("subm", 23999, 16, 8), ("subm", 24000, 32, 32), ("subm", 24001, 28, 12), ("subm", 100003, 64, 24),
+    ("subm", 299999, 16, 16), ("subm", 300001, 24, 20), ("subm", 600001, 12, 28),
+    # eight taps and one rule per position; one tap
+    ("down", 301, 16, 32), ("down", 20011, 32, 32), ("down", 120007, 48, 16), ("up", 77, 64, 32), ("up", 20011, 48, 32),
+    ("up", 25001, 16, 8), ("up", 150001, 64, 16), ("nin", 5, 16, 16), ("nin", 5003, 96, 32), ("nin", 25001, 24, 16)])
+@pytest.mark.parametrize("form", ["plain", "normalised"])
+def test_rows_owned_by_a_wavefront(kind, n, cin, cout, form):
+    import torch
+    from test_conv_split_gpu import _table
+    conv, rules, rows_in, rows_out, md = _table(kind, n, 8100 + n % 89)
+    g = torch.Generator().manual_seed(n + cout)
+
+    def normal(*shape):
+        return torch.randn(*shape, generator=g).cuda()
+
+    def bn(c):
+        return normal(c) * 0.3, torch.rand(c, generator=g).cuda() + 0.5, torch.rand(c, generator=g).cuda() + 0.5, normal(c) * 0.3, 1e-4, 0.2
+
+    def normalise(y, p):
+        mean, var, gamma, beta, eps, leak = p
+        y = (y - mean.double()) * (gamma.double() / torch.sqrt(var.double() + eps)) + beta.double()
+        return torch.where(y > 0, y, leak * y)
+    x, w, bias = normal(rows_in, cin), normal(len(rules), 1, cin, cout) * 0.1, normal(cout)
+    x[:, cin // 2] *= 1e-30  # small numbers keep their bits
+    front, post = (bn(cin), bn(cout)) if form == "normalised" and kind != "nin" else (None, None)
+    f = x.double() if front is None else normalise(x.double(), front)
+    want = bias.double().expand(rows_out, -1).clone()
+    mag = want.abs()
+    for k, r in enumerate(rules):
+        r = torch.as_tensor(r).cuda().long()
+        want.index_add_(0, r[:, 1], f[r[:, 0]] @ w[k, 0].double())
+        mag.index_add_(0, r[:, 1], f[r[:, 0]].abs() @ w[k, 0].double().abs())
+    additions = len(rules) * -(-cin // 32) + 3 + 1
+    if front is None:
+        got = conv(x, w, bias)
+        assert ((got.double() - want).abs() <= (additions + 4) * 2.0 ** -24 * mag).all()
+    else:  # the folded scale and shift round a normalised value by 4 2^-24 of its terms, here and behind the sum
+        wide = torch.full((rows_out, cout + 8), 7.0).cuda()
+        conv(x, w, bias, bn=front, post=post, out=wide[:, 4:4 + cout])
+        assert (wide[:, :4] == 7.0).all() and (wide[:, 4 + cout:] == 7.0).all()
+        terms = x.double().abs() + front[0].double().abs()
+        sc = front[2].double() / torch.sqrt(front[1].double() + front[4])
+        big = bias.double().abs().expand(rows_out, -1).clone()
+        for k, r in enumerate(rules):
+            r = torch.as_tensor(r).cuda().long()
+            big.index_add_(0, r[:, 1], (terms[r[:, 0]] * sc + front[3].double().abs()) @ w[k, 0].double().abs())
+        psc = post[2].double() / torch.sqrt(post[1].double() + post[4])
+        bound = ((additions + 4) * mag + 4 * big) * psc + 4 * ((want.abs() + post[0].double().abs()) * psc + post[3].double().abs())
+        assert ((wide[:, 4:4 + cout].double() - normalise(want, post)).abs() <= 2.0 ** -24 * bound).all()
+    kernel = md._L.scn_md_last_conv_kernel(md._h).decode()
+    assert "wave" in kernel, kernel
+
+
+@pytest.mark.parametrize("kind,n,cin,cout", [("subm", 3001, 16, 16), ("subm", 3001, 32, 24), ("subm", 60001, 64, 16),
+                                             ("subm", 610001, 16, 32), ("up", 30011, 48, 32), ("down", 3001, 12, 20)])
+def test_values_that_are_not_finite(kind, n, cin, cout):
+    """Exactly the outputs whose rules read an infinity or a NaN are not finite, rows and weights alike."""
+    import torch
+    from test_conv_split_gpu import _table, _close_where_finite
+    conv, rules, rows_in, rows_out, md = _table(kind, n, 8200 + n % 89)
+    g = torch.Generator().manual_seed(n + cout)
+    w = torch.randn(len(rules), 1, cin, cout, generator=g).cuda() * 0.1
+    for case in ("rows", "weights", "overflow"):
+        x, v = torch.randn(rows_in, cin, generator=g).cuda(), w.clone()
+        if case == "rows":
+            x[5, 3], x[rows_in // 2, 7], x[rows_in - 1, 3] = float("inf"), float("nan"), float("-inf")
+        elif case == "weights":
+            v[len(rules) // 2, 0, 2, 4], v[len(rules) - 1, 0, 1, 6] = float("inf"), float("nan")
+        else:
+            v *= 1e-3
+            x[::5, 0], v[len(rules) // 2, 0, 0] = 1e38, 16.0
+        want = torch.zeros(rows_out, cout, dtype=torch.float64, device="cuda")
+        mag = want.clone()
+        for k, r in enumerate(rules):
+            r = torch.as_tensor(r).cuda().long()
+            want.index_add_(0, r[:, 1], x[r[:, 0]].double() @ v[k, 0].double())
+            mag.index_add_(0, r[:, 1], x[r[:, 0]].double().abs() @ v[k, 0].double().abs())
+        _close_where_finite(conv(x, v, torch.zeros(cout).cuda()), want, mag, len(rules) * cin + 16)
