@@ -116,6 +116,9 @@ int scn_md_input_batch(scn_metadata *md, const int64_t *spatial, const int64_t *
 int scn_md_generate_rulebooks(scn_metadata *md, int size, void *stream);
 /* Rule header [mode, maxActive, nInputRows, nOutputRows] (Metadata/IOLayersRules.h:10-15). */
 int scn_md_input_rules_header(scn_metadata *md, int32_t hdr[4]);
+/* Points of the input layer; samples and points per sample (0, 0 unless it was a batch-by-length one).  Does not wait
+ * for the device, which the headers do for the longest run of points on one site. */
+int scn_md_input_points(scn_metadata *md, int64_t n[3]);
 /* Rule rows, device int32 [nOutputRows, 1+maxActive] = [count, input indices.., 0 pad]. */
 int scn_md_input_rules(scn_metadata *md, int32_t *rows, void *stream);
 /* Metadata::blLayer (Metadata/Metadata.cpp:426-436, Metadata/IOLayersRules.h:132-286), the rule

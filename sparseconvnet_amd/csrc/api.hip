@@ -296,73 +296,96 @@ void pinned_release(void *p, size_t bytes) {
 // A handle that is destroyed or cleared may still owe the caller the multiply-add counts of
 // convolutions that did not ask for theirs (their rule counts are on the device).  Waiting for
 // them there would stall the host on the whole forward pass each time a scene's metadata dies:
-// instead the counts are copied to pinned memory behind the work already enqueued, an event
-// marks the copy, and scn_take_released_macs folds whatever has been left behind.
+// instead the counts are added up into pinned memory behind the work already enqueued, an event
+// marks the end of that, and scn_take_released_macs folds whatever has been left behind.
 namespace {
-// The rule counts of up to 48 tables copied into one staging array by one launch: block b copies
-// table b's words.  dst is pinned host memory (hipHostMalloc: device-accessible), so that a
-// handle with forty tables costs the stream one short kernel instead of forty copies.
+// The rules of up to 48 tables, one launch: block b adds up table b's words.  dst is pinned host memory
+// (hipHostMalloc: device-accessible) in which the host has put -1, so that it can see a sum arrive without
+// a call into the runtime.
 struct CountJobs {
   const long long *src[48];
-  int off[48], words[48];
+  int words[48];
 };
-__global__ void k_gather_counts(CountJobs j, long long *dst) {
-  const int b = blockIdx.x;
-  for (int i = threadIdx.x; i < j.words[b]; i += blockDim.x) dst[j.off[b] + i] = j.src[b][i];
+__global__ __launch_bounds__(256) void k_sum_counts(CountJobs j, long long *dst) {
+  const int b = blockIdx.x, lane = threadIdx.x & 63;
+  __shared__ long long part[4];
+  long long sum = 0;
+  for (int i = threadIdx.x; i < j.words[b]; i += 256) sum += j.src[b][i];
+#pragma unroll
+  for (int o = 32; o; o >>= 1) sum += __shfl_xor(sum, o, 64);
+  if (lane == 0) part[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(dst + b, part[0] + part[1] + part[2] + part[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 struct ReleasedMacs {
   hipEvent_t ev = nullptr;
-  long long *stage = nullptr;
+  long long *stage = nullptr;  // rules of table i, -1 until they are known
   size_t stage_bytes = 0;
-  struct Item {
-    size_t off;
-    int K, slots;
-    double per_rule;
-  };
-  std::vector<Item> items;
+  std::vector<double> per_rule;
 };
 std::mutex g_released_mutex;
 std::vector<ReleasedMacs> g_released;
 double g_released_settled = 0;
 
+// Folds what the GPU is done with, so that a program that never asks for its counts does not gather pinned
+// memory, and the next handle to die finds a block.  The caller holds g_released_mutex.
+void settle_released() {
+  size_t kept = 0;
+  for (ReleasedMacs &r : g_released) {
+    double sum = 0;
+    bool done = true;
+    for (size_t i = 0; i < r.per_rule.size() && done; i++) {
+      const long long rules = __atomic_load_n(r.stage + i, __ATOMIC_RELAXED);
+      done = rules >= 0;
+      sum += (double)rules * r.per_rule[i];
+    }
+    if (!done) {
+      if (&g_released[kept] != &r) g_released[kept] = std::move(r);
+      kept++;
+      continue;
+    }
+    g_released_settled += sum;
+    (void)hipEventDestroy(r.ev);
+    pinned_release(r.stage, r.stage_bytes);
+  }
+  g_released.resize(kept);
+}
+
 void release_macs(Metadata &m) {
   double settled = m.macs_settled;
   m.macs_settled = 0;
+  {
+    std::lock_guard<std::mutex> lock(g_released_mutex);
+    settle_released();
+  }
   ReleasedMacs r;
-  size_t words = 0;
+  std::vector<Counts *> tables;  // each once, however many convolutions ran over it
   for (auto &pm : m.pending_macs) {
     Counts &c = *pm.first;
-    if (c.ready || !c.K || !c.dev.p)
+    if (c.ready || !c.K || !c.dev.p) {
       settled += (c.ready ? (double)c.total() : 0.0) * pm.second;
-    else
-      words += (size_t)c.K * c.slots;
+      continue;
+    }
+    size_t i = 0;
+    while (i < tables.size() && tables[i] != &c) i++;
+    if (i == tables.size()) tables.push_back(&c), r.per_rule.push_back(0.0);
+    r.per_rule[i] += pm.second;
   }
-  if (words) {
+  if (!tables.empty()) {
     try {
       // the stream the convolutions ran on; the rule counts are final before anything on it runs
       hipStream_t s = m.consumer_known ? m.consumer : nullptr;
       if (m.last_ready) HIP_CHECK(hipStreamWaitEvent(s, m.last_ready, 0));
-      r.stage_bytes = round_up((int64_t)(words * sizeof(long long)), 1 << 16);
+      r.stage_bytes = round_up((int64_t)(tables.size() * sizeof(long long)), 4096);
       r.stage = static_cast<long long *>(pinned_acquire(r.stage_bytes));
-      size_t off = 0;
-      CountJobs jobs{};
-      int n_jobs = 0;
-      auto flush = [&] {
-        if (!n_jobs) return;
-        k_gather_counts<<<dim3((unsigned)n_jobs), 64, 0, s>>>(jobs, r.stage);
+      for (size_t i = 0; i < tables.size(); i++) __atomic_store_n(r.stage + i, -1ll, __ATOMIC_RELAXED);
+      for (size_t i0 = 0; i0 < tables.size(); i0 += 48) {
+        CountJobs jobs{};
+        const int n = (int)std::min<size_t>(48, tables.size() - i0);
+        for (int i = 0; i < n; i++) jobs.src[i] = tables[i0 + i]->dev.p, jobs.words[i] = tables[i0 + i]->K * tables[i0 + i]->slots;
+        k_sum_counts<<<dim3((unsigned)n), 256, 0, s>>>(jobs, r.stage + i0);
         LAUNCH_CHECK();
-        n_jobs = 0;
-      };
-      for (auto &pm : m.pending_macs) {
-        Counts &c = *pm.first;
-        if (c.ready || !c.K || !c.dev.p) continue;
-        const size_t w = (size_t)c.K * c.slots;
-        jobs.src[n_jobs] = c.dev.p, jobs.off[n_jobs] = (int)off, jobs.words[n_jobs] = (int)w;
-        if (++n_jobs == 48) flush();
-        r.items.push_back({off, c.K, c.slots, pm.second});
-        off += w;
       }
-      flush();
       HIP_CHECK(hipEventCreateWithFlags(&r.ev, hipEventDisableTiming));
       HIP_CHECK(hipEventRecord(r.ev, s));
     } catch (...) {  // a lost device: the counts are not worth an error in a destructor
@@ -391,11 +414,7 @@ double take_released_macs() {
   }
   for (ReleasedMacs &r : todo) {
     if (hipEventSynchronize(r.ev) == hipSuccess) {
-      for (const auto &it : r.items) {
-        long long rules = 0;
-        for (size_t i = 0; i < (size_t)it.K * it.slots; i++) rules += r.stage[it.off + i];
-        total += (double)rules * it.per_rule;
-      }
+      for (size_t i = 0; i < r.per_rule.size(); i++) total += (double)r.stage[i] * r.per_rule[i];
     } else {
       (void)hipGetLastError();
     }
@@ -626,6 +645,13 @@ int scn_md_input_rules_header(scn_metadata *h, int32_t hdr[4]) {
     hdr[1] = input_max_active(m);
     hdr[2] = (int32_t)m.input.n_in;
     hdr[3] = (int32_t)m.input.n_out;
+  });
+}
+int scn_md_input_points(scn_metadata *h, int64_t n[3]) {
+  return guarded([&] {
+    Metadata &m = md(h);
+    if (m.input.mode < 0) throw Error("input layer rules have not been built");
+    n[0] = m.input.n_in, n[1] = m.input.bl_batch, n[2] = m.input.bl_length;
   });
 }
 int scn_md_bl_input_layer(scn_metadata *h, const int64_t *spatial, const int64_t *coords, int64_t batch,

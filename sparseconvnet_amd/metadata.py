@@ -179,11 +179,17 @@ class Metadata:
         """3^d submanifold and 3^d / stride-2 rulebooks of every level, ahead of their use."""
         _lib.check(self._L.scn_md_generate_rulebooks(self._h, 3, _stream()))
 
+    def _points(self, bl=False):
+        """Points of the input layer, samples, points per sample."""
+        n = (C.c_int64 * 3)()
+        _lib.check(self._L.scn_md_input_points(self._h, n))
+        if bl and n[2] == 0:
+            raise _lib.ScnError("batch-by-length input rules have not been built")
+        return n[0], n[1], n[2]
+
     def outputLayer(self, features):
         features = _features(features, "features")
-        hdr = (C.c_int32 * 4)()
-        _lib.check(self._L.scn_md_input_rules_header(self._h, hdr))
-        out = torch.empty((hdr[2], features.size(1)), dtype=torch.float32, device=features.device)
+        out = torch.empty((self._points()[0], features.size(1)), dtype=torch.float32, device=features.device)
         _lib.check(self._L.scn_output_layer_fwd(self._h, _ptr(features), _ptr(out), features.size(1), _stream()))
         return out
 
@@ -204,9 +210,8 @@ class Metadata:
     def blOutputLayer(self, features):
         """[nActive, planes] -> [batch, length, planes] of the batch-by-length input layer."""
         features = _features(features, "features")
-        hdr = (C.c_int32 * 5)()
-        _lib.check(self._L.scn_md_bl_rules_header(self._h, hdr))
-        out = torch.empty((hdr[2], hdr[3], features.size(1)), dtype=torch.float32, device=features.device)
+        _, batch, length = self._points(bl=True)
+        out = torch.empty((batch, length, features.size(1)), dtype=torch.float32, device=features.device)
         _lib.check(self._L.scn_output_layer_fwd(self._h, _ptr(features), _ptr(out), features.size(1), _stream()))
         return out
 
@@ -468,14 +473,8 @@ class Metadata:
         """d(features of the points) from d(features of the sites); bl: [batch, length, planes]."""
         grad_output = _features(grad_output, "grad_output")
         planes = grad_output.size(1)
-        if bl:
-            hdr = (C.c_int32 * 5)()
-            _lib.check(self._L.scn_md_bl_rules_header(self._h, hdr))
-            d_in = torch.empty((hdr[2], hdr[3], planes), dtype=torch.float32, device=grad_output.device)
-        else:
-            hdr = (C.c_int32 * 4)()
-            _lib.check(self._L.scn_md_input_rules_header(self._h, hdr))
-            d_in = torch.empty((hdr[2], planes), dtype=torch.float32, device=grad_output.device)
+        points, batch, length = self._points(bl)
+        d_in = torch.empty((batch, length, planes) if bl else (points, planes), dtype=torch.float32, device=grad_output.device)
         if d_in.numel():
             _lib.check(self._L.scn_input_layer_bwd(self._h, _ptr(d_in), _ptr(grad_output), planes, _stream()))
         return d_in
