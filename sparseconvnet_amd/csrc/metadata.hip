@@ -153,26 +153,18 @@ static void fill3(void *p0, uint32_t v0, int64_t n0, void *p1, uint32_t v1, int6
   LAUNCH_CHECK();
 }
 
-// Stable sort of (key, value) pairs by the low end_bit bits of the key.  From 32 k to 1.5 million pairs
-// this repository's own sort (sort.hip: three short launches per digit, measured 95-145 us for a
-// million pairs of 35 bits against the library's 175 us, 50-80 us against 100-150 us at 15 k to
-// 250 k pairs); above, the library's radix sort, whose tiles stage their pairs through LDS and
-// write long runs (measured faster from about two million pairs on).
+// Stable sort of (key, value) pairs by the low end_bit bits of the key.  Up to 1.5 million pairs
+// this repository's own sort (sort.hip); above, the library's radix sort, whose tiles stage their pairs through
+// LDS and write long runs (measured faster from about two million pairs on).
 using RadixAlways = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
                                                rocprim::default_config, 4096>;
 static void sort_pairs(Metadata &m, const unsigned long long *kin, unsigned long long *kout,
                        const int *vin, int *vout, int64_t n, hipStream_t s, int end_bit = 64) {
-  if ((n > 32768 && n <= 1500000) || n <= 4096) {  // up to 4096 pairs: one launch, one workgroup
+  if (n <= 1500000) {
     radix_sort_pairs(m, kin, kout, vin, vout, n, end_bit, s);
     return;
   }
   size_t bytes = 0;
-  if (n <= 32768) {  // rocPRIM's own choice at this size (a merge sort of a few passes) is the fastest measured
-    HIP_CHECK(rocprim::radix_sort_pairs(nullptr, bytes, kin, kout, vin, vout, (size_t)n, 0u, (unsigned)end_bit, s));
-    m.tmp.reserve(bytes + 16);
-    HIP_CHECK(rocprim::radix_sort_pairs(m.tmp.p, bytes, kin, kout, vin, vout, (size_t)n, 0u, (unsigned)end_bit, s));
-    return;
-  }
   HIP_CHECK(rocprim::radix_sort_pairs<RadixAlways>(nullptr, bytes, kin, kout, vin, vout, (size_t)n, 0u,
                                                    (unsigned)end_bit, s));
   m.tmp.reserve(bytes + 16);

@@ -16,8 +16,7 @@
 // ballot per digit bit, the first of them reads and bumps the wavefront's running count of that value in LDS
 // (only this wavefront touches its counts, so no barrier), which gives every pair its rank
 // inside the wavefront's quarter; a prefix over the four wavefronts' counts then orders the
-// quarters.  (Between four and thirty-two thousand pairs the library's merge sort is faster and the
-// callers use it; up to 4096 pairs k_rs_single sorts in one launch, see there.)
+// quarters.  (Up to 32 k pairs k_rs_colscan is left out, up to a few thousand k_rs_single sorts in one launch, see there.)
 // The input arrays are not written: passes alternate between the output arrays and scratch.
 // The number of pairs may live on the device only (n_dev): the launches are then sized for an
 // upper bound and tiles past the real end find nothing to do.
@@ -35,7 +34,7 @@ constexpr int RS_MAX_BITS = 10, RS_MAX_BINS = 1 << RS_MAX_BITS;  // widest digit
 // compute unit leaves most of the memory system idle (a million pairs: 9.3 -> 5 us per pass).
 template <int RS_ITEMS>
 __global__ __launch_bounds__(RS_THREADS *(RS_ITEMS >= 4 ? 4 : RS_ITEMS)) void k_rs_hist(
-    const u64 *__restrict__ keys, int64_t n, int shift, int bits, int tiles, int *__restrict__ hist,
+    const u64 *__restrict__ keys, int64_t n, int shift, int bits, int tiles, bool by_tile, int *__restrict__ hist,
     const int *__restrict__ n_dev) {
   constexpr int THREADS = RS_THREADS * (RS_ITEMS >= 4 ? 4 : RS_ITEMS), PER = RS_THREADS * RS_ITEMS / THREADS;
   __shared__ int h[RS_MAX_BINS];
@@ -52,7 +51,8 @@ __global__ __launch_bounds__(RS_THREADS *(RS_ITEMS >= 4 ? 4 : RS_ITEMS)) void k_
     if (i < n) atomicAdd(&h[(unsigned)(keys[i] >> shift) & mask], 1);
   }
   __syncthreads();
-  for (int d = threadIdx.x; d < bins; d += THREADS) hist[(size_t)d * tiles + blockIdx.x] = h[d];
+  for (int d = threadIdx.x; d < bins; d += THREADS)
+    hist[by_tile ? (size_t)blockIdx.x * bins + d : (size_t)d * tiles + blockIdx.x] = h[d];
 }
 
 // One workgroup (64 threads) per digit value: hist[d][*] becomes its exclusive prefix over tiles,
@@ -79,7 +79,9 @@ __global__ __launch_bounds__(64) void k_rs_colscan(int *__restrict__ hist, int t
   if (lane == 63) tot[blockIdx.x] = incl;
 }
 
-template <int RS_ITEMS>
+// FEW: there are few enough tiles for every workgroup to add up the counts of all of them itself (offs is the
+// histogram, tile by tile; tot is not read), and k_rs_colscan is not launched.
+template <int RS_ITEMS, bool FEW>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const u64 *__restrict__ kin, const int *__restrict__ vin,
                                                            u64 *__restrict__ kout, int *__restrict__ vout, int64_t n,
                                                            int shift, int bits, int tiles, const int *__restrict__ offs,
@@ -99,9 +101,34 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const u64 *__restrict
   const int d0 = threadIdx.x * per;
   // exclusive scan of the digit values' totals (thread t: values [t * per, (t + 1) * per)) + this tile's prefix
   {
-    int mine = 0;
-    for (int j = 0; j < per; j++)
-      if (d0 + j < bins) mine += tot[d0 + j];
+    int mine = 0, total[4] = {0, 0, 0, 0}, before[4] = {0, 0, 0, 0};
+    if (FEW) {
+      const int *h = offs + d0;
+      if (per == 4) {
+#pragma unroll 8
+        for (int t = 0; t < tiles; t++) {
+          const int4 c = *reinterpret_cast<const int4 *>(h + (size_t)t * bins);
+          const int cc[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+          for (int j = 0; j < 4; j++) total[j] += cc[j], before[j] += t < (int)blockIdx.x ? cc[j] : 0;
+        }
+      } else if (d0 < bins) {  // one or two values per thread
+        const int second = per - 1;
+#pragma unroll 8
+        for (int t = 0; t < tiles; t++) {
+          const int c0 = h[(size_t)t * bins], c1 = h[(size_t)t * bins + second];
+          total[0] += c0, before[0] += t < (int)blockIdx.x ? c0 : 0;
+          total[1] += c1, before[1] += t < (int)blockIdx.x ? c1 : 0;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        if (j < per && d0 + j < bins) total[j] = tot[d0 + j], before[j] = offs[(size_t)(d0 + j) * tiles + blockIdx.x];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (j < per && d0 + j < bins) mine += total[j];
     int incl = mine;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -116,10 +143,11 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const u64 *__restrict
     __syncthreads();
     int run = incl - mine;
     for (int w = 0; w < wave; w++) run += wsum[w];
-    for (int j = 0; j < per; j++)
-      if (d0 + j < bins) {
-        base[d0 + j] = run + offs[(size_t)(d0 + j) * tiles + blockIdx.x];
-        run += tot[d0 + j];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (j < per && d0 + j < bins) {
+        base[d0 + j] = run + before[j];
+        run += total[j];
       }
   }
   // this wavefront's quarter: pairs [q0, q0 + ITEMS * 64)
@@ -187,13 +215,13 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const u64 *__restrict
   }
 }
 
-// Up to RS1_MAX pairs: one workgroup takes them through every digit without leaving LDS
+// Up to RS1_MAX pairs (98 KB of them, 17 KB of counts): one workgroup takes them through every digit without leaving LDS
 // (sort_block.h), one launch instead of three per digit.
-constexpr int RS1_ITEMS = 4, RS1_MAX = RS1_THREADS * RS1_ITEMS;
+constexpr int RS1_MAX = RS1_THREADS * 8;
+template <int ITEMS>
 __global__ __launch_bounds__(RS1_THREADS) void k_rs_single(const u64 *__restrict__ kin, const int *__restrict__ vin,
                                                            u64 *__restrict__ kout, int *__restrict__ vout, int n,
                                                            int end_bit, int width, const int *__restrict__ n_dev) {
-  constexpr int ITEMS = RS1_ITEMS;
   if (n_dev) n = *n_dev;
   __shared__ BlockSort<ITEMS> sh;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -225,17 +253,23 @@ void radix_sort_pairs(Metadata &m, const u64 *kin, u64 *kout, const int *vin, in
   // as few digits as RS_MAX_BITS bits each allow, of equal width
   const int passes = (end_bit + RS_MAX_BITS - 1) / RS_MAX_BITS;
   const int width = (end_bit + passes - 1) / passes;
-  if (n <= RS1_MAX) {
+  // one workgroup instead of two launches per digit: 8000 pairs of 27 bits 31 us against 26 and five launches more, of 9 bits 14 against 9
+  if (n <= (end_bit <= RS_MAX_BITS ? 4096 : RS1_MAX)) {
     const int p1 = (end_bit + RS1_BITS - 1) / RS1_BITS;
-    k_rs_single<<<dim3(1), RS1_THREADS, 0, s>>>(kin, vin, kout, vout, (int)n, end_bit, (end_bit + p1 - 1) / p1, n_dev);
+    auto kern = n <= RS1_THREADS * 4 ? k_rs_single<4> : k_rs_single<8>;
+    kern<<<dim3(1), RS1_THREADS, 0, s>>>(kin, vin, kout, vout, (int)n, end_bit, (end_bit + p1 - 1) / p1, n_dev);
     LAUNCH_CHECK();
     return;
   }
   // Large inputs take tiles of 4096 pairs (longer runs per digit value in the scatter's stores: a
   // million pairs of 35 bits 145 -> 122 us, eight million 800 -> 490 us); below half a million pairs
   // there are too few of those to fill the chip and smaller tiles are faster, down to 512 pairs
-  // (30 bits: 88 000 pairs 64 -> 55 us, 15 000 pairs 60 -> 44 us, 150 000 pairs 72 -> 61 us with 1024).
-  const int items = n >= 500000 ? 16 : n >= 300000 ? 8 : n >= 120000 ? 4 : 2;
+  // (30 bits: 88 000 pairs 64 -> 55 us, 150 000 pairs 72 -> 61 us with 1024).
+  // Up to 32 k pairs (32 tiles) the scatter adds up the tiles' counts itself, two launches per digit: 12 k pairs of 9 / 27 bits
+  // 10.7 -> 9.2 / 32 -> 27 us, 16 k 11.1 -> 9.7 / 33 -> 28, 32 k the same time with a third fewer launches, 64 k 12.4 -> 14.5 / 37 -> 42.
+  // (The library's merge sort, which served 4 to 32 k pairs before, took 27 to 34 us and 6 to 9 launches whatever the bits.)
+  const bool few = n <= 32768;
+  const int items = n >= 500000 ? 16 : n >= 300000 ? 8 : n >= 120000 || (few && n > 20000) ? 4 : 2;
   const int tile = RS_THREADS * items;
   const int tiles = (int)ceil_div(n, tile);
   // scratch: a second pair of arrays (when there is more than one pass), the tile counts, the totals
@@ -259,24 +293,23 @@ void radix_sort_pairs(Metadata &m, const u64 *kin, u64 *kout, const int *vin, in
     u64 *kdst = to_out ? kout : ktmp;
     int *vdst = to_out ? vout : vtmp;
     const int shift = width * pass, bits = std::min(width, end_bit - shift);
-    switch (items) {
-#define RS_PASS(I)                                                                                                  \
-  case I:                                                                                                           \
-    k_rs_hist<I><<<dim3(tiles), RS_THREADS *(I >= 4 ? 4 : I), 0, s>>>(ksrc, n, shift, bits, tiles, hist, n_dev);    \
-    LAUNCH_CHECK();                                                                                                 \
-    k_rs_colscan<<<dim3(1 << bits), 64, 0, s>>>(hist, tiles, tot);                                                  \
-    LAUNCH_CHECK();                                                                                                 \
-    k_rs_scatter<I><<<dim3(tiles), RS_THREADS, 0, s>>>(ksrc, vsrc, kdst, vdst, n, shift, bits, tiles, hist, tot, n_dev); \
-    LAUNCH_CHECK();                                                                                                 \
-    break;
-      RS_PASS(16)
-      RS_PASS(8)
-      RS_PASS(4)
-      RS_PASS(2)
-#undef RS_PASS
-    default:
-      throw Error("sort: internal tile size");
-    }
+    auto run = [&](auto per_thread, auto by_tile) {
+      constexpr int I = decltype(per_thread)::value;
+      constexpr bool FEW = decltype(by_tile)::value;
+      k_rs_hist<I><<<dim3(tiles), RS_THREADS *(I >= 4 ? 4 : I), 0, s>>>(ksrc, n, shift, bits, tiles, FEW, hist, n_dev);
+      LAUNCH_CHECK();
+      if (!FEW) {
+        k_rs_colscan<<<dim3(1 << bits), 64, 0, s>>>(hist, tiles, tot);
+        LAUNCH_CHECK();
+      }
+      k_rs_scatter<I, FEW><<<dim3(tiles), RS_THREADS, 0, s>>>(ksrc, vsrc, kdst, vdst, n, shift, bits, tiles, hist, tot, n_dev);
+      LAUNCH_CHECK();
+    };
+    typedef std::integral_constant<bool, true> Few;
+    typedef std::integral_constant<bool, false> Many;
+    if (few) items == 2 ? run(std::integral_constant<int, 2>(), Few()) : run(std::integral_constant<int, 4>(), Few());
+    else if (items >= 8) items == 16 ? run(std::integral_constant<int, 16>(), Many()) : run(std::integral_constant<int, 8>(), Many());
+    else items == 4 ? run(std::integral_constant<int, 4>(), Many()) : run(std::integral_constant<int, 2>(), Many());
     ksrc = kdst;
     vsrc = vdst;
   }
