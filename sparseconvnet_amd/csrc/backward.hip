@@ -1044,7 +1044,7 @@ static void input_gradient(Metadata &m, const Table &t, const float *d_out, int6
   // rule per position go to another kernel first, more than 256 planes run as ranges of copied columns, and
   // many taps may not fit its tile set-up.)
   if (groups == 1 && n_in <= 256 &&
-      (conv_wave_serves(m, t, d_out, d_out_rows, n_out, n_in) ||
+      (conv_wave_serves(m, t, d_out, d_out_rows, n_out, n_in, true) ||
        (t.K <= 64 && !t.few_tap.p && !t.identity_few && conv_split_serves(m, t, d_out, d_out_rows, n_out, n_in)))) {
     m.pack_transposed = w;
     m.pack_mirror = mirror;

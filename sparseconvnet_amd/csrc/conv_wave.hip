@@ -359,7 +359,11 @@ static void dispatch_wave(Metadata &m, const Table &t, const float *in, float *o
   else WAVE(4, 1, 3);
 #undef WAVE
 }
-bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in, int n_out) {
+bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in, int n_out, bool gradient) {
+  // Forward sums over nine taps (the 3 x 3 filters of 2-D networks) stay where they were, k_conv_resident and k_conv_split: values on
+  // the edge of a ReLU change sides with any other rounding, and a 2-D network of a few thousand sites has so few that a training
+  // step's gradients differ by up to 3.5e-3 then.  Its time is the host's, so that it would not run faster either (1.21 / 1.26 ms).
+  if (t.K == 9 && !gradient) return false;
   if (m.bf16 || m.fixed_scratch || n_out > 32 || t.K > 32 || !t.gmask.p) return false;
   if (n_in <= 4 || n_in % 4 || (uintptr_t)in % 16 || n_in * 4 >= (1 << 24)) return false;
   // k_conv_resident keeps 20-32 -> up to 16 planes on small levels of few taps and on large ones
@@ -376,7 +380,7 @@ bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_
 }
 bool conv_wave_dispatch(bool pre_fused, Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi,
                         int n_in, int n_out, PreArgs pre, hipStream_t s) {
-  if (!conv_wave_serves(m, t, in, m.cur_in_rows, n_in, n_out)) return false;
+  if (!conv_wave_serves(m, t, in, m.cur_in_rows, n_in, n_out, m.pack_transposed != nullptr)) return false;
   auto run = [&](auto ncb, auto pair) {
     if (pre_fused) dispatch_wave<decltype(ncb)::value, decltype(pair)::value, true>(m, t, in, out, w, epi, n_in, n_out, pre, s);
     else dispatch_wave<decltype(ncb)::value, decltype(pair)::value, false>(m, t, in, out, w, epi, n_in, n_out, pre, s);
