@@ -267,7 +267,7 @@ bool conv_split_serves(const Metadata &m, const Table &t, const float *in, int64
 bool conv_split_dispatch(bool pre_fused, Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi,
                          int n_in, int n_out, PreArgs pre, hipStream_t s);
 const float *split_weights(Metadata &m, int K, const float *w, int n_in, int n_out, int NCB, bool half, hipStream_t s);
-// conv_wave.hip: the same for up to 32 output planes.  gradient: an input gradient over the table (weights packed transposed).
+// conv_wave.hip: the same for up to 48 output planes.  gradient: an input gradient over the table (weights packed transposed).
 bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in, int n_out, bool gradient = false);
 bool conv_wave_dispatch(bool pre_fused, Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi,
                         int n_in, int n_out, PreArgs pre, hipStream_t s);

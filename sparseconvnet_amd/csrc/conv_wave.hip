@@ -1,4 +1,4 @@
-// The split-operand convolution onto up to 32 output planes: a wavefront owns its rows from the rule to the store.  The
+// The split-operand convolution onto up to 32 output planes, and up to 48 on small levels: a wavefront owns its rows from the rule to the store.  The
 // arithmetic is that of conv_split.hip, to the bit where the additions come in the same order; see conv.hip for the family.
 #include "conv_common.h"
 
@@ -14,9 +14,10 @@ namespace scn {
 //   MFMAs            six per granule and column block, granules without the tap skipped by the table's masks
 // PAIR (up to 16 input channels): an iteration is two taps of 16 channels instead of one of 32; half an operand comes from
 // either, rows and weights alike.
-// DEAL = 4: the wavefronts of a workgroup share GW granules and take the iterations in turn; their sums meet in LDS and are
+// DEAL = 4 or 8: the wavefronts of a workgroup share GW granules and take the iterations in turn; their sums meet in LDS and are
 // added in the wavefronts' order.  A small level is as long as one wavefront's chain of iterations, and this cuts it to a
-// quarter without partial sums in memory and a launch to add them up.
+// quarter without partial sums in memory and a launch to add them up.  (A cursor finds its tap by one lane read: walking the bits of
+// a mask tap by tap, eight wavefronts spent more on that than on the rest: 1.6 k sites 48 -> 48 9.7 us, 7.8 so.)
 // What bounds it: at large levels the vector instructions of the splitting (some 60 per granule and iteration) next to the
 // MFMAs: in a loop of nothing else the two overlap by a tenth only, 155 ns per granule and iteration of 2 x 16 columns against
 // 69 and 113 apart, and the clock falls to 1.9-2.1 GHz; 32 -> 32 at a million sites is 106 us of that.  Counters there:
@@ -66,30 +67,34 @@ __global__ __launch_bounds__(64 * (DEAL > 4 ? DEAL : 4), OCC) void k_conv_wave(
   const unsigned row_bytes = (unsigned)n_in * 4u;
   const bool tail = n_in % 32 != 0;
   const int last = (int)(n - 1 - pos0);  // positions behind the last one repeat its indices and are left out
+  // the taps of `all` in order, lane i the i-th, so that a cursor finds its tap by a lane read however far it moves
+  int list = 0;
+  if (lane < 32 && ((all >> lane) & 1u)) list = lane + 1;
+  list = __builtin_amdgcn_ds_permute(4 * (list ? __popc(all & ((1u << lane) - 1u)) : 63), list) - 1;
+  const int n_taps = __popc(all);
+  constexpr int TAPS = PAIR ? 2 : 1;  // of an iteration
   // three cursors over the iterations (slab outer, tap inner), each staying on the last one
   struct Cursor {
-    unsigned rest;
-    int sl, k, k2, left;  // k2 (PAIR): the second tap, -1: none
+    int sl, pos, k, k2, left;  // pos: the tap's place in the list; k2 (PAIR): the second tap, -1: none
   };
-  auto step = [&](Cursor &c) {
-    if (c.rest == 0u) c.rest = all, c.sl++;  // (PAIR: one slab, only the first step comes here)
-    c.k = __builtin_ctz(c.rest);
-    c.rest &= c.rest - 1u;
-    if (PAIR) {
-      c.k2 = c.rest ? __builtin_ctz(c.rest) : -1;
-      c.rest &= c.rest - 1u;  // stays 0 when it is
-    }
+  auto look = [&](Cursor &c) {
+    c.k = __builtin_amdgcn_readlane(list, c.pos);
+    if (PAIR) c.k2 = c.pos + 1 < n_taps ? __builtin_amdgcn_readlane(list, c.pos + 1) : -1;
+  };
+  auto move = [&](Cursor &c, int taps) {
+    c.pos += taps;
+    if (!PAIR)
+      while (c.pos >= n_taps) c.pos -= n_taps, c.sl++;
+    look(c);
   };
   auto start = [&](Cursor &c) {
-    c = Cursor{0u, -1, 0, -1, total};
-    if (total > 0)
-      for (int i = 0; i <= (DEAL > 1 ? wave : 0); i++) step(c);
+    c = Cursor{0, 0, 0, -1, total};
+    if (total > 0) move(c, DEAL > 1 ? wave * TAPS : 0);
   };
   auto advance = [&](Cursor &c) {
     if (c.left <= 1) return;
     c.left--;
-#pragma unroll
-    for (int i = 0; i < DEAL; i++) step(c);
+    move(c, DEAL * TAPS);
   };
   Cursor at, rows, idx;
   int j[GW][PAIR ? 2 : 1];
@@ -340,6 +345,39 @@ static void launch_wave(Metadata &m, const Table &t, const float *in, float *out
   LAUNCH_CHECK();
 }
 
+// 33 to 48 output planes on small levels: every pair (granules, column group) is a workgroup whose wavefronts deal out the
+// iterations, and sums meet in LDS, where k_conv_split writes partial sums for a launch to add up.  Rows are gathered and split
+// once per column group and weights read once per workgroup, so that this ends where iterations or granules are many.
+// us, k_conv_split with its second launch / here (column blocks, granules, wavefronts of the workgroup chosen):
+//   27 taps: 1.2 k sites 48 -> 48 13.0 / 7.9 (2,1,8; three column blocks 9.5), 96 -> 48 15.1 / 10.0, 6 k 48 -> 48 21.4 / 12.9,
+//     96 -> 48 22.2 / 17.4, 12 k 48 -> 48 25 / 18, 20 k 29.9 / 24.0 (2,2,4; 30.1 with 2,1,8), 39 k 55 / 41; 300 sites and fewer gain
+//     another 1 us from one column block (1,1,8); but 400 sites 256 -> 48 16.1 / 17.9, 9 k 128 -> 48 29.1 / 29.8
+//   8 taps, stride 2, onto 25 k sites 32 -> 48 13.8 / 11.5; one rule per position, onto 3.3 k sites 80 -> 48 8.8 / 4.2, 20 k
+//     64 -> 48 9.6 / 6.8, 40 k 12.2 / 10.9; 1x1 1.5 k rows 96 -> 48 6.7 / 3.5, 20 k 8.8 / 6.9
+// (64 planes and more would gain as much on levels of a few thousand sites, 1.5 k 64 -> 64 14 / 8; they stay on k_conv_split.)
+enum WideTile { NONE, B1G1D8, B2G1D8, B2G2D4 };
+static WideTile wide_tile(const Table &t, int n_in, int n_out) {
+  if (n_in <= 16 || n_out > 48) return NONE;
+  const int64_t n = t.n, slabs = ceil_div(n_in, 32);
+  if (t.few_tap.p || t.K == 1) {
+    if (n < 5000) return n < 1500 ? B1G1D8 : B2G1D8;
+    return n < 25000 || (t.K > 1 && n < 45000 && slabs <= 2) ? B2G2D4 : NONE;
+  }
+  if (n < 500 && t.K > 9) return slabs <= 5 ? B1G1D8 : NONE;
+  if (t.K <= 9) return n < 500 ? B1G1D8 : n < 2500 ? B2G1D8 : n < 25000 ? B2G2D4 : NONE;
+  if (n < 10000) return slabs <= (n < 2500 ? 5 : 3) ? B2G1D8 : NONE;
+  return n < 40000 && slabs <= 2 ? B2G2D4 : NONE;
+}
+template <bool PRE>
+static void dispatch_wide(Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi, int n_in,
+                          int n_out, PreArgs pre, hipStream_t s) {
+  switch (wide_tile(t, n_in, n_out)) {
+  case B1G1D8: return launch_wave<1, 1, 8, 4, false, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);
+  case B2G1D8: return launch_wave<2, 1, 8, 4, false, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);
+  case B2G2D4: return launch_wave<2, 2, 4, 4, false, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);
+  case NONE: throw Error("internal: no tile for this convolution");
+  }
+}
 template <int NCB, bool PAIR, bool PRE>
 static void dispatch_wave(Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi, int n_in,
                           int n_out, PreArgs pre, hipStream_t s) {
@@ -364,8 +402,10 @@ bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_
   // the edge of a ReLU change sides with any other rounding, and a 2-D network of a few thousand sites has so few that a training
   // step's gradients differ by up to 3.5e-3 then.  Its time is the host's, so that it would not run faster either (1.21 / 1.26 ms).
   if (t.K == 9 && !gradient) return false;
-  if (m.bf16 || m.fixed_scratch || n_out > 32 || t.K > 32 || !t.gmask.p) return false;
+  if (m.bf16 || m.fixed_scratch || t.K > 32 || !t.gmask.p) return false;
   if (n_in <= 4 || n_in % 4 || (uintptr_t)in % 16 || n_in * 4 >= (1 << 24)) return false;
+  if (in_rows <= 0 || in_rows >= (1 << 24) || in_rows * n_in * 4 >= ((int64_t)1 << 31)) return false;
+  if (n_out > 32) return wide_tile(t, n_in, n_out) != NONE;
   // k_conv_resident keeps 20-32 -> up to 16 planes on small levels of few taps and on large ones
   if (n_in > 16 && n_in <= 32 && n_out <= 16 && (t.K <= 9 ? t.n < 16000 : t.n >= (n_in > 24 ? 200000 : 300000))) return false;
   // k_conv_split: wide inputs of one rule per position, and on the smallest levels chains that it cuts into more parts (500 sites
@@ -376,11 +416,15 @@ bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_
   // 250 k 22.3 / 22.1, 1 M 82 / 93
   if (t.few_tap.p && n_in == 32 && t.n >= 400000) return false;
   if (t.identity_few && (n_in == 32 || n_in == 64) && t.n >= (n_in == 32 ? 100000 : 200000)) return false;
-  return in_rows > 0 && in_rows < (1 << 24) && in_rows * n_in * 4 < ((int64_t)1 << 31);
+  return true;
 }
 bool conv_wave_dispatch(bool pre_fused, Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi,
                         int n_in, int n_out, PreArgs pre, hipStream_t s) {
   if (!conv_wave_serves(m, t, in, m.cur_in_rows, n_in, n_out, m.pack_transposed != nullptr)) return false;
+  if (n_out > 32) {
+    pre_fused ? dispatch_wide<true>(m, t, in, out, w, epi, n_in, n_out, pre, s) : dispatch_wide<false>(m, t, in, out, w, epi, n_in, n_out, pre, s);
+    return true;
+  }
   auto run = [&](auto ncb, auto pair) {
     if (pre_fused) dispatch_wave<decltype(ncb)::value, decltype(pair)::value, true>(m, t, in, out, w, epi, n_in, n_out, pre, s);
     else dispatch_wave<decltype(ncb)::value, decltype(pair)::value, false>(m, t, in, out, w, epi, n_in, n_out, pre, s);

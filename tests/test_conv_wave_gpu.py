@@ -1,4 +1,4 @@
-"""The split-operand kernel of up to 32 output planes in which a wavefront owns its rows (k_conv_wave): every form of its
+"""The split-operand kernel of up to 48 output planes in which a wavefront owns its rows (k_conv_wave): every form of its
 dispatch, at sizes around granules, workgroups and the ends of its ranges, against sums in 64 bits over the exported rules.
 
 Tolerance, as for the other split-operand kernels: sums of a chain of six products of up to 32 channels are added in fp32, one per
@@ -17,7 +17,12 @@ pytestmark = pytest.mark.gpu
     ("subm", 299999, 16, 16), ("subm", 300001, 24, 20), ("subm", 600001, 12, 28),
     # eight taps and one rule per position; one tap
     ("down", 301, 16, 32), ("down", 20011, 32, 32), ("down", 120007, 48, 16), ("up", 77, 64, 32), ("up", 20011, 48, 32),
-    ("up", 25001, 16, 8), ("up", 150001, 64, 16), ("nin", 5, 16, 16), ("nin", 5003, 96, 32), ("nin", 25001, 24, 16)])
+    ("up", 25001, 16, 8), ("up", 150001, 64, 16), ("nin", 5, 16, 16), ("nin", 5003, 96, 32), ("nin", 25001, 24, 16),
+    # 33 to 48 output planes: every tile, ragged last column groups, fewer iterations than wavefronts
+    ("subm", 7, 20, 33), ("subm", 499, 128, 48), ("subm", 500, 160, 40), ("subm", 2501, 96, 48), ("subm", 9999, 64, 36),
+    ("subm", 10001, 48, 48), ("subm", 39999, 24, 36), ("down", 900, 192, 48), ("down", 9003, 32, 40), ("down", 60011, 100, 48),
+    ("up", 300, 192, 48), ("up", 2003, 64, 48), ("up", 24001, 160, 40), ("up", 44001, 64, 44), ("nin", 77, 224, 48),
+    ("nin", 3001, 128, 34), ("nin", 24999, 96, 40)])
 @pytest.mark.parametrize("form", ["plain", "normalised"])
 def test_rows_owned_by_a_wavefront(kind, n, cin, cout, form):
     import torch
@@ -67,7 +72,8 @@ def test_rows_owned_by_a_wavefront(kind, n, cin, cout, form):
 
 
 @pytest.mark.parametrize("kind,n,cin,cout", [("subm", 3001, 16, 16), ("subm", 3001, 32, 24), ("subm", 60001, 64, 16),
-                                             ("subm", 610001, 16, 32), ("up", 30011, 48, 32), ("down", 3001, 12, 20)])
+                                             ("subm", 610001, 16, 32), ("up", 30011, 48, 32), ("down", 3001, 12, 20),
+                                             ("subm", 301, 64, 48), ("subm", 3001, 96, 40), ("up", 8001, 64, 48)])
 def test_values_that_are_not_finite(kind, n, cin, cout):
     """Exactly the outputs whose rules read an infinity or a NaN are not finite, rows and weights alike."""
     import torch
