@@ -7,7 +7,8 @@
 //
 // MFMA kernels (groups == 1, accumulators in registers for the whole filter, taps skipped per
 // 16-row granule).  fp32 layers run on split operands (three bf16 pieces each) in
-//   k_conv_wave      nOut <= 32 (48 on small levels), from 8 input planes on: wavefronts own rows from the rule to the store
+//   k_conv_wave      nOut <= 32 (48 on small levels), from 8 input planes on: wavefronts own rows from the rule to the store; bf16
+//                    operands as well, up to 128 planes
 //   k_conv_split     from 20 input planes on: rows through LDS
 // and the others (fewer planes, plane counts that are no multiple of four, arrays not 16-byte aligned or
 // of 2 GiB and more, the allocation-free entry point, bf16 operands, and the ranges conv_wave_serves and

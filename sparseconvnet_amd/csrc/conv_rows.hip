@@ -441,6 +441,17 @@ static bool dispatch_rows(Metadata &m, const Table &t, const float *in, float *o
                           Epi epi, int n_in, int n_out, PreArgs pre, hipStream_t s) {
   const int ncb = (int)ceil_div(n_out, 16);
   const bool narrow = n_in <= 16;
+  // bf16 operands: a wavefront's MFMAs of one granule take half the time of its reads of the slab, and an iteration as long as its
+  // barrier; two granules per wavefront and slabs of 64 channels on levels that have the workgroups (us): 500 k sites 64 -> 64 164 -> 148,
+  // 64 -> 96 201 -> 182, 128 -> 128 398 -> 372; 61 k 192 -> 96 110 -> 95, 256 -> 128 150 -> 131; 14 k 256 -> 128 56 -> 50
+  // (5 k 32 -> 33).  k_conv_wave serves smaller levels and, up to 32 planes, most of the larger.
+  if constexpr (VEC4) {
+    if (m.bf16 && n_in % 64 == 0 && ncb > 2 && t.n >= (n_in > 128 && ncb > 4 ? 10000 : ncb <= 4 ? 260000 : 40000)) {
+      if (ncb <= 4) return launch_rows<4, 2, 4, VEC4, 4, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);
+      if (ncb <= 6) return launch_rows<6, 2, 4, VEC4, 4, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);
+      if (ncb <= 8) return launch_rows<8, 2, 4, VEC4, 4, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);
+    }
+  }
   // 64-row workgroups where 128-row ones would leave a CU with one or two of them (a level of
   // 60 k sites is 480 such workgroups for 256 CUs: one wavefront per SIMD, nothing to run while
   // it waits for its gathers).  Measured: 13-18 % faster at 62 k sites, 5 % at 15 k and 250 k,

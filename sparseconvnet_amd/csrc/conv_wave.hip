@@ -30,13 +30,15 @@ namespace scn {
 // 8 taps, stride 2, 16 -> 32 from 60 k sites 14 / 5.8; transposed 24 -> 16 onto 20 k sites 8.0 / 4.4; 1x1 16 -> 32 60 k rows 17 / 8.
 // Sums of up to 16 channels were computed on fp32 matrix instructions before; against 64 bits (relative 2-norm) 16 -> 16 at
 // 20 k sites 2.6e-7 / 6.3e-8, 8 -> 8 1.8e-7 / 6.3e-8, 1x1 8 -> 8 5.7e-8 / 3.3e-8.
-template <int NCB, int GW, int DEAL, int OCC, bool PAIR, bool PRE>
+template <int NCB, int GW, int DEAL, int OCC, bool PAIR, bool PRE, bool BF16>
 __global__ __launch_bounds__(64 * (DEAL > 4 ? DEAL : 4), OCC) void k_conv_wave(
     const int *__restrict__ nbr, const int *__restrict__ rowmap, const unsigned *__restrict__ gmask, int64_t n, int64_t npad,
     const float *__restrict__ in, float *__restrict__ out, const v8s *__restrict__ wp, Epi epi, int n_in, int n_out, int n_slab,
     int ncb, int tiles_per_xcd, int n_tiles, const float *__restrict__ pre_sc, const float *__restrict__ pre_sh, float pre_leak,
     unsigned in_bytes) {
   constexpr int WAVES = DEAL > 4 ? DEAL : 4;
+  static_assert(!BF16 || !PAIR, "bf16 operands: whole slabs");
+  constexpr int PIECES = BF16 ? 1 : 3;  // of an operand
   static_assert(DEAL == 1 || DEAL == WAVES, "a workgroup is one group of wavefronts that share granules");
   constexpr int PART = DEAL > 1 && NCB > 2 ? NCB : 2;  // KB of LDS per wavefront and granule
   __shared__ v4f turn[WAVES][GW][PART][64];
@@ -99,7 +101,7 @@ __global__ __launch_bounds__(64 * (DEAL > 4 ? DEAL : 4), OCC) void k_conv_wave(
   Cursor at, rows, idx;
   int j[GW][PAIR ? 2 : 1];
   v4f areg[GW][2];
-  v8s breg[NCB][3];
+  v8s breg[NCB][PIECES];
   auto issue_indices = [&](const Cursor &c) {
 #pragma unroll
     for (int q = 0; q < GW; q++)
@@ -119,7 +121,7 @@ __global__ __launch_bounds__(64 * (DEAL > 4 ? DEAL : 4), OCC) void k_conv_wave(
 #pragma unroll
       for (int s = 0; s < 2; s++) {
         const int row = j[q][PAIR ? s : 0], step = PAIR ? 0 : c.sl * 2 + s;  // step: of 16 channels
-        const bool past = (PAIR || tail) && step * 16 + 4 * ld_g >= n_in;    // channels past the last
+        const bool past = !BF16 && (PAIR || tail) && step * 16 + 4 * ld_g >= n_in;  // channels past the last
         const bool there = row >= 0 && !past;
         const unsigned off = __umul24((unsigned)row, row_bytes) + 16u * (unsigned)ld_g;
         areg[q][s] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, there ? off : 0x80000000u, step * 64, 0));
@@ -145,11 +147,11 @@ __global__ __launch_bounds__(64 * (DEAL > 4 ? DEAL : 4), OCC) void k_conv_wave(
         for (int p = 0; p < 3; p++)
           breg[b][p] = __builtin_shufflevector(s0[(p * ncb + b) * 64], s1[(p * ncb + b) * 64], 0, 1, 2, 3, 4, 5, 6, 7);
     } else {
-      const v8s *src = wp + (((int64_t)c.k * n_slab + c.sl) * (3 * ncb) + cb0) * 64 + lane;
+      const v8s *src = wp + (((int64_t)c.k * n_slab + c.sl) * (PIECES * ncb) + cb0) * 64 + lane;
 #pragma unroll
       for (int b = 0; b < NCB; b++)
 #pragma unroll
-        for (int p = 0; p < 3; p++) breg[b][p] = src[(p * ncb + b) * 64];
+        for (int p = 0; p < PIECES; p++) breg[b][p] = src[(p * ncb + b) * 64];
     }
   };
   start(at);
@@ -164,13 +166,20 @@ __global__ __launch_bounds__(64 * (DEAL > 4 ? DEAL : 4), OCC) void k_conv_wave(
   }
   for (int it = 0; it < total; it++) {
 #pragma unroll
-    for (int q = 0; q < GW; q++)
+    for (int q = 0; q < GW; q++) {
+      if constexpr (BF16) {  // rounded before they turn: half the LDS traffic
+        v4f x0 = pre_act<PRE>(areg[q][0], psc[0], psh[0], pre_leak), x1 = pre_act<PRE>(areg[q][1], psc[1], psh[1], pre_leak);
+        if (PRE && !((aok >> (2 * q)) & 1u)) x0 = x1 = (v4f){0.f, 0.f, 0.f, 0.f};
+        turn[wave][q][0][wr_slot] = __builtin_bit_cast(v4f, to_bf16x8(x0, x1));
+        continue;
+      }
 #pragma unroll
       for (int s = 0; s < 2; s++) {
         v4f v = pre_act<PRE>(areg[q][s], psc[s], psh[s], pre_leak);
         if (PRE && !((aok >> (2 * q + s)) & 1u)) v = (v4f){0.f, 0.f, 0.f, 0.f};
         turn[wave][q][s][wr_slot] = v;
       }
+    }
     advance(rows);
     issue_rows(rows);
     advance(idx);
@@ -180,22 +189,28 @@ __global__ __launch_bounds__(64 * (DEAL > 4 ? DEAL : 4), OCC) void k_conv_wave(
 #pragma unroll
     for (int q = 0; q < GW; q++) {
       if (!((gm[q] >> at.k) & 1u) && (!PAIR || at.k2 < 0 || !((gm[q] >> at.k2) & 1u))) continue;  // uniform over the wavefront
-      const Split8 a = split8(turn[wave][q][0][rd_slot], turn[wave][q][1][rd_slot]);
-      v4f t[NCB];
+      if constexpr (BF16) {
+        const v8s a = __builtin_bit_cast(v8s, turn[wave][q][0][rd_slot]);
 #pragma unroll
-      for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.h, breg[c][2], (v4f){0.f, 0.f, 0.f, 0.f});
+        for (int c = 0; c < NCB; c++) acc[q][c] = mfma_bf16(a, breg[c][0], acc[q][c]);
+      } else {
+        const Split8 a = split8(turn[wave][q][0][rd_slot], turn[wave][q][1][rd_slot]);
+        v4f t[NCB];
 #pragma unroll
-      for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.l, breg[c][0], t[c]);
+        for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.h, breg[c][PIECES - 1], (v4f){0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-      for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.m, breg[c][1], t[c]);
+        for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.l, breg[c][0], t[c]);
 #pragma unroll
-      for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.h, breg[c][1], t[c]);
+        for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.m, breg[c][PIECES / 2], t[c]);
 #pragma unroll
-      for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.m, breg[c][0], t[c]);
+        for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.h, breg[c][PIECES / 2], t[c]);
 #pragma unroll
-      for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.h, breg[c][0], t[c]);
+        for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.m, breg[c][0], t[c]);
 #pragma unroll
-      for (int c = 0; c < NCB; c++) acc[q][c] += t[c];
+        for (int c = 0; c < NCB; c++) t[c] = mfma_bf16(a.h, breg[c][0], t[c]);
+#pragma unroll
+        for (int c = 0; c < NCB; c++) acc[q][c] += t[c];
+      }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -203,71 +218,73 @@ __global__ __launch_bounds__(64 * (DEAL > 4 ? DEAL : 4), OCC) void k_conv_wave(
     issue_weights(rows);
   }
 
-  float probe = 0.f;  // stays zero while every sum is finite
-#pragma unroll
-  for (int q = 0; q < GW; q++)
-#pragma unroll
-    for (int c = 0; c < NCB; c++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) probe = __builtin_fmaf(acc[q][c][r], 0.f, probe);
-  if (__ballot(probe != 0.f) != 0ull) {
-    // infinities, NaNs or values too large for pieces: again on the fp32 matrix instructions (see k_conv_split)
+  if constexpr (!BF16) {
+    float probe = 0.f;  // stays zero while every sum is finite
 #pragma unroll
     for (int q = 0; q < GW; q++)
 #pragma unroll
-      for (int c = 0; c < NCB; c++) acc[q][c] = (v4f){0.f, 0.f, 0.f, 0.f};
-    start(at);
+      for (int c = 0; c < NCB; c++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) probe = __builtin_fmaf(acc[q][c][r], 0.f, probe);
+    if (__ballot(probe != 0.f) != 0ull) {
+      // infinities, NaNs or values too large for pieces: again on the fp32 matrix instructions (see k_conv_split)
+#pragma unroll
+      for (int q = 0; q < GW; q++)
+#pragma unroll
+        for (int c = 0; c < NCB; c++) acc[q][c] = (v4f){0.f, 0.f, 0.f, 0.f};
+      start(at);
 #pragma unroll 1
-    for (int it = 0; it < (PAIR ? 2 * total : total); it++) {
-      const int k = PAIR && (it & 1) ? at.k2 : at.k, sl = at.sl;
+      for (int it = 0; it < (PAIR ? 2 * total : total); it++) {
+        const int k = PAIR && (it & 1) ? at.k2 : at.k, sl = at.sl;
 #pragma unroll
-      for (int c = 0; c < NCB; c++) {
-        if (PAIR && k < 0) break;  // uniform
-        float w[8];
-        if constexpr (PAIR) {
-          const v4s *src = reinterpret_cast<const v4s *>(wp) + ((int64_t)k * (3 * ncb) + cb0 + c) * 64 + lane;
-          const v4s wh = src[0], wm = src[ncb * 64], wl = src[2 * ncb * 64];
+        for (int c = 0; c < NCB; c++) {
+          if (PAIR && k < 0) break;  // uniform
+          float w[8];
+          if constexpr (PAIR) {
+            const v4s *src = reinterpret_cast<const v4s *>(wp) + ((int64_t)k * (3 * ncb) + cb0 + c) * 64 + lane;
+            const v4s wh = src[0], wm = src[ncb * 64], wl = src[2 * ncb * 64];
 #pragma unroll
-          for (int e = 0; e < 4; e++) w[e] = join_weight(wh[e], wm[e], wl[e]);
-        } else {
-          const v8s *src = wp + (((int64_t)k * n_slab + sl) * (3 * ncb) + cb0 + c) * 64 + lane;
-          const v8s wh = src[0], wm = src[ncb * 64], wl = src[2 * ncb * 64];
+            for (int e = 0; e < 4; e++) w[e] = join_weight(wh[e], wm[e], wl[e]);
+          } else {
+            const v8s *src = wp + (((int64_t)k * n_slab + sl) * (3 * ncb) + cb0 + c) * 64 + lane;
+            const v8s wh = src[0], wm = src[ncb * 64], wl = src[2 * ncb * 64];
 #pragma unroll
-          for (int e = 0; e < 8; e++) w[e] = join_weight(wh[e], wm[e], wl[e]);
-        }
+            for (int e = 0; e < 8; e++) w[e] = join_weight(wh[e], wm[e], wl[e]);
+          }
 #pragma unroll
-        for (int q = 0; q < GW; q++) {
-          if (!((gm[q] >> k) & 1u)) continue;  // uniform over the wavefront
-          const int *src_j = nbr + (int64_t)k * npad + pos0;
-          const int row = 16 * q + r16 <= last ? src_j[16 * q + r16] : -1;
-          v4f t = (v4f){0.f, 0.f, 0.f, 0.f};
+          for (int q = 0; q < GW; q++) {
+            if (!((gm[q] >> k) & 1u)) continue;  // uniform over the wavefront
+            const int *src_j = nbr + (int64_t)k * npad + pos0;
+            const int row = 16 * q + r16 <= last ? src_j[16 * q + r16] : -1;
+            v4f t = (v4f){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int s = 0; s < (PAIR ? 1 : 2); s++) {
-            const int ch = (sl * 2 + s) * 16 + 4 * g;
-            const bool there = row >= 0 && ch < n_in;  // n_in is a multiple of four
-            v4f x = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
-                                                rsrc, there ? (unsigned)row * row_bytes + 4u * (unsigned)ch : 0x80000000u, 0, 0));
-            if (PRE) {
-              x = pre_act<PRE>(x, *reinterpret_cast<const v4f *>(pre_sc + ch), *reinterpret_cast<const v4f *>(pre_sh + ch), pre_leak);
-              if (!there) x = (v4f){0.f, 0.f, 0.f, 0.f};
+            for (int s = 0; s < (PAIR ? 1 : 2); s++) {
+              const int ch = (sl * 2 + s) * 16 + 4 * g;
+              const bool there = row >= 0 && ch < n_in;  // n_in is a multiple of four
+              v4f x = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
+                                                  rsrc, there ? (unsigned)row * row_bytes + 4u * (unsigned)ch : 0x80000000u, 0, 0));
+              if (PRE) {
+                x = pre_act<PRE>(x, *reinterpret_cast<const v4f *>(pre_sc + ch), *reinterpret_cast<const v4f *>(pre_sh + ch), pre_leak);
+                if (!there) x = (v4f){0.f, 0.f, 0.f, 0.f};
+              }
+#pragma unroll
+              for (int e = 0; e < 4; e++) t = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], w[4 * s + e], t, 0, 0, 0);
             }
 #pragma unroll
-            for (int e = 0; e < 4; e++) t = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], w[4 * s + e], t, 0, 0, 0);
-          }
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const int p = 16 * q + 4 * g + r;
-            acc[q][c][r] += p <= last && src_j[min(p, last)] >= 0 ? t[r] : 0.f;
+            for (int r = 0; r < 4; r++) {
+              const int p = 16 * q + 4 * g + r;
+              acc[q][c][r] += p <= last && src_j[min(p, last)] >= 0 ? t[r] : 0.f;
+            }
           }
         }
+        if (!PAIR || (it & 1)) advance(at);
       }
-      if (!PAIR || (it & 1)) advance(at);
+    } else {
+#pragma unroll
+      for (int q = 0; q < GW; q++)
+#pragma unroll
+        for (int c = 0; c < NCB; c++) acc[q][c] *= SPLIT_UNSCALE;
     }
-  } else {
-#pragma unroll
-    for (int q = 0; q < GW; q++)
-#pragma unroll
-      for (int c = 0; c < NCB; c++) acc[q][c] *= SPLIT_UNSCALE;
   }
 
   // acc[q][c][r] = result for position pos0 + 16*q + 4*g + r, column 16*c + r16
@@ -330,16 +347,24 @@ __global__ __launch_bounds__(64 * (DEAL > 4 ? DEAL : 4), OCC) void k_conv_wave(
   }
 }
 
-template <int NCB, int GW, int DEAL, int OCC, bool PAIR, bool PRE>
+template <int NCB, int GW, int DEAL, int OCC, bool PAIR, bool PRE, bool BF16 = false>
 static void launch_wave(Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi, int n_in,
                         int n_out, PreArgs pre, hipStream_t s) {
   const int n_slab = (int)ceil_div(n_in, 32);
   const int groups = (int)ceil_div(n_out, 16 * NCB), ncb = groups * NCB;
-  const float *wpack = split_weights(m, t.K, w, n_in, n_out, ncb, PAIR, s);
+  const float *wpack;
+  if constexpr (BF16) {  // [K][n_slab][ncb][lane], a lane's eight channels of a slab
+    const int stride = ncb * 512;
+    wpack = packed_weights(m, {6, (int64_t)(uintptr_t)w, t.K, n_in, n_out, ncb}, (size_t)t.K * n_slab * stride / 2, [&](float *dst) {
+      launch_pack_weights(w, dst, t.K, n_in, n_out, n_slab, 2, ncb, stride, take_jobs(m), true, s);
+    });
+  } else {
+    wpack = split_weights(m, t.K, w, n_in, n_out, ncb, PAIR, s);
+  }
   const int n_tiles = (int)ceil_div(t.n, (DEAL > 1 ? 1 : 4) * GW * 16);
   const int tiles_per_xcd = t.spread ? 0 : (int)ceil_div(n_tiles, 8);
-  note_kernel(m, "split wave", {{"ncb", NCB}, {"gw", GW}, {"deal", DEAL}, {"pair", PAIR}, {"pre", PRE}, {"split", 1}});
-  k_conv_wave<NCB, GW, DEAL, OCC, PAIR, PRE><<<dim3((unsigned)(tiles_per_xcd ? tiles_per_xcd * 8 : n_tiles), groups), 64 * std::max(4, DEAL), 0, s>>>(
+  note_kernel(m, BF16 ? "wave-bf16" : "split wave", {{"ncb", NCB}, {"gw", GW}, {"deal", DEAL}, {"pair", PAIR}, {"pre", PRE}, {"split", 1}});
+  k_conv_wave<NCB, GW, DEAL, OCC, PAIR, PRE, BF16><<<dim3((unsigned)(tiles_per_xcd ? tiles_per_xcd * 8 : n_tiles), groups), 64 * std::max(4, DEAL), 0, s>>>(
       t.nbr.p, t.rowmap_ptr(), t.gmask.p, t.n, t.npad, in, out, reinterpret_cast<const v8s *>(wpack), epi, n_in, n_out, n_slab,
       ncb, tiles_per_xcd, n_tiles, pre.sc, pre.sh, pre.leak, (unsigned)(m.cur_in_rows * n_in * 4));
   LAUNCH_CHECK();
@@ -397,14 +422,64 @@ static void dispatch_wave(Metadata &m, const Table &t, const float *in, float *o
   else WAVE(4, 1, 3);
 #undef WAVE
 }
+// bf16 operands (the caller's choice; whole slabs of 32 channels): the same kernel with one instruction and no splitting.  What bounds
+// it: the rows' way from L2 (13 TB/s at 800 k sites 32 -> 32), and on small levels the chain, as above.  us, k_conv_resident,
+// k_conv_rows or k_conv_mfma, which keep the rest / here:
+//   27 taps: 1 k sites 32 -> 32 18.3 / 4.7, 64 -> 64 12.8 / 6.7, 128 -> 128 18.0 / 10.6; 14 k 32 -> 32 20.0 / 5.8, 64 -> 64 22.6 / 10.6,
+//     128 -> 128 36.4 / 27.9, but 256 -> 128 55.9 / 50.7 where 128-row tiles of slabs of 64 (k_conv_rows) take 49.6; 61 k 64 -> 32 47 / 20.5,
+//     64 -> 64 38 / 27, but 96 -> 96 60 / 61; 240 k 32 -> 32 60 / 36, 128 -> 64 144 / 134, 128 -> 128 205 / 192; 500 k 32 -> 32 86 / 65,
+//     but 64 -> 32 112 / 118; 900 k 32 -> 32 140 / 126
+//   8 taps, onto 5 k sites 32 -> 64 13.6 / 4.0, 59 k 13.9 / 12.9, 221 k 32 -> 32 63 / 26; one rule per position, onto 20 k sites
+//     64 -> 32 14.0 / 4.1, 900 k 51 / 38, 61 k 96 -> 64 12.8 / 10.9; 1x1 20 k rows 128 -> 64 8.5 / 5.8, 61 k 13.0 / 13.0
+// (Rounding the rows in a pass of its own, so that each rule reads half the bytes, takes longer than it saves: 300 k sites 64 -> 64
+// 92 -> 102, 800 k 32 -> 32 99 -> 135.)
+enum BfTile { BF_NONE, BF_2_1_4, BF_2_2_4, BF_2_2_1, BF_2_4_1, BF_4_2_4, BF_8_4_1 };  // column blocks, granules, wavefronts that share them
+static BfTile bf_tile(const Table &t, int n_in, int n_out) {
+  const int64_t n = t.n;
+  if (n_in % 32 || n_out > 128) return BF_NONE;
+  const bool one_rule = t.few_tap.p || t.K == 1, few = one_rule || t.K <= 9;
+  if (n_out <= 32) {
+    if (n < 20000) return BF_2_1_4;
+    if (n < (few ? 100000 : 300000)) return BF_2_2_4;
+    if (few) return BF_2_2_1;
+    return n_in > 32 ? BF_NONE : n < 700000 ? BF_2_2_1 : BF_2_4_1;
+  }
+  if (few) {
+    const int64_t to = t.K == 1 ? 45000 : n_out <= 64 ? (one_rule ? 100000 : 70000) : 25000;
+    return n < 8000 ? BF_2_1_4 : n < to ? BF_4_2_4 : BF_NONE;
+  }
+  if (n_out <= 64) return n < 8000 ? BF_2_1_4 : n < 260000 ? BF_4_2_4 : BF_NONE;
+  if (n < 3000) return BF_2_1_4;
+  if (n_in > 128) return BF_NONE;
+  if (n < 8000) return n_out <= 96 ? BF_2_1_4 : BF_4_2_4;
+  if (n < 40000) return BF_4_2_4;
+  return n_out > 96 && n >= 100000 ? BF_8_4_1 : BF_NONE;
+}
+template <bool PRE>
+static void dispatch_bf(Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi, int n_in,
+                        int n_out, PreArgs pre, hipStream_t s) {
+#define BF(N, G, D, O) \
+  case BF_##N##_##G##_##D: return launch_wave<N, G, D, O, false, PRE, true>(m, t, in, out, w, epi, n_in, n_out, pre, s)
+  switch (bf_tile(t, n_in, n_out)) {
+    BF(2, 1, 4, 5);
+    BF(2, 2, 4, 4);
+    BF(2, 2, 1, 5);
+    BF(2, 4, 1, 4);
+    BF(4, 2, 4, 4);
+    BF(8, 4, 1, 2);
+  case BF_NONE: throw Error("internal: no tile for this convolution");
+  }
+#undef BF
+}
 bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in, int n_out, bool gradient) {
   // Forward sums over nine taps (the 3 x 3 filters of 2-D networks) stay where they were, k_conv_resident and k_conv_split: values on
   // the edge of a ReLU change sides with any other rounding, and a 2-D network of a few thousand sites has so few that a training
   // step's gradients differ by up to 3.5e-3 then.  Its time is the host's, so that it would not run faster either (1.21 / 1.26 ms).
   if (t.K == 9 && !gradient) return false;
-  if (m.bf16 || m.fixed_scratch || t.K > 32 || !t.gmask.p) return false;
+  if (m.fixed_scratch || t.K > 32 || !t.gmask.p) return false;
   if (n_in <= 4 || n_in % 4 || (uintptr_t)in % 16 || n_in * 4 >= (1 << 24)) return false;
   if (in_rows <= 0 || in_rows >= (1 << 24) || in_rows * n_in * 4 >= ((int64_t)1 << 31)) return false;
+  if (m.bf16) return !gradient && bf_tile(t, n_in, n_out) != BF_NONE;  // (these weights are packed from a transposed copy)
   if (n_out > 32) return wide_tile(t, n_in, n_out) != NONE;
   // k_conv_resident keeps 20-32 -> up to 16 planes on small levels of few taps and on large ones
   if (n_in > 16 && n_in <= 32 && n_out <= 16 && (t.K <= 9 ? t.n < 16000 : t.n >= (n_in > 24 ? 200000 : 300000))) return false;
@@ -421,6 +496,10 @@ bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_
 bool conv_wave_dispatch(bool pre_fused, Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi,
                         int n_in, int n_out, PreArgs pre, hipStream_t s) {
   if (!conv_wave_serves(m, t, in, m.cur_in_rows, n_in, n_out, m.pack_transposed != nullptr)) return false;
+  if (m.bf16) {
+    pre_fused ? dispatch_bf<true>(m, t, in, out, w, epi, n_in, n_out, pre, s) : dispatch_bf<false>(m, t, in, out, w, epi, n_in, n_out, pre, s);
+    return true;
+  }
   if (n_out > 32) {
     pre_fused ? dispatch_wide<true>(m, t, in, out, w, epi, n_in, n_out, pre, s) : dispatch_wide<false>(m, t, in, out, w, epi, n_in, n_out, pre, s);
     return true;

@@ -97,3 +97,42 @@ def test_values_that_are_not_finite(kind, n, cin, cout):
             want.index_add_(0, r[:, 1], x[r[:, 0]].double() @ v[k, 0].double())
             mag.index_add_(0, r[:, 1], x[r[:, 0]].double().abs() @ v[k, 0].double().abs())
         _close_where_finite(conv(x, v, torch.zeros(cout).cuda()), want, mag, len(rules) * cin + 16)
+
+
+@pytest.mark.parametrize("kind,n,cin,cout", [
+    ("subm", 1, 32, 16), ("subm", 17, 64, 32), ("subm", 7999, 96, 64), ("subm", 8001, 32, 40), ("subm", 19999, 32, 32),
+    ("subm", 20001, 64, 24), ("subm", 300001, 32, 32), ("subm", 700001, 32, 20), ("subm", 2999, 256, 128), ("subm", 3001, 128, 100),
+    ("subm", 39999, 96, 96), ("subm", 100001, 64, 128), ("subm", 259999, 32, 64), ("subm", 260001, 64, 64), ("subm", 40001, 64, 72),
+    ("subm", 10001, 192, 112), ("down", 900, 64, 96), ("down", 60011, 96, 128), ("down", 500001, 32, 32), ("up", 301, 64, 64),
+    ("up", 20011, 128, 96), ("up", 120011, 64, 32), ("nin", 77, 96, 128), ("nin", 44999, 32, 64), ("nin", 120001, 64, 32)])
+@pytest.mark.parametrize("form", ["plain", "normalised"])
+def test_bf16_operands(kind, n, cin, cout, form):
+    """Operands rounded to bf16, products exact, added in fp32 by a unit that need not round to nearest: one result is off by at most
+    an ulp, 2^-23, per addition of the sum of the products' magnitudes; a normalised row's value may be rounded from the neighbouring
+    fp32 number, an ulp of bf16 (2^-7) away."""
+    import torch
+    from test_conv_split_gpu import _table
+    conv, rules, rows_in, rows_out, md = _table(kind, n, 8300 + n % 89)
+    md.setBf16(True)
+    g = torch.Generator().manual_seed(n + cout)
+    x, w = torch.randn(rows_in, cin, generator=g).cuda(), (torch.randn(len(rules), 1, cin, cout, generator=g) * 0.1).cuda()
+    bias = torch.randn(cout, generator=g).cuda()
+    front = None
+    f = x
+    if form == "normalised" and kind != "nin":
+        front = (torch.randn(cin, generator=g).cuda(), torch.rand(cin, generator=g).cuda() + 0.5, torch.rand(cin, generator=g).cuda() + 0.5,
+                 torch.randn(cin, generator=g).cuda() + 1.0, 1e-4, 0.2)
+        f = (x.double() - front[0]) * (front[2].double() / torch.sqrt(front[1].double() + front[4])) + front[3]
+        f = torch.where(f > 0, f, 0.2 * f).float()
+    f, wr = f.bfloat16().double(), w.bfloat16().double()
+    want = bias.double().expand(rows_out, -1).clone()
+    mag = want.abs()
+    for k, r in enumerate(rules):
+        r = torch.as_tensor(r).cuda().long()
+        want.index_add_(0, r[:, 1], f[r[:, 0]] @ wr[k, 0])
+        mag.index_add_(0, r[:, 1], f[r[:, 0]].abs() @ wr[k, 0].abs())
+    got = conv(x, w, bias) if front is None else conv(x, w, bias, bn=front)
+    bound = (len(rules) * cin + 8) * 2.0 ** -23 + (0 if front is None else 2.0 ** -7)
+    assert ((got.double() - want).abs() <= bound * mag + 1e-30).all()
+    kernel = md._L.scn_md_last_conv_kernel(md._h).decode()
+    assert "bf16" in kernel, kernel
