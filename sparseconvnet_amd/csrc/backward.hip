@@ -1100,6 +1100,25 @@ void strided_conv_backward(Metadata &m, const Table &fwd, const Table &other, in
 // CPU/BatchNormalization.cpp:19-40: batch mean and biased variance into save_mean / save_invstd,
 // running statistics updated with `momentum` weighting the old value and the unbiased variance;
 // coef = scale | shift for the affine pass.
+struct BnTrain {
+  float *save_mean, *save_invstd, *running_mean, *running_var;
+  const float *gamma, *beta;
+  float eps, momentum;
+};
+// Plane c from the sums of its values and of their squares.
+__device__ inline void bn_train_plane(const BnTrain &t, int c, int64_t rows, double s1, double s2, float &sc, float &sh) {
+  const double mean = s1 / (double)rows;
+  double ss = s2 - mean * mean * (double)rows;  // sum of squared deviations
+  if (ss < 0) ss = 0;
+  t.save_mean[c] = (float)mean;
+  t.running_mean[c] = t.momentum * t.running_mean[c] + (1 - t.momentum) * (float)mean;
+  t.running_var[c] = t.momentum * t.running_var[c] + (1 - t.momentum) * (float)(ss / (double)(rows - 1));
+  const float invstd = powf((float)(ss / (double)rows) + t.eps, -0.5f);
+  t.save_invstd[c] = invstd;
+  const float w = invstd * (t.gamma ? t.gamma[c] : 1.f);
+  sc = w;
+  sh = -(float)mean * w + (t.beta ? t.beta[c] : 0.f);
+}
 __global__ __launch_bounds__(1024) void k_bn_train_finish(const float *partial, int blocks, int planes, int64_t rows,
                                                           float *save_mean, float *save_invstd, float *running_mean,
                                                           float *running_var, const float *gamma, const float *beta,
@@ -1108,17 +1127,8 @@ __global__ __launch_bounds__(1024) void k_bn_train_finish(const float *partial, 
   pair_sums64(partial, blocks, planes, s1, s2);
   const int c = blockIdx.x * 64 + (threadIdx.x & 63);
   if (threadIdx.x >= 64 || c >= planes) return;
-  const double mean = s1 / (double)rows;
-  double ss = s2 - mean * mean * (double)rows;  // sum of squared deviations
-  if (ss < 0) ss = 0;
-  save_mean[c] = (float)mean;
-  running_mean[c] = momentum * running_mean[c] + (1 - momentum) * (float)mean;
-  running_var[c] = momentum * running_var[c] + (1 - momentum) * (float)(ss / (double)(rows - 1));
-  const float invstd = powf((float)(ss / (double)rows) + eps, -0.5f);
-  save_invstd[c] = invstd;
-  const float w = invstd * (gamma ? gamma[c] : 1.f);
-  coef[c] = w;
-  coef[planes + c] = -(float)mean * w + (beta ? beta[c] : 0.f);
+  bn_train_plane(BnTrain{save_mean, save_invstd, running_mean, running_var, gamma, beta, eps, momentum}, c, rows, s1, s2, coef[c],
+                 coef[planes + c]);
 }
 // out = leaky(x * sc + sh), one thread per element (rows x planes), any strides
 __global__ void k_affine_leaky(const float *in, float *out, int64_t rows, int planes, int64_t in_stride,
@@ -1132,6 +1142,14 @@ __global__ void k_affine_leaky(const float *in, float *out, int64_t rows, int pl
     out[r * out_stride + c] = y * (y > 0 ? 1.f : leak);
   }
 }
+__device__ inline v4f affine_leaky4(v4f x, v4f sc, v4f sh, float leak) {
+  v4f y = x * sc + sh;
+  y.x *= y.x > 0 ? 1.f : leak;
+  y.y *= y.y > 0 ? 1.f : leak;
+  y.z *= y.z > 0 ? 1.f : leak;
+  y.w *= y.w > 0 ? 1.f : leak;
+  return y;
+}
 // The same, four planes per thread (plane count and strides multiples of four, 16-byte aligned).
 __global__ void k_affine_leaky4(const float *__restrict__ in, float *__restrict__ out, int64_t rows, int planes,
                                 int64_t in_stride, int64_t out_stride, const float *__restrict__ coef, float leak) {
@@ -1143,44 +1161,20 @@ __global__ void k_affine_leaky4(const float *__restrict__ in, float *__restrict_
     const int c = 4 * (int)(i - r * quads);
     const v4f x = *reinterpret_cast<const v4f *>(in + r * in_stride + c);
     const v4f sc = *reinterpret_cast<const v4f *>(coef + c), sh = *reinterpret_cast<const v4f *>(coef + planes + c);
-    v4f y = x * sc + sh;
-    y.x *= y.x > 0 ? 1.f : leak;
-    y.y *= y.y > 0 ? 1.f : leak;
-    y.z *= y.z > 0 ? 1.f : leak;
-    y.w *= y.w > 0 ? 1.f : leak;
-    *reinterpret_cast<v4f *>(out + r * out_stride + c) = y;
+    *reinterpret_cast<v4f *>(out + r * out_stride + c) = affine_leaky4(x, sc, sh, leak);
   }
 }
-void bn_train_forward(Metadata *scratch, const float *in, float *out, int64_t rows, int planes, int64_t in_stride,
-                      int64_t out_stride, float *save_mean, float *save_invstd, float *running_mean,
-                      float *running_var, const float *gamma, const float *beta, float eps, float momentum,
-                      float leak, hipStream_t s) {
-  if (planes <= 0) return;
-  if (rows <= 0) {  // no rows: defined statistics (the reference divides by zero here), running ones untouched
-    fill32(save_mean, 0, planes, s);
-    fill32(save_invstd, 0, planes, s);
-    return;
-  }
-  Metadata &m = *scratch;
-  const ColsumPlan p = colsum_plan(rows, planes);
-  m.partial.reserve((size_t)p.blocks * 2 * planes);
-  m.prebuf.reserve(2 * (size_t)planes);
-  launch_colsum<1>(dim3(p.blocks, (unsigned)ceil_div(planes, p.CW)), s, in, in_stride, nullptr, nullptr, 0, nullptr,
-                                                                                 0.f, rows, planes, p.CW, p.rows_per_block,
-                                                                                 m.partial.p);
-  k_bn_train_finish<<<dim3((unsigned)ceil_div(planes, 64)), 1024, 0, s>>>(m.partial.p, p.blocks, planes, rows, save_mean,
-                                                                          save_invstd, running_mean, running_var, gamma,
-                                                                          beta, eps, momentum, m.prebuf.p);
-  LAUNCH_CHECK();
-  if (planes % 4 == 0 && in_stride % 4 == 0 && out_stride % 4 == 0 && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 16 == 0) {
-    const int64_t blocks4 = std::min<int64_t>(ceil_div(rows * (planes / 4), TB), 256 * 64);
-    k_affine_leaky4<<<dim3((unsigned)blocks4), TB, 0, s>>>(in, out, rows, planes, in_stride, out_stride, m.prebuf.p, leak);
-    LAUNCH_CHECK();
-    return;
-  }
-  const int64_t blocks = std::min<int64_t>(ceil_div(rows * planes, TB), 256 * 64);
-  k_affine_leaky<<<dim3((unsigned)blocks), TB, 0, s>>>(in, out, rows, planes, in_stride, out_stride, m.prebuf.p, leak);
-  LAUNCH_CHECK();
+struct BnBackward {
+  const float *save_invstd, *gamma;
+  float *d_gamma, *d_beta;
+};
+__device__ inline void bn_bwd_plane(const BnBackward &t, int c, int64_t rows, double sd, double dotp, float &c0, float &c1, float &c2) {
+  const float invstd = t.save_invstd[c];
+  if (t.d_beta) t.d_beta[c] = (float)sd;
+  if (t.d_gamma) t.d_gamma[c] = (float)dotp * invstd;
+  c0 = (float)(sd / (double)rows);
+  c1 = (float)dotp * invstd * invstd / (float)rows;
+  c2 = invstd * (t.gamma ? t.gamma[c] : 1.f);
 }
 // CPU/BatchNormalization.cpp:84-106: coef = gradMean | k | invstd * gamma
 __global__ __launch_bounds__(1024) void k_bn_bwd_finish(const float *partial, int blocks, int planes, int64_t rows,
@@ -1190,12 +1184,7 @@ __global__ __launch_bounds__(1024) void k_bn_bwd_finish(const float *partial, in
   pair_sums64(partial, blocks, planes, sd, dotp);
   const int c = blockIdx.x * 64 + (threadIdx.x & 63);
   if (threadIdx.x >= 64 || c >= planes) return;
-  const float invstd = save_invstd[c];
-  if (d_beta) d_beta[c] = (float)sd;
-  if (d_gamma) d_gamma[c] = (float)dotp * invstd;
-  coef[c] = (float)(sd / (double)rows);
-  coef[planes + c] = (float)dotp * invstd * invstd / (float)rows;
-  coef[2 * planes + c] = invstd * (gamma ? gamma[c] : 1.f);
+  bn_bwd_plane(BnBackward{save_invstd, gamma, d_gamma, d_beta}, c, rows, sd, dotp, coef[c], coef[planes + c], coef[2 * planes + c]);
 }
 __global__ void k_bn_bwd_apply(const float *in, float *d_in, const float *out, const float *d_out, int64_t rows,
                                int planes, int64_t in_stride, int64_t out_stride, const float *save_mean,
@@ -1210,6 +1199,19 @@ __global__ void k_bn_bwd_apply(const float *in, float *d_in, const float *out, c
     d_in[r * in_stride + c] =
         (d - coef[c] - (in[r * in_stride + c] - save_mean[c]) * coef[planes + c]) * coef[2 * planes + c];
   }
+}
+__device__ inline v4f bn_bwd4(v4f x, v4f y, v4f d, v4f mu, v4f c0, v4f c1, v4f c2, float leak) {
+  v4f g;
+  g.x = d.x * (y.x > 0.f ? 1.f : leak);
+  g.y = d.y * (y.y > 0.f ? 1.f : leak);
+  g.z = d.z * (y.z > 0.f ? 1.f : leak);
+  g.w = d.w * (y.w > 0.f ? 1.f : leak);
+  v4f o;
+  o.x = (g.x - c0.x - (x.x - mu.x) * c1.x) * c2.x;
+  o.y = (g.y - c0.y - (x.y - mu.y) * c1.y) * c2.y;
+  o.z = (g.z - c0.z - (x.z - mu.z) * c1.z) * c2.z;
+  o.w = (g.w - c0.w - (x.w - mu.w) * c1.w) * c2.w;
+  return o;
 }
 // The same, four planes per thread (plane count and strides multiples of four, arrays 16-byte aligned).
 __global__ void k_bn_bwd_apply4(const float *__restrict__ in, float *__restrict__ d_in, const float *__restrict__ out,
@@ -1227,18 +1229,145 @@ __global__ void k_bn_bwd_apply4(const float *__restrict__ in, float *__restrict_
     const v4f x = *reinterpret_cast<const v4f *>(in + r * in_stride + c);
     const v4f mu = *reinterpret_cast<const v4f *>(save_mean + c), c0 = *reinterpret_cast<const v4f *>(coef + c),
               c1 = *reinterpret_cast<const v4f *>(coef + planes + c), c2 = *reinterpret_cast<const v4f *>(coef + 2 * planes + c);
-    v4f g;
-    g.x = d.x * (y.x > 0.f ? 1.f : leak);
-    g.y = d.y * (y.y > 0.f ? 1.f : leak);
-    g.z = d.z * (y.z > 0.f ? 1.f : leak);
-    g.w = d.w * (y.w > 0.f ? 1.f : leak);
-    v4f o;
-    o.x = (g.x - c0.x - (x.x - mu.x) * c1.x) * c2.x;
-    o.y = (g.y - c0.y - (x.y - mu.y) * c1.y) * c2.y;
-    o.z = (g.z - c0.z - (x.z - mu.z) * c1.z) * c2.z;
-    o.w = (g.w - c0.w - (x.w - mu.w) * c1.w) * c2.w;
-    *reinterpret_cast<v4f *>(d_in + r * in_stride + c) = o;
+    *reinterpret_cast<v4f *>(d_in + r * in_stride + c) = bn_bwd4(x, y, d, mu, c0, c1, c2, leak);
   }
+}
+// Small levels: statistics, their use and the pass over the rows in one launch, a workgroup to sixteen planes.  The deep levels of a
+// network are hundreds of rows, and what their batch norms cost is launches (three each way, 4 us apiece and their gaps).  The sums
+// come in k_colsum's and pair_sums64's order, so that the results are theirs to the bit: part p = (row block, row mod RW) is one
+// thread's sum, the RW parts of a block are added in fp32 and the blocks in double.
+// Bound by latencies: a chain of up to 16 rows, two passes through LDS and the rows once more, from L2, all on one compute unit per
+// sixteen planes.  Forward and backward together, us, three launches each / one: 90 rows x 64 planes 14.7 / 8.5, 256 17.8 / 10.2, 768
+// 18.5 / 13.7, 1500 19.6 / 20.0 (and four launches less for the host), 2048 18.9 / 22.4: up to six row blocks, 1536 rows.
+constexpr int BN_SMALL_PARTS = 384, BN_SMALL_BLOCKS = 6;
+struct BnRows {
+  const float *in, *out, *d_out;  // of the forward pass: in alone
+  int64_t rows, in_stride, out_stride;
+  int planes, rw, blocks;
+  int64_t rows_per_block;
+};
+static bool bn_small(const BnRows &r) {
+  return r.planes % 4 == 0 && r.blocks <= BN_SMALL_BLOCKS && r.blocks * r.rw <= BN_SMALL_PARTS;
+}
+// The sums of plane blockIdx.x * 16 + threadIdx.x for threads below 16; every thread of the workgroup (1024) calls it.
+template <bool BACKWARD>
+__device__ inline void bn_small_sums(const BnRows &t, const float *mean, float leak, double &s1, double &s2) {
+  __shared__ v4f part[2][BN_SMALL_PARTS][4];
+  __shared__ float block_sum[2][BN_SMALL_BLOCKS][16];
+  const int quad = threadIdx.x & 3, c = blockIdx.x * 16 + 4 * quad, n_parts = t.blocks * t.rw;
+  if (c < t.planes) {
+    v4f mu = (v4f){0.f, 0.f, 0.f, 0.f};
+    if (BACKWARD) mu = (v4f){mean[c], mean[c + 1], mean[c + 2], mean[c + 3]};
+    for (int p = threadIdx.x >> 2; p < n_parts; p += 256) {
+      const int64_t r0 = (int64_t)(p / t.rw) * t.rows_per_block, r1 = min(t.rows, r0 + t.rows_per_block);
+      v4f a = (v4f){0.f, 0.f, 0.f, 0.f}, b = a;
+#pragma unroll 4
+      for (int64_t r = r0 + p % t.rw; r < r1; r += t.rw) {
+        const v4f x = *reinterpret_cast<const v4f *>(t.in + r * t.in_stride + c);
+        if (!BACKWARD) {
+#pragma unroll
+          for (int v = 0; v < 4; v++) a[v] += x[v], b[v] += x[v] * x[v];
+        } else {
+          const v4f d = *reinterpret_cast<const v4f *>(t.d_out + r * t.out_stride + c);
+          const v4f y = *reinterpret_cast<const v4f *>(t.out + r * t.out_stride + c);
+#pragma unroll
+          for (int v = 0; v < 4; v++) {
+            const float g = d[v] * (y[v] > 0.f ? 1.f : leak);
+            a[v] += g;
+            b[v] += (x[v] - mu[v]) * g;
+          }
+        }
+      }
+      part[0][p][quad] = a;
+      part[1][p][quad] = b;
+    }
+  }
+  __syncthreads();
+  const float *flat = reinterpret_cast<const float *>(&part[0][0][0]);
+  for (int e = threadIdx.x; e < t.blocks * 32; e += 1024) {  // (block, sum, plane)
+    const int b = e >> 5, q = (e >> 4) & 1, col = e & 15;
+    float v = 0.f;
+#pragma unroll 8
+    for (int i = 0; i < t.rw; i++) v += flat[(q * BN_SMALL_PARTS + b * t.rw + i) * 16 + col];
+    block_sum[q][b][col] = v;
+  }
+  __syncthreads();
+  s1 = s2 = 0;
+  if (threadIdx.x < 16 && blockIdx.x * 16 + (int)threadIdx.x < t.planes)
+    for (int b = 0; b < t.blocks; b++) s1 += (double)block_sum[0][b][threadIdx.x], s2 += (double)block_sum[1][b][threadIdx.x];
+}
+__global__ __launch_bounds__(1024) void k_bn_train_small(BnRows t, BnTrain p, float *out, float leak) {
+  __shared__ v4f coef[2][4];
+  double s1, s2;
+  bn_small_sums<false>(t, nullptr, leak, s1, s2);
+  const int mine = blockIdx.x * 16 + threadIdx.x;
+  if (threadIdx.x < 16 && mine < t.planes)
+    bn_train_plane(p, mine, t.rows, s1, s2, reinterpret_cast<float *>(coef[0])[threadIdx.x], reinterpret_cast<float *>(coef[1])[threadIdx.x]);
+  __syncthreads();
+  const int quad = threadIdx.x & 3, c = blockIdx.x * 16 + 4 * quad;
+  if (c >= t.planes) return;
+  const v4f sc = coef[0][quad], sh = coef[1][quad];
+#pragma unroll 4
+  for (int64_t r = threadIdx.x >> 2; r < t.rows; r += 256)
+    *reinterpret_cast<v4f *>(out + r * t.out_stride + c) = affine_leaky4(*reinterpret_cast<const v4f *>(t.in + r * t.in_stride + c), sc, sh, leak);
+}
+__global__ __launch_bounds__(1024) void k_bn_bwd_small(BnRows t, BnBackward p, const float *save_mean, float *d_in, float leak) {
+  __shared__ v4f coef[3][4];
+  double s1, s2;
+  bn_small_sums<true>(t, save_mean, leak, s1, s2);
+  const int mine = blockIdx.x * 16 + threadIdx.x;
+  if (threadIdx.x < 16 && mine < t.planes)
+    bn_bwd_plane(p, mine, t.rows, s1, s2, reinterpret_cast<float *>(coef[0])[threadIdx.x], reinterpret_cast<float *>(coef[1])[threadIdx.x],
+                 reinterpret_cast<float *>(coef[2])[threadIdx.x]);
+  __syncthreads();
+  const int quad = threadIdx.x & 3, c = blockIdx.x * 16 + 4 * quad;
+  if (c >= t.planes) return;
+  const v4f mu = (v4f){save_mean[c], save_mean[c + 1], save_mean[c + 2], save_mean[c + 3]};
+  const v4f c0 = coef[0][quad], c1 = coef[1][quad], c2 = coef[2][quad];
+#pragma unroll 4
+  for (int64_t r = threadIdx.x >> 2; r < t.rows; r += 256)
+    *reinterpret_cast<v4f *>(d_in + r * t.in_stride + c) =
+        bn_bwd4(*reinterpret_cast<const v4f *>(t.in + r * t.in_stride + c), *reinterpret_cast<const v4f *>(t.out + r * t.out_stride + c),
+                *reinterpret_cast<const v4f *>(t.d_out + r * t.out_stride + c), mu, c0, c1, c2, leak);
+}
+void bn_train_forward(Metadata *scratch, const float *in, float *out, int64_t rows, int planes, int64_t in_stride,
+                      int64_t out_stride, float *save_mean, float *save_invstd, float *running_mean,
+                      float *running_var, const float *gamma, const float *beta, float eps, float momentum,
+                      float leak, hipStream_t s) {
+  if (planes <= 0) return;
+  if (rows <= 0) {  // no rows: defined statistics (the reference divides by zero here), running ones untouched
+    fill32(save_mean, 0, planes, s);
+    fill32(save_invstd, 0, planes, s);
+    return;
+  }
+  Metadata &m = *scratch;
+  const ColsumPlan p = colsum_plan(rows, planes);
+  const bool vec = planes % 4 == 0 && in_stride % 4 == 0 && out_stride % 4 == 0 && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 16 == 0;
+  const BnRows small{in, nullptr, nullptr, rows, in_stride, out_stride, planes, 256 * 4 / p.CW, p.blocks, p.rows_per_block};
+  if (vec && bn_small(small)) {
+    k_bn_train_small<<<dim3((unsigned)ceil_div(planes, 16)), 1024, 0, s>>>(
+        small, BnTrain{save_mean, save_invstd, running_mean, running_var, gamma, beta, eps, momentum}, out, leak);
+    LAUNCH_CHECK();
+    return;
+  }
+  m.partial.reserve((size_t)p.blocks * 2 * planes);
+  m.prebuf.reserve(2 * (size_t)planes);
+  launch_colsum<1>(dim3(p.blocks, (unsigned)ceil_div(planes, p.CW)), s, in, in_stride, nullptr, nullptr, 0, nullptr,
+                                                                                 0.f, rows, planes, p.CW, p.rows_per_block,
+                                                                                 m.partial.p);
+  k_bn_train_finish<<<dim3((unsigned)ceil_div(planes, 64)), 1024, 0, s>>>(m.partial.p, p.blocks, planes, rows, save_mean,
+                                                                          save_invstd, running_mean, running_var, gamma,
+                                                                          beta, eps, momentum, m.prebuf.p);
+  LAUNCH_CHECK();
+  if (vec) {
+    const int64_t blocks4 = std::min<int64_t>(ceil_div(rows * (planes / 4), TB), 256 * 64);
+    k_affine_leaky4<<<dim3((unsigned)blocks4), TB, 0, s>>>(in, out, rows, planes, in_stride, out_stride, m.prebuf.p, leak);
+    LAUNCH_CHECK();
+    return;
+  }
+  const int64_t blocks = std::min<int64_t>(ceil_div(rows * planes, TB), 256 * 64);
+  k_affine_leaky<<<dim3((unsigned)blocks), TB, 0, s>>>(in, out, rows, planes, in_stride, out_stride, m.prebuf.p, leak);
+  LAUNCH_CHECK();
 }
 // CPU/BatchNormalization.cpp:63-107.  d_out is not modified (the reference scales it in place).
 void bn_backward(Metadata *scratch, const float *in, float *d_in, const float *out, const float *d_out, int64_t rows,
@@ -1252,6 +1381,15 @@ void bn_backward(Metadata *scratch, const float *in, float *d_in, const float *o
   }
   Metadata &m = *scratch;
   const ColsumPlan p = colsum_plan(rows, planes);
+  auto al = [](const float *p) { return (uintptr_t)p % 16 == 0; };
+  const bool vec = planes % 4 == 0 && in_stride % 4 == 0 && out_stride % 4 == 0 && al(in) && al(d_in) && al(out) && al(d_out);
+  const BnRows small{in, out, d_out, rows, in_stride, out_stride, planes, 256 * 4 / p.CW, p.blocks, p.rows_per_block};
+  if (vec && bn_small(small)) {
+    k_bn_bwd_small<<<dim3((unsigned)ceil_div(planes, 16)), 1024, 0, s>>>(small, BnBackward{save_invstd, gamma, d_gamma, d_beta}, save_mean,
+                                                                        d_in, leak);
+    LAUNCH_CHECK();
+    return;
+  }
   m.partial.reserve((size_t)p.blocks * 2 * planes);
   m.prebuf.reserve(3 * (size_t)planes);
   launch_colsum<2>(dim3(p.blocks, (unsigned)ceil_div(planes, p.CW)), s, in, in_stride, d_out, out, out_stride,
@@ -1260,9 +1398,7 @@ void bn_backward(Metadata *scratch, const float *in, float *d_in, const float *o
   k_bn_bwd_finish<<<dim3((unsigned)ceil_div(planes, 64)), 1024, 0, s>>>(m.partial.p, p.blocks, planes, rows, save_invstd,
                                                                         gamma, d_gamma, d_beta, m.prebuf.p);
   LAUNCH_CHECK();
-  auto al = [](const float *p) { return (uintptr_t)p % 16 == 0; };
-  if (planes % 4 == 0 && in_stride % 4 == 0 && out_stride % 4 == 0 && al(in) && al(d_in) && al(out) && al(d_out) &&
-      al(save_mean)) {
+  if (vec && al(save_mean)) {
     const int64_t blocks4 = std::min<int64_t>(ceil_div(rows * (planes / 4), TB), 256 * 64);
     k_bn_bwd_apply4<<<dim3((unsigned)blocks4), TB, 0, s>>>(in, d_in, out, d_out, rows, planes, in_stride, out_stride,
                                                            save_mean, m.prebuf.p, leak);
