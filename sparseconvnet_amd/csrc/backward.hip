@@ -323,15 +323,21 @@ __global__ __launch_bounds__(256) void k_conv_dw(const int *__restrict__ nbr, co
 }
 // The same sums for narrow layers (both channel counts <= 32), where the kernel above spends its
 // time re-reading: one workgroup per tap reads the rows of b once per tap, 27 times in all.  Here
-// a workgroup of eight wavefronts takes a share of the positions and a 32 x 32 channel tile for
-// ALL taps: wavefront w keeps the accumulators of taps w, w + 8, w + 16, w + 24 (16 registers
+// a workgroup of sixteen wavefronts takes a share of the positions and a 32 x 32 channel tile for
+// ALL taps: wavefront w keeps the accumulators of taps w and w + 16 (16 registers
 // each) and walks its share 16 positions (one granule of the tap masks) at a time, skipping the
-// taps the granule does not have.  Nothing goes through LDS: the MFMA contracts over four positions,
+// taps the granule does not have.  No row goes through LDS: the MFMA contracts over four positions,
 // lane (r, g) supplies position 4 g + kk of the granule and, of that position's row, the two
 // channels 2 r and 2 r + 1 as one 8-byte load (16 lanes read 128 consecutive bytes); instruction
 // i of a pair takes component i, so that it computes the gradient's rows 2 * (MFMA row) + i, and
-// likewise for the columns.  The rows of b are loaded once per granule and serve all its taps.
-constexpr int DT_NW = 8, DT_T = 32, DT_SLOTS = 4, DT_BLOCK = 8;  // DT_BLOCK granules of 16 positions per turn
+// likewise for the columns.  The rows of b are loaded once per granule and serve both taps.
+// Indices, rows and masks of a block of DT_BLOCK granules come to LDS while the block before is worked on, one barrier per
+// block; a tap's rows of the next granule are requested as soon as its MFMAs have freed the registers.
+// Bound by the matrix instructions next to that barrier: 13 of 27 taps a granule of the room surfaces has are 200 us of fp32 MFMAs
+// at a million sites if the four SIMDs share them evenly.  us, eight wavefronts of four taps, two workgroups per compute unit and
+// two memory latencies in a row per granule / this: a million sites 32 x 32 508 / 465, and half the partial sums; the whole backward
+// call, 98 k 32 x 32 98 / 91, 24 k 52 / 48, 6 k 16 x 16 42 / 33, 1 k 37 / 33.  (Eight wavefronts with these loads spill: 546.)
+constexpr int DT_NW = 16, DT_T = 32, DT_SLOTS = 2, DT_BLOCK = 8;  // DT_BLOCK granules of 16 positions per turn
 template <bool VEC2>
 __global__ __launch_bounds__(DT_NW * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_conv_dw_taps(const int *__restrict__ nbr, const int *__restrict__ rowmap,
                                                              const unsigned *__restrict__ gmask, int K, int64_t n,
@@ -375,61 +381,88 @@ __global__ __launch_bounds__(DT_NW * 64) __attribute__((amdgpu_waves_per_eu(4, 4
     if (wave + sl * DT_NW < K) own |= 1u << (wave + sl * DT_NW);
   // Workgroup x takes the blocks of DT_BLOCK granules x, x + gridDim.x, ...: every workgroup sees
   // every part of the pattern-sorted table, so that they all carry about the same number of rules.
-  const int n_granules = (int)((n + 15) >> 4), n32 = (int)n;  // the host checks that 4 K npad < 2^31
-  for (int gb = blockIdx.x * DT_BLOCK; gb < n_granules; gb += gridDim.x * DT_BLOCK) {
-    const int ge = min(n_granules, gb + DT_BLOCK);
-    for (int gi = gb; gi < ge; gi++) {
-      const unsigned present = gmask[gi] & own;
-      if (present == 0u) continue;  // uniform over the wavefront
-      const int t0 = gi << 4;
-      // this lane's four positions of the granule: t0 + 4 g + kk; first the index quads of the
-      // wavefront's taps, then all gathers, then the MFMAs: two memory latencies per granule
-      // (fetching the next granule's quads meanwhile costs more registers than there are at
-      // four wavefronts per SIMD, and measured slower with fewer)
-      int4 j4[DT_SLOTS];
-      const unsigned toff = (unsigned)(t0 + 4 * g) * 4u;
+  const int n_blocks = (int)((n + 16 * DT_BLOCK - 1) / (16 * DT_BLOCK)), n32 = (int)n;  // the host checks that 4 K npad < 2^31
+  constexpr int PER = DT_NW * DT_SLOTS * 4 * DT_BLOCK / (DT_NW * 64);  // 16-byte loads of a block's indices per thread
+  __shared__ int4 jtab[2][DT_NW * DT_SLOTS][4 * DT_BLOCK];  // [tap][position / 4]
+  __shared__ int rows[2][16 * DT_BLOCK];
+  __shared__ unsigned masks[2][DT_BLOCK];
+  int4 nj[PER];
+  int nrow = -1;
+  unsigned nmask = 0u;
+  auto fetch = [&](int blk) {  // a block's indices, rows of b and masks on their way; past the last block nothing
+    const bool there = blk < n_blocks;
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+      const int e = threadIdx.x + i * DT_NW * 64, k = e / (4 * DT_BLOCK), p = 16 * DT_BLOCK * blk + 4 * (e % (4 * DT_BLOCK));
+      nj[i] = __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(
+                                           nbr_rsrc, there && k < K && p < npad ? ((unsigned)k * (unsigned)npad + (unsigned)p) * 4u : nowhere, 0, 0));
+    }
+    const int t = 16 * DT_BLOCK * blk + (int)threadIdx.x;
+    nrow = -1;
+    if (threadIdx.x < 16 * DT_BLOCK && there && t < n32) nrow = rowmap ? rowmap[t] : t;
+    nmask = 0u;
+    if (threadIdx.x < DT_BLOCK && there && 16 * (DT_BLOCK * blk + (int)threadIdx.x) < n32) nmask = gmask[DT_BLOCK * blk + threadIdx.x];
+  };
+  auto put = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+      const int e = threadIdx.x + i * DT_NW * 64;
+      jtab[buf][e / (4 * DT_BLOCK)][e % (4 * DT_BLOCK)] = nj[i];
+    }
+    if (threadIdx.x < 16 * DT_BLOCK) rows[buf][threadIdx.x] = nrow;
+    if (threadIdx.x < DT_BLOCK) masks[buf][threadIdx.x] = nmask;
+  };
+  v2f av[DT_SLOTS][4], bv[4], bn[4];
+  auto issue_a = [&](int buf, int gl, unsigned present, int sl) {
+    const int k = wave + sl * DT_NW;
+    const bool has = (present >> k) & 1u;
+    const int4 j4 = jtab[buf][k][4 * gl + g];
+    const int j[4] = {j4.x, j4.y, j4.z, j4.w};
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) av[sl][kk] = pair_of(a_rsrc, has ? j[kk] : -1, a_row_bytes, ca0, ca1);
+  };
+  auto issue_b = [&](int buf, int gl, unsigned present, v2f (&dst)[4]) {
+    const int4 r4 = *reinterpret_cast<const int4 *>(&rows[buf][16 * gl + 4 * g]);
+    const int r[4] = {r4.x, r4.y, r4.z, r4.w};
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) dst[kk] = pair_of(b_rsrc, present ? r[kk] : -1, b_row_bytes, cb0, cb1);
+  };
+  fetch(blockIdx.x);
+  put(0);
+  __syncthreads();
+  unsigned present = __builtin_amdgcn_readfirstlane(masks[0][0]) & own;
+  issue_b(0, 0, present, bv);
+#pragma unroll
+  for (int sl = 0; sl < DT_SLOTS; sl++) issue_a(0, 0, present, sl);
+  int buf = 0;
+  for (int blk = blockIdx.x; blk < n_blocks; blk += gridDim.x, buf ^= 1) {
+    fetch(blk + gridDim.x);
+#pragma unroll 1
+    for (int gl = 0; gl < DT_BLOCK; gl++) {
+      const bool over = gl == DT_BLOCK - 1;
+      if (over) {  // nothing of the other buffer is read any more: its last granule was issued before the barrier in front of this block
+        put(buf ^ 1);
+        __syncthreads();
+      }
+      const int nb = over ? buf ^ 1 : buf, ngl = over ? 0 : gl + 1;
+      const unsigned next = __builtin_amdgcn_readfirstlane(masks[nb][ngl]) & own;
+      issue_b(nb, ngl, next, bn);
 #pragma unroll
       for (int sl = 0; sl < DT_SLOTS; sl++) {
-        const int k = wave + sl * DT_NW;
-        // a tap the granule does not have: an offset past the table, which reads zeros; made -1 below
-        j4[sl] = __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(
-                                              nbr_rsrc, ((present >> k) & 1u) ? toff : nowhere, (unsigned)k * (unsigned)npad * 4u, 0));
-      }
-      v2f bv[4];
-      if (rowmap) {
-        const int4 r4 = *reinterpret_cast<const int4 *>(rowmap + t0 + 4 * g);
-        const int r[4] = {r4.x, r4.y, r4.z, r4.w};
+        if ((present >> (wave + sl * DT_NW)) & 1u) {  // uniform over the wavefront
 #pragma unroll
-        for (int kk = 0; kk < 4; kk++) bv[kk] = pair_of(b_rsrc, t0 + 4 * g + kk < n32 ? r[kk] : -1, b_row_bytes, cb0, cb1);
-      } else {
+          for (int kk = 0; kk < 4; kk++)
 #pragma unroll
-        for (int kk = 0; kk < 4; kk++) {
-          const int t = t0 + 4 * g + kk;
-          bv[kk] = pair_of(b_rsrc, t < n32 ? t : -1, b_row_bytes, cb0, cb1);
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+              for (int jx = 0; jx < 2; jx++)
+                acc[sl][i][jx] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[sl][kk][i], bv[kk][jx], acc[sl][i][jx], 0, 0, 0);
         }
+        issue_a(nb, ngl, next, sl);  // the registers are free
       }
-      v2f av[DT_SLOTS][4];
+      present = next;
 #pragma unroll
-      for (int sl = 0; sl < DT_SLOTS; sl++) {
-        const int k = wave + sl * DT_NW;
-        const bool has = (present >> k) & 1u;
-        const int j[4] = {j4[sl].x, j4[sl].y, j4[sl].z, j4[sl].w};
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++) av[sl][kk] = pair_of(a_rsrc, has ? j[kk] : -1, a_row_bytes, ca0, ca1);
-      }
-#pragma unroll
-      for (int sl = 0; sl < DT_SLOTS; sl++) {
-        const int k = wave + sl * DT_NW;
-        if (!((present >> k) & 1u)) continue;  // uniform over the wavefront
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++)
-#pragma unroll
-          for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int jx = 0; jx < 2; jx++)
-              acc[sl][i][jx] =
-                  __builtin_amdgcn_mfma_f32_16x16x4f32(av[sl][kk][i], bv[kk][jx], acc[sl][i][jx], 0, 0, 0);
-      }
+      for (int kk = 0; kk < 4; kk++) bv[kk] = bn[kk];
     }
   }
   // acc[sl][i][jx][r] = dW[k][ct*32 + 2 (4 g + r) + i][ot*32 + 2 r16 + jx] of this chunk
@@ -870,8 +903,8 @@ static void weight_gradient(Metadata &m, const Table &t, const float *a, int64_t
       (int64_t)t.K * t.npad * 4 < ((int64_t)1 << 31)) {
     // narrow layers: all taps per workgroup
     const int tiles = (int)(ceil_div(n_a, DT_T) * ceil_div(n_b, DT_T));
-    // one resident round: two workgroups per compute unit, shared between the channel tiles
-    const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(ceil_div(t.n, 16 * DT_BLOCK), 512 / tiles));
+    // one resident round: a workgroup per compute unit, shared between the channel tiles
+    const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(ceil_div(t.n, 16 * DT_BLOCK), 256 / tiles));
     m.partial.reserve((size_t)chunks * per_chunk);
     const dim3 grid((unsigned)chunks, (unsigned)tiles);
     const bool vec2 = n_a % 2 == 0 && n_b % 2 == 0 && (uintptr_t)a % 8 == 0 && (uintptr_t)b % 8 == 0;
