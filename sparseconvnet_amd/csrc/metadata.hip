@@ -2655,8 +2655,15 @@ StridedRules &strided_rules(Metadata &m, const int64_t *in_size, const int64_t *
 // time, find a coarse row that one of them fetched still in that XCD's L2; with an eighth of a
 // million-site level per range every tap's run fetched its 4 MB of coarse rows again (counters:
 // 268 MB read for 95 MB of operands).
+// The window's workgroup writes the table as well: position t of it is position src of the schedule, its one entry, -1 in the
+// other taps, its row, and the granule masks (an OR over the 16 lanes of a granule).  Bound by the table's bytes (4 K + 17 per position)
+// and, on small levels, by launches: with the order through memory and a second kernel a million positions took 37 us and
+// six levels from a million down 147, 22 and 62 so (windows of 4096: 152, too few workgroups for the stores).
 template <int ITEMS>
-__global__ __launch_bounds__(RS1_THREADS) void k_few_order(const int *in_tap, int64_t n, int *perm) {
+__global__ __launch_bounds__(RS1_THREADS) void k_few_table(const int *__restrict__ in_tap, const int *__restrict__ in_row, int K, int64_t n,
+                                                          int64_t npad, const int *__restrict__ base_rows, int *__restrict__ nbr,
+                                                          int *__restrict__ rowmap, unsigned *__restrict__ gmask,
+                                                          unsigned char *__restrict__ few_tap, int *__restrict__ few_row) {
   __shared__ BlockSort<ITEMS> sh;
   constexpr int WINDOW = RS1_THREADS * ITEMS;
   const int64_t base = (int64_t)blockIdx.x * WINDOW;
@@ -2673,28 +2680,24 @@ __global__ __launch_bounds__(RS1_THREADS) void k_few_order(const int *in_tap, in
     val[r] = i;
   }
   block_sort<ITEMS>(sh, key, val, valid, 5, 5);
-  const int here = (int)min<int64_t>(WINDOW, n - base);
-  for (int i = threadIdx.x; i < here; i += RS1_THREADS) perm[base + i] = (int)(base + sh.sval[i]);
-}
-// Position t of the sorted table is position perm[t] of the schedule: its one entry, -1 in the
-// other taps, its row, and the granule masks (an OR over the 16 lanes of a granule).
-__global__ void k_table_expand_few(const int *in_tap, const int *in_row, int K, int64_t n, int64_t npad, const int *perm,
-                                   const int *base, int *nbr, int *rowmap, unsigned *gmask, unsigned char *few_tap,
-                                   int *few_row) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  unsigned mk = 0;
-  if (t < n) {
-    const int src = perm[t];
-    const int tap = in_tap[src], row = in_row[src];
-    few_tap[t] = tap >= 0 ? (unsigned char)tap : (unsigned char)255;
-    few_row[t] = tap >= 0 ? row : 0;
-    for (int k = 0; k < K; k++) nbr[(int64_t)k * npad + t] = k == tap ? row : -1;
-    mk = tap >= 0 ? 1u << tap : 0u;
-    rowmap[t] = base ? base[src] : src;
-  }
 #pragma unroll
-  for (int o = 1; o < 16; o <<= 1) mk |= __shfl_xor(mk, o, 64);
-  if ((threadIdx.x & 15) == 0 && t < n) gmask[t >> 4] = mk;
+  for (int q = 0; q < ITEMS; q++) {
+    const int i = q * RS1_THREADS + (int)threadIdx.x;
+    const int64_t t = base + i;
+    unsigned mk = 0;
+    if (t < n) {
+      const int64_t src = base + sh.sval[i];
+      const int tap = sh.skey[i] == 16ull ? -1 : (int)sh.skey[i], row = in_row[src];
+      few_tap[t] = tap >= 0 ? (unsigned char)tap : (unsigned char)255;
+      few_row[t] = tap >= 0 ? row : 0;
+      for (int k = 0; k < K; k++) nbr[(int64_t)k * npad + t] = k == tap ? row : -1;
+      mk = tap >= 0 ? 1u << tap : 0u;
+      rowmap[t] = base_rows ? base_rows[src] : (int)src;
+    }
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) mk |= __shfl_xor(mk, o, 64);
+    if ((threadIdx.x & 15) == 0 && t < n) gmask[t >> 4] = mk;
+  }
 }
 
 void finish_by_in(Metadata &m, StridedRules &r, hipStream_t s) {
@@ -2704,20 +2707,16 @@ void finish_by_in(Metadata &m, StridedRules &r, hipStream_t s) {
   m.builds++;
   Table &t = r.by_in;
   if (r.by_in_compact && t.n > 0) {
-    m.v1.reserve(t.n);  // the order: position t of the table is position v1[t] of the schedule
-    constexpr int FEW_ITEMS = 4;  // windows of 4096 positions (1024, 2048 and 8192 measured alike)
+    constexpr int FEW_ITEMS = 2;  // windows of 2048 positions
     const int window = RS1_THREADS * FEW_ITEMS;
     t.spread = window >= t.n;
-    k_few_order<FEW_ITEMS><<<dim3((unsigned)ceil_div(t.n, window)), RS1_THREADS, 0, s>>>(r.in_tap.p, t.n, m.v1.p);
-    LAUNCH_CHECK();
     t.nbr.reserve((size_t)t.K * t.npad);
     t.rowmap.reserve(t.npad);
     t.gmask.reserve(ceil_div(t.n, 16));
     t.few_tap.reserve(t.n);
     t.few_row.reserve(t.n);
-    k_table_expand_few<<<grid_for(t.n), TB, 0, s>>>(r.in_tap.p, r.in_row.p, t.K, t.n, t.npad, m.v1.p,
-                                                    li->second.sched_ptr(), t.nbr.p, t.rowmap.p, t.gmask.p, t.few_tap.p,
-                                                    t.few_row.p);
+    k_few_table<FEW_ITEMS><<<dim3((unsigned)ceil_div(t.n, window)), RS1_THREADS, 0, s>>>(
+        r.in_tap.p, r.in_row.p, t.K, t.n, t.npad, li->second.sched_ptr(), t.nbr.p, t.rowmap.p, t.gmask.p, t.few_tap.p, t.few_row.p);
     LAUNCH_CHECK();
     t.identity_rows = false;
     r.in_tap.release();
@@ -2747,35 +2746,60 @@ void finish_by_in(Metadata &m, StridedRules &r, hipStream_t s) {
 
 // ---- identity table -----------------------------------------------------------------------
 
-__global__ void k_identity_table(int64_t n, int64_t npad, int *nbr, unsigned *gmask) {
+constexpr int IDENT_JOBS = 16;
+struct IdentJobs {
+  int64_t n[IDENT_JOBS], npad[IDENT_JOBS];
+  int *nbr[IDENT_JOBS];
+  unsigned *gmask[IDENT_JOBS];
+};
+__global__ void k_identity_tables(IdentJobs j) {  // blockIdx.y: table
+  const int q = blockIdx.y;
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < npad) nbr[t] = t < n ? (int)t : -1;
-  if (t < (n + 15) / 16) gmask[t] = 1u;
+  if (t < j.npad[q]) j.nbr[q][t] = t < j.n[q] ? (int)t : -1;
+  if (t < (j.n[q] + 15) / 16) j.gmask[q][t] = 1u;
 }
 
 // A 1x1 convolution (NetworkInNetwork, CPU/NetworkInNetwork.cpp:7-23) is the convolution
-// over this table: one tap, position t reads row t and writes row t.
+// over this table: one tap, position t reads row t and writes row t.  The first one makes those of the handle's other
+// levels as well, by the same launch, where they are small: a network that has a 1x1 convolution on one level has one on others,
+// and each would be a launch of its own and an event that the other stream waits for, some 8 us, for what 64 k rows write in 2.
+constexpr int64_t IDENT_AHEAD = 65536;
 Table &identity_table(Metadata &m, int64_t rows, hipStream_t s) {
   auto it = m.ident.find(rows);
   if (it != m.ident.end()) return it->second;
   m.builds++;
-  Table t;
-  t.K = 1;
-  t.n = rows;
-  t.npad = round_up(std::max<int64_t>(rows, 1), 64);
-  t.identity_rows = true;
-  t.identity_few = true;
-  t.cnt = std::make_shared<Counts>();
-  t.cnt->K = 1;
-  t.cnt->host.assign(1, rows);
-  t.cnt->ready = true;
-  if (rows > 0) {
-    t.nbr.reserve(t.npad);
-    t.gmask.reserve(ceil_div(rows, 16));
-    k_identity_table<<<grid_for(t.npad), TB, 0, s>>>(rows, t.npad, t.nbr.p, t.gmask.p);
+  IdentJobs jobs{};
+  int n_jobs = 0;
+  int64_t most = 0;
+  auto make = [&](int64_t n) {
+    if (n_jobs == IDENT_JOBS || m.ident.count(n)) return;
+    Table t;
+    t.K = 1;
+    t.n = n;
+    t.npad = round_up(std::max<int64_t>(n, 1), 64);
+    t.identity_rows = true;
+    t.identity_few = true;
+    t.cnt = std::make_shared<Counts>();
+    t.cnt->K = 1;
+    t.cnt->host.assign(1, n);
+    t.cnt->ready = true;
+    if (n > 0) {
+      t.nbr.reserve(t.npad);
+      t.gmask.reserve(ceil_div(n, 16));
+      jobs.n[n_jobs] = n, jobs.npad[n_jobs] = t.npad, jobs.nbr[n_jobs] = t.nbr.p, jobs.gmask[n_jobs] = t.gmask.p;
+      n_jobs++;
+      most = std::max(most, t.npad);
+    }
+    m.ident.emplace(n, std::move(t));
+  };
+  make(rows);
+  for (const auto &l : m.levels)
+    if (l.second.n > 0 && l.second.n <= IDENT_AHEAD) make(l.second.n);
+  if (n_jobs) {
+    k_identity_tables<<<dim3((unsigned)ceil_div(most, TB), n_jobs), TB, 0, s>>>(jobs);
     LAUNCH_CHECK();
   }
-  return m.ident.emplace(rows, std::move(t)).first->second;
+  return m.ident.at(rows);
 }
 
 // ---- pair-list export (ballot / prefix compaction) --------------------------------------
