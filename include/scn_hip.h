@@ -333,6 +333,9 @@ scn_params *scn_params_create(void);
 void scn_params_destroy(scn_params *p);
 int scn_params_clear(scn_params *p);
 int scn_md_use_params(scn_metadata *md, scn_params *p);
+/* The NEXT convolution call on md is a forward pass whose output will be differentiated: it runs in the kernels whose
+ * rounding a training run has seen, not in faster ones that round differently. */
+int scn_md_next_differentiated(scn_metadata *md);
 
 /* ActivePooling_updateOutput / ActivePooling_updateGradInput (pybind.cpp:34-43,
  * CPU/ActivePooling.cpp:8-83): out [batchSize, planes] = per sample the sum of its active rows, times

@@ -1009,6 +1009,9 @@ int scn_params_clear(scn_params *p) {
 int scn_md_use_params(scn_metadata *h, scn_params *p) {
   return guarded([&] { md(h).frozen = p ? &p->p : nullptr; });
 }
+int scn_md_next_differentiated(scn_metadata *h) {
+  return guarded([&] { md(h).differentiated = true; });
+}
 int scn_active_pooling_fwd(scn_metadata *h, const int64_t *spatial, const float *in, float *out, int planes,
                            int average, void *stream) {
   return guarded([&] {

@@ -472,10 +472,11 @@ static void dispatch_bf(Metadata &m, const Table &t, const float *in, float *out
 #undef BF
 }
 bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in, int n_out, bool gradient) {
-  // Forward sums over nine taps (the 3 x 3 filters of 2-D networks) stay where they were, k_conv_resident and k_conv_split: values on
-  // the edge of a ReLU change sides with any other rounding, and a 2-D network of a few thousand sites has so few that a training
-  // step's gradients differ by up to 3.5e-3 then.  Its time is the host's, so that it would not run faster either (1.21 / 1.26 ms).
-  if (t.K == 9 && !gradient) return false;
+  // Forward sums that will be differentiated, and those over nine taps (the 3 x 3 filters of 2-D networks, whose time is the host's:
+  // 1.21 / 1.26 ms for a batch of pen strokes), keep their rounding in k_conv_resident and k_conv_split: with another one values on the edge
+  // of a ReLU change sides, and the gradients of a training step over some ten thousand sites differ by up to 9e-3 (2-D: 3.5e-3).  A
+  // million-site step takes 1 % longer for it.
+  if ((t.K == 9 || m.differentiated) && !gradient) return false;
   if (m.fixed_scratch || t.K > 32 || !t.gmask.p) return false;
   if (n_in <= 4 || n_in % 4 || (uintptr_t)in % 16 || n_in * 4 >= (1 << 24)) return false;
   if (in_rows <= 0 || in_rows >= (1 << 24) || in_rows * n_in * 4 >= ((int64_t)1 << 31)) return false;

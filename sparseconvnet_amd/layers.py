@@ -73,6 +73,7 @@ def _use_frozen(module, md, weight, bias, pre=None, post=None, second=None):
 class _NoGrad:
     """What a Function's forward is handed in place of its context when nothing will be
     differentiated: attributes can be set on it, saved tensors are dropped."""
+    needs_input_grad = ()
 
     def save_for_backward(self, *tensors):
         pass
@@ -97,6 +98,8 @@ class _ConvFunction(Function):
         ctx.has_bias = bias.numel() > 0
         ctx.save_for_backward(features, weight)
         fn = (md.submanifoldConvolution, md.convolution, md.deconvolution)[kind]
+        if any(ctx.needs_input_grad):
+            md.nextDifferentiated()
         out, _ = fn(*sizes, features, weight, bias, pre, post, want_macs=False, out=out, second=second)
         _count(out)
         return out
@@ -118,6 +121,8 @@ class _NetworkInNetworkFunction(Function):
     def forward(ctx, features, weight, bias, md):
         ctx.md, ctx.has_bias = md, bias.numel() > 0
         ctx.save_for_backward(features, weight)
+        if any(ctx.needs_input_grad):
+            md.nextDifferentiated()
         out, _ = md.networkInNetwork(features, weight, bias, want_macs=False)
         _count(out)
         return out

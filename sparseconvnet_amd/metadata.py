@@ -100,6 +100,10 @@ class Metadata:
             self._h = None
             self._L.scn_md_destroy(h)  # does not wait for the GPU; the counts it owes are kept (MacCounter)
 
+    def nextDifferentiated(self):
+        """The next convolution's output will be differentiated: its sums keep the rounding a training run has seen."""
+        _lib.check(self._L.scn_md_next_differentiated(self._h))
+
     def takeMacs(self):
         """Multiply-adds of the convolutions run on this Metadata since the last call whose
         count was not returned to the caller directly (synchronises the stream once)."""

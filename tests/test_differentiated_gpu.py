@@ -1,0 +1,29 @@
+"""A convolution whose output will be differentiated runs in the kernels that served it before k_conv_wave, for that one call."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,planes", [(3001, 16), (30001, 32), (2001, 48)])
+def test_one_call_keeps_its_rounding(n, planes):
+    import torch
+    import sparseconvnet_amd as scn
+    g = torch.Generator().manual_seed(n)
+    side = 96
+    cells = torch.randperm(side ** 3, generator=g)[:n]
+    coords = torch.stack([cells // side ** 2, cells // side % side, cells % side], 1)
+    t = scn.InputLayer(3, side, mode=0)([coords.cuda(), torch.zeros(n, 1).cuda()])
+    x = scn.SparseConvNetTensor(torch.randn(n, planes, generator=g).cuda(), t.metadata, t.spatial_size)
+    conv = scn.SubmanifoldConvolution(3, planes, planes, 3, False).cuda()
+
+    def kernel():
+        return t.metadata._L.scn_md_last_conv_kernel(t.metadata._h).decode()
+    with torch.no_grad():
+        a = conv(x).features
+    assert "split wave" in kernel()
+    b = conv(x).features
+    assert "split wave" not in kernel()
+    with torch.no_grad():
+        c = conv(x).features
+    assert "split wave" in kernel() and torch.equal(a, c)
+    assert (a - b).norm() <= 1e-6 * a.norm()
