@@ -473,11 +473,11 @@ static void dispatch_bf(Metadata &m, const Table &t, const float *in, float *out
 }
 bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in, int n_out, bool gradient) {
   // Forward sums that will be differentiated, and those over nine taps (the 3 x 3 filters of 2-D networks, whose time is the host's:
-  // 1.07 / 1.07 ms for a batch of pen strokes), keep their rounding in k_conv_resident and k_conv_split: with another one values on the edge
-  // of a ReLU change sides, and the gradients of a training step over some ten thousand sites differ by up to 9e-3 (2-D: 3.5e-3).  From
-  // 300 k sites on neither this kernel nor k_conv_split deals taps out, and more than 16 channels give the same sums to the bit.
-  const bool same_bits = !m.bf16 && t.K > 9 && t.n >= 300000 && n_in > 16;
-  if ((t.K == 9 || (m.differentiated && !same_bits)) && !gradient) return false;
+  // 1.21 / 1.26 ms for a batch of pen strokes), keep their rounding in k_conv_resident and k_conv_split: with another one values on the edge
+  // of a ReLU change sides, and the gradients of a training step over some ten thousand sites differ by up to 9e-3 (2-D: 3.5e-3).  A
+  // million-site step takes 1 % longer for it.
+  if ((t.K == 9 || m.differentiated) && !gradient) return false;
+  if (m.fixed_scratch || t.K > 32 || !t.gmask.p) return false;
   if (n_in <= 4 || n_in % 4 || (uintptr_t)in % 16 || n_in * 4 >= (1 << 24)) return false;
   if (in_rows <= 0 || in_rows >= (1 << 24) || in_rows * n_in * 4 >= ((int64_t)1 << 31)) return false;
   if (m.bf16) return !gradient && bf_tile(t, n_in, n_out) != BF_NONE;  // (these weights are packed from a transposed copy)

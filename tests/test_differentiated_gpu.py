@@ -27,23 +27,3 @@ def test_one_call_keeps_its_rounding(n, planes):
         c = conv(x).features
     assert "split wave" in kernel() and torch.equal(a, c)
     assert (a - b).norm() <= 1e-6 * a.norm()
-
-
-@pytest.mark.parametrize("n,cin,cout", [(300001, 32, 32), (300001, 64, 24), (600001, 48, 32), (310001, 20, 20)])
-def test_large_levels_have_one_rounding(n, cin, cout):
-    """From 300 k sites on k_conv_wave adds in k_conv_split's order: the same bits, so that differentiated calls use it as well."""
-    import torch
-    from test_conv_split_gpu import _table
-    conv, rules, rows_in, rows_out, md = _table("subm", n, 8400)
-    g = torch.Generator().manual_seed(n + cin)
-    x, w = torch.randn(rows_in, cin, generator=g).cuda(), torch.randn(len(rules), 1, cin, cout, generator=g).cuda() * 0.1
-    bias = torch.randn(cout, generator=g).cuda()
-    md.nextDifferentiated()
-    got = conv(x, w, bias)
-    assert "split wave" in md._L.scn_md_last_conv_kernel(md._h).decode()
-    # 52 planes of which the first cout are these: k_conv_split, a tile's columns do not depend on one another
-    wide = torch.zeros(len(rules), 1, cin, 52).cuda()
-    wide[..., :cout] = w
-    want = conv(x, wide, torch.cat([bias, torch.zeros(52 - cout).cuda()]))
-    assert "split ncbw" in md._L.scn_md_last_conv_kernel(md._h).decode()
-    assert torch.equal(got, want[:, :cout])
