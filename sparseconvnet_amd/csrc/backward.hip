@@ -334,16 +334,17 @@ __global__ __launch_bounds__(256) void k_conv_dw(const int *__restrict__ nbr, co
 // Indices, rows and masks of a block of DT_BLOCK granules come to LDS while the block before is worked on, one barrier per
 // block; a tap's rows of the next granule are requested as soon as its MFMAs have freed the registers.
 // Bound by the matrix instructions next to that barrier: 13 of 27 taps a granule of the room surfaces has are 200 us of fp32 MFMAs
-// at a million sites if the four SIMDs share them evenly.  us, eight wavefronts of four taps, two workgroups per compute unit and
-// two memory latencies in a row per granule / this: a million sites 32 x 32 508 / 465, and half the partial sums; the whole backward
-// call, 98 k 32 x 32 98 / 91, 24 k 52 / 48, 6 k 16 x 16 42 / 33, 1 k 37 / 33.  (Eight wavefronts with these loads spill: 546.)
+// at a million sites if the four SIMDs share them evenly.  The whole backward call, us (graph replays), eight wavefronts of four
+// taps, two workgroups per compute unit and two memory latencies in a row per granule / this: a million sites 32 x 32 745 / 683, 16 x 16
+// 575 / 540, 300 k 32 x 32 250 / 235, 98 k 111 / 101, 24 k 63 / 48, 6 k 16 x 16 54 / 33; the same bits.  (Eight wavefronts with these
+// loads spill.)
 constexpr int DT_NW = 16, DT_T = 32, DT_SLOTS = 2, DT_BLOCK = 8;  // DT_BLOCK granules of 16 positions per turn
 template <bool VEC2>
 __global__ __launch_bounds__(DT_NW * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_conv_dw_taps(const int *__restrict__ nbr, const int *__restrict__ rowmap,
                                                              const unsigned *__restrict__ gmask, int K, int64_t n,
                                                              int64_t npad, const float *__restrict__ a, int n_a,
                                                              unsigned a_bytes, const float *__restrict__ b, int n_b,
-                                                             unsigned b_bytes, float *__restrict__ partial) {
+                                                             unsigned b_bytes, float *__restrict__ partial, int shares) {
   const int tiles_o = (n_b + DT_T - 1) / DT_T;
   const int ct = blockIdx.y / tiles_o, ot = blockIdx.y % tiles_o;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -379,8 +380,9 @@ __global__ __launch_bounds__(DT_NW * 64) __attribute__((amdgpu_waves_per_eu(4, 4
 #pragma unroll
   for (int sl = 0; sl < DT_SLOTS; sl++)
     if (wave + sl * DT_NW < K) own |= 1u << (wave + sl * DT_NW);
-  // Workgroup x takes the blocks of DT_BLOCK granules x, x + gridDim.x, ...: every workgroup sees
-  // every part of the pattern-sorted table, so that they all carry about the same number of rules.
+  // Share x takes the blocks of DT_BLOCK granules x, x + shares, ...: every share sees every part of the
+  // pattern-sorted table, so that they all carry about the same number of rules.  A workgroup takes the shares
+  // blockIdx.x, blockIdx.x + gridDim.x, ... one after the other, each summed from zero and stored by itself.
   const int n_blocks = (int)((n + 16 * DT_BLOCK - 1) / (16 * DT_BLOCK)), n32 = (int)n;  // the host checks that 4 K npad < 2^31
   constexpr int PER = DT_NW * DT_SLOTS * 4 * DT_BLOCK / (DT_NW * 64);  // 16-byte loads of a block's indices per thread
   __shared__ int4 jtab[2][DT_NW * DT_SLOTS][4 * DT_BLOCK];  // [tap][position / 4]
@@ -427,6 +429,27 @@ __global__ __launch_bounds__(DT_NW * 64) __attribute__((amdgpu_waves_per_eu(4, 4
 #pragma unroll
     for (int kk = 0; kk < 4; kk++) dst[kk] = pair_of(b_rsrc, present ? r[kk] : -1, b_row_bytes, cb0, cb1);
   };
+  // acc[sl][i][jx][r] = dW[k][ct*32 + 2 (4 g + r) + i][ot*32 + 2 r16 + jx] of the share
+  auto store = [&](int share) {
+#pragma unroll
+    for (int sl = 0; sl < DT_SLOTS; sl++) {
+      const int k = wave + sl * DT_NW;
+      if (k >= K) continue;
+      float *pk = partial + ((size_t)share * K + k) * (size_t)n_a * n_b;
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int c = ct * DT_T + 2 * (4 * g + r) + i;
+          if (c >= n_a) continue;
+          if (cb + 0 < n_b) pk[(size_t)c * n_b + cb + 0] = acc[sl][i][0][r];
+          if (cb + 1 < n_b) pk[(size_t)c * n_b + cb + 1] = acc[sl][i][1][r];
+        }
+#pragma unroll
+        for (int jx = 0; jx < 2; jx++) acc[sl][i][jx] = (v4f){0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  };
   fetch(blockIdx.x);
   put(0);
   __syncthreads();
@@ -434,9 +457,14 @@ __global__ __launch_bounds__(DT_NW * 64) __attribute__((amdgpu_waves_per_eu(4, 4
   issue_b(0, 0, present, bv);
 #pragma unroll
   for (int sl = 0; sl < DT_SLOTS; sl++) issue_a(0, 0, present, sl);
-  int buf = 0;
-  for (int blk = blockIdx.x; blk < n_blocks; blk += gridDim.x, buf ^= 1) {
-    fetch(blk + gridDim.x);
+  int buf = 0, share = blockIdx.x;
+  for (int blk = share; blk < n_blocks; buf ^= 1) {  // (there are at least as many blocks as shares)
+    int next_share = share, next_blk = blk + shares;
+    if (next_blk >= n_blocks) {
+      next_share += gridDim.x;
+      next_blk = next_share < shares ? next_share : n_blocks;
+    }
+    fetch(next_blk);
 #pragma unroll 1
     for (int gl = 0; gl < DT_BLOCK; gl++) {
       const bool over = gl == DT_BLOCK - 1;
@@ -464,22 +492,9 @@ __global__ __launch_bounds__(DT_NW * 64) __attribute__((amdgpu_waves_per_eu(4, 4
 #pragma unroll
       for (int kk = 0; kk < 4; kk++) bv[kk] = bn[kk];
     }
-  }
-  // acc[sl][i][jx][r] = dW[k][ct*32 + 2 (4 g + r) + i][ot*32 + 2 r16 + jx] of this chunk
-#pragma unroll
-  for (int sl = 0; sl < DT_SLOTS; sl++) {
-    const int k = wave + sl * DT_NW;
-    if (k >= K) continue;
-    float *pk = partial + ((size_t)blockIdx.x * K + k) * (size_t)n_a * n_b;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int c = ct * DT_T + 2 * (4 * g + r) + i;
-        if (c >= n_a) continue;
-        if (cb + 0 < n_b) pk[(size_t)c * n_b + cb + 0] = acc[sl][i][0][r];
-        if (cb + 1 < n_b) pk[(size_t)c * n_b + cb + 1] = acc[sl][i][1][r];
-      }
+    if (next_share != share) store(share);
+    share = next_share;
+    blk = next_blk;
   }
 }
 
@@ -903,21 +918,23 @@ static void weight_gradient(Metadata &m, const Table &t, const float *a, int64_t
       (int64_t)t.K * t.npad * 4 < ((int64_t)1 << 31)) {
     // narrow layers: all taps per workgroup
     const int tiles = (int)(ceil_div(n_a, DT_T) * ceil_div(n_b, DT_T));
-    // one resident round: a workgroup per compute unit, shared between the channel tiles
-    const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(ceil_div(t.n, 16 * DT_BLOCK), 256 / tiles));
-    m.partial.reserve((size_t)chunks * per_chunk);
-    const dim3 grid((unsigned)chunks, (unsigned)tiles);
+    // one resident round: a workgroup per compute unit, shared between the channel tiles, two shares to a workgroup: the longer
+    // the fp32 sums of a share, the further off they are (relative 2-norm against 64 bits, 512 shares / 256: 700 k sites 32 x 32
+    // 5.1e-7 / 6.9e-7, 1x1 16 x 32 6.7e-7 / 9.9e-7, 300 k 32 x 32 3.6e-7 / 4.6e-7)
+    const int64_t shares = std::max<int64_t>(1, std::min<int64_t>(ceil_div(t.n, 16 * DT_BLOCK), 512 / tiles));
+    m.partial.reserve((size_t)shares * per_chunk);
+    const dim3 grid((unsigned)std::min<int64_t>(shares, 256 / tiles), (unsigned)tiles);
     const bool vec2 = n_a % 2 == 0 && n_b % 2 == 0 && (uintptr_t)a % 8 == 0 && (uintptr_t)b % 8 == 0;
     if (vec2)
       k_conv_dw_taps<true><<<grid, DT_NW * 64, 0, s>>>(t.nbr.p, t.rowmap_ptr(), t.gmask.p, t.K, t.n, t.npad, a, n_a,
                                                        (unsigned)(a_rows * n_a * 4), b, n_b,
-                                                       (unsigned)(b_rows * n_b * 4), m.partial.p);
+                                                       (unsigned)(b_rows * n_b * 4), m.partial.p, (int)shares);
     else
       k_conv_dw_taps<false><<<grid, DT_NW * 64, 0, s>>>(t.nbr.p, t.rowmap_ptr(), t.gmask.p, t.K, t.n, t.npad, a, n_a,
                                                         (unsigned)(a_rows * n_a * 4), b, n_b,
-                                                       (unsigned)(b_rows * n_b * 4), m.partial.p);
+                                                       (unsigned)(b_rows * n_b * 4), m.partial.p, (int)shares);
     LAUNCH_CHECK();
-    k_sum_blocks<float, float><<<dim3((unsigned)ceil_div(per_chunk, 64)), sum_threads(chunks), 0, s>>>(m.partial.p, (int)chunks, per_chunk, per_chunk, dw);
+    k_sum_blocks<float, float><<<dim3((unsigned)ceil_div(per_chunk, 64)), sum_threads(shares), 0, s>>>(m.partial.p, (int)shares, per_chunk, per_chunk, dw);
     LAUNCH_CHECK();
     return;
   }

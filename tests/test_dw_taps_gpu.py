@@ -35,3 +35,29 @@ def test_weight_gradient(n, dim, size, planes):
         a, b = x.detach()[j[at]].double(), dy[at].double()
         bound = (len(at) + 4) * 2.0 ** -24 * (a.abs().T @ b.abs()) + 1e-30
         assert ((got[k].double() - a.T @ b).abs() <= bound).all(), k
+
+
+@pytest.mark.parametrize("kind,n,n_a,n_b", [("nin", 700001, 16, 32), ("subm", 700001, 32, 32)])
+def test_sums_over_large_levels_are_cut_into_512_shares(kind, n, n_a, n_b):
+    """Of products of either sign the partial sums grow like the square root of their number, and a sum of m additions in fp32 is off by
+    sqrt(c m / 2) 2^-24 of its size (2-norm; c = 0.18, the mean square of a rounding error over numbers whose logarithm is uniform).
+    A tap with R rules is summed in 512 shares, m = R / 512; 256 shares would be off by 1.41 times as much, the bound is 1.2 times.
+    (Adding the shares up comes on top, in quadrature: a few percent where a share has as many rules as here.)"""
+    import torch
+    from test_conv_split_gpu import _table
+    _, rules, rows_in, rows_out, md = _table(kind, n, 9900 + n % 79)
+    g = torch.Generator().manual_seed(n + n_a)
+    x, d = torch.randn(rows_in, n_a, generator=g).cuda(), torch.randn(rows_out, n_b, generator=g).cuda()
+    w = torch.zeros(len(rules), 1, n_a, n_b).cuda()
+    if kind == "nin":
+        got = md.networkInNetworkBackward(x, d, w[0, 0], False)[1]
+    else:
+        got = md.submanifoldConvolutionBackward(torch.LongTensor([1022] * 3), torch.LongTensor([3] * 3), x, d, w, False)[1]
+    got = got.reshape(len(rules), n_a, n_b).double()
+    error = limit = 0.0
+    for k, r in enumerate(rules):
+        r = torch.as_tensor(r).cuda().long()
+        want = x[r[:, 0]].double().t().contiguous() @ d[r[:, 1]].double()
+        error += float((got[k] - want).norm()) ** 2
+        limit += 0.18 * len(r) / 512 / 2 * 2.0 ** -48 * float(want.norm()) ** 2
+    assert error <= 1.2 ** 2 * limit, (error / limit) ** 0.5
