@@ -323,28 +323,25 @@ __global__ __launch_bounds__(256) void k_conv_dw(const int *__restrict__ nbr, co
 }
 // The same sums for narrow layers (both channel counts <= 32), where the kernel above spends its
 // time re-reading: one workgroup per tap reads the rows of b once per tap, 27 times in all.  Here
-// a workgroup of sixteen wavefronts takes a share of the positions and a 32 x 32 channel tile for
-// ALL taps: wavefront w keeps the accumulators of taps w and w + 16 (16 registers
+// a workgroup of eight wavefronts takes a share of the positions and a 32 x 32 channel tile for
+// ALL taps: wavefront w keeps the accumulators of taps w, w + 8, w + 16, w + 24 (16 registers
 // each) and walks its share 16 positions (one granule of the tap masks) at a time, skipping the
-// taps the granule does not have.  No row goes through LDS: the MFMA contracts over four positions,
+// taps the granule does not have.  Nothing goes through LDS: the MFMA contracts over four positions,
 // lane (r, g) supplies position 4 g + kk of the granule and, of that position's row, the two
 // channels 2 r and 2 r + 1 as one 8-byte load (16 lanes read 128 consecutive bytes); instruction
 // i of a pair takes component i, so that it computes the gradient's rows 2 * (MFMA row) + i, and
-// likewise for the columns.  The rows of b are loaded once per granule and serve both taps.
-// Indices, rows and masks of a block of DT_BLOCK granules come to LDS while the block before is worked on, one barrier per
-// block; a tap's rows of the next granule are requested as soon as its MFMAs have freed the registers.
-// Bound by the matrix instructions next to that barrier: 13 of 27 taps a granule of the room surfaces has are 200 us of fp32 MFMAs
-// at a million sites if the four SIMDs share them evenly.  The whole backward call, us (graph replays), eight wavefronts of four
-// taps, two workgroups per compute unit and two memory latencies in a row per granule / this: a million sites 32 x 32 745 / 683, 16 x 16
-// 575 / 540, 300 k 32 x 32 250 / 235, 98 k 111 / 101, 24 k 63 / 48, 6 k 16 x 16 54 / 33; the same bits.  (Eight wavefronts with these
-// loads spill.)
-constexpr int DT_NW = 16, DT_T = 32, DT_SLOTS = 2, DT_BLOCK = 8;  // DT_BLOCK granules of 16 positions per turn
+// likewise for the columns.  The rows of b are loaded once per granule and serve all its taps.
+// (Sixteen wavefronts of two taps with indices through LDS a block of granules ahead and one barrier per block, us with the launch that adds
+// the shares up, here / so: 27 taps 32 x 32 6 k sites 30.7 / 27.9, a million 513 / 487, but 100 k 80 / 85, 64 sites 19 / 24, and where a
+// granule has few of the taps a wavefront waits for the others' blocks: transposed a million positions 281 / 357, filter 3 stride 2 222 / 424,
+// 1x1 100 k rows 16 x 16 25 / 54.)
+constexpr int DT_NW = 8, DT_T = 32, DT_SLOTS = 4, DT_BLOCK = 8;  // DT_BLOCK granules of 16 positions per turn
 template <bool VEC2>
 __global__ __launch_bounds__(DT_NW * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_conv_dw_taps(const int *__restrict__ nbr, const int *__restrict__ rowmap,
                                                              const unsigned *__restrict__ gmask, int K, int64_t n,
                                                              int64_t npad, const float *__restrict__ a, int n_a,
                                                              unsigned a_bytes, const float *__restrict__ b, int n_b,
-                                                             unsigned b_bytes, float *__restrict__ partial, int shares) {
+                                                             unsigned b_bytes, float *__restrict__ partial) {
   const int tiles_o = (n_b + DT_T - 1) / DT_T;
   const int ct = blockIdx.y / tiles_o, ot = blockIdx.y % tiles_o;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -380,121 +377,80 @@ __global__ __launch_bounds__(DT_NW * 64) __attribute__((amdgpu_waves_per_eu(4, 4
 #pragma unroll
   for (int sl = 0; sl < DT_SLOTS; sl++)
     if (wave + sl * DT_NW < K) own |= 1u << (wave + sl * DT_NW);
-  // Share x takes the blocks of DT_BLOCK granules x, x + shares, ...: every share sees every part of the
-  // pattern-sorted table, so that they all carry about the same number of rules.  A workgroup takes the shares
-  // blockIdx.x, blockIdx.x + gridDim.x, ... one after the other, each summed from zero and stored by itself.
-  const int n_blocks = (int)((n + 16 * DT_BLOCK - 1) / (16 * DT_BLOCK)), n32 = (int)n;  // the host checks that 4 K npad < 2^31
-  constexpr int PER = DT_NW * DT_SLOTS * 4 * DT_BLOCK / (DT_NW * 64);  // 16-byte loads of a block's indices per thread
-  __shared__ int4 jtab[2][DT_NW * DT_SLOTS][4 * DT_BLOCK];  // [tap][position / 4]
-  __shared__ int rows[2][16 * DT_BLOCK];
-  __shared__ unsigned masks[2][DT_BLOCK];
-  int4 nj[PER];
-  int nrow = -1;
-  unsigned nmask = 0u;
-  auto fetch = [&](int blk) {  // a block's indices, rows of b and masks on their way; past the last block nothing
-    const bool there = blk < n_blocks;
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-      const int e = threadIdx.x + i * DT_NW * 64, k = e / (4 * DT_BLOCK), p = 16 * DT_BLOCK * blk + 4 * (e % (4 * DT_BLOCK));
-      nj[i] = __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(
-                                           nbr_rsrc, there && k < K && p < npad ? ((unsigned)k * (unsigned)npad + (unsigned)p) * 4u : nowhere, 0, 0));
-    }
-    const int t = 16 * DT_BLOCK * blk + (int)threadIdx.x;
-    nrow = -1;
-    if (threadIdx.x < 16 * DT_BLOCK && there && t < n32) nrow = rowmap ? rowmap[t] : t;
-    nmask = 0u;
-    if (threadIdx.x < DT_BLOCK && there && 16 * (DT_BLOCK * blk + (int)threadIdx.x) < n32) nmask = gmask[DT_BLOCK * blk + threadIdx.x];
-  };
-  auto put = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-      const int e = threadIdx.x + i * DT_NW * 64;
-      jtab[buf][e / (4 * DT_BLOCK)][e % (4 * DT_BLOCK)] = nj[i];
-    }
-    if (threadIdx.x < 16 * DT_BLOCK) rows[buf][threadIdx.x] = nrow;
-    if (threadIdx.x < DT_BLOCK) masks[buf][threadIdx.x] = nmask;
-  };
-  v2f av[DT_SLOTS][4], bv[4], bn[4];
-  auto issue_a = [&](int buf, int gl, unsigned present, int sl) {
-    const int k = wave + sl * DT_NW;
-    const bool has = (present >> k) & 1u;
-    const int4 j4 = jtab[buf][k][4 * gl + g];
-    const int j[4] = {j4.x, j4.y, j4.z, j4.w};
-#pragma unroll
-    for (int kk = 0; kk < 4; kk++) av[sl][kk] = pair_of(a_rsrc, has ? j[kk] : -1, a_row_bytes, ca0, ca1);
-  };
-  auto issue_b = [&](int buf, int gl, unsigned present, v2f (&dst)[4]) {
-    const int4 r4 = *reinterpret_cast<const int4 *>(&rows[buf][16 * gl + 4 * g]);
-    const int r[4] = {r4.x, r4.y, r4.z, r4.w};
-#pragma unroll
-    for (int kk = 0; kk < 4; kk++) dst[kk] = pair_of(b_rsrc, present ? r[kk] : -1, b_row_bytes, cb0, cb1);
-  };
-  // acc[sl][i][jx][r] = dW[k][ct*32 + 2 (4 g + r) + i][ot*32 + 2 r16 + jx] of the share
-  auto store = [&](int share) {
-#pragma unroll
-    for (int sl = 0; sl < DT_SLOTS; sl++) {
-      const int k = wave + sl * DT_NW;
-      if (k >= K) continue;
-      float *pk = partial + ((size_t)share * K + k) * (size_t)n_a * n_b;
-#pragma unroll
-      for (int i = 0; i < 2; i++) {
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int c = ct * DT_T + 2 * (4 * g + r) + i;
-          if (c >= n_a) continue;
-          if (cb + 0 < n_b) pk[(size_t)c * n_b + cb + 0] = acc[sl][i][0][r];
-          if (cb + 1 < n_b) pk[(size_t)c * n_b + cb + 1] = acc[sl][i][1][r];
-        }
-#pragma unroll
-        for (int jx = 0; jx < 2; jx++) acc[sl][i][jx] = (v4f){0.f, 0.f, 0.f, 0.f};
-      }
-    }
-  };
-  fetch(blockIdx.x);
-  put(0);
-  __syncthreads();
-  unsigned present = __builtin_amdgcn_readfirstlane(masks[0][0]) & own;
-  issue_b(0, 0, present, bv);
-#pragma unroll
-  for (int sl = 0; sl < DT_SLOTS; sl++) issue_a(0, 0, present, sl);
-  int buf = 0, share = blockIdx.x;
-  for (int blk = share; blk < n_blocks; buf ^= 1) {  // (there are at least as many blocks as shares)
-    int next_share = share, next_blk = blk + shares;
-    if (next_blk >= n_blocks) {
-      next_share += gridDim.x;
-      next_blk = next_share < shares ? next_share : n_blocks;
-    }
-    fetch(next_blk);
-#pragma unroll 1
-    for (int gl = 0; gl < DT_BLOCK; gl++) {
-      const bool over = gl == DT_BLOCK - 1;
-      if (over) {  // nothing of the other buffer is read any more: its last granule was issued before the barrier in front of this block
-        put(buf ^ 1);
-        __syncthreads();
-      }
-      const int nb = over ? buf ^ 1 : buf, ngl = over ? 0 : gl + 1;
-      const unsigned next = __builtin_amdgcn_readfirstlane(masks[nb][ngl]) & own;
-      issue_b(nb, ngl, next, bn);
+  // Workgroup x takes the blocks of DT_BLOCK granules x, x + gridDim.x, ...: every workgroup sees
+  // every part of the pattern-sorted table, so that they all carry about the same number of rules.
+  const int n_granules = (int)((n + 15) >> 4), n32 = (int)n;  // the host checks that 4 K npad < 2^31
+  for (int gb = blockIdx.x * DT_BLOCK; gb < n_granules; gb += gridDim.x * DT_BLOCK) {
+    const int ge = min(n_granules, gb + DT_BLOCK);
+    for (int gi = gb; gi < ge; gi++) {
+      const unsigned present = gmask[gi] & own;
+      if (present == 0u) continue;  // uniform over the wavefront
+      const int t0 = gi << 4;
+      // this lane's four positions of the granule: t0 + 4 g + kk; first the index quads of the
+      // wavefront's taps, then all gathers, then the MFMAs: two memory latencies per granule
+      // (fetching the next granule's quads meanwhile costs more registers than there are at
+      // four wavefronts per SIMD, and measured slower with fewer)
+      int4 j4[DT_SLOTS];
+      const unsigned toff = (unsigned)(t0 + 4 * g) * 4u;
 #pragma unroll
       for (int sl = 0; sl < DT_SLOTS; sl++) {
-        if ((present >> (wave + sl * DT_NW)) & 1u) {  // uniform over the wavefront
-#pragma unroll
-          for (int kk = 0; kk < 4; kk++)
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-              for (int jx = 0; jx < 2; jx++)
-                acc[sl][i][jx] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[sl][kk][i], bv[kk][jx], acc[sl][i][jx], 0, 0, 0);
-        }
-        issue_a(nb, ngl, next, sl);  // the registers are free
+        const int k = wave + sl * DT_NW;
+        // a tap the granule does not have: an offset past the table, which reads zeros; made -1 below
+        j4[sl] = __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(
+                                              nbr_rsrc, ((present >> k) & 1u) ? toff : nowhere, (unsigned)k * (unsigned)npad * 4u, 0));
       }
-      present = next;
+      v2f bv[4];
+      if (rowmap) {
+        const int4 r4 = *reinterpret_cast<const int4 *>(rowmap + t0 + 4 * g);
+        const int r[4] = {r4.x, r4.y, r4.z, r4.w};
 #pragma unroll
-      for (int kk = 0; kk < 4; kk++) bv[kk] = bn[kk];
+        for (int kk = 0; kk < 4; kk++) bv[kk] = pair_of(b_rsrc, t0 + 4 * g + kk < n32 ? r[kk] : -1, b_row_bytes, cb0, cb1);
+      } else {
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) {
+          const int t = t0 + 4 * g + kk;
+          bv[kk] = pair_of(b_rsrc, t < n32 ? t : -1, b_row_bytes, cb0, cb1);
+        }
+      }
+      v2f av[DT_SLOTS][4];
+#pragma unroll
+      for (int sl = 0; sl < DT_SLOTS; sl++) {
+        const int k = wave + sl * DT_NW;
+        const bool has = (present >> k) & 1u;
+        const int j[4] = {j4[sl].x, j4[sl].y, j4[sl].z, j4[sl].w};
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) av[sl][kk] = pair_of(a_rsrc, has ? j[kk] : -1, a_row_bytes, ca0, ca1);
+      }
+#pragma unroll
+      for (int sl = 0; sl < DT_SLOTS; sl++) {
+        const int k = wave + sl * DT_NW;
+        if (!((present >> k) & 1u)) continue;  // uniform over the wavefront
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++)
+#pragma unroll
+          for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int jx = 0; jx < 2; jx++)
+              acc[sl][i][jx] =
+                  __builtin_amdgcn_mfma_f32_16x16x4f32(av[sl][kk][i], bv[kk][jx], acc[sl][i][jx], 0, 0, 0);
+      }
     }
-    if (next_share != share) store(share);
-    share = next_share;
-    blk = next_blk;
+  }
+  // acc[sl][i][jx][r] = dW[k][ct*32 + 2 (4 g + r) + i][ot*32 + 2 r16 + jx] of this chunk
+#pragma unroll
+  for (int sl = 0; sl < DT_SLOTS; sl++) {
+    const int k = wave + sl * DT_NW;
+    if (k >= K) continue;
+    float *pk = partial + ((size_t)blockIdx.x * K + k) * (size_t)n_a * n_b;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int c = ct * DT_T + 2 * (4 * g + r) + i;
+        if (c >= n_a) continue;
+        if (cb + 0 < n_b) pk[(size_t)c * n_b + cb + 0] = acc[sl][i][0][r];
+        if (cb + 1 < n_b) pk[(size_t)c * n_b + cb + 1] = acc[sl][i][1][r];
+      }
   }
 }
 
@@ -918,23 +874,23 @@ static void weight_gradient(Metadata &m, const Table &t, const float *a, int64_t
       (int64_t)t.K * t.npad * 4 < ((int64_t)1 << 31)) {
     // narrow layers: all taps per workgroup
     const int tiles = (int)(ceil_div(n_a, DT_T) * ceil_div(n_b, DT_T));
-    // one resident round: a workgroup per compute unit, shared between the channel tiles, two shares to a workgroup: the longer
-    // the fp32 sums of a share, the further off they are (relative 2-norm against 64 bits, 512 shares / 256: 700 k sites 32 x 32
-    // 5.1e-7 / 6.9e-7, 1x1 16 x 32 6.7e-7 / 9.9e-7, 300 k 32 x 32 3.6e-7 / 4.6e-7)
-    const int64_t shares = std::max<int64_t>(1, std::min<int64_t>(ceil_div(t.n, 16 * DT_BLOCK), 512 / tiles));
-    m.partial.reserve((size_t)shares * per_chunk);
-    const dim3 grid((unsigned)std::min<int64_t>(shares, 256 / tiles), (unsigned)tiles);
+    // one resident round: two workgroups per compute unit, shared between the channel tiles.  The longer the fp32 sums of a share, the
+    // further off they are: relative 2-norm against 64 bits with 512 shares / 256, 700 k sites 32 x 32 5.1e-7 / 6.9e-7, 1x1 16 x 32
+    // 6.7e-7 / 9.9e-7
+    const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(ceil_div(t.n, 16 * DT_BLOCK), 512 / tiles));
+    m.partial.reserve((size_t)chunks * per_chunk);
+    const dim3 grid((unsigned)chunks, (unsigned)tiles);
     const bool vec2 = n_a % 2 == 0 && n_b % 2 == 0 && (uintptr_t)a % 8 == 0 && (uintptr_t)b % 8 == 0;
     if (vec2)
       k_conv_dw_taps<true><<<grid, DT_NW * 64, 0, s>>>(t.nbr.p, t.rowmap_ptr(), t.gmask.p, t.K, t.n, t.npad, a, n_a,
                                                        (unsigned)(a_rows * n_a * 4), b, n_b,
-                                                       (unsigned)(b_rows * n_b * 4), m.partial.p, (int)shares);
+                                                       (unsigned)(b_rows * n_b * 4), m.partial.p);
     else
       k_conv_dw_taps<false><<<grid, DT_NW * 64, 0, s>>>(t.nbr.p, t.rowmap_ptr(), t.gmask.p, t.K, t.n, t.npad, a, n_a,
                                                         (unsigned)(a_rows * n_a * 4), b, n_b,
-                                                       (unsigned)(b_rows * n_b * 4), m.partial.p, (int)shares);
+                                                       (unsigned)(b_rows * n_b * 4), m.partial.p);
     LAUNCH_CHECK();
-    k_sum_blocks<float, float><<<dim3((unsigned)ceil_div(per_chunk, 64)), sum_threads(shares), 0, s>>>(m.partial.p, (int)shares, per_chunk, per_chunk, dw);
+    k_sum_blocks<float, float><<<dim3((unsigned)ceil_div(per_chunk, 64)), sum_threads(chunks), 0, s>>>(m.partial.p, (int)chunks, per_chunk, per_chunk, dw);
     LAUNCH_CHECK();
     return;
   }
