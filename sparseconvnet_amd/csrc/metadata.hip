@@ -2655,18 +2655,10 @@ StridedRules &strided_rules(Metadata &m, const int64_t *in_size, const int64_t *
 // time, find a coarse row that one of them fetched still in that XCD's L2; with an eighth of a
 // million-site level per range every tap's run fetched its 4 MB of coarse rows again (counters:
 // 268 MB read for 95 MB of operands).
-// The window's workgroup writes the table as well: position t of it is position src of the schedule, its one entry, -1 in the
-// other taps, its row, and the granule masks (an OR over the 16 lanes of a granule).  Bound by the table's bytes (4 K + 17 per position)
-// and, on small levels, by launches: with the order through memory and a second kernel a million positions took 37 us and
-// six levels from a million down 147, 22 and 62 so (windows of 4096: 152, too few workgroups for the stores).
+// Sorts window blockIdx.x: on return sh.sval[i] is the window's position that comes i-th, sh.skey[i] its tap (16: no rule).
 template <int ITEMS>
-__global__ __launch_bounds__(RS1_THREADS) void k_few_table(const int *__restrict__ in_tap, const int *__restrict__ in_row, int K, int64_t n,
-                                                          int64_t npad, const int *__restrict__ base_rows, int *__restrict__ nbr,
-                                                          int *__restrict__ rowmap, unsigned *__restrict__ gmask,
-                                                          unsigned char *__restrict__ few_tap, int *__restrict__ few_row) {
-  __shared__ BlockSort<ITEMS> sh;
-  constexpr int WINDOW = RS1_THREADS * ITEMS;
-  const int64_t base = (int64_t)blockIdx.x * WINDOW;
+__device__ inline void few_sort_window(BlockSort<ITEMS> &sh, const int *__restrict__ in_tap, int64_t n) {
+  const int64_t base = (int64_t)blockIdx.x * (RS1_THREADS * ITEMS);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   unsigned long long key[ITEMS];
   int val[ITEMS];
@@ -2680,24 +2672,63 @@ __global__ __launch_bounds__(RS1_THREADS) void k_few_table(const int *__restrict
     val[r] = i;
   }
   block_sort<ITEMS>(sh, key, val, valid, 5, 5);
-#pragma unroll
-  for (int q = 0; q < ITEMS; q++) {
-    const int i = q * RS1_THREADS + (int)threadIdx.x;
-    const int64_t t = base + i;
-    unsigned mk = 0;
-    if (t < n) {
-      const int64_t src = base + sh.sval[i];
-      const int tap = sh.skey[i] == 16ull ? -1 : (int)sh.skey[i], row = in_row[src];
-      few_tap[t] = tap >= 0 ? (unsigned char)tap : (unsigned char)255;
-      few_row[t] = tap >= 0 ? row : 0;
-      for (int k = 0; k < K; k++) nbr[(int64_t)k * npad + t] = k == tap ? row : -1;
-      mk = tap >= 0 ? 1u << tap : 0u;
-      rowmap[t] = base_rows ? base_rows[src] : (int)src;
-    }
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) mk |= __shfl_xor(mk, o, 64);
-    if ((threadIdx.x & 15) == 0 && t < n) gmask[t >> 4] = mk;
+}
+// Position t of the table is position src of the schedule: its one entry, -1 in the other taps, its row, and the granule masks
+// (an OR over the 16 lanes of a granule).  Whole wavefronts call it, 64 consecutive t each.
+__device__ inline void few_write(int64_t t, int64_t src, int tap, const int *__restrict__ in_row, int K, int64_t n, int64_t npad,
+                                 const int *__restrict__ base_rows, int *__restrict__ nbr, int *__restrict__ rowmap,
+                                 unsigned *__restrict__ gmask, unsigned char *__restrict__ few_tap, int *__restrict__ few_row) {
+  unsigned mk = 0;
+  if (t < n) {
+    const int row = in_row[src];
+    few_tap[t] = tap >= 0 ? (unsigned char)tap : (unsigned char)255;
+    few_row[t] = tap >= 0 ? row : 0;
+    for (int k = 0; k < K; k++) nbr[(int64_t)k * npad + t] = k == tap ? row : -1;
+    mk = tap >= 0 ? 1u << tap : 0u;
+    rowmap[t] = base_rows ? base_rows[src] : (int)src;
   }
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) mk |= __shfl_xor(mk, o, 64);
+  if ((threadIdx.x & 15) == 0 && t < n) gmask[t >> 4] = mk;
+}
+// Small levels, where launches are what it costs: a window's PARTS workgroups each sort all of it and write their part of the table.
+// Up to FEW_ONE_LAUNCH positions; six levels from 20 k positions down 44 us with two launches each, 32 so, but from a million down
+// 127-160 / 144-163, where a workgroup's sort no longer hides behind another's stores.  (Windows of 2048: 28 and 116-136, but a tile of
+// the convolutions over the table then spans more taps: transposed 224 -> 8 onto 18.5 k sites 22 -> 54, 256 -> 24 14.8 k 25 -> 38, 192 -> 16
+// 145 k 36 -> 55.)
+template <int ITEMS, int PARTS>
+__global__ __launch_bounds__(RS1_THREADS) void k_few_table(const int *__restrict__ in_tap, const int *__restrict__ in_row, int K, int64_t n,
+                                                          int64_t npad, const int *__restrict__ base_rows, int *__restrict__ nbr,
+                                                          int *__restrict__ rowmap, unsigned *__restrict__ gmask,
+                                                          unsigned char *__restrict__ few_tap, int *__restrict__ few_row) {
+  __shared__ BlockSort<ITEMS> sh;
+  const int64_t base = (int64_t)blockIdx.x * (RS1_THREADS * ITEMS);
+  few_sort_window<ITEMS>(sh, in_tap, n);
+#pragma unroll
+  for (int j = 0; j < ITEMS / PARTS; j++) {
+    const int i = ((int)blockIdx.y * (ITEMS / PARTS) + j) * RS1_THREADS + (int)threadIdx.x;
+    const bool there = base + i < n;
+    const int tap = there && sh.skey[i] != 16ull ? (int)sh.skey[i] : -1;
+    few_write(base + i, base + (there ? sh.sval[i] : 0), tap, in_row, K, n, npad, base_rows, nbr, rowmap, gmask, few_tap, few_row);
+  }
+}
+// Larger levels: the order first, then the table.
+template <int ITEMS>
+__global__ __launch_bounds__(RS1_THREADS) void k_few_order(const int *__restrict__ in_tap, int64_t n, int *__restrict__ perm) {
+  __shared__ BlockSort<ITEMS> sh;
+  constexpr int WINDOW = RS1_THREADS * ITEMS;
+  const int64_t base = (int64_t)blockIdx.x * WINDOW;
+  few_sort_window<ITEMS>(sh, in_tap, n);
+  const int here = (int)min<int64_t>(WINDOW, n - base);
+  for (int i = threadIdx.x; i < here; i += RS1_THREADS) perm[base + i] = (int)(base + sh.sval[i]);
+}
+__global__ void k_few_write(const int *__restrict__ in_tap, const int *__restrict__ in_row, int K, int64_t n, int64_t npad,
+                            const int *__restrict__ perm, const int *__restrict__ base_rows, int *__restrict__ nbr,
+                            int *__restrict__ rowmap, unsigned *__restrict__ gmask, unsigned char *__restrict__ few_tap,
+                            int *__restrict__ few_row) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int src = t < n ? perm[t] : 0;
+  few_write(t, src, t < n ? in_tap[src] : -1, in_row, K, n, npad, base_rows, nbr, rowmap, gmask, few_tap, few_row);
 }
 
 void finish_by_in(Metadata &m, StridedRules &r, hipStream_t s) {
@@ -2707,7 +2738,8 @@ void finish_by_in(Metadata &m, StridedRules &r, hipStream_t s) {
   m.builds++;
   Table &t = r.by_in;
   if (r.by_in_compact && t.n > 0) {
-    constexpr int FEW_ITEMS = 2;  // windows of 2048 positions
+    constexpr int FEW_ITEMS = 4, FEW_PARTS = 2;  // windows of 4096 positions
+    constexpr int64_t FEW_ONE_LAUNCH = 65536;
     const int window = RS1_THREADS * FEW_ITEMS;
     t.spread = window >= t.n;
     t.nbr.reserve((size_t)t.K * t.npad);
@@ -2715,8 +2747,17 @@ void finish_by_in(Metadata &m, StridedRules &r, hipStream_t s) {
     t.gmask.reserve(ceil_div(t.n, 16));
     t.few_tap.reserve(t.n);
     t.few_row.reserve(t.n);
-    k_few_table<FEW_ITEMS><<<dim3((unsigned)ceil_div(t.n, window)), RS1_THREADS, 0, s>>>(
-        r.in_tap.p, r.in_row.p, t.K, t.n, t.npad, li->second.sched_ptr(), t.nbr.p, t.rowmap.p, t.gmask.p, t.few_tap.p, t.few_row.p);
+    const dim3 windows((unsigned)ceil_div(t.n, window), t.n <= FEW_ONE_LAUNCH ? FEW_PARTS : 1);
+    if (t.n <= FEW_ONE_LAUNCH) {
+      k_few_table<FEW_ITEMS, FEW_PARTS><<<windows, RS1_THREADS, 0, s>>>(r.in_tap.p, r.in_row.p, t.K, t.n, t.npad, li->second.sched_ptr(),
+                                                                       t.nbr.p, t.rowmap.p, t.gmask.p, t.few_tap.p, t.few_row.p);
+    } else {
+      m.v1.reserve(t.n);  // the order: position t of the table is position v1[t] of the schedule
+      k_few_order<FEW_ITEMS><<<windows, RS1_THREADS, 0, s>>>(r.in_tap.p, t.n, m.v1.p);
+      LAUNCH_CHECK();
+      k_few_write<<<grid_for(t.n), TB, 0, s>>>(r.in_tap.p, r.in_row.p, t.K, t.n, t.npad, m.v1.p, li->second.sched_ptr(), t.nbr.p,
+                                               t.rowmap.p, t.gmask.p, t.few_tap.p, t.few_row.p);
+    }
     LAUNCH_CHECK();
     t.identity_rows = false;
     r.in_tap.release();

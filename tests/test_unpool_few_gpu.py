@@ -1,11 +1,12 @@
 """Unpooling over a halving rulebook (k_unpool_few): every fine site receives its parent's row, exactly, at sizes around a workgroup's
-elements, with planes dropped, and where planes or strides do not allow 16-byte loads (the general kernel)."""
+elements, to windows of 4096 positions and to the largest table made in one launch, with planes dropped, and where planes or strides do not
+allow 16-byte loads (the general kernel)."""
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 15, 255, 257, 1023, 1025, 8191, 40009])
+@pytest.mark.parametrize("n", [1, 15, 255, 257, 1023, 1025, 4095, 4097, 8191, 40009, 65536, 65537])
 @pytest.mark.parametrize("planes,drop", [(4, 0), (20, 0), (64, 0), (36, 4), (7, 0), (12, 3)])
 def test_children_receive_their_parents_row(n, planes, drop):
     import torch
