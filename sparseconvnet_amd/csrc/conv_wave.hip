@@ -192,7 +192,13 @@ __global__ __launch_bounds__(64 * (DEAL > 4 ? DEAL : 4), OCC) void k_conv_wave(
       if constexpr (BF16) {
         const v8s a = __builtin_bit_cast(v8s, turn[wave][q][0][rd_slot]);
 #pragma unroll
-        for (int c = 0; c < NCB; c++) acc[q][c] = mfma_bf16(a, breg[c][0], acc[q][c]);
+        for (int c = 0; c < NCB; c++) {
+          // Dealt out, a wavefront's chain is longer than the parts k_conv_rows gave to workgroups on small levels, and the unit does not
+          // round its sums to nearest: added up by fp32 adds instead.  Relative 2-norm against 64 bits, k_conv_rows / one chain / so:
+          // 1.5 k sites 128 -> 64 9.5e-8 / 1.22e-7 / 8.8e-8, 12 k 128 -> 128 1.58e-7 / 1.59e-7 / 8.6e-8; 1-5 % of the time on small levels
+          if constexpr (DEAL > 1) acc[q][c] += mfma_bf16(a, breg[c][0], (v4f){0.f, 0.f, 0.f, 0.f});
+          else acc[q][c] = mfma_bf16(a, breg[c][0], acc[q][c]);
+        }
       } else {
         const Split8 a = split8(turn[wave][q][0][rd_slot], turn[wave][q][1][rd_slot]);
         v4f t[NCB];

@@ -136,3 +136,27 @@ def test_bf16_operands(kind, n, cin, cout, form):
     assert ((got.double() - want).abs() <= bound * mag + 1e-30).all()
     kernel = md._L.scn_md_last_conv_kernel(md._h).decode()
     assert "bf16" in kernel, kernel
+
+
+@pytest.mark.parametrize("n,cin,cout", [(1500, 128, 64), (3001, 128, 64), (6001, 128, 128), (12001, 128, 64), (12001, 64, 64)])
+def test_bf16_sums_of_small_levels(n, cin, cout):
+    """Four wavefronts take a row's R (tap, 32 channels) products in turn and add them up by fp32 adds, R / 4 each.  Of terms of either sign
+    the partial sums grow like the square root of their number: off by sqrt(0.18 R / 8) 2^-24 of the result (2-norm; 0.18: the mean square of
+    a rounding error over numbers whose logarithm is uniform), and by sqrt(1.5) 2^-24 from the 32 products of an instruction, which are not
+    rounded to nearest.  The bound is 1.1 times that; one chain of instructions per wavefront is 1.25 to 1.4 times as far off."""
+    import torch
+    from test_conv_split_gpu import _table
+    conv, rules, rows_in, rows_out, md = _table("subm", n, 8300 + n % 89)
+    md.setBf16(True)
+    g = torch.Generator().manual_seed(n + cin)
+    x, w = torch.randn(rows_in, cin, generator=g).cuda(), (torch.randn(len(rules), 1, cin, cout, generator=g) * 0.1).cuda()
+    got = conv(x, w, torch.zeros(cout).cuda())
+    kernel = md._L.scn_md_last_conv_kernel(md._h).decode()
+    assert "wave-bf16" in kernel, kernel
+    want = torch.zeros(rows_out, cout, dtype=torch.float64, device="cuda")
+    for k, r in enumerate(rules):
+        r = torch.as_tensor(r).cuda().long()
+        want.index_add_(0, r[:, 1], x[r[:, 0]].bfloat16().double() @ w[k, 0].bfloat16().double())
+    products = sum(len(r) for r in rules) / rows_out * cin / 32
+    limit = 1.1 * (0.18 * products / 8 + 1.5) ** 0.5 * 2.0 ** -24
+    assert (got.double() - want).norm() <= limit * want.norm(), float((got.double() - want).norm() / want.norm()) / limit
