@@ -444,9 +444,17 @@ static bool dispatch_rows(Metadata &m, const Table &t, const float *in, float *o
   // bf16 operands: a wavefront's MFMAs of one granule take half the time of its reads of the slab, and an iteration as long as its
   // barrier; two granules per wavefront and slabs of 64 channels on levels that have the workgroups (us): 500 k sites 64 -> 64 164 -> 148,
   // 64 -> 96 201 -> 182, 128 -> 128 398 -> 372; 61 k 192 -> 96 110 -> 95, 256 -> 128 150 -> 131; 14 k 256 -> 128 56 -> 50
-  // (5 k 32 -> 33).  k_conv_wave serves smaller levels and, up to 32 planes, most of the larger.
+  // (5 k 32 -> 33).  k_conv_wave serves smaller levels and, up to 32 planes, most of the larger.  Not where a tile has few iterations: one
+  // rule per position (transposed 31 k sites 256 -> 128 23 / 37, 85 k 192 -> 128 31 / 36, but 939 k 256 -> 96 254 / 233; 1x1 below 100 k rows
+  // 46 k 128 -> 96 15.8 / 16.7) and, onto more than 96 planes, up to eight taps (194 k sites 320 -> 112 74 / 80, 1x1 958 k 192 -> 128 262 / 285); nor
+  // for most of the long tap lists (5^3, 500 k 192 -> 96 4993 / 5704, 16 k 320 -> 80 365 / 445; but 943 k 192 -> 48 6766 / 4941, 20 k 192 -> 96
+  // 563 / 348, 17 k 320 -> 128 706 / 509).
   if constexpr (VEC4) {
-    if (m.bf16 && n_in % 64 == 0 && ncb > 2 && t.n >= (n_in > 128 && ncb > 4 ? 10000 : ncb <= 4 ? 260000 : 40000)) {
+    bool enough = t.K > 8 || ncb <= 6;
+    if (t.few_tap.p) enough = ncb <= 6 && n_in > 128 && t.n >= 300000;
+    else if (t.K == 1) enough = ncb <= 6 && t.n >= 100000;
+    else if (t.K > 32) enough = ncb <= 4 || (n_in > 64 && t.n >= 16000 && t.n < 60000);
+    if (m.bf16 && n_in % 64 == 0 && ncb > 2 && enough && t.n >= (n_in > 128 && ncb > 4 ? 10000 : ncb <= 4 ? 260000 : 40000)) {
       if (ncb <= 4) return launch_rows<4, 2, 4, VEC4, 4, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);
       if (ncb <= 6) return launch_rows<6, 2, 4, VEC4, 4, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);
       if (ncb <= 8) return launch_rows<8, 2, 4, VEC4, 4, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);

@@ -376,6 +376,11 @@ static void launch_wave(Metadata &m, const Table &t, const float *in, float *out
   LAUNCH_CHECK();
 }
 
+// Taps a position has at most: fine sides of strided tables have few of theirs, as few as coarse and fine rows say (see launch_split).
+static int64_t likely_taps(const Table &t, int64_t in_rows) {
+  return t.few_tap.p ? 1 : std::min<int64_t>(t.K, ceil_div(t.K * in_rows, std::max<int64_t>(t.n, 1)));
+}
+
 // 33 to 48 output planes on small levels: every pair (granules, column group) is a workgroup whose wavefronts deal out the
 // iterations, and sums meet in LDS, where k_conv_split writes partial sums for a launch to add up.  Rows are gathered and split
 // once per column group and weights read once per workgroup, so that this ends where iterations or granules are many.
@@ -436,13 +441,25 @@ static void dispatch_wave(Metadata &m, const Table &t, const float *in, float *o
 //     64 -> 64 38 / 27, but 96 -> 96 60 / 61; 240 k 32 -> 32 60 / 36, 128 -> 64 144 / 134, 128 -> 128 205 / 192; 500 k 32 -> 32 86 / 65,
 //     but 64 -> 32 112 / 118; 900 k 32 -> 32 140 / 126
 //   8 taps, onto 5 k sites 32 -> 64 13.6 / 4.0, 59 k 13.9 / 12.9, 221 k 32 -> 32 63 / 26; one rule per position, onto 20 k sites
-//     64 -> 32 14.0 / 4.1, 900 k 51 / 38, 61 k 96 -> 64 12.8 / 10.9; 1x1 20 k rows 128 -> 64 8.5 / 5.8, 61 k 13.0 / 13.0
+//     64 -> 32 14.0 / 4.1, 900 k 51 / 38, 61 k 96 -> 64 12.8 / 10.9; 1x1 20 k rows 128 -> 64 8.5 / 5.8, 61 k 13.0 / 13.0, 43 k 256 -> 96 19.6 / 24.4
 // (Rounding the rows in a pass of its own, so that each rule reads half the bytes, takes longer than it saves: 300 k sites 64 -> 64
 // 92 -> 102, 800 k 32 -> 32 99 -> 135.)
+// Wide inputs on small levels, where k_conv_rows gives a tile's taps to several workgroups (there / here): 64 sites 256 -> 128 17.8 / 32.5,
+// 340 192 -> 64 15.5 / 25.9, 466 160 -> 48 15.2 / 19.0, 700 256 -> 64 18.8 / 26.1, 2.1 k 256 -> 128 28.1 / 34.3, 2.8 k 320 -> 64 31.3 / 37.5; but
+// 200 sites 64 -> 64 12.6 / 12.0, 700 96 -> 96 16.9 / 13.4, 1.5 k 128 -> 128 24.7 / 17.0, 6 k 192 -> 32 27.1 / 18.5.  The sites from which on
+// this kernel is the faster one, by (many taps) slabs of 32 channels; filter 3 stride 2 from the fine side and eight taps below.
+static int64_t bf_from(int64_t taps, int64_t slabs, int n_out) {
+  static const int64_t many[3][10] = {{0, 0, 0, 500, 850, 1250, 1800, 2000, 2500, 4500},  // onto up to 32 planes, 64, and more
+                                      {0, 0, 0, 520, 850, 1000, 1350, 1500, 4200, 6000},
+                                      {0, 0, 0, 400, 600, 700, 1000, 1500, 3000, 3000}};
+  if (taps > 16) return many[n_out <= 32 ? 0 : n_out <= 64 ? 1 : 2][std::min<int64_t>(slabs, 9)];
+  return taps > 8 ? (slabs >= 8 ? 700 : 0) : taps > 1 && slabs >= 10 ? 250 : 0;
+}
 enum BfTile { BF_NONE, BF_2_1_4, BF_2_2_4, BF_2_2_1, BF_2_4_1, BF_4_2_4, BF_8_4_1 };  // column blocks, granules, wavefronts that share them
-static BfTile bf_tile(const Table &t, int n_in, int n_out) {
+static BfTile bf_tile(const Table &t, int64_t in_rows, int n_in, int n_out) {
   const int64_t n = t.n;
   if (n_in % 32 || n_out > 128) return BF_NONE;
+  if (n < bf_from(likely_taps(t, in_rows), n_in / 32, n_out)) return BF_NONE;
   const bool one_rule = t.few_tap.p || t.K == 1, few = one_rule || t.K <= 9;
   if (n_out <= 32) {
     if (n < 20000) return BF_2_1_4;
@@ -451,7 +468,7 @@ static BfTile bf_tile(const Table &t, int n_in, int n_out) {
     return n_in > 32 ? BF_NONE : n < 700000 ? BF_2_2_1 : BF_2_4_1;
   }
   if (few) {
-    const int64_t to = t.K == 1 ? 45000 : n_out <= 64 ? (one_rule ? 100000 : 70000) : 25000;
+    const int64_t to = t.K == 1 ? (n_out <= 64 ? 45000 : 28000) : n_out <= 64 ? (one_rule ? 100000 : 70000) : 25000;
     return n < 8000 ? BF_2_1_4 : n < to ? BF_4_2_4 : BF_NONE;
   }
   if (n_out <= 64) return n < 8000 ? BF_2_1_4 : n < 260000 ? BF_4_2_4 : BF_NONE;
@@ -466,7 +483,7 @@ static void dispatch_bf(Metadata &m, const Table &t, const float *in, float *out
                         int n_out, PreArgs pre, hipStream_t s) {
 #define BF(N, G, D, O) \
   case BF_##N##_##G##_##D: return launch_wave<N, G, D, O, false, PRE, true>(m, t, in, out, w, epi, n_in, n_out, pre, s)
-  switch (bf_tile(t, n_in, n_out)) {
+  switch (bf_tile(t, m.cur_in_rows, n_in, n_out)) {
     BF(2, 1, 4, 5);
     BF(2, 2, 4, 4);
     BF(2, 2, 1, 5);
@@ -486,7 +503,7 @@ bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_
   if (m.fixed_scratch || t.K > 32 || !t.gmask.p) return false;
   if (n_in <= 4 || n_in % 4 || (uintptr_t)in % 16 || n_in * 4 >= (1 << 24)) return false;
   if (in_rows <= 0 || in_rows >= (1 << 24) || in_rows * n_in * 4 >= ((int64_t)1 << 31)) return false;
-  if (m.bf16) return !gradient && bf_tile(t, n_in, n_out) != BF_NONE;  // (these weights are packed from a transposed copy)
+  if (m.bf16) return !gradient && bf_tile(t, in_rows, n_in, n_out) != BF_NONE;  // (these weights are packed from a transposed copy)
   if (n_out > 32) return wide_tile(t, n_in, n_out) != NONE;
   // k_conv_resident keeps 20-32 -> up to 16 planes on small levels of few taps and on large ones
   if (n_in > 16 && n_in <= 32 && n_out <= 16 && (t.K <= 9 ? t.n < 16000 : t.n >= (n_in > 24 ? 200000 : 300000))) return false;

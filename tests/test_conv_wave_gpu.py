@@ -160,3 +160,33 @@ def test_bf16_sums_of_small_levels(n, cin, cout):
     products = sum(len(r) for r in rules) / rows_out * cin / 32
     limit = 1.1 * (0.18 * products / 8 + 1.5) ** 0.5 * 2.0 ** -24
     assert (got.double() - want).norm() <= limit * want.norm(), float((got.double() - want).norm() / want.norm()) / limit
+
+
+@pytest.mark.parametrize("kind,n,cin,cout,says", [
+    # many (tap, 32 channels) products per row on small levels: k_conv_rows deals them over workgroups
+    ("subm", 64, 64, 64, "wave-bf16"), ("subm", 200, 96, 96, "rows-bf16"), ("subm", 501, 96, 24, "wave-bf16"),
+    ("subm", 599, 128, 96, "rows-bf16"), ("subm", 601, 128, 96, "wave-bf16"), ("subm", 999, 160, 64, "rows-bf16"),
+    ("subm", 1001, 160, 64, "wave-bf16"), ("subm", 4199, 256, 64, "rows-bf16"), ("subm", 4201, 256, 64, "wave-bf16"),
+    ("subm", 4499, 320, 32, "rows-bf16"), ("down", 300, 320, 64, "rows-bf16"), ("up", 300, 320, 64, "wave-bf16"),
+    ("nin", 27999, 64, 96, "wave-bf16"), ("nin", 28001, 64, 96, "rows-bf16"),
+    # two granules per wavefront of k_conv_rows: not over tables of few iterations a tile, nor over most of the long tap lists
+    ("up", 31001, 256, 128, "ss=2"), ("subm", 31001, 256, 128, "ss=4"), ("subm5", 61001, 64, 96, "ss=2"), ("subm5", 17001, 320, 128, "ss=4"),
+    ("nin", 130001, 256, 128, "ss=2"), ("nin", 130001, 256, 96, "ss=4"), ("nin", 70001, 256, 96, "ss=2")])
+def test_bf16_kernel_by_size(kind, n, cin, cout, says):
+    import torch
+    from test_conv_split_gpu import _table
+    conv, rules, rows_in, rows_out, md = _table(kind, n, 8300 + n % 89)
+    md.setBf16(True)
+    g = torch.Generator().manual_seed(n + cin)
+    x, w = torch.randn(rows_in, cin, generator=g).cuda(), (torch.randn(len(rules), 1, cin, cout, generator=g) * 0.1).cuda()
+    got = conv(x, w, torch.zeros(cout).cuda())
+    kernel = md._L.scn_md_last_conv_kernel(md._h).decode()
+    assert says in kernel, kernel
+    want = torch.zeros(rows_out, cout, dtype=torch.float64, device="cuda")
+    mag = want.clone()
+    for k, r in enumerate(rules):
+        r = torch.as_tensor(r).cuda().long()
+        f, v = x[r[:, 0]].bfloat16().double(), w[k, 0].bfloat16().double()
+        want.index_add_(0, r[:, 1], f @ v)
+        mag.index_add_(0, r[:, 1], f.abs() @ v.abs())
+    assert ((got.double() - want).abs() <= (len(rules) * cin + 8) * 2.0 ** -23 * mag + 1e-30).all()
