@@ -387,27 +387,30 @@ static int64_t likely_taps(const Table &t, int64_t in_rows) {
 // us, k_conv_split with its second launch / here (column blocks, granules, wavefronts of the workgroup chosen):
 //   27 taps: 1.2 k sites 48 -> 48 13.0 / 7.9 (2,1,8; three column blocks 9.5), 96 -> 48 15.1 / 10.0, 6 k 48 -> 48 21.4 / 12.9,
 //     96 -> 48 22.2 / 17.4, 12 k 48 -> 48 25 / 18, 20 k 29.9 / 24.0 (2,2,4; 30.1 with 2,1,8), 39 k 55 / 41; 300 sites and fewer gain
-//     another 1 us from one column block (1,1,8); but 400 sites 256 -> 48 16.1 / 17.9, 9 k 128 -> 48 29.1 / 29.8
-//   8 taps, stride 2, onto 25 k sites 32 -> 48 13.8 / 11.5; one rule per position, onto 3.3 k sites 80 -> 48 8.8 / 4.2, 20 k
+//     another 1 us from one column block (1,1,8); but 60 sites 100 -> 44 14.2 / 15.8, 140 160 -> 48 15.7 / 18.8, 400 256 -> 48 16.1 / 17.9,
+//     9 k 128 -> 48 29.1 / 29.8
+//   8 taps, stride 2, onto 25 k sites 32 -> 48 13.8 / 11.5, but onto 8 k 256 -> 48 26.9 / 30.4; one rule per position, onto 3.3 k sites 80 -> 48 8.8 / 4.2, 20 k
 //     64 -> 48 9.6 / 6.8, 40 k 12.2 / 10.9; 1x1 1.5 k rows 96 -> 48 6.7 / 3.5, 20 k 8.8 / 6.9
 // (64 planes and more would gain as much on levels of a few thousand sites, 1.5 k 64 -> 64 14 / 8; they stay on k_conv_split.)
 enum WideTile { NONE, B1G1D8, B2G1D8, B2G2D4 };
-static WideTile wide_tile(const Table &t, int n_in, int n_out) {
+static WideTile wide_tile(const Table &t, int64_t in_rows, int n_in, int n_out) {
   if (n_in <= 16 || n_out > 48) return NONE;
   const int64_t n = t.n, slabs = ceil_div(n_in, 32);
   if (t.few_tap.p || t.K == 1) {
     if (n < 5000) return n < 1500 ? B1G1D8 : B2G1D8;
     return n < 25000 || (t.K > 1 && n < 45000 && slabs <= 2) ? B2G2D4 : NONE;
   }
+  // long chains on the smallest levels: k_conv_split deals them over more workgroups
+  if (slabs >= 4 && n < (slabs == 4 ? 450 : 500) && likely_taps(t, in_rows) > 16) return NONE;
   if (n < 500 && t.K > 9) return slabs <= 5 ? B1G1D8 : NONE;
-  if (t.K <= 9) return n < 500 ? B1G1D8 : n < 2500 ? B2G1D8 : n < 25000 ? B2G2D4 : NONE;
+  if (t.K <= 9) return n < 500 ? B1G1D8 : n < 2500 ? B2G1D8 : n < 25000 && slabs <= 6 ? B2G2D4 : NONE;
   if (n < 10000) return slabs <= (n < 2500 ? 5 : 3) ? B2G1D8 : NONE;
   return n < 40000 && slabs <= 2 ? B2G2D4 : NONE;
 }
 template <bool PRE>
 static void dispatch_wide(Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi, int n_in,
                           int n_out, PreArgs pre, hipStream_t s) {
-  switch (wide_tile(t, n_in, n_out)) {
+  switch (wide_tile(t, m.cur_in_rows, n_in, n_out)) {
   case B1G1D8: return launch_wave<1, 1, 8, 4, false, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);
   case B2G1D8: return launch_wave<2, 1, 8, 4, false, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);
   case B2G2D4: return launch_wave<2, 2, 4, 4, false, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s);
@@ -504,12 +507,17 @@ bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_
   if (n_in <= 4 || n_in % 4 || (uintptr_t)in % 16 || n_in * 4 >= (1 << 24)) return false;
   if (in_rows <= 0 || in_rows >= (1 << 24) || in_rows * n_in * 4 >= ((int64_t)1 << 31)) return false;
   if (m.bf16) return !gradient && bf_tile(t, in_rows, n_in, n_out) != BF_NONE;  // (these weights are packed from a transposed copy)
-  if (n_out > 32) return wide_tile(t, n_in, n_out) != NONE;
+  if (n_out > 32) return wide_tile(t, in_rows, n_in, n_out) != NONE;
   // k_conv_resident keeps 20-32 -> up to 16 planes on small levels of few taps and on large ones
   if (n_in > 16 && n_in <= 32 && n_out <= 16 && (t.K <= 9 ? t.n < 16000 : t.n >= (n_in > 24 ? 200000 : 300000))) return false;
   // k_conv_split: wide inputs of one rule per position, and on the smallest levels chains that it cuts into more parts (500 sites
-  // 64 -> 32 11.9 there, 11.1 here, 128 -> 32 13.7 / 18.5)
+  // 64 -> 32 11.9 there, 11.1 here, 128 -> 32 13.7 / 18.5, 1.01 k 128 -> 24 17.6 / 21.8, 1.05 k 224 -> 32 21.5 / 33.5, 1.7 k 192 -> 32 22.6 / 29.1,
+  // 3.5 k 256 -> 24 37.0 / 43.8, 4.5 k 256 -> 17 35.9 / 41.0, 1.4 k 224 -> 12 23.5 / 29.1; 80 coarse sites of eight taps 256 -> 17 16.5 / 17.4): the
+  // sites from which on this kernel is the faster one, by slabs of 32 channels
+  static const int64_t many[] = {0, 0, 1000, 1000, 2000, 2500, 3700, 5000, 5500};
   if ((t.few_tap.p && n_in > 64) || (t.K > 9 && t.n < 1000 && n_in > 32)) return false;
+  if (likely_taps(t, in_rows) > 16 && t.n < many[std::min<int64_t>(ceil_div(n_in, 32), 8)] * (n_out <= 16 ? 3 : 4) / 4) return false;
+  if (t.K > 1 && t.K <= 9 && !t.few_tap.p && t.n < 150 && n_in > 224) return false;
   // k_deconv_few, all weights in LDS (there / here): transposed 32 -> 32 onto 250 k sites 18.0 / 17.4, 500 k 28.0 / 28.5, 1 M 47 / 49, but
   // 64 -> 32 1 M 71 / 64, 60 k 14.4 / 9.6; 1x1 32 -> 32 60 k rows 8.9 / 7.1, 120 k 10.1 / 10.2, 1 M 45 / 58; 64 -> 32 120 k 14.5 / 13.2,
   // 250 k 22.3 / 22.1, 1 M 82 / 93

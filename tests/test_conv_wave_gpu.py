@@ -190,3 +190,29 @@ def test_bf16_kernel_by_size(kind, n, cin, cout, says):
         want.index_add_(0, r[:, 1], f @ v)
         mag.index_add_(0, r[:, 1], f.abs() @ v.abs())
     assert ((got.double() - want).abs() <= (len(rules) * cin + 8) * 2.0 ** -23 * mag + 1e-30).all()
+
+
+@pytest.mark.parametrize("kind,n,cin,cout,says", [
+    ("subm", 1050, 224, 32, "split ncbw"), ("subm", 1999, 128, 32, "split ncbw"), ("subm", 2001, 128, 32, "split wave"),
+    ("subm", 1499, 128, 16, "split ncbw"), ("subm", 1501, 128, 16, "split wave"), ("subm", 3699, 192, 24, "split ncbw"),
+    ("subm", 3701, 192, 24, "split wave"), ("subm", 5499, 256, 20, "split ncbw"), ("subm", 5501, 256, 20, "split wave"),
+    ("subm", 449, 100, 44, "split ncbw"), ("subm", 451, 100, 44, "split wave"), ("subm", 499, 160, 48, "split ncbw"),
+    ("subm", 140, 96, 48, "split wave"), ("down", 100, 256, 17, "split ncbw"), ("down", 1500, 256, 17, "split wave"),
+    ("down", 33001, 256, 48, "split ncbw")])
+def test_kernel_by_length_of_the_chain(kind, n, cin, cout, says):
+    """Many (tap, 32 channels) products per row on small levels: k_conv_split deals them over workgroups."""
+    import torch
+    from test_conv_split_gpu import _table
+    conv, rules, rows_in, rows_out, md = _table(kind, n, 8100 + n % 89)
+    g = torch.Generator().manual_seed(n + cout)
+    x, w = torch.randn(rows_in, cin, generator=g).cuda(), (torch.randn(len(rules), 1, cin, cout, generator=g) * 0.1).cuda()
+    got = conv(x, w, torch.zeros(cout).cuda())
+    kernel = md._L.scn_md_last_conv_kernel(md._h).decode()
+    assert says in kernel, kernel
+    want = torch.zeros(rows_out, cout, dtype=torch.float64, device="cuda")
+    mag = want.clone()
+    for k, r in enumerate(rules):
+        r = torch.as_tensor(r).cuda().long()
+        want.index_add_(0, r[:, 1], x[r[:, 0]].double() @ w[k, 0].double())
+        mag.index_add_(0, r[:, 1], x[r[:, 0]].double().abs() @ w[k, 0].double().abs())
+    assert ((got.double() - want).abs() <= (len(rules) * -(-cin // 32) + 3 + 1 + 4) * 2.0 ** -24 * mag).all()
