@@ -331,17 +331,20 @@ __global__ __launch_bounds__(256) void k_conv_dw(const int *__restrict__ nbr, co
 // channels 2 r and 2 r + 1 as one 8-byte load (16 lanes read 128 consecutive bytes); instruction
 // i of a pair takes component i, so that it computes the gradient's rows 2 * (MFMA row) + i, and
 // likewise for the columns.  The rows of b are loaded once per granule and serve all its taps.
-// (Sixteen wavefronts of two taps with indices through LDS a block of granules ahead and one barrier per block, us with the launch that adds
-// the shares up, here / so: 27 taps 32 x 32 6 k sites 30.7 / 27.9, a million 513 / 487, but 100 k 80 / 85, 64 sites 19 / 24, and where a
-// granule has few of the taps a wavefront waits for the others' blocks: transposed a million positions 281 / 357, filter 3 stride 2 222 / 424,
-// 1x1 100 k rows 16 x 16 25 / 54.)
-constexpr int DT_NW = 8, DT_T = 32, DT_SLOTS = 4, DT_BLOCK = 8;  // DT_BLOCK granules of 16 positions per turn
-template <bool VEC2>
+// NW = 16, small levels, where the launch is as long as one workgroup's block of DT_BLOCK granules: sixteen wavefronts of two taps; the block's
+// indices, rows and masks come to LDS first, and a granule's rows are requested behind the MFMAs of the one before (one memory latency per
+// granule instead of two).  With the launch that adds the shares up, us, eight wavefronts / sixteen, the same bits: 27 taps 16 x 16 150 sites
+// 29.7 / 27.9, 32 x 32 6 k 31.0 / 28.5, 24 k 37.3 / 30.9; nine taps 16 x 16 6 k 22.7 / 20.4; eight onto 24 k 32 x 32 28.7 / 22.7.  Not with
+// several blocks per workgroup, a barrier each (27 taps 32 x 32 100 k 80 / 85, a million 513 / 487), nor where granules have few taps or
+// blocks few granules (transposed 600 positions 13.7 / 18.8, filter 3 stride 2 19 / 21, 1x1 15 / 18, 64 sites 19 / 23).
+constexpr int DT_T = 32, DT_TAPS = 32, DT_BLOCK = 8;  // DT_BLOCK granules of 16 positions per turn
+template <bool VEC2, int DT_NW>
 __global__ __launch_bounds__(DT_NW * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_conv_dw_taps(const int *__restrict__ nbr, const int *__restrict__ rowmap,
                                                              const unsigned *__restrict__ gmask, int K, int64_t n,
                                                              int64_t npad, const float *__restrict__ a, int n_a,
                                                              unsigned a_bytes, const float *__restrict__ b, int n_b,
                                                              unsigned b_bytes, float *__restrict__ partial) {
+  constexpr int DT_SLOTS = DT_TAPS / DT_NW;
   const int tiles_o = (n_b + DT_T - 1) / DT_T;
   const int ct = blockIdx.y / tiles_o, ot = blockIdx.y % tiles_o;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -380,6 +383,61 @@ __global__ __launch_bounds__(DT_NW * 64) __attribute__((amdgpu_waves_per_eu(4, 4
   // Workgroup x takes the blocks of DT_BLOCK granules x, x + gridDim.x, ...: every workgroup sees
   // every part of the pattern-sorted table, so that they all carry about the same number of rules.
   const int n_granules = (int)((n + 15) >> 4), n32 = (int)n;  // the host checks that 4 K npad < 2^31
+  auto multiply = [&](int sl, unsigned present, const v2f (&av)[DT_SLOTS][4], const v2f (&bv)[4]) {
+    if (!((present >> (wave + sl * DT_NW)) & 1u)) return;  // uniform over the wavefront
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int jx = 0; jx < 2; jx++)
+          acc[sl][i][jx] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[sl][kk][i], bv[kk][jx], acc[sl][i][jx], 0, 0, 0);
+  };
+  if constexpr (DT_NW == 16) {  // the workgroup's one block
+    __shared__ int4 jtab[DT_TAPS][4 * DT_BLOCK];  // [tap][position / 4]
+    __shared__ int rows[16 * DT_BLOCK];
+    __shared__ unsigned masks[DT_BLOCK + 1];
+    const int t0 = 16 * DT_BLOCK * blockIdx.x, tid = threadIdx.x;
+    const int k = tid / (4 * DT_BLOCK), p = t0 + 4 * (tid % (4 * DT_BLOCK));
+    static_assert(DT_NW * 64 == DT_TAPS * 4 * DT_BLOCK, "a thread per quad of indices");
+    jtab[k][tid % (4 * DT_BLOCK)] = __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(
+        nbr_rsrc, k < K && p < npad ? ((unsigned)k * (unsigned)npad + (unsigned)p) * 4u : nowhere, 0, 0));
+    if (tid < 16 * DT_BLOCK) rows[tid] = t0 + tid < n32 ? (rowmap ? rowmap[t0 + tid] : t0 + tid) : -1;
+    if (tid <= DT_BLOCK) masks[tid] = tid < DT_BLOCK && t0 + 16 * tid < n32 ? gmask[t0 / 16 + tid] : 0u;
+    __syncthreads();
+    v2f av[DT_SLOTS][4], bv[4], bn[4];
+    auto issue_a = [&](int gl, unsigned present, int sl) {
+      const int kt = wave + sl * DT_NW;
+      const bool has = (present >> kt) & 1u;
+      const int4 j4 = jtab[kt][4 * min(gl, DT_BLOCK - 1) + g];
+      const int j[4] = {j4.x, j4.y, j4.z, j4.w};
+#pragma unroll
+      for (int kk = 0; kk < 4; kk++) av[sl][kk] = pair_of(a_rsrc, has ? j[kk] : -1, a_row_bytes, ca0, ca1);
+    };
+    auto issue_b = [&](int gl, unsigned present, v2f (&dst)[4]) {
+      const int4 r4 = *reinterpret_cast<const int4 *>(&rows[16 * min(gl, DT_BLOCK - 1) + 4 * g]);
+      const int r[4] = {r4.x, r4.y, r4.z, r4.w};
+#pragma unroll
+      for (int kk = 0; kk < 4; kk++) dst[kk] = pair_of(b_rsrc, present ? r[kk] : -1, b_row_bytes, cb0, cb1);
+    };
+    unsigned present = __builtin_amdgcn_readfirstlane(masks[0]) & own;
+    issue_b(0, present, bv);
+#pragma unroll
+    for (int sl = 0; sl < DT_SLOTS; sl++) issue_a(0, present, sl);
+#pragma unroll 1
+    for (int gl = 0; gl < DT_BLOCK; gl++) {
+      const unsigned next = __builtin_amdgcn_readfirstlane(masks[gl + 1]) & own;  // behind the last granule none
+      issue_b(gl + 1, next, bn);
+#pragma unroll
+      for (int sl = 0; sl < DT_SLOTS; sl++) {
+        multiply(sl, present, av, bv);
+        issue_a(gl + 1, next, sl);  // the registers are free
+      }
+      present = next;
+#pragma unroll
+      for (int kk = 0; kk < 4; kk++) bv[kk] = bn[kk];
+    }
+  } else
   for (int gb = blockIdx.x * DT_BLOCK; gb < n_granules; gb += gridDim.x * DT_BLOCK) {
     const int ge = min(n_granules, gb + DT_BLOCK);
     for (int gi = gb; gi < ge; gi++) {
@@ -422,18 +480,7 @@ __global__ __launch_bounds__(DT_NW * 64) __attribute__((amdgpu_waves_per_eu(4, 4
         for (int kk = 0; kk < 4; kk++) av[sl][kk] = pair_of(a_rsrc, has ? j[kk] : -1, a_row_bytes, ca0, ca1);
       }
 #pragma unroll
-      for (int sl = 0; sl < DT_SLOTS; sl++) {
-        const int k = wave + sl * DT_NW;
-        if (!((present >> k) & 1u)) continue;  // uniform over the wavefront
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++)
-#pragma unroll
-          for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int jx = 0; jx < 2; jx++)
-              acc[sl][i][jx] =
-                  __builtin_amdgcn_mfma_f32_16x16x4f32(av[sl][kk][i], bv[kk][jx], acc[sl][i][jx], 0, 0, 0);
-      }
+      for (int sl = 0; sl < DT_SLOTS; sl++) multiply(sl, present, av, bv);
     }
   }
   // acc[sl][i][jx][r] = dW[k][ct*32 + 2 (4 g + r) + i][ot*32 + 2 r16 + jx] of this chunk
@@ -869,7 +916,7 @@ static void weight_gradient(Metadata &m, const Table &t, const float *a, int64_t
   }
   // up to 32 channels on both sides; from there on the per-wavefront kernel below is faster
   // (64 -> 64 at 1 M sites: 1.97 against 1.3 ms)
-  if (t.K <= DT_NW * DT_SLOTS && t.gmask.p && n_a <= DT_T && n_b <= DT_T && t.npad % 4 == 0 &&
+  if (t.K <= DT_TAPS && t.gmask.p && n_a <= DT_T && n_b <= DT_T && t.npad % 4 == 0 &&
       a_rows * n_a * 4 < ((int64_t)1 << 31) && b_rows * n_b * 4 < ((int64_t)1 << 31) &&
       (int64_t)t.K * t.npad * 4 < ((int64_t)1 << 31)) {
     // narrow layers: all taps per workgroup
@@ -881,14 +928,15 @@ static void weight_gradient(Metadata &m, const Table &t, const float *a, int64_t
     m.partial.reserve((size_t)chunks * per_chunk);
     const dim3 grid((unsigned)chunks, (unsigned)tiles);
     const bool vec2 = n_a % 2 == 0 && n_b % 2 == 0 && (uintptr_t)a % 8 == 0 && (uintptr_t)b % 8 == 0;
-    if (vec2)
-      k_conv_dw_taps<true><<<grid, DT_NW * 64, 0, s>>>(t.nbr.p, t.rowmap_ptr(), t.gmask.p, t.K, t.n, t.npad, a, n_a,
-                                                       (unsigned)(a_rows * n_a * 4), b, n_b,
-                                                       (unsigned)(b_rows * n_b * 4), m.partial.p);
+    auto run = [&](auto kern, int waves) {
+      kern<<<grid, waves * 64, 0, s>>>(t.nbr.p, t.rowmap_ptr(), t.gmask.p, t.K, t.n, t.npad, a, n_a, (unsigned)(a_rows * n_a * 4), b, n_b,
+                                       (unsigned)(b_rows * n_b * 4), m.partial.p);
+    };
+    // sixteen wavefronts: one block per workgroup, and a compute unit has at most one of those; fine sides gather from fewer rows
+    if (t.K >= 8 && a_rows >= t.n && t.n >= 100 && t.n <= 256 * 16 * DT_BLOCK)
+      vec2 ? run(k_conv_dw_taps<true, 16>, 16) : run(k_conv_dw_taps<false, 16>, 16);
     else
-      k_conv_dw_taps<false><<<grid, DT_NW * 64, 0, s>>>(t.nbr.p, t.rowmap_ptr(), t.gmask.p, t.K, t.n, t.npad, a, n_a,
-                                                        (unsigned)(a_rows * n_a * 4), b, n_b,
-                                                       (unsigned)(b_rows * n_b * 4), m.partial.p);
+      vec2 ? run(k_conv_dw_taps<true, 8>, 8) : run(k_conv_dw_taps<false, 8>, 8);
     LAUNCH_CHECK();
     k_sum_blocks<float, float><<<dim3((unsigned)ceil_div(per_chunk, 64)), sum_threads(chunks), 0, s>>>(m.partial.p, (int)chunks, per_chunk, per_chunk, dw);
     LAUNCH_CHECK();
