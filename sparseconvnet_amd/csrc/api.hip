@@ -125,7 +125,11 @@ void *pool_alloc(size_t bytes, int pool) {
       std::lock_guard<std::mutex> lock(g_pool_mutex);
       release_idle_locked();
     }
-    HIP_CHECK(hipMalloc(&p, cls));
+    e = hipMalloc(&p, cls);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();  // reported here, not by the next launch's check
+      hip_check(e, "hipMalloc(&p, cls)", __FILE__, __LINE__);
+    }
   }
   std::lock_guard<std::mutex> lock(g_pool_mutex);
   g_block_bytes[p] = cls;
