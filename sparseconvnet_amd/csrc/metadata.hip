@@ -2804,6 +2804,8 @@ __global__ void k_identity_tables(IdentJobs j) {  // blockIdx.y: table
 // over this table: one tap, position t reads row t and writes row t.  The first one makes those of the handle's other
 // levels as well, by the same launch, where they are small: a network that has a 1x1 convolution on one level has one on others,
 // and each would be a launch of its own and an event that the other stream waits for, some 8 us, for what 64 k rows write in 2.
+// The tables are kept once they have been filled: a call that fails leaves none behind, and memory that is short for a level ahead of
+// its use is no error of this call.
 constexpr int64_t IDENT_AHEAD = 65536;
 Table &identity_table(Metadata &m, int64_t rows, hipStream_t s) {
   auto it = m.ident.find(rows);
@@ -2812,8 +2814,8 @@ Table &identity_table(Metadata &m, int64_t rows, hipStream_t s) {
   IdentJobs jobs{};
   int n_jobs = 0;
   int64_t most = 0;
+  std::map<int64_t, Table> made;
   auto make = [&](int64_t n) {
-    if (n_jobs == IDENT_JOBS || m.ident.count(n)) return;
     Table t;
     t.K = 1;
     t.n = n;
@@ -2828,18 +2830,26 @@ Table &identity_table(Metadata &m, int64_t rows, hipStream_t s) {
       t.nbr.reserve(t.npad);
       t.gmask.reserve(ceil_div(n, 16));
       jobs.n[n_jobs] = n, jobs.npad[n_jobs] = t.npad, jobs.nbr[n_jobs] = t.nbr.p, jobs.gmask[n_jobs] = t.gmask.p;
-      n_jobs++;
-      most = std::max(most, t.npad);
     }
-    m.ident.emplace(n, std::move(t));
+    made.emplace(n, std::move(t));
+    if (n > 0) {
+      n_jobs++;
+      most = std::max(most, round_up(n, 64));
+    }
   };
   make(rows);
-  for (const auto &l : m.levels)
-    if (l.second.n > 0 && l.second.n <= IDENT_AHEAD) make(l.second.n);
+  try {
+    for (const auto &l : m.levels) {
+      const int64_t n = l.second.n;
+      if (n_jobs < IDENT_JOBS && n > 0 && n <= IDENT_AHEAD && !made.count(n) && !m.ident.count(n)) make(n);
+    }
+  } catch (const std::exception &) {  // those that have their memory are made
+  }
   if (n_jobs) {
     k_identity_tables<<<dim3((unsigned)ceil_div(most, TB), n_jobs), TB, 0, s>>>(jobs);
     LAUNCH_CHECK();
   }
+  for (auto &e : made) m.ident.emplace(e.first, std::move(e.second));
   return m.ident.at(rows);
 }
 

@@ -76,9 +76,60 @@ static void failed_allocation() {
   CHECK(threw && mallocs == 2 && hipGetLastError() == hipSuccess);
 }
 
+static void add_level(Metadata &m, int64_t side, int64_t n) {
+  Level &l = m.levels[SizeKey{side, side, side}];
+  l.n = n;
+  l.npad = round_up(n, 64);
+}
+
+// A table is kept for later calls only once the kernel that fills it has been launched, and a level nobody asked about yet does not
+// fail the call.
+static void identity_tables() {
+  for (int ok = 0; ok < 8; ok++) {  // how many allocations succeed: two per table, four tables
+    Metadata m;
+    m.dim = 3;
+    add_level(m, 64, 5000), add_level(m, 32, 90000), add_level(m, 16, 700), add_level(m, 8, 30);
+    mallocs = launches = 0;
+    fail_malloc = ok;
+    bool threw = false;
+    try {
+      Table &t = identity_table(m, 90000, nullptr);
+      CHECK(t.n == 90000 && t.nbr.p && t.gmask.p && launches == 1);
+    } catch (const std::exception &) {
+      threw = true;
+    }
+    fail_malloc = -1;
+    CHECK(threw == (ok < 2));
+    if (threw) CHECK(m.ident.empty() && launches == 0);
+    for (auto &e : m.ident) CHECK(e.second.nbr.p && e.second.gmask.p);
+    const int before = launches;
+    for (int64_t n : {90000, 5000, 700, 30}) {
+      const bool had = m.ident.count(n);
+      Table &t = identity_table(m, n, nullptr);
+      CHECK(t.n == n && t.K == 1 && t.nbr.p && t.gmask.p);
+      CHECK(had || launches > before);
+    }
+    m.ident.clear();
+    scn_release_cache();  // the next round allocates again
+  }
+  Metadata m;
+  m.dim = 3;
+  add_level(m, 16, 700);
+  fail_launch = true;
+  bool threw = false;
+  try {
+    identity_table(m, 5000, nullptr);
+  } catch (const std::exception &) {
+    threw = true;
+  }
+  fail_launch = false;
+  CHECK(threw && m.ident.empty());
+}
+
 int main(int argc, char **argv) {
   const char *name = argc > 1 ? argv[1] : "";
   if (!strcmp(name, "failed_allocation")) failed_allocation();
+  else if (!strcmp(name, "identity_tables")) identity_tables();
   else return printf("no check of that name\n"), 2;
   printf("ok\n");
   return 0;
