@@ -514,6 +514,14 @@ static Level *find_level(Metadata &m, const int64_t *spatial) {
   return it == m.levels.end() ? nullptr : &it->second;
 }
 
+// A forward convolution's entry point: what was said of the next convolution's output (scn_md_next_differentiated) ends with it, also
+// where it fails in front of its kernel.
+template <class F> static int convolution(scn_metadata *h, F f) {
+  const int status = guarded(f);
+  if (h) h->m.differentiated = false;
+  return status;
+}
+
 extern "C" {
 
 const char *scn_last_error(void) { return g_error.c_str(); }
@@ -859,14 +867,14 @@ static void deconv(scn_metadata *h, const int64_t *in_size, const int64_t *out_s
 int scn_subm_conv_fwd(scn_metadata *h, const int64_t *spatial, const int64_t *filter, const float *in,
                       float *out, const float *weight, const float *bias, int n_in, int n_out,
                       int groups, void *stream, double *macs) {
-  return guarded([&] {
+  return convolution(h, [&] {
     subm_conv(h, spatial, filter, in, out, weight, bias, n_in, n_out, groups, nullptr, nullptr, stream, macs);
   });
 }
 int scn_subm_conv_fwd_noalloc(scn_metadata *h, const int64_t *spatial, const int64_t *filter, const float *in,
                               float *out, const float *weight, const float *bias, int n_in, int n_out,
                               void *stream) {
-  return guarded([&] {
+  return convolution(h, [&] {
     Metadata &m = md(h);
     auto it = m.subm.find(mk(m.dim, spatial, filter));
     if (it == m.subm.end())
@@ -885,7 +893,7 @@ int scn_subm_conv_fwd_noalloc(scn_metadata *h, const int64_t *spatial, const int
 int scn_conv_fwd(scn_metadata *h, const int64_t *in_size, const int64_t *out_size, const int64_t *filter,
                  const int64_t *stride, const float *in, float *out, const float *weight,
                  const float *bias, int n_in, int n_out, int groups, void *stream, double *macs) {
-  return guarded([&] {
+  return convolution(h, [&] {
     strided_conv(h, in_size, out_size, filter, stride, in, out, weight, bias, n_in, n_out, groups, nullptr, nullptr,
                  stream, macs);
   });
@@ -893,7 +901,7 @@ int scn_conv_fwd(scn_metadata *h, const int64_t *in_size, const int64_t *out_siz
 int scn_deconv_fwd(scn_metadata *h, const int64_t *in_size, const int64_t *out_size, const int64_t *filter,
                    const int64_t *stride, const float *in, float *out, const float *weight,
                    const float *bias, int n_in, int n_out, int groups, void *stream, double *macs) {
-  return guarded([&] {
+  return convolution(h, [&] {
     deconv(h, in_size, out_size, filter, stride, in, out, weight, bias, n_in, n_out, groups, nullptr, nullptr, stream,
            macs);
   });
@@ -902,7 +910,7 @@ int scn_conv_bn_fwd(scn_metadata *h, int kind, const int64_t *a, const int64_t *
                     const int64_t *d, const float *in, float *out, const float *weight, const float *bias,
                     int n_in, int n_out, int groups, const scn_bn_params *pre, const scn_bn_params *post,
                     void *stream, double *macs) {
-  return guarded([&] {
+  return convolution(h, [&] {
     BnArgs pre_a{}, post_a{};
     auto conv = [](const scn_bn_params *p, BnArgs &o) -> const BnArgs * {
       if (!p) return nullptr;
@@ -923,7 +931,7 @@ int scn_conv_bn_fwd(scn_metadata *h, int kind, const int64_t *a, const int64_t *
 }
 int scn_nin_fwd(scn_metadata *h, const float *in, float *out, const float *weight, const float *bias,
                 int64_t rows, int n_in, int n_out, void *stream, double *macs) {
-  return guarded([&] {
+  return convolution(h, [&] {
     Metadata &m = md(h);
     if (rows < 0 || rows >= ((int64_t)1 << 31)) throw Error("network in network: row count out of range");
     Table *tp;

@@ -308,7 +308,6 @@ void conv_forward(Metadata &m, const Table &t, const float *in, int64_t n_in_row
       m.next_out2 = nullptr;
       m.before_pack = nullptr;
       m.pack_transposed = nullptr;
-      m.differentiated = false;
       m.wkey_ptr = 0;
     }
   } frozen_reset{m};

@@ -237,7 +237,7 @@ struct Metadata {
   // in reverse order): the packing reads them so (k_pack_weights_split), no transposed copy is made.
   const float *pack_transposed = nullptr;
   bool pack_mirror = false;
-  bool differentiated = false;  // the next convolution call's output will be differentiated (scn_md_next_differentiated); serves one call
+  bool differentiated = false;  // the next forward convolution's output will be differentiated (scn_md_next_differentiated); serves one call (api.hip: convolution)
   std::function<void()> before_pack;  // work the packing of the running convolution's weights needs first (the column-range path's copy), run at most once
   // while a column range of a wide layer runs: addresses in the scratch copy (from wkey_from) stand for
   // addresses from wkey_ptr in the caller's weights in a frozen set's keys

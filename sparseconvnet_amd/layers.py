@@ -98,9 +98,8 @@ class _ConvFunction(Function):
         ctx.has_bias = bias.numel() > 0
         ctx.save_for_backward(features, weight)
         fn = (md.submanifoldConvolution, md.convolution, md.deconvolution)[kind]
-        if any(ctx.needs_input_grad):
-            md.nextDifferentiated()
-        out, _ = fn(*sizes, features, weight, bias, pre, post, want_macs=False, out=out, second=second)
+        out, _ = fn(*sizes, features, weight, bias, pre, post, want_macs=False, out=out, second=second,
+                    differentiated=any(ctx.needs_input_grad))
         _count(out)
         return out
 
@@ -121,9 +120,7 @@ class _NetworkInNetworkFunction(Function):
     def forward(ctx, features, weight, bias, md):
         ctx.md, ctx.has_bias = md, bias.numel() > 0
         ctx.save_for_backward(features, weight)
-        if any(ctx.needs_input_grad):
-            md.nextDifferentiated()
-        out, _ = md.networkInNetwork(features, weight, bias, want_macs=False)
+        out, _ = md.networkInNetwork(features, weight, bias, want_macs=False, differentiated=any(ctx.needs_input_grad))
         _count(out)
         return out
 

@@ -219,7 +219,8 @@ class Metadata:
         _lib.check(self._L.scn_output_layer_fwd(self._h, _ptr(features), _ptr(out), features.size(1), _stream()))
         return out
 
-    def _conv(self, kind, size_args, n_rows, features, weight, bias, bn, post, want_macs, out=None, second=None):
+    def _conv(self, kind, size_args, n_rows, features, weight, bias, bn, post, want_macs, out=None, second=None,
+              differentiated=False):
         """kind 0 / 1 / 2: submanifold / strided / transposed convolution.  bn, post: None, or
         (running_mean, running_var, weight, bias, eps, leakiness) of an eval-mode batch
         normalisation in front of / behind the convolution, applied inside it.  want_macs:
@@ -228,7 +229,8 @@ class Metadata:
         out: a [rows, planes] range of columns of a wider float32 matrix to write the result into
         (the convolution's part of a concatenation), or None for a new tensor.
         second: None, or (batch norm arguments, columns as for `out`): the convolution also writes
-        its output there, taken before `post` and normalised with that batch norm instead."""
+        its output there, taken before `post` and normalised with that batch norm instead.
+        differentiated: the output will be (nextDifferentiated)."""
         features = _features(features, "features")
         weight = _features(weight, "weight")
         K, groups, ip, op = weight.shape
@@ -255,18 +257,20 @@ class Metadata:
                 if n_rows and out.stride(0) != out.size(1):
                     resets.append(lambda: self._L.scn_md_next_output_stride(self._h, 0))
                     _lib.check(self._L.scn_md_next_output_stride(self._h, out.stride(0)))
-            return self._conv_into(kind, size_args, features, weight, bias_t, bn, post, want_macs, out)
+            return self._conv_into(kind, size_args, features, weight, bias_t, bn, post, want_macs, out, differentiated)
         finally:
             for r in resets:
                 r()
 
-    def _conv_into(self, kind, size_args, features, weight, bias_t, bn, post, want_macs, out):
+    def _conv_into(self, kind, size_args, features, weight, bias_t, bn, post, want_macs, out, differentiated):
         K, groups, ip, op = weight.shape
         macs = C.c_double(0)
         macs_p = C.byref(macs) if want_macs else None
         tail = (_ptr(features), _ptr(out), _ptr(weight), _ptr(bias_t), groups * ip, groups * op, groups)
         if bn is None and post is None:
             fn = (self._L.scn_subm_conv_fwd, self._L.scn_conv_fwd, self._L.scn_deconv_fwd)[kind]
+            if differentiated:
+                self.nextDifferentiated()
             _lib.check(fn(self._h, *size_args, *tail, _stream(), macs_p))
         else:
             keep = []  # tensors behind the raw pointers stay alive until the call has been issued
@@ -282,30 +286,35 @@ class Metadata:
                 keep.extend(t)
                 return C.byref(_lib.BnParams(*[_ptr(x) for x in t], float(eps), float(leak)))
             sizes = list(size_args) + [None] * (4 - len(size_args))
-            _lib.check(self._L.scn_conv_bn_fwd(self._h, kind, *sizes, *tail, params(bn, groups * ip),
-                                               params(post, groups * op), _stream(), macs_p))
+            bns = params(bn, groups * ip), params(post, groups * op)
+            if differentiated:
+                self.nextDifferentiated()
+            _lib.check(self._L.scn_conv_bn_fwd(self._h, kind, *sizes, *tail, *bns, _stream(), macs_p))
         return out, (macs.value if want_macs else None)
 
     def submanifoldConvolution(self, spatial_size, filter_size, features, weight, bias, bn=None, post=None,
-                               want_macs=True, out=None, second=None):
+                               want_macs=True, out=None, second=None, differentiated=False):
         sp, fs = self._s(spatial_size), self._s(filter_size)
         _lib.check(self._L.scn_md_submanifold_rules(self._h, sp, fs, _stream()))
-        return self._conv(0, (sp, fs), self.getNActive(spatial_size), features, weight, bias, bn, post, want_macs, out, second)
+        return self._conv(0, (sp, fs), self.getNActive(spatial_size), features, weight, bias, bn, post, want_macs, out, second,
+                          differentiated)
 
     def convolution(self, in_size, out_size, filter_size, stride, features, weight, bias, bn=None, post=None,
-                    want_macs=True, out=None, second=None):
+                    want_macs=True, out=None, second=None, differentiated=False):
         a = [self._s(v) for v in (in_size, out_size, filter_size, stride)]
         _lib.check(self._L.scn_md_strided_rules(self._h, *a, _stream()))
-        return self._conv(1, a, self.getNActive(out_size), features, weight, bias, bn, post, want_macs, out, second)
+        return self._conv(1, a, self.getNActive(out_size), features, weight, bias, bn, post, want_macs, out, second,
+                          differentiated)
 
     def deconvolution(self, in_size, out_size, filter_size, stride, features, weight, bias, bn=None, post=None,
-                      want_macs=True, out=None, second=None):
+                      want_macs=True, out=None, second=None, differentiated=False):
         a = [self._s(v) for v in (in_size, out_size, filter_size, stride)]
         rb = [self._s(v) for v in (out_size, in_size, filter_size, stride)]
         _lib.check(self._L.scn_md_strided_rules(self._h, *rb, _stream()))
-        return self._conv(2, a, self.getNActive(out_size), features, weight, bias, bn, post, want_macs, out, second)
+        return self._conv(2, a, self.getNActive(out_size), features, weight, bias, bn, post, want_macs, out, second,
+                          differentiated)
 
-    def networkInNetwork(self, features, weight, bias, want_macs=True):
+    def networkInNetwork(self, features, weight, bias, want_macs=True, differentiated=False):
         """out = bias + features @ weight (weight [nIn, nOut]): a convolution with one tap."""
         features = _features(features, "features")
         weight = _features(weight, "weight")
@@ -314,6 +323,8 @@ class Metadata:
         assert features.size(0) == 0 or features.size(1) == n_in, (features.shape, weight.shape)
         out = torch.empty((features.size(0), n_out), dtype=torch.float32, device=features.device)
         macs = C.c_double(0)
+        if differentiated:
+            self.nextDifferentiated()
         _lib.check(self._L.scn_nin_fwd(self._h, _ptr(features), _ptr(out), _ptr(weight), _ptr(bias_t),
                                        features.size(0), n_in, n_out, _stream(),
                                        C.byref(macs) if want_macs else None))

@@ -27,3 +27,26 @@ def test_one_call_keeps_its_rounding(n, planes):
         c = conv(x).features
     assert "split wave" in kernel() and torch.equal(a, c)
     assert (a - b).norm() <= 1e-6 * a.norm()
+
+
+@pytest.mark.parametrize("fails", ["operands", "call"])
+def test_a_call_that_fails_leaves_nothing_behind(fails):
+    import ctypes as C
+    import torch
+    import sparseconvnet_amd as scn
+    g = torch.Generator().manual_seed(5)
+    cells = torch.randperm(96 ** 3, generator=g)[:3001]
+    coords = torch.stack([cells // 96 ** 2, cells // 96 % 96, cells % 96], 1)
+    t = scn.InputLayer(3, 96, mode=0)([coords.cuda(), torch.zeros(3001, 1).cuda()])
+    md = t.metadata
+    conv = scn.SubmanifoldConvolution(3, 16, 16, 3, False).cuda()
+    x = torch.randn(3001, 16, generator=g).cuda()
+    if fails == "operands":  # refused in Python
+        with pytest.raises(Exception):
+            conv(scn.SparseConvNetTensor(x.double(), md, t.spatial_size))
+    else:  # refused by the library in front of its kernel
+        md.nextDifferentiated()
+        assert md._L.scn_conv_bn_fwd(md._h, 9, None, None, None, None, None, None, None, None, 16, 16, 1, None, None, C.c_void_p(0), None) != 0
+    with torch.no_grad():
+        conv(scn.SparseConvNetTensor(x, md, t.spatial_size))
+    assert "split wave" in md._L.scn_md_last_conv_kernel(md._h).decode()
