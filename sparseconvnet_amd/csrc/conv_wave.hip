@@ -356,6 +356,9 @@ __global__ __launch_bounds__(64 * (DEAL > 4 ? DEAL : 4), OCC) void k_conv_wave(
 template <int NCB, int GW, int DEAL, int OCC, bool PAIR, bool PRE, bool BF16 = false>
 static void launch_wave(Metadata &m, const Table &t, const float *in, float *out, const float *w, Epi epi, int n_in,
                         int n_out, PreArgs pre, hipStream_t s) {
+  // what the kernel reads without looking: a slip in the dispatch is an error here, not a read through a null pointer
+  if (!t.gmask.p || t.K > 32 || m.fixed_scratch || n_in % 4 || (uintptr_t)in % 16 || m.cur_in_rows * n_in * 4 >= ((int64_t)1 << 31))
+    throw Error("internal: this convolution does not fit the kernel chosen for it");
   const int n_slab = (int)ceil_div(n_in, 32);
   const int groups = (int)ceil_div(n_out, 16 * NCB), ncb = groups * NCB;
   const float *wpack;
@@ -503,6 +506,8 @@ bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_
   // of a ReLU change sides, and the gradients of a training step over some ten thousand sites differ by up to 9e-3 (2-D: 3.5e-3).  A
   // million-site step takes 1 % longer for it.
   if ((t.K == 9 || m.differentiated) && !gradient) return false;
+  // The kernel reads granule masks of 32 bits, which tables of more taps do not have (gmask is null there), and keeps its taps in the lanes of
+  // half a wavefront; the allocation-free entry has no room for its weights.
   if (m.fixed_scratch || t.K > 32 || !t.gmask.p) return false;
   if (n_in <= 4 || n_in % 4 || (uintptr_t)in % 16 || n_in * 4 >= (1 << 24)) return false;
   if (in_rows <= 0 || in_rows >= (1 << 24) || in_rows * n_in * 4 >= ((int64_t)1 << 31)) return false;

@@ -126,10 +126,47 @@ static void identity_tables() {
   CHECK(threw && m.ident.empty());
 }
 
+// Calls whose tables, operands or scratch k_conv_wave cannot read are refused, whatever else they are: forward or gradient, either operand type.
+static void wave_refuses() {
+  Metadata m;
+  Table t;
+  t.n = 3000, t.npad = 3008;
+  t.gmask.reserve(188);
+  const float *in = (const float *)4096;
+  for (bool bf16 : {false, true})
+    for (bool gradient : {false, true}) {
+      m.bf16 = bf16;
+      const int n_in = 32;
+      for (int K : {1, 8, 27, 32}) {
+        t.K = K;
+        CHECK(conv_wave_serves(m, t, in, 3000, n_in, 32, gradient) == !(bf16 && gradient));
+        for (int64_t rows : {(int64_t)0, (int64_t)1 << 24, (int64_t)1 << 31}) CHECK(!conv_wave_serves(m, t, in, rows, n_in, 32, gradient));
+        CHECK(!conv_wave_serves(m, t, in + 1, 3000, n_in, 32, gradient));
+        CHECK(!conv_wave_serves(m, t, in, 3000, 33, 32, gradient) && !conv_wave_serves(m, t, in, 3000, 30, 32, gradient));
+        m.fixed_scratch = (unsigned char *)&m;
+        CHECK(!conv_wave_serves(m, t, in, 3000, n_in, 32, gradient));
+        m.fixed_scratch = nullptr;
+        Table bare;
+        bare.n = t.n, bare.npad = t.npad, bare.K = K;
+        CHECK(!conv_wave_serves(m, bare, in, 3000, n_in, 32, gradient));
+      }
+      for (int K : {33, 49, 64, 125}) {
+        t.K = K;
+        for (int64_t n : {500, 3000, 300001}) {
+          t.n = n;
+          for (int planes : {8, 20, 32, 48, 64, 128})
+            for (int out : {8, 32, 40, 48, 64}) CHECK(!conv_wave_serves(m, t, in, n, planes, out, gradient));
+        }
+        t.n = 3000;
+      }
+    }
+}
+
 int main(int argc, char **argv) {
   const char *name = argc > 1 ? argv[1] : "";
   if (!strcmp(name, "failed_allocation")) failed_allocation();
   else if (!strcmp(name, "identity_tables")) identity_tables();
+  else if (!strcmp(name, "wave_refuses")) wave_refuses();
   else return printf("no check of that name\n"), 2;
   printf("ok\n");
   return 0;
