@@ -70,16 +70,16 @@ def test_calls_without_granule_masks_and_without_scratch_do_not_take_the_kernel(
         x = scn.SparseConvNetTensor(torch.randn(3000, planes, generator=g).cuda(), md, t.spatial_size)
         conv = scn.SubmanifoldConvolution(3, planes, out, 5, False).cuda()
         y = conv(x).features
-        assert "wave" not in kernel(), kernel()
+        assert "split wave" not in kernel(), kernel()
         y.sum().backward()
         with torch.no_grad():
             assert torch.equal(conv(x).features, y.detach())
-        assert "wave" not in kernel(), kernel()
+        assert "split wave" not in kernel(), kernel()
     x, w = torch.randn(3000, 32, generator=g).cuda(), torch.randn(27, 1, 32, 32, generator=g).cuda()
     sp, fs = md._s(t.spatial_size), md._s(torch.LongTensor([3, 3, 3]))
     _lib.check(md._L.scn_md_submanifold_rules(md._h, sp, fs, C.c_void_p(0)))
     y = torch.empty(3000, 32).cuda()
     _lib.check(md._L.scn_subm_conv_fwd_noalloc(md._h, sp, fs, C.c_void_p(x.data_ptr()), C.c_void_p(y.data_ptr()), C.c_void_p(w.data_ptr()), None,
                                                32, 32, C.c_void_p(torch.cuda.current_stream().cuda_stream)))
-    assert "wave" not in kernel(), kernel()
+    assert "split wave" not in kernel(), kernel()
     torch.cuda.synchronize()
