@@ -129,8 +129,9 @@ __global__ __launch_bounds__(256, OCC) void k_conv_split(
 #pragma unroll
       for (int s = 0; s < 2; s++) {
         const bool past = tail && (sl * 2 + s) * 16 + 4 * ld_g >= n_in;  // channels past the last
-        areg[i][s] = __builtin_bit_cast(
-            v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, past ? 0x80000000u : voff, (sl * 2 + s) * 64, 0));
+        // (the range check takes the scalar offset from the size: a step past the last channel stays within the one row there may be)
+        const unsigned at = min((unsigned)(sl * 2 + s) * 64u, row_bytes);
+        areg[i][s] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, past ? 0x80000000u : voff, at, 0));
         if (PRE && j >= 0 && !past) aok |= 1u << (2 * i + s);
       }
     }

@@ -124,7 +124,9 @@ __global__ __launch_bounds__(64 * (DEAL > 4 ? DEAL : 4), OCC) void k_conv_wave(
         const bool past = !BF16 && (PAIR || tail) && step * 16 + 4 * ld_g >= n_in;  // channels past the last
         const bool there = row >= 0 && !past;
         const unsigned off = __umul24((unsigned)row, row_bytes) + 16u * (unsigned)ld_g;
-        areg[q][s] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, there ? off : 0x80000000u, step * 64, 0));
+        // (the range check takes the scalar offset from the size: a step past the last channel stays within the one row there may be)
+        const unsigned at = BF16 ? (unsigned)step * 64u : min((unsigned)step * 64u, row_bytes);
+        areg[q][s] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, there ? off : 0x80000000u, at, 0));
         if (PRE && there) aok |= 1u << (2 * q + s);
       }
     }

@@ -68,7 +68,7 @@ def test_rows_owned_by_a_wavefront(kind, n, cin, cout, form):
         bound = ((additions + 4) * mag + 4 * big) * psc + 4 * ((want.abs() + post[0].double().abs()) * psc + post[3].double().abs())
         assert ((wide[:, 4:4 + cout].double() - normalise(want, post)).abs() <= 2.0 ** -24 * bound).all()
     kernel = md._L.scn_md_last_conv_kernel(md._h).decode()
-    assert "wave" in kernel, kernel
+    assert "split wave" in kernel, kernel
 
 
 @pytest.mark.parametrize("kind,n,cin,cout", [("subm", 3001, 16, 16), ("subm", 3001, 32, 24), ("subm", 60001, 64, 16),
@@ -216,3 +216,24 @@ def test_kernel_by_length_of_the_chain(kind, n, cin, cout, says):
         want.index_add_(0, r[:, 1], x[r[:, 0]].double() @ w[k, 0].double())
         mag.index_add_(0, r[:, 1], x[r[:, 0]].double().abs() @ w[k, 0].double().abs())
     assert ((got.double() - want).abs() <= (len(rules) * -(-cin // 32) + 3 + 1 + 4) * 2.0 ** -24 * mag).all()
+
+
+@pytest.mark.parametrize("cin", [12, 20, 36, 40, 44, 100, 132, 140])
+@pytest.mark.parametrize("cout", [8, 32, 40, 96])
+@pytest.mark.parametrize("kind", ["subm", "down", "up", "nin"])
+def test_one_input_row(kind, cin, cout):
+    """A level of one site, plane counts whose last 32 channels are mostly padding: the loads of steps past the last channel are further from the
+    row's start than the input is long."""
+    import torch
+    from test_conv_split_gpu import _table
+    conv, rules, rows_in, rows_out, md = _table(kind, 1, 8400)
+    assert rows_in == rows_out == 1
+    g = torch.Generator().manual_seed(cin + cout)
+    x, w, bias = torch.randn(1, cin, generator=g).cuda(), torch.randn(len(rules), 1, cin, cout, generator=g).cuda(), torch.randn(cout, generator=g).cuda()
+    got = conv(x, w, bias)
+    want, mag = bias.double()[None].clone(), bias.double().abs()[None].clone()
+    for k, r in enumerate(rules):
+        if len(r):
+            want += x.double() @ w[k, 0].double()
+            mag += x.double().abs() @ w[k, 0].double().abs()
+    assert ((got.double() - want).abs() <= (cin + 4) * 2.0 ** -24 * mag).all()
