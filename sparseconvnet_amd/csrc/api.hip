@@ -330,6 +330,27 @@ struct ReleasedMacs {
 std::mutex g_released_mutex;
 std::vector<ReleasedMacs> g_released;
 double g_released_settled = 0;
+// Counts of handles that died while their stream was being captured, still on the device: a launch there would become part of the graph, read
+// tables that are gone and write into a block that another handle has by then, at every replay.  They are fetched when somebody asks, or
+// when this many have gathered.
+std::vector<std::pair<std::shared_ptr<Counts>, double>> g_unread;
+constexpr size_t UNREAD_MOST = 256;
+
+// The multiply-adds behind `unread`; waits for the device.
+double read_counts(std::vector<std::pair<std::shared_ptr<Counts>, double>> &unread) {
+  double total = 0;
+  if (unread.empty()) return total;
+  try {
+    HIP_CHECK(hipDeviceSynchronize());
+    for (auto &u : unread) {
+      ensure_counts(*u.first, use_build_stream() ? device_build_stream() : nullptr);
+      total += (double)u.first->total() * u.second;
+    }
+  } catch (...) {  // a lost device
+    (void)hipGetLastError();
+  }
+  return total;
+}
 
 // Folds what the GPU is done with, so that a program that never asks for its counts does not gather pinned
 // memory, and the next handle to die finds a block.  The caller holds g_released_mutex.
@@ -375,10 +396,23 @@ void release_macs(Metadata &m) {
     if (i == tables.size()) tables.push_back(&c), r.per_rule.push_back(0.0);
     r.per_rule[i] += pm.second;
   }
+  // the stream the convolutions ran on; the rule counts are final before anything on it runs
+  hipStream_t s = m.consumer_known ? m.consumer : nullptr;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (!tables.empty() && hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
+  std::vector<std::pair<std::shared_ptr<Counts>, double>> unread;
+  if (capture != hipStreamCaptureStatusNone) {
+    std::lock_guard<std::mutex> lock(g_released_mutex);
+    for (auto &pm : m.pending_macs)
+      if (!pm.first->ready && pm.first->K && pm.first->dev.p) g_unread.push_back(pm);
+    tables.clear();
+  } else {
+    std::lock_guard<std::mutex> lock(g_released_mutex);
+    if (g_unread.size() > UNREAD_MOST) unread.swap(g_unread);
+  }
+  settled += read_counts(unread);
   if (!tables.empty()) {
     try {
-      // the stream the convolutions ran on; the rule counts are final before anything on it runs
-      hipStream_t s = m.consumer_known ? m.consumer : nullptr;
       if (m.last_ready) HIP_CHECK(hipStreamWaitEvent(s, m.last_ready, 0));
       r.stage_bytes = round_up((int64_t)(tables.size() * sizeof(long long)), 4096);
       r.stage = static_cast<long long *>(pinned_acquire(r.stage_bytes));
@@ -409,10 +443,12 @@ void release_macs(Metadata &m) {
 
 double take_released_macs() {
   std::vector<ReleasedMacs> todo;
+  std::vector<std::pair<std::shared_ptr<Counts>, double>> unread;
   double total;
   {
     std::lock_guard<std::mutex> lock(g_released_mutex);
     todo.swap(g_released);
+    unread.swap(g_unread);
     total = g_released_settled;
     g_released_settled = 0;
   }
@@ -425,7 +461,7 @@ double take_released_macs() {
     (void)hipEventDestroy(r.ev);
     pinned_release(r.stage, r.stage_bytes);
   }
-  return total;
+  return total + read_counts(unread);
 }
 }  // namespace
 

@@ -20,7 +20,7 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("name", ["failed_allocation", "identity_tables", "wave_refuses"])
+@pytest.mark.parametrize("name", ["failed_allocation", "identity_tables", "wave_refuses", "counts_under_capture"])
 def test_host_code(program, name):
     r = subprocess.run([program, name], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, timeout=60)
     assert r.returncode == 0, r.stdout.decode()
