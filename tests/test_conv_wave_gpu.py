@@ -99,6 +99,60 @@ def test_values_that_are_not_finite(kind, n, cin, cout):
         _close_where_finite(conv(x, v, torch.zeros(cout).cuda()), want, mag, len(rules) * cin + 16)
 
 
+@pytest.mark.parametrize("kind,n,cin,cout", [("subm", 3001, 16, 16), ("subm", 30001, 12, 24), ("subm", 3001, 64, 24), ("subm", 60001, 48, 16),
+                                             ("down", 3001, 16, 20), ("up", 30011, 48, 32), ("subm", 3001, 96, 40), ("up", 8001, 64, 48)])
+def test_values_that_are_not_finite_behind_a_batch_norm(kind, n, cin, cout):
+    """The same with a batch norm in the gather, which the second computation applies as well, one behind the sums and a second output."""
+    import torch
+    from test_conv_split_gpu import _table, test_values_that_are_not_finite_in_every_form_of_the_call as every_form
+    every_form(kind, n, cin, cout, True)
+    conv, rules, rows_in, rows_out, md = _table(kind, n, 9600 + n % 91)  # the table it used
+    front = (torch.zeros(cin).cuda(), torch.ones(cin).cuda(), torch.ones(cin).cuda(), torch.zeros(cin).cuda(), 1e-4, 0.2)
+    conv(torch.zeros(rows_in, cin).cuda(), torch.zeros(len(rules), 1, cin, cout).cuda(), torch.zeros(cout).cuda(), bn=front)
+    kernel = md._L.scn_md_last_conv_kernel(md._h).decode()
+    assert "split wave" in kernel and "pre=1" in kernel, kernel
+
+
+@pytest.mark.parametrize("kind,n,cin,cout", [
+    # the gradient's sums run over the layer's output planes and onto its input planes: two taps of up to 16 planes together, slabs of 32,
+    # more than 32 planes
+    ("subm", 17, 8, 16), ("subm", 3001, 16, 16), ("subm", 3001, 12, 8), ("subm", 60001, 20, 12), ("subm", 3001, 32, 64), ("subm", 24001, 24, 48),
+    ("subm", 2501, 48, 40), ("down", 20011, 20, 16), ("down", 20011, 16, 32), ("down", 3001, 48, 64), ("up", 20011, 32, 16),
+    ("up", 20011, 24, 48), ("up", 20011, 40, 64), ("nin", 5003, 16, 96), ("nin", 25001, 24, 12), ("nin", 3001, 36, 128)])
+def test_input_gradients(kind, n, cin, cout):
+    """Weights packed transposed, those of a submanifold convolution with the taps in reverse order."""
+    import torch
+    from test_conv_split_gpu import _table, _rules_of
+    conv, rules, rows_in, rows_out, md = _table(kind, n, 8500 + n % 89)
+    g = torch.Generator().manual_seed(n + cin)
+    d, w = torch.randn(rows_out, cout, generator=g).cuda(), torch.randn(len(rules), 1, cin, cout, generator=g).cuda() * 0.1
+    conv(torch.zeros(rows_in, cin).cuda(), w, torch.zeros(cout).cuda())
+    p, size = _rules_of(md), 126 if n < 30000 else 1022
+    x, d_out, weight = torch.zeros(rows_in, cin).numpy(), d.cpu().numpy(), w.cpu().numpy()
+    if kind == "subm":
+        got = p.subm_conv_bwd(size, 3, x, d_out, weight)[0]
+    elif kind == "down":
+        got = p.conv_bwd(size, size // 2, 2, 2, x, d_out, weight)[0]
+    elif kind == "up":
+        got = p.deconv_bwd(size // 2, size, 2, 2, x, d_out, weight)[0]
+    else:
+        got = p.nin_bwd(x, d_out, weight[0, 0])[0]
+    kernel = md._L.scn_md_last_conv_kernel(md._h).decode()
+    assert "split wave" in kernel and ("pair=1" in kernel) == (cout <= 16), kernel
+    want = torch.zeros(rows_in, cin, dtype=torch.float64, device="cuda")
+    mag = want.clone()
+    for k, r in enumerate(rules):
+        r = torch.as_tensor(r).cuda().long()
+        want.index_add_(0, r[:, 0], d[r[:, 1]].double() @ w[k, 0].double().t().contiguous())
+        mag.index_add_(0, r[:, 0], d[r[:, 1]].double().abs() @ w[k, 0].double().abs().t().contiguous())
+    additions = len(rules) * -(-cout // 32) + 3
+    assert ((torch.as_tensor(got).cuda().double() - want).abs() <= (additions + 4) * 2.0 ** -24 * mag).all()
+
+
+# left to k_conv_rows: large levels of 64 and more planes, wide inputs on small ones
+BF16_ROWS = {("subm", 260001, 64, 64), ("subm", 40001, 64, 72), ("subm", 10001, 192, 112), ("subm", 2999, 256, 128)}
+
+
 @pytest.mark.parametrize("kind,n,cin,cout", [
     ("subm", 1, 32, 16), ("subm", 17, 64, 32), ("subm", 7999, 96, 64), ("subm", 8001, 32, 40), ("subm", 19999, 32, 32),
     ("subm", 20001, 64, 24), ("subm", 300001, 32, 32), ("subm", 700001, 32, 20), ("subm", 2999, 256, 128), ("subm", 3001, 128, 100),
@@ -109,7 +163,8 @@ def test_values_that_are_not_finite(kind, n, cin, cout):
 def test_bf16_operands(kind, n, cin, cout, form):
     """Operands rounded to bf16, products exact, added in fp32 by a unit that need not round to nearest: one result is off by at most
     an ulp, 2^-23, per addition of the sum of the products' magnitudes; a normalised row's value may be rounded from the neighbouring
-    fp32 number, an ulp of bf16 (2^-7) away."""
+    fp32 number, an ulp of bf16 (2^-7) away.  That needs a value within some 4 2^-24 of its terms of the middle between two bf16 numbers,
+    which one in 2^13 is: the 2-norm of all results is off by 2^-8 / 2^6.5, twice that for values smaller than their terms."""
     import torch
     from test_conv_split_gpu import _table
     conv, rules, rows_in, rows_out, md = _table(kind, n, 8300 + n % 89)
@@ -134,8 +189,10 @@ def test_bf16_operands(kind, n, cin, cout, form):
     got = conv(x, w, bias) if front is None else conv(x, w, bias, bn=front)
     bound = (len(rules) * cin + 8) * 2.0 ** -23 + (0 if front is None else 2.0 ** -7)
     assert ((got.double() - want).abs() <= bound * mag + 1e-30).all()
+    if rows_out >= 1000:  # enough results for a share of them
+        assert (got.double() - want).norm() <= 2.0 ** -13.5 * want.norm(), float((got.double() - want).norm() / want.norm())
     kernel = md._L.scn_md_last_conv_kernel(md._h).decode()
-    assert "bf16" in kernel, kernel
+    assert ("rows-bf16" if (kind, n, cin, cout) in BF16_ROWS else "wave-bf16") in kernel, kernel
 
 
 @pytest.mark.parametrize("n,cin,cout", [(1500, 128, 64), (3001, 128, 64), (6001, 128, 128), (12001, 128, 64), (12001, 64, 64)])
