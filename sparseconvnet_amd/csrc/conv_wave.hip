@@ -21,7 +21,7 @@ namespace scn {
 // What bounds it: at large levels the vector instructions of the splitting (some 60 per granule and iteration) next to the
 // MFMAs: in a loop of nothing else the two overlap by a tenth only, 155 ns per granule and iteration of 2 x 16 columns against
 // 69 and 113 apart, and the clock falls to 1.9-2.1 GHz; 32 -> 32 at a million sites is 106 us of that.  Counters there:
-// vector unit 53 %, matrix unit 28 % of the time, 2.1 TB/s from beyond L2.
+// vector unit 52 %, matrix unit 27 % of the time, 1.9 TB/s from beyond L2.
 // Against k_conv_split and k_conv_resident, which served these shapes (us, graph replays, room surfaces, 27 taps):
 //   sites       1 M        400 k      100 k      24 k       8 k        2 k
 //   32 -> 32    262 / 213  105 / 86   44 / 31    24 / 12    18 / 7.6   13 / 7.2
@@ -374,6 +374,7 @@ static void launch_wave(Metadata &m, const Table &t, const float *in, float *out
   }
   const int n_tiles = (int)ceil_div(t.n, (DEAL > 1 ? 1 : 4) * GW * 16);
   const int tiles_per_xcd = t.spread ? 0 : (int)ceil_div(n_tiles, 8);
+  // (split: workgroups that share a tile's iterations through partial sums in memory, as k_conv_split says it: here never)
   note_kernel(m, BF16 ? "wave-bf16" : "split wave", {{"ncb", NCB}, {"gw", GW}, {"deal", DEAL}, {"pair", PAIR}, {"pre", PRE}, {"split", 1}});
   k_conv_wave<NCB, GW, DEAL, OCC, PAIR, PRE, BF16><<<dim3((unsigned)(tiles_per_xcd ? tiles_per_xcd * 8 : n_tiles), groups), 64 * std::max(4, DEAL), 0, s>>>(
       t.nbr.p, t.rowmap_ptr(), t.gmask.p, t.n, t.npad, in, out, reinterpret_cast<const v8s *>(wpack), epi, n_in, n_out, n_slab,
@@ -432,7 +433,7 @@ static void dispatch_wave(Metadata &m, const Table &t, const float *in, float *o
   // are enough of them (us: one granule dealt out / two dealt out / two / four):
   //   27 taps 32 -> 32: 8 k sites 7.6 / 9.8 / 25 / 41, 24 k 12.2 / 12.7 / 26 / 42, 100 k 36 / 31 / 36 / 47, 200 k 64 / 52 / 53 / 57,
   //     400 k 120 / 99 / 86 / 90, 1 M 360 / 274 / 230 / 213
-  //   9 taps (2-D) 16 -> 16: 12 k 4.7 / 5.4 / 8.4 / 13, 50 k 9.4 / 8.5 / 9.4 / 14, 200 k 31 / 24 / 22 / 26
+  //   9 taps (input gradients only, see conv_wave_serves) 16 -> 16: 12 k 4.7 / 5.4 / 8.4 / 13, 50 k 9.4 / 8.5 / 9.4 / 14, 200 k 31 / 24 / 22 / 26
   //   one rule per position 24 -> 16: 20 k 4.4 / 4.5 / 5.4 / 7.7, 60 k 7.3 / 6.6 / 6.2 / 8.5, 1 M 81 / 55 / 33 / 38
 #define WAVE(G, D, O) launch_wave<NCB, G, D, O, PAIR, PRE>(m, t, in, out, w, epi, n_in, n_out, pre, s)
   if (t.n < 24000) WAVE(1, 4, O1);
@@ -442,7 +443,8 @@ static void dispatch_wave(Metadata &m, const Table &t, const float *in, float *o
 #undef WAVE
 }
 // bf16 operands (the caller's choice; whole slabs of 32 channels): the same kernel with one instruction and no splitting.  What bounds
-// it: the rows' way from L2 (13 TB/s at 800 k sites 32 -> 32), and on small levels the chain, as above.  us, k_conv_resident,
+// it: what comes from L2, rows and, per wavefront, weights (300 k sites 128 -> 128 269 us: 2.8 GB of read requests, 10.4 TB/s, 1.66 GB of it
+// rows; 900 k 32 -> 32 126 us: 1.2 GB of rows, 9.7 TB/s), and on small levels the chain, as above.  us, k_conv_resident,
 // k_conv_rows or k_conv_mfma, which keep the rest / here:
 //   27 taps: 1 k sites 32 -> 32 18.3 / 4.7, 64 -> 64 12.8 / 6.7, 128 -> 128 18.0 / 10.6; 14 k 32 -> 32 20.0 / 5.8, 64 -> 64 22.6 / 10.6,
 //     128 -> 128 36.4 / 27.9, but 256 -> 128 55.9 / 50.7 where 128-row tiles of slabs of 64 (k_conv_rows) take 49.6; 61 k 64 -> 32 47 / 20.5,
@@ -503,10 +505,12 @@ static void dispatch_bf(Metadata &m, const Table &t, const float *in, float *out
 #undef BF
 }
 bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_t in_rows, int n_in, int n_out, bool gradient) {
-  // Forward sums that will be differentiated, and those over nine taps (the 3 x 3 filters of 2-D networks, whose time is the host's:
-  // 1.21 / 1.26 ms for a batch of pen strokes), keep their rounding in k_conv_resident and k_conv_split: with another one values on the edge
+  // Forward sums that will be differentiated keep their rounding in k_conv_resident and k_conv_split: with another one values on the edge
   // of a ReLU change sides, and the gradients of a training step over some ten thousand sites differ by up to 9e-3 (2-D: 3.5e-3).  A
-  // million-site step takes 1 % longer for it.
+  // million-site step takes 1 % longer for it.  So do those over nine taps, whatever the filter's shape, differentiated or not: they are
+  // the 3 x 3 filters of 2-D networks, whose time is the host's (1.21 / 1.26 ms for a batch of pen strokes).  The kernels that keep them are slower
+  // by themselves (us, there / here, filter 3 x 3 x 1): 4 k sites 16 -> 16 11.7 / 4.6, 32 -> 32 16.4 / 5.3, 48 -> 48 14.0 / 8.2, 100 k 28 / 13, 22 / 19
+  // and, bf16 operands, 31 / 14, a million 130 / 73, 141 / 130 and 152 / 101, 64 -> 32 227 / 232.
   if ((t.K == 9 || m.differentiated) && !gradient) return false;
   // The kernel reads granule masks of 32 bits, which tables of more taps do not have (gmask is null there), and keeps its taps in the lanes of
   // half a wavefront; the allocation-free entry has no room for its weights.
@@ -515,11 +519,14 @@ bool conv_wave_serves(const Metadata &m, const Table &t, const float *in, int64_
   if (in_rows <= 0 || in_rows >= (1 << 24) || in_rows * n_in * 4 >= ((int64_t)1 << 31)) return false;
   if (m.bf16) return !gradient && bf_tile(t, in_rows, n_in, n_out) != BF_NONE;  // (these weights are packed from a transposed copy)
   if (n_out > 32) return wide_tile(t, in_rows, n_in, n_out) != NONE;
-  // k_conv_resident keeps 20-32 -> up to 16 planes on small levels of few taps and on large ones
+  // k_conv_resident keeps 20-32 -> up to 16 planes on small levels of few taps and on large ones, where it was faster than k_conv_split, and
+  // test_kernel_and_shares_by_size holds the lines.  Here they would be faster still (us, there / here): eight taps onto 1 k to 5 k sites 24 -> 16
+  // 11.6-13.1 / 4.3-4.5; 27 taps 32 -> 16 200 k 65 / 41, 300 k 74 / 57, a million 165 / 157, 24 -> 16 300 k 84 / 65, a million 190 / 190.
   if (n_in > 16 && n_in <= 32 && n_out <= 16 && (t.K <= 9 ? t.n < 16000 : t.n >= (n_in > 24 ? 200000 : 300000))) return false;
-  // k_conv_split: wide inputs of one rule per position, and on the smallest levels chains that it cuts into more parts (500 sites
-  // 64 -> 32 11.9 there, 11.1 here, 128 -> 32 13.7 / 18.5, 1.01 k 128 -> 24 17.6 / 21.8, 1.05 k 224 -> 32 21.5 / 33.5, 1.7 k 192 -> 32 22.6 / 29.1,
-  // 3.5 k 256 -> 24 37.0 / 43.8, 4.5 k 256 -> 17 35.9 / 41.0, 1.4 k 224 -> 12 23.5 / 29.1; 80 coarse sites of eight taps 256 -> 17 16.5 / 17.4): the
+  // k_conv_split: wide inputs of one rule per position (test_kernel_and_shares_by_size holds them there; transposed 96 -> 32 onto 4 k
+  // sites 11.7 us there, 4.6 here, 100 k 20.7 / 15.6, a million 112 / 87, 160 -> 32 13.7 / 5.3, 27.5 / 21.1, 161 / 148), and on the
+  // smallest levels chains that it cuts into more parts (500 sites 64 -> 32 11.9 there, 11.1 here, 128 -> 32 13.7 / 18.5, 1.01 k 128 -> 24 17.6 / 21.8,
+  // 1.05 k 224 -> 32 21.5 / 33.5, 1.7 k 192 -> 32 22.6 / 29.1, 3.5 k 256 -> 24 37.0 / 43.8, 4.5 k 256 -> 17 35.9 / 41.0, 1.4 k 224 -> 12 23.5 / 29.1; 80 coarse sites of eight taps 256 -> 17 16.5 / 17.4): the
   // sites from which on this kernel is the faster one, by slabs of 32 channels
   static const int64_t many[] = {0, 0, 1000, 1000, 2000, 2500, 3700, 5000, 5500};
   if ((t.few_tap.p && n_in > 64) || (t.K > 9 && t.n < 1000 && n_in > 32)) return false;

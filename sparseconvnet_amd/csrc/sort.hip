@@ -265,7 +265,7 @@ void radix_sort_pairs(Metadata &m, const u64 *kin, u64 *kout, const int *vin, in
   // million pairs of 35 bits 145 -> 122 us, eight million 800 -> 490 us); below half a million pairs
   // there are too few of those to fill the chip and smaller tiles are faster, down to 512 pairs
   // (30 bits: 88 000 pairs 64 -> 55 us, 150 000 pairs 72 -> 61 us with 1024).
-  // Up to 32 k pairs (32 tiles) the scatter adds up the tiles' counts itself, two launches per digit: 12 k pairs of 9 / 27 bits
+  // Up to 32 k pairs (40 tiles at most) the scatter adds up the tiles' counts itself, two launches per digit: 12 k pairs of 9 / 27 bits
   // 10.7 -> 9.2 / 32 -> 27 us, 16 k 11.1 -> 9.7 / 33 -> 28, 32 k the same time with a third fewer launches, 64 k 12.4 -> 14.5 / 37 -> 42.
   // (The library's merge sort, which served 4 to 32 k pairs before, took 27 to 34 us and 6 to 9 launches whatever the bits.)
   const bool few = n <= 32768;
