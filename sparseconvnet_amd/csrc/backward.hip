@@ -334,7 +334,7 @@ __global__ __launch_bounds__(256) void k_conv_dw(const int *__restrict__ nbr, co
 // NW = 16, small levels, where the launch is as long as one workgroup's block of DT_BLOCK granules: sixteen wavefronts of two taps; the block's
 // indices, rows and masks come to LDS first, and a granule's rows are requested behind the MFMAs of the one before (one memory latency per
 // granule instead of two).  With the launch that adds the shares up, us, eight wavefronts / sixteen, the same bits: 27 taps 16 x 16 150 sites
-// 29.7 / 27.9, 32 x 32 6 k 31.0 / 28.5, 24 k 37.3 / 30.9; nine taps 16 x 16 6 k 22.7 / 20.4; eight onto 24 k 32 x 32 28.7 / 22.7.  Not with
+// 29.7 / 27.9 (where every site has most of its taps), 32 x 32 6 k 31.0 / 28.5, 24 k 37.3 / 30.9; nine taps 16 x 16 6 k 22.7 / 20.4; eight onto 24 k 32 x 32 28.7 / 22.7.  Not with
 // several blocks per workgroup, a barrier each (27 taps 32 x 32 100 k 80 / 85, a million 513 / 487), nor where granules have few taps or
 // blocks few granules (transposed 600 positions 13.7 / 18.8, filter 3 stride 2 19 / 21, 1x1 15 / 18, 64 sites 19 / 23).
 constexpr int DT_T = 32, DT_TAPS = 32, DT_BLOCK = 8;  // DT_BLOCK granules of 16 positions per turn
@@ -932,8 +932,10 @@ static void weight_gradient(Metadata &m, const Table &t, const float *a, int64_t
       kern<<<grid, waves * 64, 0, s>>>(t.nbr.p, t.rowmap_ptr(), t.gmask.p, t.K, t.n, t.npad, a, n_a, (unsigned)(a_rows * n_a * 4), b, n_b,
                                        (unsigned)(b_rows * n_b * 4), m.partial.p);
     };
-    // sixteen wavefronts: one block per workgroup, and a compute unit has at most one of those; fine sides gather from fewer rows
-    if (t.K >= 8 && a_rows >= t.n && t.n >= 100 && t.n <= 256 * 16 * DT_BLOCK)
+    // sixteen wavefronts: one block per workgroup, and a compute unit has at most one of those; fine sides gather from fewer rows; the blocks
+    // of the smallest levels have few granules with many of their taps (12 x 32, whole call, eight / sixteen: eight taps onto 116 positions
+    // 22.8 / 28.2, 201 24.9 / 27.9, 338 29.8 / 29.3; nine taps 180 32.6 / 33.4, 400 35.3 / 34.2; 27 taps 180 29.1 / 29.6, 266 34.2 / 32.1)
+    if (t.K >= 8 && a_rows >= t.n && t.n >= 300 && t.n <= 256 * 16 * DT_BLOCK)
       vec2 ? run(k_conv_dw_taps<true, 16>, 16) : run(k_conv_dw_taps<false, 16>, 16);
     else
       vec2 ? run(k_conv_dw_taps<true, 8>, 8) : run(k_conv_dw_taps<false, 8>, 8);

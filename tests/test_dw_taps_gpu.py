@@ -8,7 +8,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 16, 127, 128, 129, 257, 5003, 32767, 32769, 70001])
+@pytest.mark.parametrize("n", [1, 16, 127, 128, 129, 257, 299, 300, 5003, 32767, 32769, 70001])
 @pytest.mark.parametrize("dim,size,planes", [(3, 3, (8, 8)), (3, 3, (32, 32)), (3, 3, (7, 9)), (2, 3, (16, 24)), (3, 1, (5, 32)), (2, 5, (20, 12))])
 def test_weight_gradient(n, dim, size, planes):
     import torch
