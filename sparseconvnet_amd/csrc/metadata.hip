@@ -155,25 +155,16 @@ static void fill3(void *p0, uint32_t v0, int64_t n0, void *p1, uint32_t v1, int6
 
 // Stable sort of (key, value) pairs by the low end_bit bits of the key.  Up to 1.5 million pairs
 // this repository's own sort (sort.hip); above, the library's radix sort, whose tiles stage their pairs through
-// LDS and write long runs (measured faster from about two million pairs on).  So are 4 to 32 thousand pairs of more than three digits
-// (input layers of fields from 1024^3 on), for which it merges a few sorted blocks whatever the bits: own / library, us, one call and its wait:
-// 8 k pairs of 31 bits 44 / 37, of 40 53 / 39, 16 k 46 / 39 and 52 / 41, 32 k 52 / 48 and 60 / 50; but of 27 bits 38 / 37, 41 / 39, 46 / 49.
+// LDS and write long runs (measured faster from about two million pairs on).
 using RadixAlways = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
                                                rocprim::default_config, 4096>;
 static void sort_pairs(Metadata &m, const unsigned long long *kin, unsigned long long *kout,
                        const int *vin, int *vout, int64_t n, hipStream_t s, int end_bit = 64) {
-  const bool merge = n > 4096 && n <= 32768 && end_bit > 30;
-  if (n <= 1500000 && !merge) {
+  if (n <= 1500000) {
     radix_sort_pairs(m, kin, kout, vin, vout, n, end_bit, s);
     return;
   }
   size_t bytes = 0;
-  if (merge) {  // what rocPRIM chooses by itself at this size
-    HIP_CHECK(rocprim::radix_sort_pairs(nullptr, bytes, kin, kout, vin, vout, (size_t)n, 0u, (unsigned)end_bit, s));
-    m.tmp.reserve(bytes + 16);
-    HIP_CHECK(rocprim::radix_sort_pairs(m.tmp.p, bytes, kin, kout, vin, vout, (size_t)n, 0u, (unsigned)end_bit, s));
-    return;
-  }
   HIP_CHECK(rocprim::radix_sort_pairs<RadixAlways>(nullptr, bytes, kin, kout, vin, vout, (size_t)n, 0u,
                                                    (unsigned)end_bit, s));
   m.tmp.reserve(bytes + 16);

@@ -215,9 +215,9 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const u64 *__restrict
   }
 }
 
-// Up to RS1_MAX pairs (98 KB of LDS for eight per thread, 17 KB of counts): one workgroup takes them through every digit without leaving LDS
+// Up to RS1_MAX pairs (98 KB of them, 17 KB of counts): one workgroup takes them through every digit without leaving LDS
 // (sort_block.h), one launch instead of three per digit.
-constexpr int RS1_MAX = RS1_THREADS * 6;
+constexpr int RS1_MAX = RS1_THREADS * 8;
 template <int ITEMS>
 __global__ __launch_bounds__(RS1_THREADS) void k_rs_single(const u64 *__restrict__ kin, const int *__restrict__ vin,
                                                            u64 *__restrict__ kout, int *__restrict__ vout, int n,
@@ -253,8 +253,7 @@ void radix_sort_pairs(Metadata &m, const u64 *kin, u64 *kout, const int *vin, in
   // as few digits as RS_MAX_BITS bits each allow, of equal width
   const int passes = (end_bit + RS_MAX_BITS - 1) / RS_MAX_BITS;
   const int width = (end_bit + passes - 1) / passes;
-  // one workgroup instead of two launches per digit, while that is no slower: 6000 pairs of 22 bits 31 us against 35, of 27 36 / 37; but 8000 of 18
-  // bits 32 / 28, of 27 41 / 37, of 9 14 / 9
+  // one workgroup instead of two launches per digit: 8000 pairs of 27 bits 31 us against 26 and five launches more, of 9 bits 14 against 9
   if (n <= (end_bit <= RS_MAX_BITS ? 4096 : RS1_MAX)) {
     const int p1 = (end_bit + RS1_BITS - 1) / RS1_BITS;
     auto kern = n <= RS1_THREADS * 4 ? k_rs_single<4> : k_rs_single<8>;
@@ -268,7 +267,7 @@ void radix_sort_pairs(Metadata &m, const u64 *kin, u64 *kout, const int *vin, in
   // (30 bits: 88 000 pairs 64 -> 55 us, 150 000 pairs 72 -> 61 us with 1024).
   // Up to 32 k pairs (40 tiles at most) the scatter adds up the tiles' counts itself, two launches per digit: 12 k pairs of 9 / 27 bits
   // 10.7 -> 9.2 / 32 -> 27 us, 16 k 11.1 -> 9.7 / 33 -> 28, 32 k the same time with a third fewer launches, 64 k 12.4 -> 14.5 / 37 -> 42.
-  // (The library's merge sort takes 27 to 38 us and 6 to 9 launches whatever the bits; sort_pairs leaves it those of more than three digits.)
+  // (The library's merge sort, which served 4 to 32 k pairs before, took 27 to 34 us and 6 to 9 launches whatever the bits.)
   const bool few = n <= 32768;
   const int items = n >= 500000 ? 16 : n >= 300000 ? 8 : n >= 120000 || (few && n > 20000) ? 4 : 2;
   const int tile = RS_THREADS * items;
