@@ -267,7 +267,9 @@ void radix_sort_pairs(Metadata &m, const u64 *kin, u64 *kout, const int *vin, in
   // (30 bits: 88 000 pairs 64 -> 55 us, 150 000 pairs 72 -> 61 us with 1024).
   // Up to 32 k pairs (40 tiles at most) the scatter adds up the tiles' counts itself, two launches per digit: 12 k pairs of 9 / 27 bits
   // 10.7 -> 9.2 / 32 -> 27 us, 16 k 11.1 -> 9.7 / 33 -> 28, 32 k the same time with a third fewer launches, 64 k 12.4 -> 14.5 / 37 -> 42.
-  // (The library's merge sort, which served 4 to 32 k pairs before, took 27 to 34 us and 6 to 9 launches whatever the bits.)
+  // (The library's merge sort, which served 4 to 32 k pairs before, takes 27 to 38 us and 6 to 9 launches whatever the bits.  From 31 bits on that is
+  // less: one call and its wait, us, here / there, 8 k pairs of 31 bits 44 / 37, 10 k of 40 bits 52 / 40, 32 k 60 / 50.  An input layer of 10 k points in
+  // 1024^3 through the modules takes the same with either, 152-177 / 155-180 over four processes each, so that there is one sort.)
   const bool few = n <= 32768;
   const int items = n >= 500000 ? 16 : n >= 300000 ? 8 : n >= 120000 || (few && n > 20000) ? 4 : 2;
   const int tile = RS_THREADS * items;
