@@ -334,7 +334,7 @@ void scn_params_destroy(scn_params *p);
 int scn_params_clear(scn_params *p);
 int scn_md_use_params(scn_metadata *md, scn_params *p);
 /* The NEXT convolution call on md is a forward pass whose output will be differentiated: it runs in the kernels whose
- * rounding a training run has seen, not in faster ones that round differently. */
+ * rounding a training run has seen, not in faster ones that round differently.  Taken back by that call, also where it fails. */
 int scn_md_next_differentiated(scn_metadata *md);
 
 /* ActivePooling_updateOutput / ActivePooling_updateGradInput (pybind.cpp:34-43,

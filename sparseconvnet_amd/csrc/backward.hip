@@ -333,8 +333,8 @@ __global__ __launch_bounds__(256) void k_conv_dw(const int *__restrict__ nbr, co
 // likewise for the columns.  The rows of b are loaded once per granule and serve all its taps.
 // NW = 16, small levels, where the launch is as long as one workgroup's block of DT_BLOCK granules: sixteen wavefronts of two taps; the block's
 // indices, rows and masks come to LDS first, and a granule's rows are requested behind the MFMAs of the one before (one memory latency per
-// granule instead of two).  With the launch that adds the shares up, us, eight wavefronts / sixteen, the same bits: 27 taps 16 x 16 150 sites
-// 29.7 / 27.9 (where every site has most of its taps), 32 x 32 6 k 31.0 / 28.5, 24 k 37.3 / 30.9; nine taps 16 x 16 6 k 22.7 / 20.4; eight onto 24 k 32 x 32 28.7 / 22.7.  Not with
+// granule instead of two).  With the launch that adds the shares up, us, eight wavefronts / sixteen, the same bits: 27 taps 32 x 32
+// 6 k sites 31.0 / 28.5, 24 k 37.3 / 30.9; nine taps 16 x 16 6 k 22.7 / 20.4; eight onto 24 k 32 x 32 28.7 / 22.7.  Not with
 // several blocks per workgroup, a barrier each (27 taps 32 x 32 100 k 80 / 85, a million 513 / 487), nor where granules have few taps or
 // blocks few granules (transposed 600 positions 13.7 / 18.8, filter 3 stride 2 19 / 21, 1x1 15 / 18, 64 sites 19 / 23).
 constexpr int DT_T = 32, DT_TAPS = 32, DT_BLOCK = 8;  // DT_BLOCK granules of 16 positions per turn
